@@ -1,16 +1,16 @@
 // SC-MXFP4 weight quantizer on the device: float weights -> packed codes, block codes and row scales.
 //
-// Restates, in float64 exactly as the host procedure computes it, sim/mx_int8.py:39-109 (block exponent search,
-// spread constraint, E2M1 rounding, INT8 embedding) followed by the packing of sim/make_testcase.py:26-44 and
-// e2e/sc_format.py:93-111.  One workgroup quantizes one row; a lane holds one weight, a group of BLOCK lanes one
-// block.
+// Restates, bit for bit, sim/mx_int8.py:39-109 (block exponent search, spread constraint, E2M1 rounding, INT8
+// embedding) followed by the packing of sim/make_testcase.py:26-44 and e2e/sc_format.py:93-111.  A thread owns one
+// block: its weights stay in registers from the search to the packing, sums over a block need no cross-lane traffic,
+// and a workgroup takes as many whole rows as give its 256 threads a block each.
 //
-// Bit-exactness rests on three things: every quantity is a float64 (weights arrive as float32 or bf16, both exact
-// in float64); scaling by block steps is a multiplication by a power of two (exact); and the squared error of a
-// block is summed in the order of the host's pairwise reduction over BLOCK contiguous values: eight running sums
-// r[j] = ((a[j] + a[8+j]) + a[16+j]) + a[24+j], then ((r0+r1)+(r2+r3)) + ((r4+r5)+(r6+r7)).  The candidate
-// comparison is a strict "<" on those sums, so a different order could flip a near tie.
+// The host decides between exponents by a strict "<" on float64 sums taken in a fixed order.  Here the sums are formed
+// in float32 first (which scaling by powers of two leaves exact up to the sums' own rounding), and only where two of
+// them are too close for float32 to tell apart is the block summed again in float64 in the host's order: eight running
+// sums r[j] = ((a[j] + a[8+j]) + a[16+j]) + a[24+j], then ((r0+r1)+(r2+r3)) + ((r4+r5)+(r6+r7)).
 #include <climits>
+#include <type_traits>
 
 #include "scmx_common.h"
 
@@ -30,116 +30,199 @@ __device__ __forceinline__ double e2m1_level(int idx) {   // 0, .5, 1, 1.5, 2, 3
     return idx <= 4 ? 0.5 * idx : (idx == 5 ? 3.0 : (idx == 6 ? 4.0 : 6.0));
 }
 
-// Squared error of the block this lane belongs to when quantized at exponent e (sim/mx_int8.py:34-36), summed in the
-// host's order; every lane of the block returns the same value.
+// Squared error of BLOCK consecutive weights quantized at exponent e (sim/mx_int8.py:34-36), in float64 and summed in
+// the host's order.  Reads the weights again: it decides near ties only.
+template <int BLOCK, typename W>
+__device__ double block_sq_err(W&& weight, int e) {
+    double r[8];
+#pragma unroll 1
+    for (int i = 0; i < BLOCK; i += 8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const double b = double(weight(i + j));
+            const double x = b * pow2_f64(-e);
+            const double q = e2m1_level(e2m1_index(x));
+            const double d = (x < 0.0 ? -q : q) * pow2_f64(e) - b;
+            r[j] = i == 0 ? d * d : r[j] + d * d;
+        }
+    }
+    return ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
+}
+
+// BLOCK consecutive weights into registers; vec: the address is 16-byte aligned.
+template <int BLOCK, bool BF16>
+__device__ __forceinline__ void load_block(const void* __restrict__ w, size_t at, bool vec, float (&v)[BLOCK]) {
+    if (BF16) {
+        const uint16_t* p = reinterpret_cast<const uint16_t*>(w) + at;
+        if (vec) {
+#pragma unroll
+            for (int i = 0; i < BLOCK / 8; ++i) {
+                const u32x4 u = reinterpret_cast<const u32x4*>(p)[i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[8 * i + 2 * j] = __uint_as_float(u[j] << 16);
+                    v[8 * i + 2 * j + 1] = __uint_as_float(u[j] & 0xFFFF0000u);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < BLOCK; ++i) v[i] = bf16_to_f32(p[i]);
+        }
+    } else {
+        const float* p = reinterpret_cast<const float*>(w) + at;
+        if (vec) {
+#pragma unroll
+            for (int i = 0; i < BLOCK / 4; ++i) {
+                const f32x4 u = reinterpret_cast<const f32x4*>(p)[i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[4 * i + j] = u[j];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < BLOCK; ++i) v[i] = p[i];
+        }
+    }
+}
+
+// The code words of a block leave in 16- or 8-byte stores where the pointer allows it.
 template <int BLOCK>
-__device__ __forceinline__ double block_sq_err(double b, int e) {
-    const double x = b * pow2_f64(-e);
-    const double lv = e2m1_level(e2m1_index(x));
-    const double v = x < 0.0 ? -lv : lv;
-    const double d = v * pow2_f64(e) - b;
-    const double sq = d * d;
-    double r = sq + __shfl_down(sq, 8, BLOCK);
-    if (BLOCK == 32) {
-        r = r + __shfl_down(sq, 16, BLOCK);
-        r = r + __shfl_down(sq, 24, BLOCK);
+__device__ __forceinline__ void store_codes(uint32_t* __restrict__ dst, bool vec, const uint32_t (&c)[BLOCK / 8]) {
+    if (BLOCK == 32 && vec) {
+        *reinterpret_cast<u32x4*>(dst) = u32x4{c[0], c[1], c[BLOCK / 8 - 2], c[BLOCK / 8 - 1]};
+    } else if (vec) {
+        *reinterpret_cast<u32x2*>(dst) = u32x2{c[0], c[1]};
+    } else {
+#pragma unroll
+        for (int i = 0; i < BLOCK / 8; ++i) dst[i] = c[i];
     }
-    r = r + __shfl_xor(r, 1, BLOCK);
-    r = r + __shfl_xor(r, 2, BLOCK);
-    r = r + __shfl_xor(r, 4, BLOCK);
-    return __shfl(r, 0, BLOCK);
 }
 
-template <bool MAXOP>
-__device__ __forceinline__ int wg_reduce(int v, int* red) {
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+// Squared error, in units of the square of 2^e0, of the block x * 2^e0 at exponent e0 + log2(scale).  The FP4 conversion
+// does the rounding: it takes a tie to the even code where the host takes the lower one, which is the same distance away.
+template <int BLOCK>
+__device__ __forceinline__ float fp4_sq_err(const float (&x)[BLOCK], float scale) {
+    float r0 = 0.0f, r1 = 0.0f;
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const int o = __shfl_xor(v, off, WAVE);
-        v = MAXOP ? max(v, o) : min(v, o);
+    for (int i = 0; i < BLOCK; i += 2) {
+        const uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[i], x[i + 1], scale, 0);
+        const f32x2_t v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 0);
+        const float d0 = v[0] - x[i], d1 = v[1] - x[i + 1];   // exact: the difference fits 24 bits
+        r0 = __builtin_fmaf(d0, d0, r0);
+        r1 = __builtin_fmaf(d1, d1, r1);
     }
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    int r = red[0];
-#pragma unroll
-    for (int i = 1; i < QNT / 64; ++i) r = MAXOP ? max(r, red[i]) : min(r, red[i]);
-    return r;
+    return r0 + r1;
 }
 
+// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: HBM (the weights are read once) and about 25 vector
+// instructions per weight.  12288 x 2048 bf16: 44.5 us (1.4 TB/s); 234 us with a lane per weight and every candidate in
+// float64 across lanes.
 template <int BLOCK, bool BF16>
 __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                          uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
-                                                         int K) {
-    extern __shared__ int s_e[];   // K / BLOCK block exponents, then 4 ints of reduction scratch
+                                                         int64_t N, int K, int rows, bool vec) {
+    extern __shared__ int s_e[];   // rows x nb block exponents, then the rows' smallest allowed and lowest exponents
     const int nb = K / BLOCK;
-    int* red = s_e + nb;
-    const size_t row = blockIdx.x;
-    const int tid = threadIdx.x;
+    const size_t row0 = size_t(blockIdx.x) * rows;
+    const int live = int(min(int64_t(rows), N - int64_t(row0)));
+    const int total = live * nb, tid = threadIdx.x, lane = tid & 63;
+    int* s_floor = s_e + rows * nb;
+    int* s_lo = s_floor + rows;
     constexpr int EMPTY = INT_MIN;   // an all-zero block: the host's -inf
-    auto weight = [&](int k) -> double {
-        if (BF16) return double(bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[row * K + k]));
-        return double(reinterpret_cast<const float*>(w)[row * K + k]);
-    };
+    const size_t base = row0 * K;
 
-    // ---- pass 1: exponent of every block (sim/mx_int8.py:39-65, rule "search") ------------------------------------
-    // QNT is a multiple of BLOCK and K a multiple of BLOCK, so a block is entirely inside or outside the row.
-    for (int k0 = 0; k0 < K; k0 += QNT) {
-        const int k = k0 + tid;
-        const bool in = k < K;
-        const double b = in ? weight(k) : 0.0;
-        double amax = fabs(b);
+    // ---- exponent of every block (sim/mx_int8.py:39-65, rule "search") --------------------------------------------
+    float v[BLOCK];
+    for (int b = tid; b < total; b += QNT) {
+        const size_t at = base + size_t(b) * BLOCK;
+        load_block<BLOCK, BF16>(w, at, vec, v);
+        float amax = 0.0f;
 #pragma unroll
-        for (int off = BLOCK / 2; off >= 1; off >>= 1) amax = fmax(amax, __shfl_xor(amax, off, BLOCK));
-        // floor(log2 amax) of a float32-born value is its binary exponent
-        const int e0 = amax > 0.0 ? int((__double_as_longlong(amax) >> 52) & 0x7FF) - 1023 - 2 : 0;
-        double best = block_sq_err<BLOCK>(b, e0);
-        int chosen = e0;
-        double t = block_sq_err<BLOCK>(b, e0 - 1);
-        if (t < best) {
-            best = t;
-            chosen = e0 - 1;
+        for (int i = 0; i < BLOCK; ++i) amax = fmaxf(amax, fabsf(v[i]));
+        int chosen = EMPTY;
+        if (amax > 0.0f) {
+            // floor(log2 amax) of a float32-born value is its binary exponent
+            const int e0 = int((__double_as_longlong(double(amax)) >> 52) & 0x7FF) - 1023 - 2;
+            float x[BLOCK];
+#pragma unroll
+            for (int i = 0; i < BLOCK; ++i) x[i] = __builtin_amdgcn_ldexpf(v[i], -e0);
+            const float s0 = fp4_sq_err<BLOCK>(x, 1.0f), sm = fp4_sq_err<BLOCK>(x, 0.5f), sp = fp4_sq_err<BLOCK>(x, 2.0f);
+            // A float32 sum of 32 squares of exact differences is within 32 half-ulps (2e-6) of the exact one, the host's
+            // float64 sum within 1e-14: apart by more than 1e-5, the sums order alike.  (Below 1e-30 squares underflow.)
+            auto close = [](float a, float b) { return !(fabsf(a - b) > 1e-5f * fmaxf(a, b)) || fmaxf(a, b) < 1e-30f; };
+            const float s1 = sm < s0 ? sm : s0;
+            if (close(sm, s0) || close(sp, s1)) {
+                auto weight = [&](int i) -> float {
+                    if (BF16) return bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[at + i]);
+                    return reinterpret_cast<const float*>(w)[at + i];
+                };
+                double best = block_sq_err<BLOCK>(weight, e0);
+                chosen = e0;
+                double t = block_sq_err<BLOCK>(weight, e0 - 1);
+                if (t < best) {
+                    best = t;
+                    chosen = e0 - 1;
+                }
+                t = block_sq_err<BLOCK>(weight, e0 + 1);
+                if (t < best) chosen = e0 + 1;
+            } else {
+                chosen = sp < s1 ? e0 + 1 : sm < s0 ? e0 - 1 : e0;
+            }
         }
-        t = block_sq_err<BLOCK>(b, e0 + 1);
-        if (t < best) chosen = e0 + 1;
-        if (in && tid % BLOCK == 0) s_e[k / BLOCK] = amax > 0.0 ? chosen : EMPTY;
+        s_e[b] = chosen;
     }
     __syncthreads();
 
-    // ---- row constraint (sim/mx_int8.py:68-81) and the row's lowest exponent (sim/mx_int8.py:92-109) ---------------
-    int top = EMPTY;
-    for (int i = tid; i < nb; i += QNT) top = max(top, s_e[i]);
-    top = wg_reduce<true>(top, red);
-    if (top == EMPTY) top = 0;   // all-zero row
-    const int floor_e = top - MAX_SPREAD;
-    int lo = INT_MAX;
-    for (int i = tid; i < nb; i += QNT) lo = min(lo, max(s_e[i], floor_e));
-    lo = wg_reduce<false>(lo, red);
-
-    // ---- pass 2: codes (sim/make_testcase.py:36-39, e2e/sc_format.py:72-73) ---------------------------------------
-    for (int k0 = 0; k0 < K; k0 += QNT) {
-        const int k = k0 + tid;
-        const bool in = k < K;
-        uint32_t c = 0;
-        if (in) {
-            const int e = max(s_e[k / BLOCK], floor_e);
-            const double x = weight(k) * pow2_f64(-e);
-            const int idx = e2m1_index(x);
-            c = uint32_t(idx) | ((x < 0.0 && idx > 0) ? 8u : 0u);
+    // ---- row constraint (sim/mx_int8.py:68-81) and the row's lowest exponent (sim/mx_int8.py:92-109): a wave per row ---
+    for (int r = tid >> 6; r < live; r += QNT / 64) {
+        int top = EMPTY;
+        for (int i = lane; i < nb; i += 64) top = max(top, s_e[r * nb + i]);
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) top = max(top, __shfl_xor(top, off, WAVE));
+        if (top == EMPTY) top = 0;   // all-zero row
+        const int floor_e = top - MAX_SPREAD;
+        int lo = INT_MAX;
+        for (int i = lane; i < nb; i += 64) lo = min(lo, max(s_e[r * nb + i], floor_e));
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) lo = min(lo, __shfl_xor(lo, off, WAVE));
+        if (lane == 0) {
+            s_floor[r] = floor_e;
+            s_lo[r] = lo;
+            wscale[row0 + r] = float(pow2_f64(lo - 1));   // 2^(E_lo - 1), sim/mx_int8.py:101
         }
-        c <<= 4 * (tid & 7);
-        c |= __shfl_xor(c, 1, 8);
-        c |= __shfl_xor(c, 2, 8);
-        c |= __shfl_xor(c, 4, 8);
-        if (in && (tid & 7) == 0) codes[(row * K + k) >> 3] = c;
+    }
+    __syncthreads();
+
+    // ---- codes (sim/make_testcase.py:36-39, e2e/sc_format.py:72-73) ------------------------------------------------
+    for (int b = tid; b < total; b += QNT) {
+        const size_t at = base + size_t(b) * BLOCK;
+        if (total > QNT) load_block<BLOCK, BF16>(w, at, vec, v);   // more than one block per thread: read them again
+        const int e = max(s_e[b], s_floor[b / nb]);
+        uint32_t c[BLOCK / 8];
+#pragma unroll
+        for (int i = 0; i < BLOCK / 8; ++i) c[i] = 0u;
+#pragma unroll
+        for (int i = 0; i < BLOCK; ++i) {
+            // index of the E2M1 level nearest to a = |w| 2^-e, saturating at 7, a midpoint to the lower level
+            // (sim/mx_int8.py:23-25): levels are t / 2 apart from t = 2^max(floor(log2 a), 0) on, so the index is
+            // ceil(2 a / t - 1/2) plus two per octave above the first
+            const float a = fabsf(__builtin_amdgcn_ldexpf(v[i], -e));
+            const uint32_t t = max(__float_as_uint(a) & 0x7F800000u, 0x3F800000u);
+            const float m = ceilf(__builtin_fmaf(a, __uint_as_float(0x7F800000u - t), -0.5f));
+            const int idx = min(int(m) + 2 * (int(t >> 23) - 127), 7);
+            c[i >> 3] |= (uint32_t(idx) | ((v[i] < 0.0f && idx > 0) ? 8u : 0u)) << (4 * (i & 7));
+        }
+        store_codes<BLOCK>(codes + at / 8, vec, c);
     }
     // block codes: shift = e - lo in 0..3, 2 bits each, four blocks per byte (e2e/sc_format.py:14)
-    for (int j = tid; j < nb / 4; j += QNT) {
+    for (int j = tid; j < total / 4; j += QNT) {
+        const int r = 4 * j / nb;
         uint32_t byte = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) byte |= uint32_t(max(s_e[4 * j + i], floor_e) - lo) << (2 * i);
-        bcodes[row * (nb / 4) + j] = uint8_t(byte);
+        for (int i = 0; i < 4; ++i) byte |= uint32_t(max(s_e[4 * j + i], s_floor[r]) - s_lo[r]) << (2 * i);
+        bcodes[row0 * (nb / 4) + j] = uint8_t(byte);
     }
-    if (tid == 0) wscale[row] = float(pow2_f64(lo - 1));   // 2^(E_lo - 1), sim/mx_int8.py:101
 }
 
 // ---- the integer-exact format family: w = base[row] * mult[block] * sign * code ------------------------------------
@@ -147,7 +230,7 @@ __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict
 // peak / (largest multiplier * largest code); 8 bases per octave below it are tried in descending order, each with
 // the per-block multiplier of least squared error (first minimum), and a candidate replaces the best so far only
 // when its total error over the row is strictly smaller.  Block errors and row totals are summed in the order of
-// the host's pairwise reduction.  One workgroup per row, one lane per weight.
+// the host's pairwise reduction.  A thread owns one block and keeps its magnitudes in registers over all trials.
 struct FamilyArgs {
     float cb[8];      // code magnitudes
     float cut[7];     // midpoints between neighbouring magnitudes
@@ -156,27 +239,35 @@ struct FamilyArgs {
 };
 
 // numpy's pairwise sum of n contiguous float32 values (n <= 128: eight strided running sums, a fixed tree, then the
-// n % 8 tail; longer inputs are split in two at a multiple of 8 below the middle).
-__device__ float np_pairwise_sum(const float* a, int n) {
+// n % 8 tail; longer inputs are split in two at a multiple of 8 below the middle).  DEPTH splits at most: four bring
+// any n <= 1024 down to 128.
+template <int DEPTH>
+__device__ __forceinline__ float np_pairwise_sum(const float* a, int n) {
+    if constexpr (DEPTH > 0) {
+        if (n > 128) {
+            int n2 = n / 2;
+            n2 -= n2 % 8;
+            const float lower = np_pairwise_sum<DEPTH - 1>(a, n2);
+            return __fadd_rn(lower, np_pairwise_sum<DEPTH - 1>(a + n2, n - n2));
+        }
+    }
     if (n < 8) {
         float r = 0.0f;
         for (int i = 0; i < n; ++i) r = __fadd_rn(r, a[i]);
         return r;
     }
-    if (n <= 128) {
-        float r[8];
-        for (int j = 0; j < 8; ++j) r[j] = a[j];
-        int i = 8;
-        for (; i < n - (n % 8); i += 8)
-            for (int j = 0; j < 8; ++j) r[j] = __fadd_rn(r[j], a[i + j]);
-        float res = __fadd_rn(__fadd_rn(__fadd_rn(r[0], r[1]), __fadd_rn(r[2], r[3])),
-                              __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
-        for (; i < n; ++i) res = __fadd_rn(res, a[i]);
-        return res;
+    float r[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = a[j];
+    int i = 8;
+    for (; i < n - (n % 8); i += 8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) r[j] = __fadd_rn(r[j], a[i + j]);
     }
-    int n2 = n / 2;
-    n2 -= n2 % 8;
-    return __fadd_rn(np_pairwise_sum(a, n2), np_pairwise_sum(a + n2, n - n2));
+    float res = __fadd_rn(__fadd_rn(__fadd_rn(r[0], r[1]), __fadd_rn(r[2], r[3])),
+                          __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
+    for (; i < n; ++i) res = __fadd_rn(res, a[i]);
+    return res;
 }
 
 __device__ __forceinline__ int family_index(const FamilyArgs& f, float x) {   // nearest code, ties to the lower one
@@ -186,122 +277,188 @@ __device__ __forceinline__ int family_index(const FamilyArgs& f, float x) {   //
     for (int i = 0; i < 7; ++i) idx += int(a > f.cut[i]);
     return idx;
 }
+__device__ __forceinline__ float family_level(const FamilyArgs& f, float a) {   // its magnitude, for a >= 0
+    float v = f.cb[0];
+#pragma unroll
+    for (int i = 0; i < 7; ++i) v = a > f.cut[i] ? f.cb[i + 1] : v;
+    return v;
+}
 
-template <int BLOCK, bool BF16>
+// Squared error of the block of magnitudes aw at scale sc, as the host evaluates it (float32, its order of sums).
+template <int BLOCK>
+__device__ __forceinline__ float family_sq_err(const FamilyArgs& f, const float (&aw)[BLOCK], float sc) {
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < BLOCK; ++i) {
+        const float v = family_level(f, __fdiv_rn(aw[i], sc));
+        const float d = __fsub_rn(__fmul_rn(v, sc), aw[i]);
+        const float sq = __fmul_rn(d, d);
+        r[i & 7] = i < 8 ? sq : __fadd_rn(r[i & 7], sq);
+    }
+    return __fadd_rn(__fadd_rn(__fadd_rn(r[0], r[1]), __fadd_rn(r[2], r[3])),
+                     __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
+}
+
+// The same for the E2M1 codebook (0, 1, 2, 3, 4, 6, 8, 12 = twice the FP4 values) through the FP4 conversion: about 8
+// instructions per weight instead of 40.  The quotient is formed twice with an approximate reciprocal, 2^-20 too large
+// and 2^-20 too small: where both round to the same code so does the correctly rounded quotient, whose error lies
+// between; where they differ (a quotient next to a midpoint) *same is cleared and the caller takes the form above.
+template <int BLOCK>
+__device__ __forceinline__ float family_sq_err_e2m1(const float (&aw)[BLOCK], float sc, bool* same) {
+    const float h = 0.5f * __builtin_amdgcn_rcpf(sc);
+    const float up = h * 1.00000095367431640625f, dn = h * 0.99999904632568359375f;
+    float r[8];
+    uint32_t diff = 0;
+#pragma unroll
+    for (int i = 0; i < BLOCK; i += 2) {
+        const uint32_t cu = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, aw[i] * up, aw[i + 1] * up, 1.0f, 0);
+        const uint32_t cd = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, aw[i] * dn, aw[i + 1] * dn, 1.0f, 0);
+        diff |= cu ^ cd;
+        const f32x2_t v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cd, 2.0f, 0);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float d = __fsub_rn(__fmul_rn(v[k], sc), aw[i + k]);
+            const float sq = __fmul_rn(d, d);
+            r[(i + k) & 7] = i < 8 ? sq : __fadd_rn(r[(i + k) & 7], sq);
+        }
+    }
+    *same = diff == 0u;
+    return __fadd_rn(__fadd_rn(__fadd_rn(r[0], r[1]), __fadd_rn(r[2], r[3])),
+                     __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
+}
+
+constexpr int FAM_ROWS = 4;   // rows per workgroup at most: more are needed only for K < 1024, and their tables cost LDS
+
+// Bound: vector ALU (8 bases x n_mult trials per weight).  2048 x 2048 bf16, ten multipliers: 130 us; 520 us with a lane
+// per weight, a correctly rounded division per trial and the sums across lanes.
+template <int BLOCK, bool BF16, bool E2M1>
 __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                              uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
-                                                             int K, const FamilyArgs f) {
-    extern __shared__ float s_f[];   // 8 x nb block errors, 8 totals, 8 reduction slots, then 8 x nb multiplier indices
+                                                             int64_t N, int K, int rows, bool vec, const FamilyArgs f) {
+    extern __shared__ float s_f[];   // per row: 8 x nb block errors; then 8 x nb multiplier indices per row
+    __shared__ uint32_t s_peak[FAM_ROWS];
+    __shared__ float s_tot[FAM_ROWS][8];
+    __shared__ int s_best[FAM_ROWS];
     const int nb = K / BLOCK;
     float* s_err = s_f;
-    float* s_tot = s_f + 8 * nb;
-    float* s_red = s_tot + 8;
-    uint8_t* s_mi = reinterpret_cast<uint8_t*>(s_red + 8);
-    __shared__ int s_best;
-    const size_t row = blockIdx.x;
-    const int tid = threadIdx.x;
-    auto weight = [&](int k) -> float {
-        if (BF16) return bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[row * K + k]);
-        return reinterpret_cast<const float*>(w)[row * K + k];
-    };
-    // row peak
-    float peak = 0.0f;
-    for (int k = tid; k < K; k += QNT) peak = fmaxf(peak, fabsf(weight(k)));
-    peak = wave_max(peak);
-    if ((tid & 63) == 0) s_red[tid >> 6] = peak;
+    uint8_t* s_mi = reinterpret_cast<uint8_t*>(s_f + size_t(rows) * 8 * nb);
+    const size_t row0 = size_t(blockIdx.x) * rows;
+    const int live = int(min(int64_t(rows), N - int64_t(row0)));
+    const int total = live * nb, tid = threadIdx.x;
+    const size_t wbase = row0 * K;
+    // row peaks (bit patterns of non-negative floats order like the floats)
+    if (tid < FAM_ROWS) s_peak[tid] = 0u;
     __syncthreads();
-    peak = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-    if (peak == 0.0f) peak = 1.0f;
-    const float top = __fdiv_rn(peak, __fmul_rn(f.mult[f.n_mult - 1], f.cb[7]));
+    float v[BLOCK];
+    for (int b = tid; b < total; b += QNT) {
+        load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < BLOCK; ++i) amax = fmaxf(amax, fabsf(v[i]));
+        atomicMax(&s_peak[b / nb], __float_as_uint(amax));
+    }
+    __syncthreads();
     // 2^(-j/8) rounded to float32: the candidate ladder of one octave
     const float ladder[8] = {1.0f, 0.9170040488243103f, 0.8408964276313782f, 0.7711054086685181f, 0.7071067690849304f,
                              0.6484197974205017f, 0.5946035385131836f, 0.5452538728713989f};
+    auto row_top = [&](int r) {
+        float peak = __uint_as_float(s_peak[r]);
+        if (peak == 0.0f) peak = 1.0f;
+        return __fdiv_rn(peak, __fmul_rn(f.mult[f.n_mult - 1], f.cb[7]));
+    };
 
     // ---- per candidate base and block: the best multiplier and its error ------------------------------------------
-    for (int k0 = 0; k0 < K; k0 += QNT) {
-        const int k = k0 + tid;
-        const bool in = k < K;
-        const float wv = in ? weight(k) : 0.0f;
+    for (int b = tid; b < total; b += QNT) {
+        if (total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+        const int r = b / nb, kb = b - r * nb;
+        const float top = row_top(r);
+        float aw[BLOCK];
+#pragma unroll
+        for (int i = 0; i < BLOCK; ++i) aw[i] = fabsf(v[i]);
 #pragma unroll 1
         for (int j = 0; j < 8; ++j) {
             const float base = __fmul_rn(top, ladder[j]);
             float best = 0.0f;
             int best_i = 0;
+#pragma unroll 1
             for (int i = 0; i < f.n_mult; ++i) {
                 const float sc = __fmul_rn(base, f.mult[i]);
-                const float x = __fdiv_rn(wv, sc);
-                const float lv = f.cb[family_index(f, x)];
-                const float v = x > 0.0f ? lv : (x < 0.0f ? -lv : 0.0f * lv);
-                const float d = __fsub_rn(__fmul_rn(v, sc), wv);
-                const float sq = __fmul_rn(d, d);
-                float r = __fadd_rn(sq, __shfl_down(sq, 8, BLOCK));
-                if (BLOCK == 32) {
-                    r = __fadd_rn(r, __shfl_down(sq, 16, BLOCK));
-                    r = __fadd_rn(r, __shfl_down(sq, 24, BLOCK));
-                }
-                r = __fadd_rn(r, __shfl_xor(r, 1, BLOCK));
-                r = __fadd_rn(r, __shfl_xor(r, 2, BLOCK));
-                r = __fadd_rn(r, __shfl_xor(r, 4, BLOCK));
-                r = __shfl(r, 0, BLOCK);
-                if (i == 0 || r < best) {
-                    best = r;
+                bool same = false;
+                float e = 0.0f;
+                // (a scale near the ends of the float32 range leaves its reciprocal no room)
+                if (E2M1 && sc > 1e-30f && sc < 1e30f) e = family_sq_err_e2m1<BLOCK>(aw, sc, &same);
+                if (!same) e = family_sq_err<BLOCK>(f, aw, sc);
+                if (i == 0 || e < best) {
+                    best = e;
                     best_i = i;
                 }
             }
-            if (in && tid % BLOCK == 0) {
-                s_err[j * nb + k / BLOCK] = best;
-                s_mi[j * nb + k / BLOCK] = uint8_t(best_i);
-            }
+            s_err[(r * 8 + j) * nb + kb] = best;
+            s_mi[(r * 8 + j) * nb + kb] = uint8_t(best_i);
         }
     }
     __syncthreads();
-    if (tid < 8) s_tot[tid] = np_pairwise_sum(s_err + tid * nb, nb);
+    if (tid < 8 * live) s_tot[tid >> 3][tid & 7] = np_pairwise_sum<4>(s_err + tid * nb, nb);
     __syncthreads();
-    if (tid == 0) {
+    if (tid < live) {
         float best = __builtin_inff();
         int bj = 0;
         for (int j = 0; j < 8; ++j)
-            if (s_tot[j] < best) {
-                best = s_tot[j];
+            if (s_tot[tid][j] < best) {
+                best = s_tot[tid][j];
                 bj = j;
             }
-        s_best = bj;
+        s_best[tid] = bj;
+        wscale[row0 + tid] = __fmul_rn(row_top(tid), ladder[bj]);
     }
     __syncthreads();
-    const int bj = s_best;
-    const float base = __fmul_rn(top, ladder[bj]);
-    const bool dead = base == 0.0f;   // a vanishing row underflows its base: it is exactly zero (e2e/pack_format.py:55-58)
 
     // ---- codes ----------------------------------------------------------------------------------------------------
-    for (int k0 = 0; k0 < K; k0 += QNT) {
-        const int k = k0 + tid;
-        const bool in = k < K;
-        uint32_t c = 0;
-        if (in && !dead) {
-            const float sc = __fmul_rn(base, f.mult[s_mi[bj * nb + k / BLOCK]]);
-            const float x = __fdiv_rn(weight(k), sc);
-            const int idx = family_index(f, x);
-            c = uint32_t(idx) | ((x < 0.0f && f.cb[idx] > 0.0f) ? 8u : 0u);
+    for (int b = tid; b < total; b += QNT) {
+        if (total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+        const int r = b / nb, kb = b - r * nb, bj = s_best[r];
+        const float base = __fmul_rn(row_top(r), ladder[bj]);
+        const bool dead = base == 0.0f;   // a vanishing row underflows its base: it is exactly zero (e2e/pack_format.py:55-58)
+        const float sc = __fmul_rn(base, f.mult[s_mi[(r * 8 + bj) * nb + kb]]);
+        uint32_t c[BLOCK / 8];
+#pragma unroll
+        for (int i = 0; i < BLOCK / 8; ++i) c[i] = 0u;
+        if (!dead) {
+#pragma unroll
+            for (int i = 0; i < BLOCK; ++i) {
+                const float x = __fdiv_rn(v[i], sc);
+                const bool minus = x < 0.0f && family_level(f, fabsf(x)) > 0.0f;
+                c[i >> 3] |= (uint32_t(family_index(f, x)) | (minus ? 8u : 0u)) << (4 * (i & 7));
+            }
         }
-        c <<= 4 * (tid & 7);
-        c |= __shfl_xor(c, 1, 8);
-        c |= __shfl_xor(c, 2, 8);
-        c |= __shfl_xor(c, 4, 8);
-        if (in && (tid & 7) == 0) codes[(row * K + k) >> 3] = c;
+        store_codes<BLOCK>(codes + (wbase + size_t(b) * BLOCK) / 8, vec, c);
     }
     // block codes: index into the multiplier table, bc_bits each (e2e/sc_format.py:14); a dead row takes multiplier 1
-    const int per_byte = 8 / f.bc_bits;
+    const int per_byte = 8 / f.bc_bits, row_bytes = nb / per_byte;
     int one = 0;
     for (int i = 0; i < f.n_mult; ++i)
         if (f.mult[i] == 1.0f) one = i;
-    for (int b = tid; b < nb / per_byte; b += QNT) {
+    for (int q = tid; q < live * row_bytes; q += QNT) {
+        const int r = q / row_bytes, kb = (q - r * row_bytes) * per_byte, bj = s_best[r];
+        const bool dead = __fmul_rn(row_top(r), ladder[bj]) == 0.0f;
         uint32_t byte = 0;
         for (int i = 0; i < per_byte; ++i)
-            byte |= uint32_t(dead ? one : s_mi[bj * nb + b * per_byte + i]) << (f.bc_bits * i);
-        bcodes[row * (nb / per_byte) + b] = uint8_t(byte);
+            byte |= uint32_t(dead ? one : s_mi[(r * 8 + bj) * nb + kb + i]) << (f.bc_bits * i);
+        bcodes[row0 * row_bytes + q] = uint8_t(byte);
     }
-    if (tid == 0) wscale[row] = base;
 }
+
+// fn(block width, is bf16) as compile-time constants.
+template <typename Fn>
+static void by_block_and_type(int block, int bf16, Fn&& fn) {
+    using B32 = std::integral_constant<int, 32>;
+    using B16 = std::integral_constant<int, 16>;
+    if (block == 32) bf16 ? fn(B32{}, std::true_type{}) : fn(B32{}, std::false_type{});
+    else bf16 ? fn(B16{}, std::true_type{}) : fn(B16{}, std::false_type{});
+}
+
+// Rows per workgroup: as many whole rows as give each of its threads one block, which then stays in registers.
+static int rows_per_group(int nb, int most) { return nb >= QNT ? 1 : (QNT / nb < most ? QNT / nb : most); }
 
 }  // namespace scmx
 
@@ -341,16 +498,21 @@ extern "C" int scmx_quantize_family(const scmx_format* fmt, const void* w, int w
     f.bc_bits = fmt->bc_bits;
     if (N == 0) return SCMX_OK;
     const int nb = K / block;
-    const size_t smem = size_t(8 * nb + 16) * sizeof(float) + size_t(8 * nb);
-    const dim3 grid((unsigned)N), wg(QNT);
-    hipStream_t st = (hipStream_t)stream;
-    if (block == 32) {
-        if (w_is_bf16) quantize_family_kernel<32, true><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K, f);
-        else quantize_family_kernel<32, false><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K, f);
-    } else {
-        if (w_is_bf16) quantize_family_kernel<16, true><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K, f);
-        else quantize_family_kernel<16, false><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K, f);
-    }
+    const int rows = rows_per_group(nb, FAM_ROWS);
+    const size_t smem = size_t(rows) * 8 * nb * (sizeof(float) + 1);
+    const dim3 grid((unsigned)((N + rows - 1) / rows)), wg(QNT);
+    const bool vec = uintptr_t(w) % 16 == 0 && uintptr_t(codes) % 16 == 0;
+    const bool e2m1 = df.lut_lo == 0x03020100u && df.lut_hi == 0x0C080604u;
+    auto go = [&](auto kernel) {
+        kernel<<<grid, wg, smem, (hipStream_t)stream>>>(w, codes, bcodes, wscale, N, K, rows, vec, f);
+    };
+    auto typed = [&](auto blk, auto bf) {
+        constexpr int B = decltype(blk)::value;
+        constexpr bool BF = decltype(bf)::value;
+        if (e2m1) go(quantize_family_kernel<B, BF, true>);
+        else go(quantize_family_kernel<B, BF, false>);
+    };
+    by_block_and_type(block, w_is_bf16, typed);
     return check_launch("quantize_family");
 }
 
@@ -370,15 +532,13 @@ extern "C" int scmx_quantize_sc(const void* w, int w_is_bf16, int64_t N, int K, 
         return SCMX_ERR_ARG;
     }
     if (N == 0) return SCMX_OK;
-    const dim3 grid((unsigned)N), wg(QNT);
-    const size_t smem = (size_t(K / block) + 4) * sizeof(int);
-    hipStream_t st = (hipStream_t)stream;
-    if (block == 32) {
-        if (w_is_bf16) quantize_sc_kernel<32, true><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K);
-        else quantize_sc_kernel<32, false><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K);
-    } else {
-        if (w_is_bf16) quantize_sc_kernel<16, true><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K);
-        else quantize_sc_kernel<16, false><<<grid, wg, smem, st>>>(w, codes, bcodes, wscale, K);
-    }
+    const int nb = K / block, rows = rows_per_group(nb, QNT / 4);
+    const dim3 grid((unsigned)((N + rows - 1) / rows)), wg(QNT);
+    const size_t smem = size_t(rows) * (nb + 2) * sizeof(int);
+    const bool vec = uintptr_t(w) % 16 == 0 && uintptr_t(codes) % 16 == 0;
+    by_block_and_type(block, w_is_bf16, [&](auto blk, auto bf) {
+        quantize_sc_kernel<decltype(blk)::value, decltype(bf)::value>
+            <<<grid, wg, smem, (hipStream_t)stream>>>(w, codes, bcodes, wscale, N, K, rows, vec);
+    });
     return check_launch("quantize_sc");
 }
