@@ -217,6 +217,17 @@ int scmx_attn_prefill(const uint16_t* q, const uint16_t* kcache, const uint16_t*
 int scmx_qkv_fullnorm(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q,
                       uint16_t* k, uint16_t* v, int L, int h, int d, void* stream);
 
+/* scmx_qkv_fullnorm followed by the rotary embedding of q and k and the append to the KV cache; the remaining arguments as
+ * in scmx_qkv_headnorm_rope (hq = hk = h; d <= 512).  Fuses what the model integration does with array ops after qkv_fullnorm_y
+ * (e2e/fused_olmoe.py:197-203). */
+int scmx_qkv_fullnorm_rope(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q,
+                           uint16_t* kcache, uint16_t* vcache, int L, int h, int d, const float* inv_freq,
+                           const int64_t* pos_dev, int64_t pos0, int cache_rows, int q_token_major, void* stream);
+
+/* RMSNorm(x, w, eps) of T rows [M, K] -> T[M, K]: the model's final norm (the array op before the output head,
+ * e2e/fused_qwen3.py:224-255). */
+int scmx_rmsnorm(const uint16_t* x, const uint16_t* w, float eps, uint16_t* out, int M, int K, void* stream);
+
 /* ---- decode --------------------------------------------------------------------------------------------------- */
 
 /* W4A8 GEMV on packed weights, `batch` input rows sharing one weight stream (batch 1, 2, 4 or 8; the reference has

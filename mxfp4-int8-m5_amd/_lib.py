@@ -47,6 +47,8 @@ SIGNATURES = {
     "scmx_attn_decode_qkv": (_I, [_P, _P, _P, _F, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _F, _P, _I, _P]),
     "scmx_qkv_headnorm_rope": (_I, [_P, _P, _P, _P, _P, _P, _F, _P, _P, _P, _I, _I, _I, _I, _P, _P, _L, _I, _I, _P]),
     "scmx_qkv_fullnorm": (_I, [_P, _P, _P, _F, _P, _P, _P, _I, _I, _I, _P]),
+    "scmx_qkv_fullnorm_rope": (_I, [_P, _P, _P, _F, _P, _P, _P, _I, _I, _I, _P, _P, _L, _I, _I, _P]),
+    "scmx_rmsnorm": (_I, [_P, _P, _F, _P, _I, _I, _P]),
     "scmx_gemv": (_I, [_FMT, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _F, _I, _I, _I, _P, _I, _I, _I, _P]),
     "scmx_route_topk": (_I, [_P, _P, _I, _I, _I, _I, _P, _P, _P]),
     "scmx_route_sort": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P]),

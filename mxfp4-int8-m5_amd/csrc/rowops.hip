@@ -113,14 +113,84 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const uint16_t* __res
     block_quant_row(srow, K, qrow, xs + row, red);
 }
 
+// Sum of squares of a row held by one wave, lane l owning the 16-byte pieces l, l + 64, ... (CH of them, K = 512 * CH),
+// taken in the order of block_inv_rms: there, thread (wave g, lane t) adds the squares of elements 256 g + 4 t .. + 3 in
+// sequence, a butterfly over lane distances 32 ... 1 gives the sum of group g, and a second butterfly over the group sums
+// (zeros beyond the last group) gives the total.  Here piece l + 64 j holds the elements of lanes 2 (l % 32) and
+// 2 (l % 32) + 1 of group 2 j + l / 32: the two four-element sums stay apart through the butterfly over lane distances
+// 16 ... 1 (= 32 ... 2 there) and are added last (= distance 1); lane l then picks up the sum of group l and the second
+// butterfly runs as it does there.
+template <int CH>
+__device__ __forceinline__ float wave_row_sumsq(const u32x4 (&v)[CH]) {
+    const int lane = threadIdx.x & 63;
+    auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
+    auto hi = [](uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); };
+    float r = 0.0f;   // lane l < 2 CH: the sum of group l
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        float a = __fmul_rn(lo(v[j][0]), lo(v[j][0]));
+        a = __fadd_rn(a, __fmul_rn(hi(v[j][0]), hi(v[j][0])));
+        a = __fadd_rn(a, __fmul_rn(lo(v[j][1]), lo(v[j][1])));
+        a = __fadd_rn(a, __fmul_rn(hi(v[j][1]), hi(v[j][1])));
+        float b = __fmul_rn(lo(v[j][2]), lo(v[j][2]));
+        b = __fadd_rn(b, __fmul_rn(hi(v[j][2]), hi(v[j][2])));
+        b = __fadd_rn(b, __fmul_rn(lo(v[j][3]), lo(v[j][3])));
+        b = __fadd_rn(b, __fmul_rn(hi(v[j][3]), hi(v[j][3])));
+#pragma unroll
+        for (int off = 16; off >= 1; off >>= 1) {
+            a = __fadd_rn(a, __shfl_xor(a, off, WAVE));
+            b = __fadd_rn(b, __shfl_xor(b, off, WAVE));
+        }
+        const float mine = __fadd_rn(a, b);                 // group 2 j + lane / 32
+        const float other = __shfl_xor(mine, 32, WAVE);     // the other group of this j
+        const float even = lane < 32 ? mine : other, odd = lane < 32 ? other : mine;
+        if ((lane >> 1) == j) r = (lane & 1) ? odd : even;
+    }
+    return wave_sum(r);
+}
+__device__ __forceinline__ float inv_rms(float sumsq, int n, float eps) {
+    return __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sumsq, float(n)), eps)));
+}
+// Eight bf16 values x of a row normalised: bf16(w * bf16(x * inv)).
+__device__ __forceinline__ u32x4 norm8(const u32x4& x, const u32x4& w, float inv) {
+    u32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float n0 = __fmul_rn(__uint_as_float(w[e] << 16), round_bf16(__fmul_rn(__uint_as_float(x[e] << 16), inv)));
+        const float n1 = __fmul_rn(__uint_as_float(w[e] & 0xFFFF0000u),
+                                   round_bf16(__fmul_rn(__uint_as_float(x[e] & 0xFFFF0000u), inv)));
+        r[e] = uint32_t(f32_to_bf16(n0)) | (uint32_t(f32_to_bf16(n1)) << 16);
+    }
+    return r;
+}
+
+// ---- rmsnorm: the normalised rows alone ------------------------------------------------------------------------------
+// One wave per row, the row in registers (K = 512 * CH); any other K: a workgroup per row.
+template <int CH>
+__global__ __launch_bounds__(256) void rmsnorm_wave_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                           float eps, uint16_t* __restrict__ out, int M) {
+    constexpr int K = 512 * CH;
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= M) return;
+    u32x4 v[CH], wv[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) v[j] = reinterpret_cast<const u32x4*>(x + size_t(row) * K)[lane + 64 * j];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) wv[j] = reinterpret_cast<const u32x4*>(w)[lane + 64 * j];
+    const float inv = inv_rms(wave_row_sumsq(v), K, eps);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) reinterpret_cast<u32x4*>(out + size_t(row) * K)[lane + 64 * j] = norm8(v[j], wv[j], inv);
+}
+__global__ __launch_bounds__(NT) void rmsnorm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, float eps,
+                                                     uint16_t* __restrict__ out, int K) {
+    __shared__ float red[72];
+    const size_t at = size_t(blockIdx.x) * K;
+    const float inv = block_inv_rms(x + at, K, eps, red);
+    block_norm_row(x + at, w, inv, out + at, nullptr, K);
+}
+
 // The same with the row in registers: one wave per row, lane l owns the 16-byte pieces l, l + 64, ... (CH of them,
-// K = 512 * CH), four rows per workgroup, no LDS and no workgroup barrier.  The sum of squares is taken in the order of
-// block_inv_rms, so both kernels give the same bits: there, thread (wave g, lane t) adds the squares of elements
-// 256 g + 4 t .. + 3 in sequence, a butterfly over lane distances 32 ... 1 gives the sum of group g, and a second
-// butterfly over the group sums (zeros beyond the last group) gives the total.  Here piece l + 64 j holds the
-// elements of lanes 2 (l % 32) and 2 (l % 32) + 1 of group 2 j + l / 32: the two four-element sums stay apart through
-// the butterfly over lane distances 16 ... 1 (= 32 ... 2 there) and are added last (= distance 1); lane l then picks
-// up the sum of group l and the second butterfly runs as it does there.
+// K = 512 * CH), four rows per workgroup, no LDS and no workgroup barrier.  Same bits (wave_row_sumsq).
 // BLK: xq leaves in the blocked layout of the dense GEMM (32 x 32 blocks in MFMA operand order, Mp % 32 == 0): eight
 // rows per workgroup, whose codes meet in LDS -- the 16 bytes of row r, k 16 c ... at slot c * 8 + (r + c / 2) % 8 -- and
 // are stored as whole 128-byte lines (8 rows x 16 bytes are adjacent in a block).  Same codes and scales.
@@ -168,39 +238,13 @@ __global__ __launch_bounds__(BLK ? 512 : 256) void rmsnorm_quant_wave_kernel(con
     for (int j = 0; j < CH; ++j) wv[j] = wrow[lane + 64 * j];
     auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
     auto hi = [](uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); };
-    float r = 0.0f;   // lane l < 2 CH: the sum of group l
-#pragma unroll
-    for (int j = 0; j < CH; ++j) {
-        float a = __fmul_rn(lo(v[j][0]), lo(v[j][0]));
-        a = __fadd_rn(a, __fmul_rn(hi(v[j][0]), hi(v[j][0])));
-        a = __fadd_rn(a, __fmul_rn(lo(v[j][1]), lo(v[j][1])));
-        a = __fadd_rn(a, __fmul_rn(hi(v[j][1]), hi(v[j][1])));
-        float b = __fmul_rn(lo(v[j][2]), lo(v[j][2]));
-        b = __fadd_rn(b, __fmul_rn(hi(v[j][2]), hi(v[j][2])));
-        b = __fadd_rn(b, __fmul_rn(lo(v[j][3]), lo(v[j][3])));
-        b = __fadd_rn(b, __fmul_rn(hi(v[j][3]), hi(v[j][3])));
-#pragma unroll
-        for (int off = 16; off >= 1; off >>= 1) {
-            a = __fadd_rn(a, __shfl_xor(a, off, WAVE));
-            b = __fadd_rn(b, __shfl_xor(b, off, WAVE));
-        }
-        const float mine = __fadd_rn(a, b);                 // group 2 j + lane / 32
-        const float other = __shfl_xor(mine, 32, WAVE);     // the other group of this j
-        const float even = lane < 32 ? mine : other, odd = lane < 32 ? other : mine;
-        if ((lane >> 1) == j) r = (lane & 1) ? odd : even;
-    }
-    const float tot = wave_sum(r);
-    const float inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(tot, float(K)), eps)));
+    const float inv = inv_rms(wave_row_sumsq(v), K, eps);
     float amax = 0.0f;
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
+        v[j] = norm8(v[j], wv[j], inv);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float n0 = round_bf16(__fmul_rn(lo(wv[j][e]), round_bf16(__fmul_rn(lo(v[j][e]), inv))));
-            const float n1 = round_bf16(__fmul_rn(hi(wv[j][e]), round_bf16(__fmul_rn(hi(v[j][e]), inv))));
-            amax = fmaxf(amax, fmaxf(fabsf(n0), fabsf(n1)));
-            v[j][e] = (__float_as_uint(n0) >> 16) | (__float_as_uint(n1) & 0xFFFF0000u);
-        }
+        for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fmaxf(fabsf(lo(v[j][e])), fabsf(hi(v[j][e]))));
         if (nrow) nrow[lane + 64 * j] = v[j];
     }
     amax = wave_max(amax);
@@ -438,16 +482,22 @@ __global__ __launch_bounds__(NT) void qkv_headnorm128_kernel(const uint16_t* __r
 }
 
 // ---- OLMoE q/k/v split with RMSNorm over the full h*d width ------------------------------------------------------
+// With inv_freq != NULL also the rotary embedding of q and k and the append to the caches (RopeArgs, as above).
 __global__ __launch_bounds__(NT) void qkv_fullnorm_kernel(const uint16_t* __restrict__ y, const uint16_t* __restrict__ qn,
                                                           const uint16_t* __restrict__ kn, float eps, uint16_t* __restrict__ q,
                                                           uint16_t* __restrict__ k, uint16_t* __restrict__ v, int L, int h,
-                                                          int d) {
-    extern __shared__ __attribute__((aligned(16))) uint16_t srow[];   // W bf16 + 72 floats
+                                                          int d, const RopeArgs rope) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t srow[];   // W bf16, 72 floats, d sines and cosines
     const int W = h * d, row = blockIdx.x;
     float* red = reinterpret_cast<float*>(srow + W);
+    float* s_sin = red + 72;
+    float* s_cos = s_sin + d / 2;
+    const int64_t pos = rope.inv_freq ? (rope.pos_dev ? rope.pos_dev[0] : rope.pos0) + row : row;
+    const int kv_rows = rope.inv_freq ? rope.kv_rows : L;
+    if (rope.inv_freq)
+        for (int i = threadIdx.x; i < d / 2; i += NT) sincosf(float(pos) * rope.inv_freq[i], &s_sin[i], &s_cos[i]);
     for (int part = 0; part < 3; ++part) {
         const uint16_t* yr = y + size_t(row) * 3 * W + size_t(part) * W;
-        uint16_t* out = part == 0 ? q : (part == 1 ? k : v);
         const uint16_t* src = yr;
         if (part < 2) {
             const float inv = block_inv_rms(yr, W, eps, red);
@@ -456,9 +506,84 @@ __global__ __launch_bounds__(NT) void qkv_fullnorm_kernel(const uint16_t* __rest
         }
         for (int c = threadIdx.x; c < W / 4; c += NT) {
             const int col = 4 * c, hh = col / d, dd = col % d;
-            *reinterpret_cast<u32x2*>(out + (size_t(hh) * L + row) * d + dd) = *reinterpret_cast<const u32x2*>(src + col);
+            u32x2 o = *reinterpret_cast<const u32x2*>(src + col);
+            if (rope.inv_freq && part < 2) {   // element e pairs with e +- d / 2 of its head
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int e = (dd + i) % (d / 2);
+                    const float a = bf16_to_f32(src[hh * d + e]), b = bf16_to_f32(src[hh * d + e + d / 2]);
+                    const float r = dd + i < d / 2 ? __fsub_rn(__fmul_rn(a, s_cos[e]), __fmul_rn(b, s_sin[e]))
+                                                   : __fadd_rn(__fmul_rn(b, s_cos[e]), __fmul_rn(a, s_sin[e]));
+                    const uint32_t bits = f32_to_bf16(r);
+                    o[i >> 1] = i & 1 ? (o[i >> 1] & 0xFFFFu) | (bits << 16) : (o[i >> 1] & 0xFFFF0000u) | bits;
+                }
+            }
+            uint16_t* out = part > 0             ? (part == 1 ? k : v) + (size_t(hh) * kv_rows + size_t(pos)) * d + dd
+                            : rope.q_token_major ? q + size_t(row) * W + col
+                                                 : q + (size_t(hh) * L + row) * d + dd;
+            *reinterpret_cast<u32x2*>(out) = o;
         }
         __syncthreads();
+    }
+}
+
+// The same for W = 512 * CH and head dims of 16 ... 512 that are powers of two: a wave per part (q, k, v) of a row, the part
+// in registers, 16-byte accesses, and a rotation partner d / 16 lanes away.  Same bits (wave_row_sumsq).  Bound: HBM
+// (read 3 W, write 3 W bf16 per row).  The array operations it replaces after a norm kernel of its own were 22 launches a
+// block: two blocks of an OLMoE prompt of 3000 tokens 1591 -> 1130 us, of a decode step 752 -> 319 us.
+template <int CH>
+__global__ __launch_bounds__(192) void qkv_fullnorm_wave_kernel(const uint16_t* __restrict__ y, const uint16_t* __restrict__ qn,
+                                                                const uint16_t* __restrict__ kn, float eps,
+                                                                uint16_t* __restrict__ q, uint16_t* __restrict__ k,
+                                                                uint16_t* __restrict__ v, int L, int d, const RopeArgs rope) {
+    constexpr int W = 512 * CH;
+    __shared__ float s_sin[256], s_cos[256];
+    const int row = blockIdx.x, part = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t pos = rope.inv_freq ? (rope.pos_dev ? rope.pos_dev[0] : rope.pos0) + row : row;
+    const int kv_rows = rope.inv_freq ? rope.kv_rows : L;
+    u32x4 x[CH], wv[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+        x[j] = reinterpret_cast<const u32x4*>(y + size_t(row) * 3 * W + size_t(part) * W)[lane + 64 * j];
+    if (part < 2) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) wv[j] = reinterpret_cast<const u32x4*>(part ? kn : qn)[lane + 64 * j];
+    }
+    if (rope.inv_freq) {
+        for (int i = threadIdx.x; i < d / 2; i += 192) sincosf(float(pos) * rope.inv_freq[i], &s_sin[i], &s_cos[i]);
+        __syncthreads();
+    }
+    if (part < 2) {
+        const float inv = inv_rms(wave_row_sumsq(x), W, eps);
+        const bool low = (lane & (d / 16)) == 0;   // the lane's elements lie in the lower half of their head
+        const int e0 = (8 * lane) & (d / 2 - 1);   // first rotation angle of the lane's pieces (512 % d == 0: of all of them)
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            x[j] = norm8(x[j], wv[j], inv);
+            if (!rope.inv_freq) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t other = uint32_t(__shfl_xor(int(x[j][i]), d / 16, WAVE));
+                uint32_t bits[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const float me = __uint_as_float(t ? x[j][i] & 0xFFFF0000u : x[j][i] << 16);
+                    const float ot = __uint_as_float(t ? other & 0xFFFF0000u : other << 16);
+                    const float sn = s_sin[e0 + 2 * i + t], cs = s_cos[e0 + 2 * i + t];
+                    bits[t] = f32_to_bf16(low ? __fsub_rn(__fmul_rn(me, cs), __fmul_rn(ot, sn))
+                                              : __fadd_rn(__fmul_rn(me, cs), __fmul_rn(ot, sn)));
+                }
+                x[j][i] = bits[0] | (bits[1] << 16);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const int col = 8 * (lane + 64 * j), hh = col / d, dd = col & (d - 1);
+        uint16_t* out = part > 0             ? (part == 1 ? k : v) + (size_t(hh) * kv_rows + size_t(pos)) * d + dd
+                        : rope.q_token_major ? q + size_t(row) * W + col
+                                             : q + (size_t(hh) * L + row) * d + dd;
+        *reinterpret_cast<u32x4*>(out) = x[j];
     }
 }
 
@@ -660,6 +785,21 @@ __global__ __launch_bounds__(NT) void moe_combine_kernel(const uint16_t* __restr
     block_quant_row(nrow_s, K, xq + size_t(row) * K, xs + row, red);
 }
 
+// fn(K / 512 as a compile-time constant), 1 ... 8: the kernels that keep a row in a wave's registers.
+template <typename Fn>
+static void by_chunks(int chunks, Fn&& fn) {
+    switch (chunks) {
+        case 1: return fn(std::integral_constant<int, 1>{});
+        case 2: return fn(std::integral_constant<int, 2>{});
+        case 3: return fn(std::integral_constant<int, 3>{});
+        case 4: return fn(std::integral_constant<int, 4>{});
+        case 5: return fn(std::integral_constant<int, 5>{});
+        case 6: return fn(std::integral_constant<int, 6>{});
+        case 7: return fn(std::integral_constant<int, 7>{});
+        default: return fn(std::integral_constant<int, 8>{});
+    }
+}
+
 static bool row_shape_ok(const char* who, int rows, int K, int max_k) {
     if (rows < 0 || K <= 0 || K % 4 || K > max_k) {
         set_error("%s: need rows >= 0 and K %% 4 == 0, K <= %d (rows=%d K=%d)", who, max_k, rows, K);
@@ -754,16 +894,9 @@ int scmx_rmsnorm_quant_blocked(const uint16_t* x, const uint16_t* w, float eps, 
     if (Mp == 0) return SCMX_OK;
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid(unsigned(Mp) / 8u), block(512);
-    switch (K / 512) {
-        case 1: rmsnorm_quant_wave_kernel<1, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-        case 2: rmsnorm_quant_wave_kernel<2, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-        case 3: rmsnorm_quant_wave_kernel<3, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-        case 4: rmsnorm_quant_wave_kernel<4, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-        case 5: rmsnorm_quant_wave_kernel<5, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-        case 6: rmsnorm_quant_wave_kernel<6, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-        case 7: rmsnorm_quant_wave_kernel<7, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-        default: rmsnorm_quant_wave_kernel<8, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); break;
-    }
+    by_chunks(K / 512, [&](auto ch) {
+        rmsnorm_quant_wave_kernel<decltype(ch)::value, true><<<grid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp);
+    });
     return check_launch("rmsnorm_quant_blocked");
 }
 
@@ -775,20 +908,13 @@ int scmx_rmsnorm_quant(const uint16_t* x, const uint16_t* w, float eps, int8_t* 
     }
     if (Mp == 0) return SCMX_OK;
     hipStream_t st = (hipStream_t)stream;
-    if (K % 512 == 0 && (uintptr_t(x) | uintptr_t(w) | uintptr_t(xn)) % 16 == 0 && uintptr_t(xq) % 8 == 0) {
+    if (K % 512 == 0 && K <= 4096 && (uintptr_t(x) | uintptr_t(w) | uintptr_t(xn)) % 16 == 0 && uintptr_t(xq) % 8 == 0) {
         // rows of up to 4096 elements stay in registers (one wave per row)
-        const dim3 wgrid((unsigned(Mp) + 3u) / 4u), block(256);
-        switch (K / 512) {
-            case 1: rmsnorm_quant_wave_kernel<1><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            case 2: rmsnorm_quant_wave_kernel<2><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            case 3: rmsnorm_quant_wave_kernel<3><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            case 4: rmsnorm_quant_wave_kernel<4><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            case 5: rmsnorm_quant_wave_kernel<5><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            case 6: rmsnorm_quant_wave_kernel<6><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            case 7: rmsnorm_quant_wave_kernel<7><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            case 8: rmsnorm_quant_wave_kernel<8><<<wgrid, block, 0, st>>>(x, w, eps, xq, xs, xn, M, Mp); return check_launch("rmsnorm_quant");
-            default: break;
-        }
+        by_chunks(K / 512, [&](auto ch) {
+            rmsnorm_quant_wave_kernel<decltype(ch)::value>
+                <<<dim3((unsigned(Mp) + 3u) / 4u), dim3(256), 0, st>>>(x, w, eps, xq, xs, xn, M, Mp);
+        });
+        return check_launch("rmsnorm_quant");
     }
     rmsnorm_quant_kernel<<<dim3(Mp), dim3(NT), size_t(K) * 2 + 72 * 4, st>>>(x, w, eps, xq, xs, xn, M, K);
     return check_launch("rmsnorm_quant");
@@ -887,20 +1013,67 @@ int scmx_qkv_headnorm_rope(const int32_t* acc, const float* xscale, const float*
     return check_launch("qkv_headnorm_rope");
 }
 
-int scmx_qkv_fullnorm(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q, uint16_t* k,
-                      uint16_t* v, int L, int h, int d, void* stream) {
+static int qkv_fullnorm(const char* who, const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q,
+                        uint16_t* k, uint16_t* v, int L, int h, int d, const RopeArgs& rope, hipStream_t st) {
     if (!y || !qn || !kn || !q || !k || !v) {
-        set_error("qkv_fullnorm: null pointer argument");
+        set_error("%s: null pointer argument", who);
         return SCMX_ERR_ARG;
     }
     if (L < 0 || h < 1 || d < 4 || d % 4 || d > 16384 || h > 16384 / d) {
-        set_error("qkv_fullnorm: need L >= 0, h >= 1, d %% 4 == 0 and h * d <= 16384 (L=%d h=%d d=%d)", L, h, d);
+        set_error("%s: need L >= 0, h >= 1, d %% 4 == 0 and h * d <= 16384 (L=%d h=%d d=%d)", who, L, h, d);
         return SCMX_ERR_ARG;
     }
     if (L == 0) return SCMX_OK;
-    qkv_fullnorm_kernel<<<dim3(L), dim3(NT), size_t(h) * d * 2 + 72 * 4, (hipStream_t)stream>>>(y, qn, kn, eps, q, k, v, L,
-                                                                                                 h, d);
-    return check_launch("qkv_fullnorm");
+    const int W = h * d;
+    const bool aligned = (uintptr_t(y) | uintptr_t(qn) | uintptr_t(kn) | uintptr_t(q) | uintptr_t(k) | uintptr_t(v)) % 16 == 0;
+    if (aligned && W % 512 == 0 && W <= 4096 && d >= 16 && d <= 512 && (d & (d - 1)) == 0) {
+        auto go = [&](auto ch) {
+            qkv_fullnorm_wave_kernel<decltype(ch)::value><<<dim3(L), dim3(192), 0, st>>>(y, qn, kn, eps, q, k, v, L, d, rope);
+        };
+        by_chunks(W / 512, go);
+    } else {
+        qkv_fullnorm_kernel<<<dim3(L), dim3(NT), size_t(W) * 2 + (72 + (rope.inv_freq ? d : 0)) * 4, st>>>(
+            y, qn, kn, eps, q, k, v, L, h, d, rope);
+    }
+    return check_launch(who);
+}
+
+int scmx_qkv_fullnorm(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q, uint16_t* k,
+                      uint16_t* v, int L, int h, int d, void* stream) {
+    return qkv_fullnorm("qkv_fullnorm", y, qn, kn, eps, q, k, v, L, h, d, RopeArgs{nullptr, nullptr, 0, 0, 0},
+                        (hipStream_t)stream);
+}
+
+int scmx_qkv_fullnorm_rope(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q,
+                           uint16_t* kcache, uint16_t* vcache, int L, int h, int d, const float* inv_freq,
+                           const int64_t* pos_dev, int64_t pos0, int cache_rows, int q_token_major, void* stream) {
+    if (!inv_freq || d > 512) {
+        set_error("qkv_fullnorm_rope: null pointer argument or a head dim above 512 (d=%d)", d);
+        return SCMX_ERR_ARG;
+    }
+    if (cache_rows < L || (!pos_dev && (pos0 < 0 || pos0 > int64_t(cache_rows) - L))) {
+        set_error("qkv_fullnorm_rope: rows %lld..%lld do not fit a cache of %d rows", (long long)pos0, (long long)(pos0 + L),
+                  cache_rows);
+        return SCMX_ERR_ARG;
+    }
+    return qkv_fullnorm("qkv_fullnorm_rope", y, qn, kn, eps, q, kcache, vcache, L, h, d,
+                        RopeArgs{inv_freq, pos_dev, pos0, cache_rows, q_token_major}, (hipStream_t)stream);
+}
+
+int scmx_rmsnorm(const uint16_t* x, const uint16_t* w, float eps, uint16_t* out, int M, int K, void* stream) {
+    if (!x || !w || !out || !row_shape_ok("rmsnorm", M, K, 16384)) {
+        if (!(x && w && out)) set_error("rmsnorm: null pointer argument");
+        return SCMX_ERR_ARG;
+    }
+    if (M == 0) return SCMX_OK;
+    hipStream_t st = (hipStream_t)stream;
+    if (K % 512 == 0 && K <= 4096 && (uintptr_t(x) | uintptr_t(w) | uintptr_t(out)) % 16 == 0)
+        by_chunks(K / 512, [&](auto ch) {
+            rmsnorm_wave_kernel<decltype(ch)::value><<<dim3((unsigned(M) + 3u) / 4u), dim3(256), 0, st>>>(x, w, eps, out, M);
+        });
+    else
+        rmsnorm_kernel<<<dim3(M), dim3(NT), 0, st>>>(x, w, eps, out, K);
+    return check_launch("rmsnorm");
 }
 
 int scmx_route_topk(const uint16_t* logits, const uint16_t* shared_logit, int M, int n_experts, int topk, int renorm,

@@ -2,8 +2,9 @@
 counterpart of e2e/fused_olmoe.py:130-298 (FusedOlmoe) and e2e/decode.py:102-165 (DecodeOlmoe).
 
 Per transformer block (e2e/fused_olmoe.py:1-16):
-  y = mm_epi(xq, Wq|Wk|Wv) -> q, k, v = qkv_fullnorm_y(y)        q/k RMSNorm over the full width
-  rope, KV cache, attention                                        torch ops (MLX ops in the reference)
+  y = mm_epi(xq, Wq|Wk|Wv)
+  q = qkv_fullnorm_rope(y)                                         q/k RMSNorm over the full width, rope, KV-cache append
+  o = attn_prefill / attn_decode                                   (array ops in the reference, as rope and the cache)
   h = mm_epi(act_quant(o), Wo, + h)                                residual add in the GEMM epilogue
   xq, xs, xn = rmsnorm_quant_n(h)                                  INT8 for the experts, bf16 for the router
   router: bf16 linear (torch), softmax + top-k (+ renorm) kernel   route
@@ -20,7 +21,7 @@ from . import sc_decode as G
 from . import sc_format as F
 from . import sc_kernels as S
 from . import sc_moe
-from .fused_qwen3 import BF, KVCache, rms_norm
+from .fused_qwen3 import BF, KVCache, embed_rows
 from .sc_weights import PackedWeight
 
 # the reference keeps these two in its fused_olmoe module (e2e/fused_olmoe.py:74-97); the kernels live in sc_moe here
@@ -103,21 +104,19 @@ class FusedOlmoe:
     def make_cache(self, max_len=4096):
         return [KVCache(self.args, max_len, self.device) for _ in self.layers]
 
-    def rope(self, x, offset):
-        L = x.shape[1]
-        ang = torch.arange(offset, offset + L, device=x.device, dtype=torch.float32)[:, None] * self.inv_freq[None]
-        cos, sin = ang.cos()[None], ang.sin()[None]
-        x1, x2 = x.float().chunk(2, -1)
-        return torch.cat([x1 * cos - x2 * sin, x2 * cos + x1 * sin], -1).to(x.dtype)
-
-    def _attention(self, c, q, k, v, L):
-        off = c.offset
-        q, k = self.rope(q, off), self.rope(k, off)
-        k, v = c.update_and_fetch(k, v)
+    def _attention(self, c, nw, y, L):
+        """q/k norm, rotary embedding and cache append of the q|k|v rows y, then attention -> bf16 [L, H * d]."""
+        a, off = self.args, c.offset
+        if off + L > c.k.shape[1]:
+            raise ValueError("KV cache is full")
+        q = S.qkv_fullnorm_rope(y, nw["self_attn.q_norm"], nw["self_attn.k_norm"], self.eps, L, a.num_attention_heads,
+                                a.head_dim, c.k, c.v, off, self.inv_freq)
+        c.offset = off + L
         if L == 1:
             return S.attn_decode(q, c.k, c.v, off + 1)
-        if q.shape[-1] == 128:   # this library's causal attention (head dim 128 only; q is copied to token-major)
+        if a.head_dim == 128:   # this library's causal attention (head dim 128 only)
             return S.attn_prefill(q, c.k, c.v, off)
+        k, v = c.k[:, :off + L], c.v[:, :off + L]
         if off == 0:
             o = TF.scaled_dot_product_attention(q[None], k[None], v[None], is_causal=True)
         else:
@@ -166,18 +165,15 @@ class FusedOlmoe:
         """Final normed hidden states [L, D] for prompt ids [L]."""
         S.set_format(self.fmt)
         a = self.args
-        H, d = a.num_attention_heads, a.head_dim
         cache = cache if cache is not None else self.make_cache(max(4096, ids.numel()))
-        h = self.embed[ids.reshape(-1)]
-        L = h.shape[0]
+        L = ids.numel()
         Mp = S.pad_rows(L)
-        h = (TF.pad(h, (0, 0, 0, Mp - L)) if Mp != L else h).contiguous()
+        h = embed_rows(self.embed, ids, Mp)
         nl = len(self.layers)
         xq, xs = S.rmsnorm_quant(h, self.layers[0][0]["input_layernorm"], self.eps, Mp)
         for i, (nw, ws, ex) in enumerate(self.layers):
             y = S.mm_epi(xq, ws["qkv"].unpack(), xs, ws["qkv"].wscale, 1)
-            q, k, v = S.qkv_fullnorm_y(y, nw["self_attn.q_norm"], nw["self_attn.k_norm"], self.eps, L, H, d)
-            o = self._attention(cache[i], q, k, v, L)
+            o = self._attention(cache[i], nw, y, L)
             wo = ws["o"].unpack()   # a prefill-sized GEMM on packed weights reads its activations in 32x32 blocks
             blocked = isinstance(wo, S.PackedWq) and S.prefers_blocked(Mp, ws["o"].N, ws["o"].K)
             xq, xs = S.act_quant_blocked(o, Mp) if blocked else S.act_quant(o, Mp)
@@ -188,7 +184,7 @@ class FusedOlmoe:
                 self.record.append((inds, scores))
             nn = self.layers[i + 1][0]["input_layernorm"] if i + 1 < nl else self.norm
             h, xq, xs = self._experts(xq, xs, inds, scores, h, nn, ex, L)
-        return rms_norm(h[:L], self.norm, self.eps)
+        return S.rmsnorm(h[:L], self.norm, self.eps)
 
     def logits(self, h):
         return h @ self.lm_head.T
@@ -221,8 +217,7 @@ class DecodeOlmoe:
             else:
                 xq, xs = S.rmsnorm_quant(h, nw["input_layernorm"], f.eps, 1)
                 y = G.gemv(xq, w.codes, w.bcodes, xs, w.wscale, 3 * H * d, 1, fmt=f.fmt)
-            q, kk, v = S.qkv_fullnorm_y(y[None], nw["self_attn.q_norm"], nw["self_attn.k_norm"], f.eps, 1, H, d)
-            o = f._attention(cache[i], q, kk, v, 1)
+            o = f._attention(cache[i], nw, y[None], 1)
             wo = ws["o"]
             if self.fuse:
                 h = G.gemv(o, wo.codes, wo.bcodes, None, wo.wscale, D, 2, res=h, pro=1, fmt=f.fmt)[None]
@@ -241,5 +236,5 @@ class DecodeOlmoe:
                 xq2, xs2 = S.act_quant(act, k)
                 yd = G.gemv(xq2, cd, bd, xs2, sd, D, 1, eidx=e, xstride=1, fmt=f.fmt)
             h = sc_moe.moe_combine(yd, self.pos, scores, h, nw["post_attention_layernorm"], f.eps, 1, quant=False)[0]
-        hn = rms_norm(h, f.norm, f.eps)
+        hn = S.rmsnorm(h, f.norm, f.eps)
         return f.logits(hn) if self.head else hn

@@ -60,9 +60,14 @@ class KVCache:
         return self.k[:, :self.offset], self.v[:, :self.offset]
 
 
-def rms_norm(x, w, eps):
-    v = x.float()
-    return (v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + eps)).to(x.dtype) * w
+def embed_rows(embed, ids, Mp):
+    """The embeddings of ids [L] followed by zero rows up to Mp."""
+    ids = ids.reshape(-1).to(embed.device)
+    h = torch.empty((Mp, embed.shape[1]), dtype=embed.dtype, device=embed.device)
+    torch.index_select(embed, 0, ids, out=h[:ids.numel()])
+    if Mp > ids.numel():
+        h[ids.numel():].zero_()
+    return h
 
 
 class FusedQwen3:
@@ -142,12 +147,9 @@ class FusedQwen3:
         return o[0].transpose(0, 1).reshape(L, -1).contiguous()
 
     def _embed(self, ids):
-        h = self.embed[ids.reshape(-1)]
-        L = h.shape[0]
+        L = ids.numel()
         Mp = S.pad_rows(L)
-        if Mp != L:
-            h = TF.pad(h, (0, 0, 0, Mp - L))
-        return h.contiguous(), L, Mp
+        return embed_rows(self.embed, ids, Mp), L, Mp
 
     # ---- prefill ------------------------------------------------------------------------------------------------
     def hidden(self, ids, cache=None):
@@ -178,7 +180,7 @@ class FusedQwen3:
             h = S.mm_epi(xq, ws["down"].unpack(), xs, ws["down"].wscale, 2, res=h)
             if i + 1 < nl:
                 xq, xs = S.rmsnorm_quant(h, self.layers[i + 1][0]["input_layernorm"], self.eps, blocked=blk["qkv"])
-        return rms_norm(h[:L], self.norm, self.eps)
+        return S.rmsnorm(h[:L], self.norm, self.eps)
 
     def _hidden_row_epi(self, ids, cache):
         a = self.args
@@ -202,7 +204,7 @@ class FusedQwen3:
                                              self.eps)
             else:
                 h = S.res_epilogue(acc, xs, ws["down"].wscale, h)
-        return rms_norm(h[:L], self.norm, self.eps)
+        return S.rmsnorm(h[:L], self.norm, self.eps)
 
     def logits(self, h):
         return h @ self.lm_head.T
@@ -240,13 +242,11 @@ class DecodeQwen3:
 
     def _logits(self, h):
         f = self.f
-        hn = rms_norm(h, f.norm, f.eps)
-        if not self.head:
-            return hn
-        if self.packed_head is None:
-            return f.logits(hn)
-        codes, bc, ws, n = self.packed_head
-        return G.gemv(hn, codes, bc, None, ws, n, 1, pro=1, fmt=self.head_fmt)[None]
+        if self.head and self.packed_head is not None:   # the final norm in the GEMV's prologue
+            codes, bc, ws, n = self.packed_head
+            return G.gemv(h, codes, bc, None, ws, n, 1, pro=2, nw=f.norm, eps=f.eps, fmt=self.head_fmt)[None]
+        hn = S.rmsnorm(h, f.norm, f.eps)
+        return f.logits(hn) if self.head else hn
 
     def _pre(self, h, nw, w, c, pos):
         f = self.f

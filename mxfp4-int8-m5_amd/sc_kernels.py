@@ -216,6 +216,15 @@ def rmsnorm_quant_n(x, w, eps, Mp=None, deps=(), blocked=False):
     return _rms(x, w, eps, Mp, True, blocked)
 
 
+def rmsnorm(x, w, eps):
+    """RMSNorm of bf16 rows x [M, K] -> bf16 [M, K]."""
+    M, K = x.shape
+    assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+    out = torch.empty_like(x)
+    _lib.call("scmx_rmsnorm", _lib.ptr(x), _lib.ptr(w), _eps(eps), _lib.ptr(out), M, K, _lib.stream())
+    return out
+
+
 def prefers_blocked(M, N, K):
     """Whether a dense [M, K] x [N, K]^T problem on packed weights runs faster from blocked activations."""
     return bool(_lib.load().scmx_mm_w4a8_prefers_blocked(M, N, K))
@@ -363,3 +372,19 @@ def qkv_fullnorm_y(y, qn, kn, eps, L, h, d, deps=()):
     _lib.call("scmx_qkv_fullnorm", _lib.ptr(y), _lib.ptr(qn), _lib.ptr(kn), _eps(eps), _lib.ptr(q), _lib.ptr(k),
               _lib.ptr(v), L, h, d, _lib.stream())
     return q, k, v
+
+
+def qkv_fullnorm_rope(y, qn, kn, eps, L, h, d, kcache, vcache, pos, inv_freq):
+    """qkv_fullnorm_y fused with the rotary embedding of q and k and the KV-cache append: k and v go to rows
+    pos..pos+L-1 of kcache / vcache [h, rows, d]; returns the [h, L, d] view of q stored as [L, h, d].  pos: int, or an
+    int64 device tensor."""
+    q = torch.empty((L, h, d), dtype=torch.bfloat16, device=y.device)
+    assert kcache.shape == vcache.shape and kcache.shape[0] == h and kcache.shape[2] == d
+    assert y.dtype == torch.bfloat16 and kcache.dtype == torch.bfloat16
+    assert inv_freq.dtype == torch.float32 and inv_freq.numel() == d // 2
+    dev_pos = pos if torch.is_tensor(pos) else None
+    assert dev_pos is None or dev_pos.dtype == torch.int64
+    _lib.call("scmx_qkv_fullnorm_rope", _lib.ptr(y), _lib.ptr(qn), _lib.ptr(kn), _eps(eps), _lib.ptr(q), _lib.ptr(kcache),
+              _lib.ptr(vcache), L, h, d, _lib.ptr(inv_freq), _lib.ptr(dev_pos), 0 if dev_pos is not None else int(pos),
+              kcache.shape[1], 1, _lib.stream())
+    return q.transpose(0, 1)
