@@ -242,6 +242,12 @@ int scmx_gemv(const scmx_format* fmt, const void* x, const float* xscale, const 
               const uint16_t* nw, float eps, int batch, int N, int K, const int32_t* eidx, int n_eidx, int xstride,
               int shared_expert, void* stream);
 
+/* scmx_gemv without the expert gather for ANY number of rows from 1 to 8 (three rows run the four-row kernel, five to seven
+ * the eight-row one, without padding the operands: rows past the last are neither read nor written). */
+int scmx_gemv_rows(const scmx_format* fmt, const void* x, const float* xscale, const uint32_t* codes,
+                   const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi, int pro,
+                   const uint16_t* nw, float eps, int rows, int N, int K, void* stream);
+
 /* ---- mixture of experts ----------------------------------------------------------------------------------------- */
 
 /* Router: bf16 logits [M, n_experts] -> the topk experts of largest softmax probability per token and their scores.

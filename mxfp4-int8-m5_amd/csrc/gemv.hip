@@ -34,6 +34,7 @@ struct GemvArgs {
     const uint16_t* nw;       // pro 2: RMSNorm weight
     float eps;
     int epi, pro, N, K, bc_row_bytes;
+    int rows;                 // activation rows (<= BATCH of the kernel that runs; those beyond are neither read nor written)
     const int32_t* eidx;      // MoE: expert of each slot
     int n_eidx, xstride, shared_expert;
     DevFormat fmt;
@@ -605,6 +606,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a) {
                 constexpr int LOG = NV == 1 ? 0 : NV == 2 ? 1 : NV == 4 ? 2 : NV == 8 ? 3 : NV == 16 ? 4 : NV == 32 ? 5 : 6;
                 const int idx = LOG == 0 ? 0 : int(__builtin_bitreverse32(uint32_t(lane)) >> (32 - (LOG == 0 ? 1 : LOG)));
                 const int r = idx / BATCH, b = idx % BATCH;
+                if (BATCH > 1 && b >= a.rows) return;
                 const float y = __fmul_rn(__fmul_rn(float(tot), sxs[b]), a.wscale[erow + n0 + r]);
                 const size_t o = size_t(orow0 + b) * N + n0 + r;
                 if (a.epi == SCMX_EPI_SCALE)
@@ -623,6 +625,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a) {
             for (int r = 0; r < R; ++r) wsr[r] = a.wscale[erow + n0 + r];
 #pragma unroll
             for (int b = 0; b < BATCH; ++b) {
+                if (BATCH > 1 && b >= a.rows) break;
                 const float xsb = sxs[b];
                 const size_t orow = size_t(orow0 + b);
                 float y[R];
@@ -688,6 +691,10 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a) {
 
 #pragma unroll
     for (int b = 0; b < BATCH; ++b) {
+        if (BATCH > 1 && b >= a.rows) {   // its products are dropped: any finite values do
+            for (int c = tid; c < Kp * XB / 4; c += NT) reinterpret_cast<uint32_t*>(sx + size_t(b) * Kp * XB)[c] = 0u;
+            continue;
+        }
         const float s = stage_row<NT, FP4 ? X_HALF : X_PERM8, KEEP>(a, xrow0 + b, sx + size_t(b) * Kp * XB, red, xpre, have_pre && b == 0);
         for (int c = K * XB / 4 + tid; c < Kp * XB / 4; c += NT) reinterpret_cast<uint32_t*>(sx + size_t(b) * Kp * XB)[c] = 0u;
         if (tid == 0) sxs[b] = s;
@@ -799,7 +806,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(const GemvArgs a) {
         const int tot = select_reduce<NV, 4>(vals, lane);
         const int brow = NSET == 1 ? 2 * (blk & 1) + ((blk >> 1) & 1)
                                    : 4 * (blk & 1) + 2 * ((blk >> 1) & 1) + ((blk >> 2) & 1);
-        const bool emit = brow < BATCH && (blk >> (NSET == 1 ? 2 : 3)) == 0;   // one of the lanes that hold this total
+        const bool emit = brow < a.rows && (blk >> (NSET == 1 ? 2 : 3)) == 0;   // one of the lanes that hold this total
         const int n = g * 4 + j;
         float y = 0.0f;
         if (emit) y = __fmul_rn(__fmul_rn(float(tot), sxs[brow]), a.wscale[n]);
@@ -833,7 +840,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(const GemvArgs a) {
     const WavePre<1> xpre = {};   // (no early request here: the extra registers would cost this kernel a wave of occupancy)
 
     for (int b = wave; b < XR; b += NT / 64) {   // a wave per activation row, side by side (rows beyond the batch are zero)
-        if (b < BATCH) {
+        if (b < a.rows) {
             const float s = stage_row_wave<X_PLAIN8>(a, b, sx + size_t(b) * Kp, xpre, false);
             for (int c = K / 4 + lane; c < Kp / 4; c += 64) reinterpret_cast<uint32_t*>(sx + size_t(b) * Kp)[c] = 0u;
             if (lane == 0) sxs[b] = s;
@@ -883,10 +890,17 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 // SPLIT (narrow layers): one row group per workgroup, the waves take the 512-wide pieces of K in turn (wave, wave + 4, ...)
 // and their INT32 partial totals meet in LDS: the layer's few rows are spread over 4 x N / 16 waves with one or a few
 // pieces each instead of N / 16 waves walking all of K.
-// E8: a standard MXFP4 tensor in place -- the piece's 16 blocks bring 16 E8M0 bytes per row instead of 4 code bytes.
-template <int BATCH, int POL, bool SPLIT, int WAVE_PRE, bool E8 = false>
-__global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma_kernel(const GemvArgs a) {
+// FMT: the published format; a standard MXFP4 tensor in place (the piece's 16 blocks bring 16 E8M0 bytes per row instead of
+// 4 code bytes); the codebook and shifts on 16-element blocks (8 code bytes, a scale per two code words); that codebook on
+// 16-element blocks with 4-bit codes for consecutive integer multipliers (16 bytes; the multiplier is applied to the
+// converted half-precision pairs, whose products stay integers up to 127).
+enum { H_SC = 0, H_E8 = 1, H_B16 = 2, H_B16M = 3 };
+template <int BATCH, int POL, bool SPLIT, int WAVE_PRE, int FMT = H_SC>
+__global__ __launch_bounds__(256, (FMT != H_SC && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma_kernel(const GemvArgs a) {
     constexpr int NT = 256;
+    constexpr bool E8 = FMT == H_E8, B16M = FMT == H_B16M;
+    constexpr bool BYTES = E8 || B16M;        // one scale byte per 32 weights
+    constexpr bool OWN4 = FMT != H_SC;        // which blocks a lane group multiplies, below
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     const int K = a.K, N = a.N;
     const int Kp = (K + 511) & ~511;                  // whole pieces of 512, zero padded
@@ -905,12 +919,12 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
     const int groups = N / 16;
     const int CI = Kp / 512;                           // pieces per row group
     const int g_stride = gridDim.x * (NT / 64);
-    const int brow = r < BATCH ? r : 0;                // the batch row this lane's MFMA column reads
-    // E8, wide layers (E8T; at least 3 pieces per row group): a row group's exponent bytes, 16 rows x K / 32, are at most
+    const int brow = r < a.rows ? r : 0;               // the batch row this lane's MFMA column reads
+    // BYTES, wide layers (E8T; at least 3 pieces per row group): a row group's scale bytes, 16 rows x K / 32, are at most
     // 1 KiB -- ONE wave-wide 16-byte load per row group instead of a strided 4-byte load per piece (whose 16 cache lines per
     // instruction cost the batch-4 output head a quarter of its rate).  They wait in registers (`e8n`) until the group's
     // first piece is multiplied, then sit in a wave-private LDS tile of 16 rows x 80 bytes (conflict-free 4-byte reads).
-    constexpr bool E8T = E8 && !SPLIT;
+    constexpr bool E8T = BYTES && !SPLIT;
     constexpr int EPITCH = 80;
     int8_t* e8tile = reinterpret_cast<int8_t*>(sxs + ((BATCH + 3) & ~3)) + size_t(NT / 64) * 16 * WPITCH + size_t(wave) * 16 * EPITCH;
     [[maybe_unused]] u32x4 e8n = u32x4{0u, 0u, 0u, 0u};
@@ -919,7 +933,8 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
     struct Item {
         u32x4 w[4];     // loads i = 0..3 of the piece: the 32-weight block 4 i + c of row r
         uint32_t bc;    // the piece's four block-code bytes of row r (byte i: blocks 4 i .. 4 i + 3)
-        uint32_t rmin;  // E8: the row's lowest exponent byte (bc then holds the exponent bytes of blocks 4 c .. 4 c + 3)
+        uint32_t rmin;  // E8: the row's lowest exponent byte
+                        // (OWN4: bc holds the bytes of the 32-weight runs 4 c .. 4 c + 3)
     };
     const auto load_item = [&](Item& it, int g, int ci) {
         const uint8_t* crow = reinterpret_cast<const uint8_t*>(a.codes) + size_t(g) * 16 * (K / 2);   // uniform
@@ -934,11 +949,13 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
         if constexpr (E8T) {
             if (ci == 0) {   // the first piece of a row group brings the group's exponent bytes and lowest exponents
                 e8n = __builtin_amdgcn_raw_buffer_load_b128(rb, r * a.bc_row_bytes + 16 * c, 0, 0);
-                rmin_next = e8m0_row_min(a.wscale[size_t(g) * 16 + r]);
+                if (E8) rmin_next = e8m0_row_min(a.wscale[size_t(g) * 16 + r]);
             }
-        } else if constexpr (E8) {
+        } else if constexpr (BYTES) {
             it.bc = __builtin_amdgcn_raw_buffer_load_b32(rb, r * a.bc_row_bytes + 4 * c, ci * 16, 0);
-            it.rmin = e8m0_row_min(a.wscale[size_t(g) * 16 + r]);
+            if (E8) it.rmin = e8m0_row_min(a.wscale[size_t(g) * 16 + r]);
+        } else if constexpr (FMT == H_B16) {
+            it.bc = __builtin_amdgcn_raw_buffer_load_b16(rb, r * a.bc_row_bytes + 2 * c, ci * 8, 0);
         } else {
             it.bc = __builtin_amdgcn_raw_buffer_load_b32(rb, r * a.bc_row_bytes, ci * 4, 0);
         }
@@ -951,15 +968,16 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
         acc0 = acc1 = f4{0.0f, 0.0f, 0.0f, 0.0f};
     };
     // Which of the piece's 16 blocks a lane multiplies is free (the MFMA sums over the four lane groups): group c takes
-    // blocks 4 i + c, or with E8M0 bytes blocks 4 c + i, whose four exponent bytes are one aligned 4-byte load.
+    // blocks 4 i + c, or (OWN4) runs 4 c + i of 32 weights, whose scale bytes are one aligned load.
+    const int m0 = int(a.fmt.mult[0] & 0xFFu);
     const auto compute_item = [&](const Item& it, int ci) {
-        const int8_t* xrow = sx + size_t(brow) * pitch + (size_t(ci) * 512 + (E8 ? 128 : 32) * c) * 2;
+        const int8_t* xrow = sx + size_t(brow) * pitch + (size_t(ci) * 512 + (OWN4 ? 128 : 32) * c) * 2;
 #pragma unroll
         for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(slot + (4 * i + c) * WPITCH + 16 * r) = it.w[i];
-        u32x4 wt[4];   // row r, blocks 4 i + c (E8: 4 c + i): bytes 64 i + 16 c (64 c + 16 i) of the row's 256
+        u32x4 wt[4];   // row r, blocks 4 i + c (OWN4: 4 c + i): bytes 64 i + 16 c (64 c + 16 i) of the row's 256
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            wt[i] = *reinterpret_cast<const u32x4*>(slot + r * WPITCH + (E8 ? 64 * c + 16 * i : 64 * i + 16 * c));
+            wt[i] = *reinterpret_cast<const u32x4*>(slot + r * WPITCH + (OWN4 ? 64 * c + 16 * i : 64 * i + 16 * c));
         uint32_t ebytes = it.bc, elow = it.rmin;
         if constexpr (E8T) {
             if (ci == 0) {
@@ -971,17 +989,40 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float scale = E8 ? fp4_scale((((ebytes >> (8 * i)) & 0xFFu) - elow) & 0x7Fu)
-                                   : fp4_scale((it.bc >> (8 * i + 2 * c)) & 3u);
+            float scale[2];   // of code words 0-1 and 2-3
+            h2 mul[2];        // B16M: their multipliers
+            if (E8) {
+                scale[0] = scale[1] = fp4_scale((((ebytes >> (8 * i)) & 0xFFu) - elow) & 0x7Fu);
+            } else if (FMT == H_SC) {
+                scale[0] = scale[1] = fp4_scale((it.bc >> (8 * i + 2 * c)) & 3u);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    if (B16M) {
+                        const _Float16 m = _Float16(float(m0 + int((ebytes >> (8 * i + 4 * t)) & 15u)));
+                        mul[t] = h2{m, m};
+                        scale[t] = 2.0f;
+                    } else {
+                        scale[t] = fp4_scale((it.bc >> (4 * i + 2 * t)) & 3u);
+                    }
+                }
+            }
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
                 const uint32_t w = wt[i][d];
-                const h2 q0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 0);
-                const h2 q1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 1);
-                const h2 q2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 2);
-                const h2 q3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 3);
+                const float sc = scale[d >> 1];
+                h2 q0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, sc, 0);
+                h2 q1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, sc, 1);
+                h2 q2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, sc, 2);
+                h2 q3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, sc, 3);
+                if (B16M) {
+                    q0 *= mul[d >> 1];
+                    q1 *= mul[d >> 1];
+                    q2 *= mul[d >> 1];
+                    q3 *= mul[d >> 1];
+                }
                 const h8 wv = h8{q0[0], q0[1], q1[0], q1[1], q2[0], q2[1], q3[0], q3[1]};
-                const h8 xv = *reinterpret_cast<const h8*>(xrow + ((E8 ? 32 : 128) * i + 8 * d) * 2);
+                const h8 xv = *reinterpret_cast<const h8*>(xrow + ((OWN4 ? 32 : 128) * i + 8 * d) * 2);
                 if (d & 1) acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv, acc1, 0, 0, 0);
                 else acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv, acc0, 0, 0, 0);
             }
@@ -989,7 +1030,7 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
         flush();   // 8 MFMAs per chain and piece: far below the 43 that keep a chain exact
     };
     const auto finish = [&](int g) {
-        if (r >= BATCH) return;
+        if (r >= a.rows) return;
         const int n = g * 16 + 4 * c;
         const f4 ws = *reinterpret_cast<const f4*>(a.wscale + n);
         const float xs = sxs[r];
@@ -1039,7 +1080,7 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
     constexpr int RPW = BATCH > 4 ? 2 : 1;   // activation rows per wave
     WavePre<WAVE_PRE> xpre[RPW];
 #pragma unroll
-    for (int j = 0; j < RPW; ++j) wave_prefetch_row(a, wave + 4 * j, wave + 4 * j < BATCH, xpre[j]);
+    for (int j = 0; j < RPW; ++j) wave_prefetch_row(a, wave + 4 * j, wave + 4 * j < a.rows, xpre[j]);
     const bool have_pre = a.pro == 1 && a.K <= 512 * WAVE_PRE;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -1048,7 +1089,7 @@ __global__ __launch_bounds__(256, (E8 && WAVE_PRE <= 4) ? 4 : 1) void gemv_hmfma
 #pragma unroll
     for (int j = 0; j < RPW; ++j) {   // a wave per row, side by side
         const int b = wave + 4 * j;
-        if (b >= BATCH) break;
+        if (b >= a.rows) break;
         const float s = stage_row_wave<X_HALF>(a, b, sx + size_t(b) * pitch, xpre[j], have_pre);
         for (int i = K / 2 + lane; i < Kp / 2; i += 64) reinterpret_cast<uint32_t*>(sx + size_t(b) * pitch)[i] = 0u;
         if (lane == 0) sxs[b] = s;
@@ -1148,44 +1189,50 @@ static void launch_gemv_mfma(const GemvArgs& a, hipStream_t s) {
     gemv_mfma_kernel<BATCH><<<grid, block, smem, s>>>(a);
 }
 
-template <int BATCH, bool E8 = false>
+template <int BATCH, int FMT>
 static void launch_gemv_hmfma(const GemvArgs& a, bool split, hipStream_t s) {
     const int groups = a.N / 16;
     const int want = (groups + 3) / 4;
     const int rounds = (want + 1535) / 1536;   // 6 waves per SIMD are resident
     const dim3 grid(split ? groups : (want + rounds - 1) / rounds), block(256);
     const size_t smem = size_t(BATCH) * (((a.K + 511) & ~511) * 2 + 16) + (68 + ((BATCH + 3) & ~3)) * sizeof(float) + 4 * 16 * 272 +
-                        (E8 ? 4 * 16 * 80 : 0);
+                        (FMT == H_E8 || FMT == H_B16M ? 4 * 16 * 80 : 0);
     auto go = [&](auto kernel) {
         if (smem > 64 * 1024)
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
         kernel<<<grid, block, smem, s>>>(a);
     };
     // the early request of the activation rows holds K / 512 chunks per lane: 4 for K <= 2048, 12 up to 6144
-    if (!split) go(gemv_hmfma_kernel<BATCH, W_STREAM, false, 4, E8>);
-    else if (a.K <= 2048) go(gemv_hmfma_kernel<BATCH, W_STREAM, true, 4, E8>);
-    else go(gemv_hmfma_kernel<BATCH, W_STREAM, true, 12, E8>);
+    if (!split) go(gemv_hmfma_kernel<BATCH, W_STREAM, false, 4, FMT>);
+    else if (a.K <= 2048) go(gemv_hmfma_kernel<BATCH, W_STREAM, true, 4, FMT>);
+    else go(gemv_hmfma_kernel<BATCH, W_STREAM, true, 12, FMT>);
 }
 
 template <int BATCH>
 static void launch_gemv_rows(const GemvArgs& a, int slots, int dflt, hipStream_t s) {
-    // wide layers in the published format: half-precision MFMA dot products (whole row groups of 16, pieces of 512)
-    // (several activation rows, K up to 2048: beyond that its half-precision activations cost too much LDS)
-    if (BATCH > 1 && dflt == 4 && !a.eidx && a.N % 16 == 0 && a.K % 512 == 0 && a.K <= 8192 && size_t(BATCH) * a.K <= 32768 &&
-        uintptr_t(a.bcodes) % 4 == 0) {   // the same two kernels reading E8M0 bytes (4 per lane and piece, one aligned load)
-        // wide layers: the form that loads a row group's exponent bytes at once needs 3 pieces per group (K >= 1536)
-        if (a.N >= HMFMA_MIN_ROWS && a.K <= 2048 && a.K >= 1536) return launch_gemv_hmfma<BATCH, true>(a, false, s);
-        return launch_gemv_hmfma<BATCH, true>(a, true, s);
-    }
-    // (both half-precision MFMA kernels read a row's block codes of a piece with one 4-byte load: aligned codes only)
+    // Several activation rows, whole row groups of 16 and pieces of 512: half-precision MFMA dot products, for every format
+    // the FP4 conversion decodes (all of them read a row's block codes of a piece with one load of up to 4 bytes: aligned
+    // codes only).  Wide layers walk row groups; the byte-scaled forms then need 3 pieces per group (K >= 1536), and beyond
+    // K = 2048 the half-precision activations cost too much LDS.  Narrow layers split K over the waves of a workgroup.
+    // (Batch 1 measured no faster this way than with the per-row kernels: qkv 4.70 against 4.40 us, down 7.32 against 6.34.
+    // The 16-block forms gain most, they ran with table decode: four rows, e2m1/B16/M1..10: output head
+    // 116 -> 35 us, 12288 x 2048 with SwiGLU 17.4 -> 8.0, 2048 x 6144 16.1 -> 8.4.)
     const bool bc4 = uintptr_t(a.bcodes) % 4 == 0;
-    if (BATCH > 1 && dflt == 1 && bc4 && !a.eidx && a.N % 16 == 0 && a.K % 512 == 0 && a.K <= 2048 && a.N >= HMFMA_MIN_ROWS)
-        return launch_gemv_hmfma<BATCH>(a, false, s);
-    // narrow layers with several activation rows: the same kernel with K split over the waves of a workgroup
-    // (batch 1 measured no faster this way than with the per-row kernels: qkv 4.70 against 4.40 us, down 7.32 against 6.34)
-    if (BATCH > 1 && dflt == 1 && bc4 && !a.eidx && a.N % 16 == 0 && a.K % 512 == 0 && a.K <= 8192 && a.N < HMFMA_MIN_ROWS &&
-        size_t(BATCH) * a.K <= 32768)
-        return launch_gemv_hmfma<BATCH>(a, true, s);
+    if constexpr (BATCH > 1) {
+        if (dflt && bc4 && !a.eidx && a.N % 16 == 0 && a.K % 512 == 0 && a.K <= 8192) {
+            const bool bytes = dflt == 4 || dflt == 3;
+            const bool wide = a.N >= HMFMA_MIN_ROWS && a.K <= 2048 && (!bytes || a.K >= 1536);
+            const bool narrow = (a.N < HMFMA_MIN_ROWS || bytes) && size_t(BATCH) * a.K <= 32768;
+            if (wide || narrow) {
+                switch (dflt) {
+                    case 1: return launch_gemv_hmfma<BATCH, H_SC>(a, !wide, s);
+                    case 2: return launch_gemv_hmfma<BATCH, H_B16>(a, !wide, s);
+                    case 3: return launch_gemv_hmfma<BATCH, H_B16M>(a, !wide, s);
+                    default: return launch_gemv_hmfma<BATCH, H_E8>(a, !wide, s);
+                }
+            }
+        }
+    }
     if (BATCH > 1 && dflt == 1 && bc4 && !a.eidx && a.N % 4 == 0 && a.K % 512 == 0)
         return launch_gemv_mfma<BATCH>(a, s);
     // more rows per wave = more loads in flight per lane; fewer = more waves for narrow layers
@@ -1201,10 +1248,10 @@ static void launch_gemv_rows(const GemvArgs& a, int slots, int dflt, hipStream_t
 
 using namespace scmx;
 
-extern "C" int scmx_gemv(const scmx_format* fmt, const void* x, const float* xscale, const uint32_t* codes,
-                         const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi,
-                         int pro, const uint16_t* nw, float eps, int batch, int N, int K, const int32_t* eidx,
-                         int n_eidx, int xstride, int shared_expert, void* stream) {
+static int gemv_any(const scmx_format* fmt, const void* x, const float* xscale, const uint32_t* codes,
+                    const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi,
+                    int pro, const uint16_t* nw, float eps, int batch, int N, int K, const int32_t* eidx,
+                    int n_eidx, int xstride, int shared_expert, void* stream) {
     DevFormat f;
     if (int rc = make_dev_format(fmt, &f)) return rc;
     if (!x || !codes || !bcodes || !wscale || !out || (pro == 0 && !xscale) || (pro == 2 && !nw) ||
@@ -1238,15 +1285,17 @@ extern "C" int scmx_gemv(const scmx_format* fmt, const void* x, const float* xsc
         slots = n_eidx + (shared_expert >= 0 ? 1 : 0);
         if (slots == 0) return SCMX_OK;
     }
-    if (!(batch == 1 || batch == 2 || batch == 4 || batch == 8)) {
-        set_error("gemv: batch %d not in {1,2,4,8}", batch);
+    if (batch < 1 || batch > 8) {
+        set_error("gemv: %d rows outside 1..8", batch);
         return SCMX_ERR_ARG;
     }
-    if (size_t(batch) * ((K + 2047) & ~2047) * 2 + 80 * sizeof(float) > 160 * 1024) {
+    const int kernel_rows = batch <= 2 ? batch : batch <= 4 ? 4 : 8;   // rows of the kernel that runs
+    if (size_t(kernel_rows) * ((K + 2047) & ~2047) * 2 + 80 * sizeof(float) > 160 * 1024) {
         set_error("gemv: batch * K = %zu activations exceed what one workgroup can stage (80 Ki)", size_t(batch) * K);
         return SCMX_ERR_ARG;
     }
     GemvArgs a = {};
+    a.rows = batch;
     a.x = x; a.xscale = xscale; a.codes = codes; a.bcodes = bcodes; a.wscale = wscale; a.res = res; a.out = out;
     a.nw = nw; a.eps = eps; a.epi = epi; a.pro = pro; a.N = N; a.K = K;
     a.bc_row_bytes = K / f.block * f.bc_bits / 8;
@@ -1258,11 +1307,29 @@ extern "C" int scmx_gemv(const scmx_format* fmt, const void* x, const float* xsc
                      : is_block16_range_format(f) ? 3
                                                   : 0;
     hipStream_t s = (hipStream_t)stream;
-    switch (batch) {
+    switch (kernel_rows) {
         case 1: launch_gemv_rows<1>(a, slots, dflt, s); break;
         case 2: launch_gemv_rows<2>(a, slots, dflt, s); break;
         case 4: launch_gemv_rows<4>(a, slots, dflt, s); break;
         default: launch_gemv_rows<8>(a, slots, dflt, s); break;
     }
     return check_launch("gemv");
+}
+
+extern "C" int scmx_gemv(const scmx_format* fmt, const void* x, const float* xscale, const uint32_t* codes,
+                         const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi,
+                         int pro, const uint16_t* nw, float eps, int batch, int N, int K, const int32_t* eidx,
+                         int n_eidx, int xstride, int shared_expert, void* stream) {
+    if (!(batch == 1 || batch == 2 || batch == 4 || batch == 8)) {
+        set_error("gemv: batch %d not in {1,2,4,8}", batch);
+        return SCMX_ERR_ARG;
+    }
+    return gemv_any(fmt, x, xscale, codes, bcodes, wscale, res, out, epi, pro, nw, eps, batch, N, K, eidx, n_eidx, xstride,
+                    shared_expert, stream);
+}
+
+extern "C" int scmx_gemv_rows(const scmx_format* fmt, const void* x, const float* xscale, const uint32_t* codes,
+                              const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi,
+                              int pro, const uint16_t* nw, float eps, int rows, int N, int K, void* stream) {
+    return gemv_any(fmt, x, xscale, codes, bcodes, wscale, res, out, epi, pro, nw, eps, rows, N, K, nullptr, 0, 0, -1, stream);
 }
