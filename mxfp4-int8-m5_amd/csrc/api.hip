@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "scmx_common.h"
 
@@ -151,6 +152,27 @@ __global__ __launch_bounds__(256) void unpack_i8_word_kernel(DevFormat f, const 
     wq[i] = u32x2{a, b};
 }
 
+// The largest magnitude of eight bf16 values and m; their INT8 codes.
+__device__ __forceinline__ float amax8(const u32x4& v, float m) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        m = fmaxf(m, fabsf(__uint_as_float(v[e] << 16)));
+        m = fmaxf(m, fabsf(__uint_as_float(v[e] & 0xFFFF0000u)));
+    }
+    return m;
+}
+__device__ __forceinline__ u32x2 codes8(const u32x4& v, float qi) {
+    uint32_t o[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int q0 = quant_code(__uint_as_float(v[e] << 16), qi);
+        const int q1 = quant_code(__uint_as_float(v[e] & 0xFFFF0000u), qi);
+        o[e >> 1] |= (uint32_t(q0) & 0xFFu) << (16 * (e & 1));
+        o[e >> 1] |= (uint32_t(q1) & 0xFFu) << (16 * (e & 1) + 8);
+    }
+    return u32x2{o[0], o[1]};
+}
+
 // ---- act_quant: one workgroup per token row ---------------------------------------------------------------------
 // Lanes read 8 bf16 (16 bytes) per step; the row maximum goes through LDS; the second sweep re-reads the row
 // (cache hit) and writes 8 codes per lane.
@@ -167,12 +189,7 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
     const u32x4* xrow = reinterpret_cast<const u32x4*>(x + size_t(row) * K);
     float amax = 0.0f;
     for (int c = tid; c < K / 8; c += 256) {
-        const u32x4 v = xrow[c];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            amax = fmaxf(amax, fabsf(__uint_as_float(v[j] << 16)));
-            amax = fmaxf(amax, fabsf(__uint_as_float(v[j] & 0xFFFF0000u)));
-        }
+        amax = amax8(xrow[c], amax);
     }
     amax = wave_max(amax);
     if ((tid & 63) == 0) red[tid >> 6] = amax;
@@ -181,94 +198,89 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
     const float s = __fdiv_rn(amax, 127.0f);
     const float qi = s > 0.0f ? __fdiv_rn(1.0f, s) : 0.0f;
     for (int c = tid; c < K / 8; c += 256) {
-        const u32x4 v = xrow[c];
-        uint32_t o[2] = {0u, 0u};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int q0 = quant_code(__uint_as_float(v[j] << 16), qi);
-            const int q1 = quant_code(__uint_as_float(v[j] & 0xFFFF0000u), qi);
-            o[j >> 1] |= (uint32_t(q0) & 0xFFu) << (16 * (j & 1));
-            o[j >> 1] |= (uint32_t(q1) & 0xFFu) << (16 * (j & 1) + 8);
-        }
-        qrow[c] = u32x2{o[0], o[1]};
+        qrow[c] = codes8(xrow[c], qi);
     }
     if (tid == 0) xs[row] = s;
 }
 
-// The same with the row held in registers: one wave per row, lane l owns the 16-byte pieces l, l + 64, ... (CH of
-// them, K = 512 * CH), so the row is read once and the only reduction is inside the wave.  Four rows per workgroup.
+// The same with the row held in registers: one wave per row, lane l owns the 16-byte pieces l, l + 64, ... (up to CH of
+// them, K <= 512 * CH, K % 32 == 0), so the row is read once and the only reduction is inside the wave.  Four rows per
+// workgroup.
 // BLK: xq leaves in the blocked layout of the dense GEMM's large tiles (32 x 32 blocks in MFMA operand order, described at
 // act_quant_blocked_kernel below; Mp % 32 == 0): eight rows per workgroup, whose codes meet in LDS -- the 16 bytes of row
 // r, k 16 c ... at slot c * 8 + (r + c / 2) % 8 -- and are stored as whole 128-byte lines (8 rows x 16 bytes are adjacent
 // in a block).  The loads stay what they are by rows: 16 contiguous bytes per lane.
-template <int CH, bool BLK = false>
-__global__ __launch_bounds__(BLK ? 512 : 256) void act_quant_wave_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
-                                                                         float* __restrict__ xs, int M, int Mp) {
-    constexpr int K = 512 * CH, RPW = BLK ? 8 : 4;
-    __shared__ u32x2 tile[BLK ? CH * 64 * 8 : 1];
+// (Registers are held to what lets four waves share a SIMD up to 6144 values, three up to 8192: 4000 rows x 6144 blocked 16.6
+// us at three, 13.0 at four.)
+template <int CH, bool BLK, bool WHOLE>
+__global__ __launch_bounds__(BLK ? 512 : 256, CH <= 12 ? 4 : CH <= 16 ? 3 : 1) void act_quant_wave_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
+                                                                         float* __restrict__ xs, int M, int Mp, int K_any) {
+    const int K = WHOLE ? 512 * CH : K_any;   // WHOLE: every lane has all of its CH pieces
+    constexpr int RPW = BLK ? 8 : 4;
+    constexpr int TURN = CH > 16 ? CH / 2 : CH;   // pieces whose codes are in LDS at once (at most 64 KB)
+    __shared__ u32x2 tile[BLK ? TURN * 64 * 8 : 1];
     const int wid = threadIdx.x >> 6, row0 = blockIdx.x * RPW, row = row0 + wid, lane = threadIdx.x & 63;
-    auto gather_store = [&]() {   // BLK: after every wave's codes are in LDS
+    auto gather_store = [&](int j0) {   // BLK: the codes of pieces j0 .. j0 + TURN - 1 of every row, after all are in LDS
         __syncthreads();
         int8_t* const blk = xq + (size_t(row0 >> 5) * size_t(K >> 5)) * 1024;
         const u32x4* t16 = reinterpret_cast<const u32x4*>(tile);
 #pragma unroll
-        for (int j = 0; j < CH / 2 + CH % 2; ++j) {   // K / 16 pieces x 8 rows of 16 bytes, 512 per pass
-            const int idx = int(threadIdx.x) + 512 * j, c = idx >> 3, r = idx & 7;
-            if (CH % 2 == 0 || c < K / 16)
+        for (int j = 0; j < TURN / 2 + TURN % 2; ++j) {   // 32 TURN chunks of 16 k x 8 rows, 512 per pass
+            const int idx = int(threadIdx.x) + 512 * j, cl = idx >> 3, r = idx & 7, c = cl + 32 * j0;
+            if ((WHOLE && TURN % 2 == 0) || (cl < 32 * TURN && c < K / 16))
                 *reinterpret_cast<u32x4*>(blk + size_t(c >> 1) * 1024 + (c & 1) * 512 + ((row0 + r) & 31) * 16) =
-                    t16[c * 8 + ((r + (c >> 1)) & 7)];
+                    t16[cl * 8 + ((r + (cl >> 1)) & 7)];
         }
+        if (TURN < CH) __syncthreads();
     };
-    // piece p (8 codes) of this wave's row: half p % 2 of the 16-byte slot of chunk p / 2
+    // piece p (8 codes, counted from the turn's first) of this wave's row: half p % 2 of the 16-byte slot of chunk p / 2
     auto slot = [&](int p) { return ((p >> 1) * 8 + ((wid + (p >> 2)) & 7)) * 2 + (p & 1); };
+    auto mine = [&](int j) { return WHOLE || lane + 64 * j < K / 8; };
     if (!BLK && row >= Mp) return;
     u32x2* qrow = reinterpret_cast<u32x2*>(xq + size_t(row) * K);
     if (row >= M) {
 #pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            if (BLK) tile[slot(lane + 64 * j)] = u32x2{0u, 0u}; else qrow[lane + 64 * j] = u32x2{0u, 0u};
+        for (int j0 = 0; j0 < CH; j0 += TURN) {
+#pragma unroll
+            for (int j = j0; j < j0 + TURN; ++j)
+                if (mine(j)) {
+                    if (BLK) tile[slot(lane + 64 * (j - j0))] = u32x2{0u, 0u}; else qrow[lane + 64 * j] = u32x2{0u, 0u};
+                }
+            if (BLK) gather_store(j0);
         }
         if (lane == 0) xs[row] = 0.0f;
-        if (BLK) gather_store();
         return;
     }
     const u32x4* xrow = reinterpret_cast<const u32x4*>(x + size_t(row) * K);
     u32x4 v[CH];
 #pragma unroll
-    for (int j = 0; j < CH; ++j) v[j] = xrow[lane + 64 * j];
+    for (int j = 0; j < CH; ++j) v[j] = mine(j) ? xrow[lane + 64 * j] : u32x4{0u, 0u, 0u, 0u};
     float amax = 0.0f;
 #pragma unroll
-    for (int j = 0; j < CH; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            amax = fmaxf(amax, fabsf(__uint_as_float(v[j][e] << 16)));
-            amax = fmaxf(amax, fabsf(__uint_as_float(v[j][e] & 0xFFFF0000u)));
-        }
+    for (int j = 0; j < CH; ++j) amax = amax8(v[j], amax);
     amax = wave_max(amax);
     const float s = __fdiv_rn(amax, 127.0f);
     const float qi = s > 0.0f ? __fdiv_rn(1.0f, s) : 0.0f;
 #pragma unroll
-    for (int j = 0; j < CH; ++j) {
-        uint32_t o[2] = {0u, 0u};
+    for (int j0 = 0; j0 < CH; j0 += TURN) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int q0 = quant_code(__uint_as_float(v[j][e] << 16), qi);
-            const int q1 = quant_code(__uint_as_float(v[j][e] & 0xFFFF0000u), qi);
-            o[e >> 1] |= (uint32_t(q0) & 0xFFu) << (16 * (e & 1));
-            o[e >> 1] |= (uint32_t(q1) & 0xFFu) << (16 * (e & 1) + 8);
+        for (int j = j0; j < j0 + TURN; ++j) {
+            const u32x2 o = codes8(v[j], qi);
+            if (mine(j)) {
+                if (BLK) tile[slot(lane + 64 * (j - j0))] = o; else qrow[lane + 64 * j] = o;
+            }
         }
-        if (BLK) tile[slot(lane + 64 * j)] = u32x2{o[0], o[1]}; else qrow[lane + 64 * j] = u32x2{o[0], o[1]};
+        if (BLK) gather_store(j0);
     }
     if (lane == 0) xs[row] = s;
-    if (BLK) gather_store();
 }
 
 // ---- act_quant into the blocked layout ---------------------------------------------------------------------------
 // xq as the large dense GEMM tiles take it: blocks of 32 rows x 32 k (1 KB), block (m / 32, k / 32) at
 // ((m / 32) * (K / 32) + k / 32) KB, and inside a block the 16 bytes of row r, k half h at (32 h + r) * 16 -- the order
 // in which the 64 lanes of a wave hold a 32x32x32 MFMA operand, so that a wave fetches one block with one coalesced load.
-// Rows of K = 512 ... 8192 in steps of 512 go through act_quant_wave_kernel<CH, true> above; this is the kernel for every
-// other K % 32 == 0: one wave per row, eight rows per workgroup, the row read twice, every lane writing the 16 bytes of
+// Rows of K <= 12288 go through act_quant_wave_kernel above, few rows through act_quant_row_kernel below; this is the kernel
+// for longer rows: one wave per row, eight rows per workgroup, the row read twice, every lane writing the 16 bytes of
 // its own 16 elements.  Same codes and scales as act_quant_kernel: the row maximum does not depend on the order it is
 // taken in.
 __global__ __launch_bounds__(512) void act_quant_blocked_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
@@ -283,25 +295,6 @@ __global__ __launch_bounds__(512) void act_quant_blocked_kernel(const uint16_t* 
         if (lane == 0) xs[row] = 0.0f;
         return;
     }
-    auto amax8 = [](const u32x4& v, float m) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            m = fmaxf(m, fabsf(__uint_as_float(v[e] << 16)));
-            m = fmaxf(m, fabsf(__uint_as_float(v[e] & 0xFFFF0000u)));
-        }
-        return m;
-    };
-    auto codes8 = [](const u32x4& v, float qi) {
-        uint32_t o[2] = {0u, 0u};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int q0 = quant_code(__uint_as_float(v[e] << 16), qi);
-            const int q1 = quant_code(__uint_as_float(v[e] & 0xFFFF0000u), qi);
-            o[e >> 1] |= (uint32_t(q0) & 0xFFu) << (16 * (e & 1));
-            o[e >> 1] |= (uint32_t(q1) & 0xFFu) << (16 * (e & 1) + 8);
-        }
-        return u32x2{o[0], o[1]};
-    };
     const u32x4* xrow = reinterpret_cast<const u32x4*>(x + size_t(row) * K);
     float amax = 0.0f;
     for (int c = lane; c < pieces; c += 64) amax = amax8(xrow[2 * c + 1], amax8(xrow[2 * c], amax));
@@ -313,6 +306,52 @@ __global__ __launch_bounds__(512) void act_quant_blocked_kernel(const uint16_t* 
         *at(c) = u32x4{lo[0], lo[1], hi[0], hi[1]};
     }
     if (lane == 0) xs[row] = s;
+}
+
+// Either layout for few rows and, by rows, for rows too long for a wave's registers: a workgroup of WAVES waves per row, P pieces of 16 values per thread in registers (K % 32 == 0, K <= 1024 * WAVES * P).  A
+// handful of rows is a matter of latency: with a wave per row the rounding of 6144 values is a chain of 96 per lane (40 rows
+// blocked: 4.6 us, 2.9 here), and rows of 12288 values were read twice (9.0, 3.7).
+template <int WAVES, int P, bool BLK>
+__global__ __launch_bounds__(WAVES * 64) void act_quant_row_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
+                                                                   float* __restrict__ xs, int M, int K) {
+    __shared__ float red[WAVES];
+    const int row = blockIdx.x, tid = threadIdx.x, pieces = K / 16;
+    int8_t* const dst = BLK ? xq + (size_t(row >> 5) * size_t(K >> 5)) * 1024 + size_t(row & 31) * 16 : xq + size_t(row) * K;
+    auto at = [&](int c) { return reinterpret_cast<u32x4*>(BLK ? dst + size_t(c >> 1) * 1024 + (c & 1) * 512 : dst + 16 * c); };
+    if (row >= M) {
+        for (int c = tid; c < pieces; c += WAVES * 64) *at(c) = u32x4{0u, 0u, 0u, 0u};
+        if (tid == 0) xs[row] = 0.0f;
+        return;
+    }
+    const u32x4* xrow = reinterpret_cast<const u32x4*>(x + size_t(row) * K);
+    u32x4 v[P][2];
+    float amax = 0.0f;
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int c = tid + j * WAVES * 64;
+        v[j][0] = v[j][1] = u32x4{0u, 0u, 0u, 0u};
+        if (c < pieces) {
+            v[j][0] = xrow[2 * c];
+            v[j][1] = xrow[2 * c + 1];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < P; ++j) amax = amax8(v[j][1], amax8(v[j][0], amax));
+    amax = wave_max(amax);
+    if ((tid & 63) == 0) red[tid >> 6] = amax;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) amax = fmaxf(amax, red[w]);
+    const float s = __fdiv_rn(amax, 127.0f);
+    const float qi = s > 0.0f ? __fdiv_rn(1.0f, s) : 0.0f;
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int c = tid + j * WAVES * 64;
+        if (c >= pieces) break;
+        const u32x2 lo = codes8(v[j][0], qi), hi = codes8(v[j][1], qi);
+        *at(c) = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
+    if (tid == 0) xs[row] = s;
 }
 
 // ---- rot_quant: randomized Hadamard rotation of every 32-wide block, then per-token INT8 ---------------------------
@@ -411,6 +450,46 @@ __global__ __launch_bounds__(256) void mxfp4_to_sc_kernel(const uint8_t* __restr
 
 using namespace scmx;
 
+// A workgroup per row while the rows are few (by rows from 2049 values on: 8 rows x 2048 2.2 us with a wave per row, 2.4 with
+// a workgroup; 4096 2.6 and 2.4), and for rows beyond a wave's registers (4000 rows x 12288 by rows: 36 us read twice, 23).
+// Blocked, its 16-byte stores of a single row fill no line: the wave kernel then, up to 12288 values (4000
+// rows x 12288: 40 us read twice, 29).
+static bool act_quant_rows_fit(int Mp, int K, bool blocked) {
+    if (K % 32 || K > 16384) return false;
+    if (K <= 2048) return blocked && Mp <= 128 && K > 512;
+    return Mp <= 256 || K > (blocked ? 12288 : 8192);
+}
+template <bool BLK>
+static void launch_act_quant_rows(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int K, hipStream_t st) {
+    if (K <= 1024) act_quant_row_kernel<1, 1, BLK><<<dim3(Mp), dim3(64), 0, st>>>(x, xq, xs, M, K);
+    else if (K <= 4096) act_quant_row_kernel<4, 1, BLK><<<dim3(Mp), dim3(256), 0, st>>>(x, xq, xs, M, K);
+    else if (K <= 8192) act_quant_row_kernel<8, 1, BLK><<<dim3(Mp), dim3(512), 0, st>>>(x, xq, xs, M, K);
+    else act_quant_row_kernel<8, 2, BLK><<<dim3(Mp), dim3(512), 0, st>>>(x, xq, xs, M, K);
+}
+// A wave per row: the smallest number of register pieces that holds it.  False: the row is too long (or K % 32 != 0).
+template <bool BLK>
+static bool launch_act_quant_waves(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int K, hipStream_t st) {
+    if (K % 32 || K > (BLK ? 12288 : 8192)) return false;
+    const dim3 grid(BLK ? unsigned(Mp) / 8u : (unsigned(Mp) + 3u) / 4u), block(BLK ? 512 : 256);
+    auto go = [&](auto ch) {
+        constexpr int CH = decltype(ch)::value;
+        if (K == 512 * CH) act_quant_wave_kernel<CH, BLK, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K);
+        else act_quant_wave_kernel<CH, BLK, false><<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K);
+    };
+    const int ch = (K + 511) / 512;
+    if (ch <= 1) go(std::integral_constant<int, 1>{});
+    else if (ch <= 2) go(std::integral_constant<int, 2>{});
+    else if (ch <= 3) go(std::integral_constant<int, 3>{});
+    else if (ch <= 4) go(std::integral_constant<int, 4>{});
+    else if (ch <= 6) go(std::integral_constant<int, 6>{});
+    else if (ch <= 8) go(std::integral_constant<int, 8>{});
+    else if (ch <= 10) go(std::integral_constant<int, 10>{});
+    else if (ch <= 12) go(std::integral_constant<int, 12>{});
+    else if (ch <= 16) go(std::integral_constant<int, 16>{});
+    else if constexpr (BLK) go(std::integral_constant<int, 24>{});
+    return true;
+}
+
 extern "C" {
 
 #ifndef SCMX_BUILD_ID
@@ -481,19 +560,10 @@ int scmx_act_quant_blocked(const uint16_t* x, int8_t* xq, float* xs, int M, int 
         return SCMX_ERR_ARG;
     }
     if (Mp == 0) return SCMX_OK;
-    const dim3 grid(unsigned(Mp) / 8u), block(512);
     hipStream_t st = (hipStream_t)stream;
-    switch (K % 512 ? 0 : K / 512) {   // rows of up to 8192 elements stay in registers, loaded as by rows
-        case 1: act_quant_wave_kernel<1, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 2: act_quant_wave_kernel<2, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 3: act_quant_wave_kernel<3, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 4: act_quant_wave_kernel<4, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 6: act_quant_wave_kernel<6, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 8: act_quant_wave_kernel<8, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 12: act_quant_wave_kernel<12, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 16: act_quant_wave_kernel<16, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        default: act_quant_blocked_kernel<<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K); break;
-    }
+    if (act_quant_rows_fit(Mp, K, true)) launch_act_quant_rows<true>(x, xq, xs, M, Mp, K, st);
+    else if (!launch_act_quant_waves<true>(x, xq, xs, M, Mp, K, st))
+        act_quant_blocked_kernel<<<dim3(unsigned(Mp) / 8u), dim3(512), 0, st>>>(x, xq, xs, M, Mp, K);
     return check_launch("act_quant_blocked");
 }
 
@@ -503,19 +573,10 @@ int scmx_act_quant(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int 
         return SCMX_ERR_ARG;
     }
     if (Mp == 0) return SCMX_OK;
-    const dim3 wgrid((unsigned(Mp) + 3u) / 4u), block(256);
     hipStream_t st = (hipStream_t)stream;
-    switch (K % 512 ? 0 : K / 512) {   // rows of up to 8192 elements stay in registers
-        case 1: act_quant_wave_kernel<1><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 2: act_quant_wave_kernel<2><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 3: act_quant_wave_kernel<3><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 4: act_quant_wave_kernel<4><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 6: act_quant_wave_kernel<6><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 8: act_quant_wave_kernel<8><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 12: act_quant_wave_kernel<12><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        case 16: act_quant_wave_kernel<16><<<wgrid, block, 0, st>>>(x, xq, xs, M, Mp); break;
-        default: act_quant_kernel<<<dim3(Mp), block, 0, st>>>(x, xq, xs, M, K); break;
-    }
+    if (uintptr_t(xq) % 16 == 0 && act_quant_rows_fit(Mp, K, false)) launch_act_quant_rows<false>(x, xq, xs, M, Mp, K, st);
+    else if (!launch_act_quant_waves<false>(x, xq, xs, M, Mp, K, st))
+        act_quant_kernel<<<dim3(Mp), dim3(256), 0, st>>>(x, xq, xs, M, K);
     return check_launch("act_quant");
 }
 
