@@ -105,14 +105,15 @@ int scmx_mm_w4a8(const scmx_format* fmt, const int8_t* xq, const float* xscale, 
 
 /* scmx_mm_w4a8 on activations in the blocked layout of scmx_act_quant_blocked (xq: ceil(M / 32) * 32 rows, 16-byte
  * aligned): the waves of the large tiles load their activation fragments straight from memory, and only the weights
- * pass through LDS.  Same results as scmx_mm_w4a8 (same integers, same epilogues).  Meant for prefill-sized M: every
- * shape runs, on 128x128 tiles at least.  The same pair of reference calls as scmx_mm_w4a8 (e2e/fused_qwen3.py:161-172). */
+ * pass through LDS.  Same results as scmx_mm_w4a8 (same integers, same epilogues).  Meant for prefill-sized M and for few
+ * rows (a kernel that splits K over the waves of a workgroup, up to 128 rows): every other shape runs too, on 128x128
+ * tiles at least.  The same pair of reference calls as scmx_mm_w4a8 (e2e/fused_qwen3.py:161-172). */
 int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* xscale, const uint32_t* codes,
                          const uint8_t* bcodes, const float* wscale, const uint16_t* res, void* out, int epi, int M,
                          int N, int K, void* stream);
 
 /* 1 when a dense problem of this shape runs faster from blocked activations (it is large enough for the tiles that read
- * them), 0 when the row layout is the one to quantize into; what scmx_linear_w4a8 decides by.  No device work. */
+ * them, or small enough for the few-row kernel), 0 when the row layout is the one to quantize into; what scmx_linear_w4a8 decides by.  No device work. */
 int scmx_mm_w4a8_prefers_blocked(int M, int N, int K);
 
 /* Whole dense W4A8 linear on a bf16 input: activation quantization prologue + scmx_mm_w4a8, one call (the activations
@@ -243,10 +244,15 @@ int scmx_gemv(const scmx_format* fmt, const void* x, const float* xscale, const 
               int shared_expert, void* stream);
 
 /* scmx_gemv without the expert gather for ANY number of rows from 1 to 8 (three rows run the four-row kernel, five to seven
- * the eight-row one, without padding the operands: rows past the last are neither read nor written). */
+ * the eight-row one, without padding the operands: rows past the last are neither read nor written).  Several bf16 rows
+ * (pro 1) of a shape whose kernels here would decode every weight per row, or stage long rows in every workgroup, run as
+ * scmx_linear_w4a8 when `workspace` holds scmx_gemv_rows_workspace(...) bytes (256-byte aligned; 0 = not such a shape);
+ * workspace may be NULL.  Same results either way. */
+size_t scmx_gemv_rows_workspace(const scmx_format* fmt, int pro, int rows, int N, int K);
 int scmx_gemv_rows(const scmx_format* fmt, const void* x, const float* xscale, const uint32_t* codes,
                    const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi, int pro,
-                   const uint16_t* nw, float eps, int rows, int N, int K, void* stream);
+                   const uint16_t* nw, float eps, int rows, int N, int K, void* workspace, size_t workspace_bytes,
+                   void* stream);
 
 /* ---- mixture of experts ----------------------------------------------------------------------------------------- */
 

@@ -11,38 +11,9 @@
 #include <atomic>
 #include <type_traits>
 
-#include "scmx_common.h"
+#include "gemm_args.h"
 
 namespace scmx {
-
-struct GemmArgs {
-    const int8_t* xq;        // activations INT8 [rows, K] (blocked: 32 x 32 blocks in MFMA operand order, see AD)
-    const float* xscale;     // [rows]
-    const int32_t* gather;   // optional: logical row r reads xq[gather[r]], xscale[gather[r]]
-    const uint32_t* codes;   // packed weights [E][N*K/8]
-    const uint8_t* bcodes;   // [E][N][bc_row_bytes]
-    const int8_t* wq;        // INT8 weights [E*N, K] when the tile is fed from unpacked weights
-    const float* wscale;     // [E][N]
-    const uint16_t* res;     // [M, N] residual (epilogue 2)
-    void* out;
-    int M, N, K;             // M = number of logical rows (R for the grouped GEMM)
-    int bc_row_bytes;
-    int epi;
-    const int32_t* off;      // grouped: expert segment offsets [E+1]; dense: NULL
-    const uint16_t* silu;    // SwiGLU epilogue: lookup table over bf16 gate values
-    const int32_t* tstart;   // grouped: first row tile of each expert [E+1]
-    int n_experts;
-    int blocked;             // dense: xq is in the blocked layout
-    DevFormat fmt;
-};
-
-// B_PACKED_DEFAULT / B_PACKED_B16: the published codebook with power-of-two shifts on 32- / 16-element blocks (decoded
-// with the FP4 conversion); B_PACKED_B16M: that codebook on 16-element blocks with 4-bit codes for consecutive integer
-// multipliers (FP4 conversion, then one fused multiply-add); B_PACKED_GENERIC: any member of the format family (table
-// decode).
-// B_PACKED_E8M0: a standard MXFP4 tensor in place -- B_PACKED_DEFAULT's decode with the block's shift taken from its
-// E8M0 byte minus the row's lowest one (which the row scale carries).
-enum { B_INT8 = 0, B_PACKED_DEFAULT = 1, B_PACKED_GENERIC = 2, B_PACKED_B16 = 3, B_PACKED_B16M = 4, B_PACKED_E8M0 = 5 };
 
 // FD = number of fragment register buffers: fragments are fetched FD - 1 k slices ahead of their MFMAs.
 // SKIP (grouped launches): a row tile that ends inside its expert's segment multiplies only the 32-row blocks that hold
@@ -954,6 +925,7 @@ static int dense_choice(long M, long N, long K, bool blocked) {
 }
 
 static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
+    if (a.blocked && skinny_fits(a.M, a.N, a.K, bmode)) return launch_skinny(a, bmode, s);
     const int best = dense_choice(a.M, a.N, a.K, a.blocked != 0);
     if (a.blocked) {
         switch (best) {
@@ -1078,7 +1050,8 @@ int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* 
 }
 
 int scmx_mm_w4a8_prefers_blocked(int M, int N, int K) {
-    return M > 0 && N > 0 && K > 0 && K % 128 == 0 && dense_choice(M, N, K, false) <= 2;
+    return M > 0 && N > 0 && K > 0 && K % 128 == 0 &&
+           (skinny_fits(M, N, K, B_PACKED_DEFAULT) || dense_choice(M, N, K, false) <= 2);
 }
 
 // The fused layer quantizes into whichever layout suits the shape: blocked where the row-layout model would run one of its

@@ -12,7 +12,7 @@
 // the GEMM's.  `BATCH` activation rows share one pass over the weights; for the published format they go through
 // gemv_mfma_kernel below, which hands the dot products to the 4x4x4 INT8 MFMA so that the vector work per weight
 // does not grow with the number of rows.
-#include "scmx_common.h"
+#include "gemm_args.h"
 
 namespace scmx {
 
@@ -1208,6 +1208,20 @@ static void launch_gemv_hmfma(const GemvArgs& a, bool split, hipStream_t s) {
     else go(gemv_hmfma_kernel<BATCH, W_STREAM, true, 12, FMT>);
 }
 
+// Shapes of the half-precision MFMA kernel (dflt: weight format as launch_gemv counts them, 0 = none it decodes).
+static bool hmfma_wide(int dflt, int N, int K) {
+    const bool bytes = dflt == 4 || dflt == 3;
+    return dflt && N % 16 == 0 && K % 512 == 0 && N >= HMFMA_MIN_ROWS && K <= 2048 && (!bytes || K >= 1536);
+}
+static bool hmfma_narrow(int dflt, int kernel_rows, int N, int K) {
+    const bool bytes = dflt == 4 || dflt == 3;
+    return dflt && N % 16 == 0 && K % 512 == 0 && K <= 8192 && (N < HMFMA_MIN_ROWS || bytes) && size_t(kernel_rows) * K <= 32768;
+}
+static int format_kind(const DevFormat& f) {
+    return is_mxfp4_e8m0_format(f) ? 4 : is_default_format(f) ? 1 : is_pow2_block16_format(f) ? 2 : is_block16_range_format(f) ? 3 : 0;
+}
+static int kernel_rows_of(int rows) { return rows <= 2 ? rows : rows <= 4 ? 4 : 8; }
+
 template <int BATCH>
 static void launch_gemv_rows(const GemvArgs& a, int slots, int dflt, hipStream_t s) {
     // Several activation rows, whole row groups of 16 and pieces of 512: half-precision MFMA dot products, for every format
@@ -1219,11 +1233,9 @@ static void launch_gemv_rows(const GemvArgs& a, int slots, int dflt, hipStream_t
     // 116 -> 35 us, 12288 x 2048 with SwiGLU 17.4 -> 8.0, 2048 x 6144 16.1 -> 8.4.)
     const bool bc4 = uintptr_t(a.bcodes) % 4 == 0;
     if constexpr (BATCH > 1) {
-        if (dflt && bc4 && !a.eidx && a.N % 16 == 0 && a.K % 512 == 0 && a.K <= 8192) {
-            const bool bytes = dflt == 4 || dflt == 3;
-            const bool wide = a.N >= HMFMA_MIN_ROWS && a.K <= 2048 && (!bytes || a.K >= 1536);
-            const bool narrow = (a.N < HMFMA_MIN_ROWS || bytes) && size_t(BATCH) * a.K <= 32768;
-            if (wide || narrow) {
+        if (dflt && bc4 && !a.eidx) {
+            const bool wide = hmfma_wide(dflt, a.N, a.K);
+            if (wide || hmfma_narrow(dflt, BATCH, a.N, a.K)) {
                 switch (dflt) {
                     case 1: return launch_gemv_hmfma<BATCH, H_SC>(a, !wide, s);
                     case 2: return launch_gemv_hmfma<BATCH, H_B16>(a, !wide, s);
@@ -1289,7 +1301,7 @@ static int gemv_any(const scmx_format* fmt, const void* x, const float* xscale, 
         set_error("gemv: %d rows outside 1..8", batch);
         return SCMX_ERR_ARG;
     }
-    const int kernel_rows = batch <= 2 ? batch : batch <= 4 ? 4 : 8;   // rows of the kernel that runs
+    const int kernel_rows = kernel_rows_of(batch);   // rows of the kernel that runs
     if (size_t(kernel_rows) * ((K + 2047) & ~2047) * 2 + 80 * sizeof(float) > 160 * 1024) {
         set_error("gemv: batch * K = %zu activations exceed what one workgroup can stage (80 Ki)", size_t(batch) * K);
         return SCMX_ERR_ARG;
@@ -1301,11 +1313,7 @@ static int gemv_any(const scmx_format* fmt, const void* x, const float* xscale, 
     a.bc_row_bytes = K / f.block * f.bc_bits / 8;
     a.eidx = eidx; a.n_eidx = n_eidx; a.xstride = xstride; a.shared_expert = eidx ? shared_expert : -1;
     a.fmt = f;
-    const int dflt = is_mxfp4_e8m0_format(f)    ? 4
-                     : is_default_format(f)       ? 1
-                     : is_pow2_block16_format(f)  ? 2
-                     : is_block16_range_format(f) ? 3
-                                                  : 0;
+    const int dflt = format_kind(f);
     hipStream_t s = (hipStream_t)stream;
     switch (kernel_rows) {
         case 1: launch_gemv_rows<1>(a, slots, dflt, s); break;
@@ -1328,8 +1336,32 @@ extern "C" int scmx_gemv(const scmx_format* fmt, const void* x, const float* xsc
                     shared_expert, stream);
 }
 
+// Several bf16 rows that no half-precision MFMA kernel takes: quantizing them once and running the few-row GEMM beats the
+// kernels that decode with byte tables or stage the rows in every workgroup (4 rows, 4096 x 12288: 20.4 us against 15.0; 8
+// rows, 2048 x 6144: 17.8 against 9.5; 4 rows, 896 x 896: 6.5 against 5.2).
+extern "C" size_t scmx_gemv_rows_workspace(const scmx_format* fmt, int pro, int rows, int N, int K) {
+    DevFormat f;
+    if (pro != 1 || rows < 2 || rows > 8 || N <= 0 || K <= 0 || K % 128 || make_dev_format(fmt, &f)) return 0;
+    const int dflt = format_kind(f);
+    // The narrow form stages all rows in each of its N / 16 workgroups: up to about 10 M values in all (eight rows, 12288 x
+    // 2048: 12.6 M, 11.8 us against 9.8 this way; 24576 x 4096: 50 M, 48 against 22; four rows, 12288 x 2048: 6.3 M, 7.3
+    // against 9).
+    const bool narrow = hmfma_narrow(dflt, kernel_rows_of(rows), N, K) && long(kernel_rows_of(rows)) * K * (N / 16) <= 10000000;
+    if (hmfma_wide(dflt, N, K) || narrow || !skinny_fits(rows, N, K, -1)) return 0;
+    return scmx_linear_w4a8_workspace(rows, K);
+}
+
 extern "C" int scmx_gemv_rows(const scmx_format* fmt, const void* x, const float* xscale, const uint32_t* codes,
                               const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi,
-                              int pro, const uint16_t* nw, float eps, int rows, int N, int K, void* stream) {
+                              int pro, const uint16_t* nw, float eps, int rows, int N, int K, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+    if (workspace && wscale && epi >= 1 && N % 4 == 0 && (epi != SCMX_EPI_SWIGLU || N % 8 == 0) &&
+        (uintptr_t(x) | uintptr_t(out) | uintptr_t(wscale) | uintptr_t(codes)) % 16 == 0 && uintptr_t(res) % 8 == 0 &&
+        uintptr_t(workspace) % 256 == 0) {
+        const size_t need = scmx_gemv_rows_workspace(fmt, pro, rows, N, K);
+        if (need && workspace_bytes >= need)
+            return scmx_linear_w4a8(fmt, reinterpret_cast<const uint16_t*>(x), codes, bcodes, wscale, res, out, epi, rows, N, K,
+                                    workspace, workspace_bytes, stream);
+    }
     return gemv_any(fmt, x, xscale, codes, bcodes, wscale, res, out, epi, pro, nw, eps, rows, N, K, nullptr, 0, 0, -1, stream);
 }

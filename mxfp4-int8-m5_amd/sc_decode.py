@@ -46,7 +46,9 @@ def gemv(xq, codes, bcodes, xscale, wscale, N, epi, dtype=torch.bfloat16, res=No
             _lib.ptr(wscale), _lib.ptr(res) if epi == 2 else None, _lib.ptr(out), epi, pro, _lib.ptr(nw) if pro == 2 else None,
             S._eps(eps) if pro == 2 else 0.0, batch, N, K)
     if eidx is None:
-        _lib.call("scmx_gemv_rows", *args, _lib.stream())
+        need = _lib.load().scmx_gemv_rows_workspace(args[0], pro, batch, N, K) if batch > 1 else 0
+        work = torch.empty(need, dtype=torch.uint8, device=xq.device) if need else None
+        _lib.call("scmx_gemv_rows", *args, _lib.ptr(work), need, _lib.stream())
     else:
         _lib.call("scmx_gemv", *args, _lib.ptr(eidx), nslot, xstride, -1 if shared is None else int(shared), _lib.stream())
     return out
