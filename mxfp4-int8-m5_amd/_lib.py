@@ -1,9 +1,8 @@
-"""ctypes binding of libscmx.so (the C ABI declared in include/scmx.h).  There is no fallback: a missing or
-incomplete library raises, and so does every call that returns a negative status."""
+"""Access to libscmx.so (the C ABI declared in include/scmx.h): `native()` is what the wrappers call, tensors in, one native
+call per launch (csrc/torch_binding.cpp); `load()` the whole ABI through ctypes, for the queries and for foreign callers.
+There is no fallback: a missing or incomplete library raises, and so does every call that returns a negative status."""
 import ctypes as C
 import os
-
-import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libscmx.so")
@@ -81,24 +80,19 @@ def load():
     return _lib
 
 
-def call(name, *args):
-    lib = load()
-    rc = getattr(lib, name)(*args)
-    if rc != 0:
-        msg = lib.scmx_last_error().decode()
-        raise (ValueError if rc in (-1, -2, -4) else RuntimeError)(f"{name} failed ({rc}): {msg}")
+_native = None
 
 
-def ptr(t):
-    """Device pointer of a contiguous CUDA tensor (None -> NULL)."""
-    if t is None:
-        return None
-    if not t.is_cuda:
-        raise ValueError("scmx kernels take CUDA (ROCm) tensors; got a CPU tensor")
-    if not t.is_contiguous():
-        raise ValueError("scmx kernels take contiguous tensors")
-    return t.data_ptr()
-
-
-def stream():
-    return torch.cuda.current_stream().cuda_stream
+def native():
+    """The torch binding of the library (_binding.so): its entry points under their own names, on tensors and the current
+    stream, and the allocation helpers."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _binding
+        except ImportError as exc:
+            raise RuntimeError(f"the torch binding beside {LIB_PATH} cannot be loaded ({exc}): build it with `python "
+                               f"{os.path.join(HERE, 'build.py')}` (there is no fallback)") from exc
+        _native = _binding
+    return _native

@@ -1,4 +1,5 @@
-"""Builds csrc/*.hip into libscmx.so (gfx950) next to this file.  `python build.py` or build.build()."""
+"""Builds csrc/*.hip into libscmx.so (gfx950) and csrc/torch_binding.cpp into _binding.so next to this file.
+`python build.py` or build.build()."""
 import os
 import subprocess
 import sys
@@ -7,6 +8,8 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libscmx.so")
+BINDING = os.path.join(HERE, "_binding.so")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 SOURCES = ["api.hip", "gemm.hip", "gemm_skinny.hip", "gemv.hip", "rowops.hip", "quantize.hip", "attn.hip", "attn_prefill.hip", "silu_table.hip"]
 # packed FP32 instructions are kept off (they have misbehaved on this hardware pool); no FMA contraction, so the
 # FP32 epilogues and norms round exactly like a plain IEEE evaluation
@@ -50,7 +53,19 @@ def build(verbose=False):
             if verbose and out.strip():
                 print(out)
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
+    build_binding()
     return LIB
+
+
+def build_binding():
+    """The torch binding of the C ABI (host code only): _binding.so, linked to libscmx.so beside it."""
+    import sysconfig
+    from torch.utils import cpp_extension as ext
+    inc = ["-I" + p for p in [*ext.include_paths(), sysconfig.get_paths()["include"], os.path.join(ROCM, "include")]]
+    libs = ["-L" + p for p in ext.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", *inc,
+          os.path.join(CSRC, "torch_binding.cpp"), "-o", BINDING, "-L" + HERE, "-l:libscmx.so", "-Wl,-rpath,$ORIGIN", *libs])
+    return BINDING
 
 
 def build_host_check(driver, out=None):

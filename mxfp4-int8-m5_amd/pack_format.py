@@ -55,9 +55,8 @@ def pack_matrix(w, name, fmt=None):
         w = w.float()
     w = w.contiguous()
     n, k = w.shape
-    codes = torch.empty(n * k // 8, dtype=torch.int32, device=w.device)
-    bc = torch.empty((n, k // fmt.block // fmt.per_byte), dtype=torch.uint8, device=w.device)
-    ws = torch.empty(n, dtype=torch.float32, device=w.device)
-    _lib.call("scmx_quantize_family", fmt.c_struct(), _lib.ptr(w), int(w.dtype == torch.bfloat16), n, k, _lib.ptr(codes),
-              _lib.ptr(bc), _lib.ptr(ws), _lib.stream())
+    codes = _lib.native().empty_i32(w, n * k // 8)
+    bc = _lib.native().empty_u8(w, n, k // fmt.block // fmt.per_byte)
+    ws = _lib.native().empty_f32(w, n)
+    _lib.native().scmx_quantize_family(fmt.c, w, int(w.dtype == torch.bfloat16), n, k, codes, bc, ws)
     return codes, bc, ws, dict(exact_q=True)

@@ -30,7 +30,7 @@ def gemv(xq, codes, bcodes, xscale, wscale, N, epi, dtype=torch.bfloat16, res=No
         nslot = eidx.numel()
         slots = nslot + (shared is not None)
         eidx = eidx if eidx.dtype == torch.int32 else eidx.view(torch.int32) if eidx.element_size() == 4 else eidx.to(torch.int32)
-        out = torch.empty((slots, no), dtype=torch.bfloat16, device=xq.device)
+        out = _lib.native().empty_bf16(xq, slots, no)
     elif xq.dim() == 2 and xq.shape[0] > 8:   # more rows than one pass takes: eight at a time
         cut = lambda t, i: None if t is None else t[i:i + 8]   # noqa: E731
         return torch.cat([gemv(xq[i:i + 8], codes, bcodes, cut(xscale, i), wscale, N, epi, dtype, cut(res, i), nsg, None,
@@ -38,17 +38,19 @@ def gemv(xq, codes, bcodes, xscale, wscale, N, epi, dtype=torch.bfloat16, res=No
                           for i in range(0, xq.shape[0], 8)])
     elif xq.dim() == 2 and xq.shape[0] > 1:
         batch = xq.shape[0]
-        out = torch.empty((batch, no), dtype=torch.bfloat16, device=xq.device)
+        out = _lib.native().empty_bf16(xq, batch, no)
     else:
-        out = torch.empty(no, dtype=torch.bfloat16, device=xq.device)
+        out = _lib.native().empty_bf16(xq, no)
     assert (pro == 0 and xq.dtype == torch.int8) or (pro in (1, 2) and xq.dtype == torch.bfloat16)
-    args = (fmt.c_struct(), _lib.ptr(xq), _lib.ptr(xscale) if pro == 0 else None, _lib.ptr(codes), _lib.ptr(bcodes),
-            _lib.ptr(wscale), _lib.ptr(res) if epi == 2 else None, _lib.ptr(out), epi, pro, _lib.ptr(nw) if pro == 2 else None,
-            S._eps(eps) if pro == 2 else 0.0, batch, N, K)
+    nat = _lib.native()
+    xscale = xscale if pro == 0 else None
+    res = res if epi == 2 else None
+    nw, eps = (nw, S._eps(eps)) if pro == 2 else (None, 0.0)
     if eidx is None:
-        need = _lib.load().scmx_gemv_rows_workspace(args[0], pro, batch, N, K) if batch > 1 else 0
-        work = torch.empty(need, dtype=torch.uint8, device=xq.device) if need else None
-        _lib.call("scmx_gemv_rows", *args, _lib.ptr(work), need, _lib.stream())
+        need = nat.scmx_gemv_rows_workspace(fmt.c, pro, batch, N, K) if batch > 1 else 0
+        nat.scmx_gemv_rows(fmt.c, xq, xscale, codes, bcodes, wscale, res, out, epi, pro, nw, eps, batch, N, K,
+                           nat.empty_u8(xq, need) if need else None, need)
     else:
-        _lib.call("scmx_gemv", *args, _lib.ptr(eidx), nslot, xstride, -1 if shared is None else int(shared), _lib.stream())
+        nat.scmx_gemv(fmt.c, xq, xscale, codes, bcodes, wscale, res, out, epi, pro, nw, eps, batch, N, K, eidx, nslot, xstride,
+                      -1 if shared is None else int(shared))
     return out

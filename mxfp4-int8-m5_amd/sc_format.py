@@ -8,6 +8,7 @@ Layouts (row-major over N, K contiguous):
   wscale  f32 [N]
 """
 from dataclasses import dataclass
+from functools import cached_property
 
 import numpy as np
 import torch
@@ -43,8 +44,13 @@ class Format:
     def bits_per_weight(self, K):
         return 4 + self.bc_bits / self.block + 32 / K
 
+    @cached_property
+    def c(self):
+        """c_struct(), made once."""
+        return self.c_struct()
+
     def c_struct(self):
-        """The scmx_format passed across the C ABI."""
+        """The scmx_format passed across the C ABI (a new one)."""
         if len(self.mult) > 16:
             raise ValueError("the kernels take at most 16 block multipliers")
         f = _lib.CFormat()
@@ -125,10 +131,10 @@ def from_mxfp4(nibbles, e8m0):
     n, nb = e8m0.shape
     k = nb * 32
     assert nibbles.shape == (n, k // 2) and nibbles.dtype == torch.uint8 and e8m0.dtype == torch.uint8
-    bc = torch.empty((n, nb // 4), dtype=torch.uint8, device=e8m0.device)
-    ws = torch.empty(n, dtype=torch.float32, device=e8m0.device)
+    bc = _lib.native().empty_u8(e8m0, n, nb // 4)
+    ws = _lib.native().empty_f32(e8m0, n)
     status = torch.zeros(1, dtype=torch.int32, device=e8m0.device)
-    _lib.call("scmx_mxfp4_to_sc", _lib.ptr(e8m0), _lib.ptr(bc), _lib.ptr(ws), _lib.ptr(status), n, k, _lib.stream())
+    _lib.native().scmx_mxfp4_to_sc(e8m0, bc, ws, status, n, k)
     if int(status.item()) & 1:
         raise ValueError("a row's block exponents span more than 3: not INT8-embeddable")
     return nibbles.contiguous().view(torch.int32).reshape(-1), bc, ws
@@ -139,9 +145,9 @@ def mxfp4_row_scales(e8m0):
     2^(lowest E8M0 byte of the row - 128).  Raises if a row's exponents span more than 3 or hold the bytes 0 / 255."""
     n, nb = e8m0.shape
     assert e8m0.dtype == torch.uint8
-    ws = torch.empty(n, dtype=torch.float32, device=e8m0.device)
+    ws = _lib.native().empty_f32(e8m0, n)
     status = torch.zeros(1, dtype=torch.int32, device=e8m0.device)
-    _lib.call("scmx_mxfp4_to_sc", _lib.ptr(e8m0), None, _lib.ptr(ws), _lib.ptr(status), n, nb * 32, _lib.stream())
+    _lib.native().scmx_mxfp4_to_sc(e8m0, None, ws, status, n, nb * 32)
     st = int(status.item())
     if st & 1:
         raise ValueError("a row's block exponents span more than 3: not INT8-embeddable")
@@ -170,13 +176,12 @@ def quantize(w, fmt=None, with_q=True):
         w = w.float()
     w = w.contiguous()
     n, k = w.shape
-    codes = torch.empty(n * k // 8, dtype=torch.int32, device=w.device)
-    bc = torch.empty((n, k // (4 * fmt.block)), dtype=torch.uint8, device=w.device)
-    ws = torch.empty(n, dtype=torch.float32, device=w.device)
-    _lib.call("scmx_quantize_sc", _lib.ptr(w), int(w.dtype == torch.bfloat16), n, k, fmt.block, _lib.ptr(codes),
-              _lib.ptr(bc), _lib.ptr(ws), _lib.stream())
+    codes = _lib.native().empty_i32(w, n * k // 8)
+    bc = _lib.native().empty_u8(w, n, k // (4 * fmt.block))
+    ws = _lib.native().empty_f32(w, n)
+    _lib.native().scmx_quantize_sc(w, int(w.dtype == torch.bfloat16), n, k, fmt.block, codes, bc, ws)
     q = None
     if with_q:
-        q = torch.empty((n, k), dtype=torch.int8, device=w.device)
-        _lib.call("scmx_unpack_i8", fmt.c_struct(), _lib.ptr(codes), _lib.ptr(bc), _lib.ptr(q), n, k, _lib.stream())
+        q = _lib.native().empty_i8(w, n, k)
+        _lib.native().scmx_unpack_i8(fmt.c, codes, bc, q, n, k)
     return codes, bc, ws, q

@@ -64,8 +64,8 @@ def unpack_i8(codes, bcodes, N, K, deps=(), lazy=None, fmt=None, wscale=None):
     if FUSE_UNPACK if lazy is None else lazy:
         return PackedWq(codes, bcodes, N, K, fmt, wscale)
     assert codes.numel() * codes.element_size() == N * K // 2, "codes must hold N*K/2 bytes"
-    wq = torch.empty((N, K), dtype=torch.int8, device=codes.device)
-    _lib.call("scmx_unpack_i8", fmt.c_struct(), _lib.ptr(codes), _lib.ptr(bcodes), _lib.ptr(wq), N, K, _lib.stream())
+    wq = _lib.native().empty_i8(codes, N, K)
+    _lib.native().scmx_unpack_i8(fmt.c, codes, bcodes, wq, N, K)
     return wq
 
 
@@ -74,9 +74,9 @@ def act_quant(x, Mp=None, nt=256, deps=()):
     M, K = x.shape
     Mp = Mp or pad_rows(M)
     assert x.dtype == torch.bfloat16
-    xq = torch.empty((Mp, K), dtype=torch.int8, device=x.device)
-    xs = torch.empty(Mp, dtype=torch.float32, device=x.device)
-    _lib.call("scmx_act_quant", _lib.ptr(x), _lib.ptr(xq), _lib.ptr(xs), M, Mp, K, _lib.stream())
+    xq = _lib.native().empty_i8(x, Mp, K)
+    xs = _lib.native().empty_f32(x, Mp)
+    _lib.native().scmx_act_quant(x, xq, xs, M, Mp, K)
     return xq, xs
 
 
@@ -92,36 +92,35 @@ def rot_quant(x, signs, Mp=None, nt=512, deps=()):
     M, K = x.shape
     Mp = Mp or pad_rows(M)
     assert x.dtype == torch.bfloat16 and signs.dtype == torch.float32 and signs.numel() == K
-    xq = torch.empty((Mp, K), dtype=torch.int8, device=x.device)
-    xs = torch.empty(Mp, dtype=torch.float32, device=x.device)
-    _lib.call("scmx_rot_quant", _lib.ptr(x), _lib.ptr(signs), _lib.ptr(xq), _lib.ptr(xs), M, Mp, K, _lib.stream())
+    xq = _lib.native().empty_i8(x, Mp, K)
+    xs = _lib.native().empty_f32(x, Mp)
+    _lib.native().scmx_rot_quant(x, signs, xq, xs, M, Mp, K)
     return xq, xs
 
 
 def _gemm(xq, wq, xscale, wscale, epi, res):
     (M, K), N = xq.shape, wq.shape[0]
     assert xq.dtype == torch.int8 and wq.shape[1] == K
+    blocked = isinstance(xq, BlockedXq)
+    like = xq.data if blocked else xq
     if epi == 0:
-        out = torch.empty((M, N), dtype=torch.int32, device=xq.device)
+        out = _lib.native().empty_i32(like, M, N)
     else:
-        out = torch.empty((M, N // 2 if epi == 3 else N), dtype=torch.bfloat16, device=xq.device)
+        out = _lib.native().empty_bf16(like, M, N // 2 if epi == 3 else N)
     if epi == 2:
         assert res is not None and tuple(res.shape) == (M, N) and res.dtype == torch.bfloat16
-    r = _lib.ptr(res) if epi == 2 else None
-    if isinstance(xq, BlockedXq):
+    r = res if epi == 2 else None
+    if blocked:
         if not isinstance(wq, PackedWq):
             raise ValueError("blocked activations multiply packed weights (unpack_i8's lazy handle)")
-        _lib.call("scmx_mm_w4a8_blocked", wq.fmt.c_struct(), _lib.ptr(xq.data), _lib.ptr(xscale), _lib.ptr(wq.codes),
-                  _lib.ptr(wq.bcodes), _lib.ptr(wscale if wscale is not None else wq.wscale), r, _lib.ptr(out), epi, M, N,
-                  K, _lib.stream())
+        _lib.native().scmx_mm_w4a8_blocked(wq.fmt.c, xq.data, xscale, wq.codes, wq.bcodes,
+                                           wscale if wscale is not None else wq.wscale, r, out, epi, M, N, K)
     elif isinstance(wq, PackedWq):
-        _lib.call("scmx_mm_w4a8", wq.fmt.c_struct(), _lib.ptr(xq), _lib.ptr(xscale), _lib.ptr(wq.codes),
-                  _lib.ptr(wq.bcodes), _lib.ptr(wscale if wscale is not None else wq.wscale), r, _lib.ptr(out), epi, M, N,
-                  K, _lib.stream())
+        _lib.native().scmx_mm_w4a8(wq.fmt.c, xq, xscale, wq.codes, wq.bcodes, wscale if wscale is not None else wq.wscale, r,
+                                   out, epi, M, N, K)
     else:
         assert wq.dtype == torch.int8
-        _lib.call("scmx_mm_epi", _lib.ptr(xq), _lib.ptr(wq), _lib.ptr(xscale), _lib.ptr(wscale), r, _lib.ptr(out), epi,
-                  M, N, K, _lib.stream())
+        _lib.native().scmx_mm_epi(xq, wq, xscale, wscale, r, out, epi, M, N, K)
     return out
 
 
@@ -157,9 +156,9 @@ def act_quant_blocked(x, Mp=None):
     M, K = x.shape
     Mp = Mp or pad_rows(M)
     assert x.dtype == torch.bfloat16 and Mp % 32 == 0
-    xq = torch.empty(Mp * K, dtype=torch.int8, device=x.device)
-    xs = torch.empty(Mp, dtype=torch.float32, device=x.device)
-    _lib.call("scmx_act_quant_blocked", _lib.ptr(x), _lib.ptr(xq), _lib.ptr(xs), M, Mp, K, _lib.stream())
+    xq = _lib.native().empty_i8(x, Mp * K)
+    xs = _lib.native().empty_f32(x, Mp)
+    _lib.native().scmx_act_quant_blocked(x, xq, xs, M, Mp, K)
     return BlockedXq(xq, Mp, K), xs   # Mp rows like act_quant's tensor: the padding rows are zeros
 
 
@@ -174,13 +173,12 @@ def linear_w4a8(x, codes, bcodes, wscale, N, epi=1, res=None, fmt=None, workspac
     fmt = fmt or F.DEFAULT
     M, K = x.shape
     assert x.dtype == torch.bfloat16 and epi in (1, 2, 3)
-    need = _lib.load().scmx_linear_w4a8_workspace(M, K)
+    need = _lib.native().scmx_linear_w4a8_workspace(M, K)
     if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-    out = torch.empty((M, N // 2 if epi == 3 else N), dtype=torch.bfloat16, device=x.device)
-    _lib.call("scmx_linear_w4a8", fmt.c_struct(), _lib.ptr(x), _lib.ptr(codes), _lib.ptr(bcodes), _lib.ptr(wscale),
-              _lib.ptr(res) if epi == 2 else None, _lib.ptr(out), epi, M, N, K, _lib.ptr(workspace),
-              workspace.numel() * workspace.element_size(), _lib.stream())
+        workspace = _lib.native().empty_u8(x, need)
+    out = _lib.native().empty_bf16(x, M, N // 2 if epi == 3 else N)
+    _lib.native().scmx_linear_w4a8(fmt.c, x, codes, bcodes, wscale, res if epi == 2 else None, out, epi, M, N, K, workspace,
+                                   workspace.numel() * workspace.element_size())
     return out
 
 
@@ -195,11 +193,11 @@ def _rms(x, w, eps, Mp, want_xn, blocked=False):
     Mp = Mp or pad_rows(M)
     assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
     blocked = blocked and Mp % 32 == 0 and K % 512 == 0 and K <= 4096
-    xq = torch.empty((Mp, K), dtype=torch.int8, device=x.device)
-    xs = torch.empty(Mp, dtype=torch.float32, device=x.device)
-    xn = torch.empty((Mp, K), dtype=torch.bfloat16, device=x.device) if want_xn else None
-    _lib.call("scmx_rmsnorm_quant_blocked" if blocked else "scmx_rmsnorm_quant", _lib.ptr(x), _lib.ptr(w), _eps(eps),
-              _lib.ptr(xq), _lib.ptr(xs), _lib.ptr(xn), M, Mp, K, _lib.stream())
+    xq = _lib.native().empty_i8(x, Mp, K)
+    xs = _lib.native().empty_f32(x, Mp)
+    xn = _lib.native().empty_bf16(x, Mp, K) if want_xn else None
+    quantize = _lib.native().scmx_rmsnorm_quant_blocked if blocked else _lib.native().scmx_rmsnorm_quant
+    quantize(x, w, _eps(eps), xq, xs, xn, M, Mp, K)
     if blocked:
         xq = BlockedXq(xq.reshape(-1), Mp, K)   # Mp rows like the tensor it stands for: the padding rows are zeros
     return (xq, xs, xn) if want_xn else (xq, xs)
@@ -221,13 +219,13 @@ def rmsnorm(x, w, eps):
     M, K = x.shape
     assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
     out = torch.empty_like(x)
-    _lib.call("scmx_rmsnorm", _lib.ptr(x), _lib.ptr(w), _eps(eps), _lib.ptr(out), M, K, _lib.stream())
+    _lib.native().scmx_rmsnorm(x, w, _eps(eps), out, M, K)
     return out
 
 
 def prefers_blocked(M, N, K):
     """Whether a dense [M, K] x [N, K]^T problem on packed weights runs faster from blocked activations."""
-    return bool(_lib.load().scmx_mm_w4a8_prefers_blocked(M, N, K))
+    return bool(_lib.native().scmx_mm_w4a8_prefers_blocked(M, N, K))
 
 
 def res_norm_quant(acc, xscale, wscale, res, w, eps, deps=()):
@@ -235,10 +233,9 @@ def res_norm_quant(acc, xscale, wscale, res, w, eps, deps=()):
     Mp, K = acc.shape
     assert tuple(res.shape) == (Mp, K) and acc.dtype == torch.int32
     h = torch.empty_like(res)
-    xq = torch.empty((Mp, K), dtype=torch.int8, device=acc.device)
-    xs = torch.empty(Mp, dtype=torch.float32, device=acc.device)
-    _lib.call("scmx_res_norm_quant", _lib.ptr(acc), _lib.ptr(xscale), _lib.ptr(wscale), _lib.ptr(res), _lib.ptr(w),
-              _eps(eps), _lib.ptr(h), _lib.ptr(xq), _lib.ptr(xs), Mp, K, _lib.stream())
+    xq = _lib.native().empty_i8(acc, Mp, K)
+    xs = _lib.native().empty_f32(acc, Mp)
+    _lib.native().scmx_res_norm_quant(acc, xscale, wscale, res, w, _eps(eps), h, xq, xs, Mp, K)
     return h, xq, xs
 
 
@@ -246,8 +243,7 @@ def res_epilogue(acc, xscale, wscale, res, deps=()):
     """h = res + bf16(acc * xscale * wscale)."""
     Mp, N = acc.shape
     h = torch.empty_like(res)
-    _lib.call("scmx_res_norm_quant", _lib.ptr(acc), _lib.ptr(xscale), _lib.ptr(wscale), _lib.ptr(res), None, 0.0,
-              _lib.ptr(h), None, None, Mp, N, _lib.stream())
+    _lib.native().scmx_res_norm_quant(acc, xscale, wscale, res, None, 0.0, h, None, None, Mp, N)
     return h
 
 
@@ -256,31 +252,30 @@ def swiglu_quant(acc, xscale, wscale, dtype=torch.bfloat16, nt=512, deps=()):
     _check_dtype(dtype)
     Mp, F2 = acc.shape
     Fh = F2 // 2
-    xq = torch.empty((Mp, Fh), dtype=torch.int8, device=acc.device)
-    xs = torch.empty(Mp, dtype=torch.float32, device=acc.device)
-    _lib.call("scmx_swiglu_quant", _lib.ptr(acc), _lib.ptr(xscale), _lib.ptr(wscale), _lib.ptr(xq), _lib.ptr(xs), Mp, Fh,
-              _lib.stream())
+    xq = _lib.native().empty_i8(acc, Mp, Fh)
+    xs = _lib.native().empty_f32(acc, Mp)
+    _lib.native().scmx_swiglu_quant(acc, xscale, wscale, xq, xs, Mp, Fh)
     return xq, xs
 
 
-def _headnorm(acc, xscale, wscale, y, qn, kn, eps, L, hq, hk, d, dev):
-    q = torch.empty((hq, L, d), dtype=torch.bfloat16, device=dev)
-    k = torch.empty((hk, L, d), dtype=torch.bfloat16, device=dev)
-    v = torch.empty((hk, L, d), dtype=torch.bfloat16, device=dev)
-    _lib.call("scmx_qkv_headnorm", _lib.ptr(acc), _lib.ptr(xscale), _lib.ptr(wscale), _lib.ptr(y), _lib.ptr(qn),
-              _lib.ptr(kn), _eps(eps), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), L, hq, hk, d, _lib.stream())
+def _headnorm(acc, xscale, wscale, y, qn, kn, eps, L, hq, hk, d):
+    like = y if y is not None else acc
+    q = _lib.native().empty_bf16(like, hq, L, d)
+    k = _lib.native().empty_bf16(like, hk, L, d)
+    v = _lib.native().empty_bf16(like, hk, L, d)
+    _lib.native().scmx_qkv_headnorm(acc, xscale, wscale, y, qn, kn, _eps(eps), q, k, v, L, hq, hk, d)
     return q, k, v
 
 
 def qkv_epilogue_headnorm(acc, xscale, wscale, qn, kn, eps, L, hq, hk, d, dtype=torch.bfloat16, deps=()):
     """Qwen3: acc [Mp, (hq + 2 hk) d] -> q [hq, L, d], k [hk, L, d], v [hk, L, d] (q/k per-head RMSNorm)."""
     _check_dtype(dtype)
-    return _headnorm(acc, xscale, wscale, None, qn, kn, eps, L, hq, hk, d, acc.device)
+    return _headnorm(acc, xscale, wscale, None, qn, kn, eps, L, hq, hk, d)
 
 
 def qkv_headnorm_y(y, qn, kn, eps, L, hq, hk, d, deps=()):
     """Qwen3: bf16 y [Mp, (hq + 2 hk) d] -> q, k, v head-major with per-head RMSNorm of q and k."""
-    return _headnorm(None, None, None, y, qn, kn, eps, L, hq, hk, d, y.device)
+    return _headnorm(None, None, None, y, qn, kn, eps, L, hq, hk, d)
 
 
 def qkv_headnorm_rope(y, qn, kn, eps, L, hq, hk, d, kcache, vcache, pos, inv_freq, acc=None, xscale=None, wscale=None,
@@ -291,14 +286,14 @@ def qkv_headnorm_rope(y, qn, kn, eps, L, hq, hk, d, kcache, vcache, pos, inv_fre
     and returns the [hq, L, d] view of it: an attention output that inherits this layout is [L, hq * d] without a
     transposing copy."""
     src = y if y is not None else acc
-    q = torch.empty((L, hq, d) if token_major else (hq, L, d), dtype=torch.bfloat16, device=src.device)
+    q = _lib.native().empty_bf16(src, *((L, hq, d) if token_major else (hq, L, d)))
     assert kcache.shape == vcache.shape and kcache.shape[0] == hk and kcache.shape[2] == d
     assert kcache.dtype == torch.bfloat16 and inv_freq.dtype == torch.float32 and inv_freq.numel() == d // 2
     dev_pos = pos if torch.is_tensor(pos) else None
     assert dev_pos is None or dev_pos.dtype == torch.int64
-    _lib.call("scmx_qkv_headnorm_rope", _lib.ptr(acc), _lib.ptr(xscale), _lib.ptr(wscale), _lib.ptr(y), _lib.ptr(qn),
-              _lib.ptr(kn), _eps(eps), _lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache), L, hq, hk, d, _lib.ptr(inv_freq),
-              _lib.ptr(dev_pos), 0 if dev_pos is not None else int(pos), kcache.shape[1], int(token_major), _lib.stream())
+    _lib.native().scmx_qkv_headnorm_rope(acc, xscale, wscale, y, qn, kn, _eps(eps), q, kcache, vcache, L, hq, hk, d,
+                                         inv_freq, dev_pos, 0 if dev_pos is not None else int(pos), kcache.shape[1],
+                                         int(token_major))
     return q.transpose(0, 1) if token_major else q
 
 
@@ -311,8 +306,8 @@ def attn_splits(rows):
     return 1 if rows <= 1024 else 8 if rows <= 8192 else 16
 
 
-def _split_workspace(splits, hq, d, device):
-    return torch.empty(splits * hq * (d + 2), dtype=torch.float32, device=device) if splits > 1 else None
+def _split_workspace(splits, hq, d, like):
+    return _lib.native().empty_f32(like, splits * hq * (d + 2)) if splits > 1 else None
 
 
 def attn_decode(q, kcache, vcache, n, scale=None, splits=None):
@@ -321,14 +316,13 @@ def attn_decode(q, kcache, vcache, n, scale=None, splits=None):
     splits: row ranges per head (default: by n, or by the cache size when n lives on the device)."""
     hq, d = q.shape[0], q.shape[-1]
     hk, rows, _ = kcache.shape
-    out = torch.empty((1, hq * d), dtype=torch.bfloat16, device=q.device)
+    out = _lib.native().empty_bf16(q, 1, hq * d)
     dev_pos = n if torch.is_tensor(n) else None
     if splits is None:
         splits = attn_splits(rows if dev_pos is not None else int(n))
-    work = _split_workspace(splits, hq, d, q.device)
-    _lib.call("scmx_attn_decode", _lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(dev_pos),
-              0 if dev_pos is not None else int(n), _lib.ptr(out), hq, hk, d, rows,
-              float(scale if scale is not None else d ** -0.5), _lib.ptr(work), splits, _lib.stream())
+    work = _split_workspace(splits, hq, d, q)
+    _lib.native().scmx_attn_decode(q, kcache, vcache, dev_pos, 0 if dev_pos is not None else int(n), out, hq, hk, d, rows,
+                                   float(scale if scale is not None else d ** -0.5), work, splits)
     return out
 
 
@@ -340,9 +334,9 @@ def attn_prefill(q, kcache, vcache, off, scale=None):
     L, hq, d = q.shape
     hk, rows, _ = kcache.shape
     assert q.dtype == torch.bfloat16 and kcache.dtype == torch.bfloat16 and kcache.shape == vcache.shape
-    out = torch.empty((L, hq * d), dtype=torch.bfloat16, device=q.device)
-    _lib.call("scmx_attn_prefill", _lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(out), L, int(off), hq, hk, d,
-              rows, float(scale if scale is not None else d ** -0.5), _lib.stream())
+    out = _lib.native().empty_bf16(q, L, hq * d)
+    _lib.native().scmx_attn_prefill(q, kcache, vcache, out, L, int(off), hq, hk, d, rows,
+                                    float(scale if scale is not None else d ** -0.5))
     return out
 
 
@@ -353,24 +347,22 @@ def attn_decode_qkv(y, qn, kn, eps, hq, hk, d, kcache, vcache, pos, inv_freq, sc
     assert kcache.shape == vcache.shape and kcache.shape[0] == hk and kcache.shape[2] == d
     assert y.dtype == torch.bfloat16 and y.numel() == (hq + 2 * hk) * d and kcache.dtype == torch.bfloat16
     assert inv_freq.dtype == torch.float32 and inv_freq.numel() == d // 2
-    out = torch.empty((1, hq * d), dtype=torch.bfloat16, device=y.device)
+    out = _lib.native().empty_bf16(y, 1, hq * d)
     dev_pos = pos if torch.is_tensor(pos) else None
     assert dev_pos is None or dev_pos.dtype == torch.int64
     if splits is None:
         splits = attn_splits(kcache.shape[1] if dev_pos is not None else int(pos) + 1)
-    work = _split_workspace(splits, hq, d, y.device)
-    _lib.call("scmx_attn_decode_qkv", _lib.ptr(y), _lib.ptr(qn), _lib.ptr(kn), _eps(eps), _lib.ptr(inv_freq),
-              _lib.ptr(dev_pos), 0 if dev_pos is not None else int(pos), _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(out),
-              hq, hk, d, kcache.shape[1], float(scale if scale is not None else d ** -0.5), _lib.ptr(work), splits,
-              _lib.stream())
+    work = _split_workspace(splits, hq, d, y)
+    _lib.native().scmx_attn_decode_qkv(y, qn, kn, _eps(eps), inv_freq, dev_pos, 0 if dev_pos is not None else int(pos),
+                                       kcache, vcache, out, hq, hk, d, kcache.shape[1],
+                                       float(scale if scale is not None else d ** -0.5), work, splits)
     return out
 
 
 def qkv_fullnorm_y(y, qn, kn, eps, L, h, d, deps=()):
     """OLMoE: bf16 y [Mp, 3 h d] -> q, k, v [h, L, d] with RMSNorm over the full h*d-wide q and k."""
-    q, k, v = (torch.empty((h, L, d), dtype=torch.bfloat16, device=y.device) for _ in range(3))
-    _lib.call("scmx_qkv_fullnorm", _lib.ptr(y), _lib.ptr(qn), _lib.ptr(kn), _eps(eps), _lib.ptr(q), _lib.ptr(k),
-              _lib.ptr(v), L, h, d, _lib.stream())
+    q, k, v = (_lib.native().empty_bf16(y, h, L, d) for _ in range(3))
+    _lib.native().scmx_qkv_fullnorm(y, qn, kn, _eps(eps), q, k, v, L, h, d)
     return q, k, v
 
 
@@ -378,13 +370,12 @@ def qkv_fullnorm_rope(y, qn, kn, eps, L, h, d, kcache, vcache, pos, inv_freq):
     """qkv_fullnorm_y fused with the rotary embedding of q and k and the KV-cache append: k and v go to rows
     pos..pos+L-1 of kcache / vcache [h, rows, d]; returns the [h, L, d] view of q stored as [L, h, d].  pos: int, or an
     int64 device tensor."""
-    q = torch.empty((L, h, d), dtype=torch.bfloat16, device=y.device)
+    q = _lib.native().empty_bf16(y, L, h, d)
     assert kcache.shape == vcache.shape and kcache.shape[0] == h and kcache.shape[2] == d
     assert y.dtype == torch.bfloat16 and kcache.dtype == torch.bfloat16
     assert inv_freq.dtype == torch.float32 and inv_freq.numel() == d // 2
     dev_pos = pos if torch.is_tensor(pos) else None
     assert dev_pos is None or dev_pos.dtype == torch.int64
-    _lib.call("scmx_qkv_fullnorm_rope", _lib.ptr(y), _lib.ptr(qn), _lib.ptr(kn), _eps(eps), _lib.ptr(q), _lib.ptr(kcache),
-              _lib.ptr(vcache), L, h, d, _lib.ptr(inv_freq), _lib.ptr(dev_pos), 0 if dev_pos is not None else int(pos),
-              kcache.shape[1], 1, _lib.stream())
+    _lib.native().scmx_qkv_fullnorm_rope(y, qn, kn, _eps(eps), q, kcache, vcache, L, h, d, inv_freq, dev_pos,
+                                         0 if dev_pos is not None else int(pos), kcache.shape[1], 1)
     return q.transpose(0, 1)

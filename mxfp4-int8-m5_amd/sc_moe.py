@@ -24,10 +24,9 @@ def route(logits, k, renorm=True, shared_logit=None):
     if shared_logit is not None:
         shared_logit = shared_logit.reshape(M).contiguous()
     width = k + (shared_logit is not None)
-    inds = torch.empty((M, width), dtype=torch.int32, device=logits.device)
-    scores = torch.empty((M, width), dtype=torch.bfloat16, device=logits.device)
-    _lib.call("scmx_route_topk", _lib.ptr(logits), _lib.ptr(shared_logit), M, E, k, int(bool(renorm)), _lib.ptr(inds),
-              _lib.ptr(scores), _lib.stream())
+    inds = _lib.native().empty_i32(logits, M, width)
+    scores = _lib.native().empty_bf16(logits, M, width)
+    _lib.native().scmx_route_topk(logits, shared_logit, M, E, k, int(bool(renorm)), inds, scores)
     return inds, scores
 
 
@@ -36,14 +35,12 @@ def route_sort(inds, n_experts, tm):
     M, k = inds.shape
     R = M * k
     inds = inds.to(torch.int32).contiguous()
-    dev = inds.device
-    pos = torch.empty(R, dtype=torch.int32, device=dev)
-    tok = torch.empty(R + tm, dtype=torch.int32, device=dev)
-    es = torch.empty(R, dtype=torch.int32, device=dev)
-    off = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
-    ts = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
-    _lib.call("scmx_route_sort", _lib.ptr(inds), M, k, n_experts, tm, _lib.ptr(pos), _lib.ptr(tok), _lib.ptr(es),
-              _lib.ptr(off), _lib.ptr(ts), _lib.stream())
+    pos = _lib.native().empty_i32(inds, R)
+    tok = _lib.native().empty_i32(inds, R + tm)
+    es = _lib.native().empty_i32(inds, R)
+    off = _lib.native().empty_i32(inds, n_experts + 1)
+    ts = _lib.native().empty_i32(inds, n_experts + 1)
+    _lib.native().scmx_route_sort(inds, M, k, n_experts, tm, pos, tok, es, off, ts)
     return pos, tok, es, off, ts, -(-R // tm) + n_experts
 
 
@@ -65,10 +62,10 @@ def segments(expert_sorted, n_experts, tm):
     return off, tstart, -(-R // tm) + n_experts
 
 
-def _out(R, N, epi, dev):
+def _out(R, N, epi, like):
     if epi == 0:
-        return torch.empty((R, N), dtype=torch.int32, device=dev)
-    return torch.empty((R, N // 2 if epi == 3 else N), dtype=torch.bfloat16, device=dev)
+        return _lib.native().empty_i32(like, R, N)
+    return _lib.native().empty_bf16(like, R, N // 2 if epi == 3 else N)
 
 
 def moe_mm(xq, R, codes, bcodes, wscale, off, tstart, max_tiles, N, epi, xscale=None, dtype=torch.bfloat16,
@@ -80,10 +77,8 @@ def moe_mm(xq, R, codes, bcodes, wscale, off, tstart, max_tiles, N, epi, xscale=
     K = xq.shape[1]
     E = wscale.shape[0]
     assert xq.dtype == torch.int8 and (gather is not None or xq.shape[0] >= R)
-    out = _out(R, N, epi, xq.device)
-    _lib.call("scmx_moe_mm", fmt.c_struct(), _lib.ptr(xq), _lib.ptr(xscale), _lib.ptr(gather), R, _lib.ptr(codes),
-              _lib.ptr(bcodes), _lib.ptr(wscale), _lib.ptr(off), _lib.ptr(tstart), E, tile[0], N, K, epi, _lib.ptr(out),
-              _lib.stream())
+    out = _out(R, N, epi, xq)
+    _lib.native().scmx_moe_mm(fmt.c, xq, xscale, gather, R, codes, bcodes, wscale, off, tstart, E, tile[0], N, K, epi, out)
     return out
 
 
@@ -95,9 +90,8 @@ def moe_mm_i8(xq, R, wq, wscale, off, tstart, max_tiles, N, epi, xscale=None, dt
     if isinstance(wq, S.PackedWq):
         wq = wq.materialize()
     assert tuple(wq.shape) == (E * N, K)
-    out = _out(R, N, epi, xq.device)
-    _lib.call("scmx_moe_mm_i8", _lib.ptr(xq), _lib.ptr(xscale), _lib.ptr(gather), R, _lib.ptr(wq), _lib.ptr(wscale),
-              _lib.ptr(off), _lib.ptr(tstart), E, tile[0], N, K, epi, _lib.ptr(out), _lib.stream())
+    out = _out(R, N, epi, xq)
+    _lib.native().scmx_moe_mm_i8(xq, xscale, gather, R, wq, wscale, off, tstart, E, tile[0], N, K, epi, out)
     return out
 
 
@@ -123,9 +117,8 @@ def _combine(y, pos, scores, sscore, res, w, eps, M, quant):
     Mp, K = res.shape
     topk = scores.shape[1] + (1 if sscore is not None else 0)
     h = torch.empty_like(res)
-    xq = torch.empty((Mp, K), dtype=torch.int8, device=res.device) if quant else None
-    xs = torch.empty(Mp, dtype=torch.float32, device=res.device) if quant else None
-    _lib.call("scmx_moe_combine", _lib.ptr(y), _lib.ptr(pos), _lib.ptr(scores), _lib.ptr(sscore), _lib.ptr(res),
-              _lib.ptr(w) if quant else None, S._eps(eps) if quant else 0.0, _lib.ptr(h), _lib.ptr(xq), _lib.ptr(xs), M,
-              Mp, K, topk, _lib.stream())
+    xq = _lib.native().empty_i8(res, Mp, K) if quant else None
+    xs = _lib.native().empty_f32(res, Mp) if quant else None
+    _lib.native().scmx_moe_combine(y, pos, scores, sscore, res, w if quant else None, S._eps(eps) if quant else 0.0, h, xq,
+                                   xs, M, Mp, K, topk)
     return h, xq, xs
