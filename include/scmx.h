@@ -229,6 +229,10 @@ int scmx_qkv_fullnorm_rope(const uint16_t* y, const uint16_t* qn, const uint16_t
  * e2e/fused_qwen3.py:224-255). */
 int scmx_rmsnorm(const uint16_t* x, const uint16_t* w, float eps, uint16_t* out, int M, int K, void* stream);
 
+/* out = x w^T of T rows x [M, K], w [N, K] -> T[M, N] with float32 sums: the linears of a model that stay T (output head,
+ * router; array ops in the reference), for M <= 16 rows.  K % 64 == 0, x and w 16-byte aligned. */
+int scmx_linear_bf16(const uint16_t* x, const uint16_t* w, uint16_t* out, int M, int N, int K, void* stream);
+
 /* ---- decode --------------------------------------------------------------------------------------------------- */
 
 /* W4A8 GEMV on packed weights, `batch` input rows sharing one weight stream (batch 1, 2, 4 or 8; the reference has

@@ -48,6 +48,7 @@ SIGNATURES = {
     "scmx_qkv_fullnorm": (_I, [_P, _P, _P, _F, _P, _P, _P, _I, _I, _I, _P]),
     "scmx_qkv_fullnorm_rope": (_I, [_P, _P, _P, _F, _P, _P, _P, _I, _I, _I, _P, _P, _L, _I, _I, _P]),
     "scmx_rmsnorm": (_I, [_P, _P, _F, _P, _I, _I, _P]),
+    "scmx_linear_bf16": (_I, [_P, _P, _P, _I, _I, _I, _P]),
     "scmx_gemv": (_I, [_FMT, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _F, _I, _I, _I, _P, _I, _I, _I, _P]),
     "scmx_gemv_rows_workspace": (_Z, [_FMT, _I, _I, _I, _I]),
     "scmx_gemv_rows": (_I, [_FMT, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _F, _I, _I, _I, _P, _Z, _P]),

@@ -167,7 +167,7 @@ PyMODINIT_FUNC PyInit__binding() {
     static PyMethodDef methods[] = {
         ENTRY(scmx_unpack_i8), ENTRY(scmx_act_quant), ENTRY(scmx_act_quant_blocked), ENTRY(scmx_mm_i8_i32), ENTRY(scmx_mm_epi),
         ENTRY(scmx_mm_w4a8), ENTRY(scmx_mm_w4a8_blocked), ENTRY(scmx_linear_w4a8), ENTRY(scmx_linear_w4a8_static),
-        ENTRY(scmx_rmsnorm_quant), ENTRY(scmx_rmsnorm_quant_blocked), ENTRY(scmx_rmsnorm), ENTRY(scmx_res_norm_quant),
+        ENTRY(scmx_rmsnorm_quant), ENTRY(scmx_rmsnorm_quant_blocked), ENTRY(scmx_rmsnorm), ENTRY(scmx_linear_bf16), ENTRY(scmx_res_norm_quant),
         ENTRY(scmx_swiglu_quant), ENTRY(scmx_qkv_headnorm), ENTRY(scmx_qkv_headnorm_rope), ENTRY(scmx_qkv_fullnorm),
         ENTRY(scmx_qkv_fullnorm_rope), ENTRY(scmx_attn_decode), ENTRY(scmx_attn_decode_qkv), ENTRY(scmx_attn_prefill),
         ENTRY(scmx_gemv), ENTRY(scmx_gemv_rows), ENTRY(scmx_route_topk), ENTRY(scmx_route_sort), ENTRY(scmx_moe_mm),

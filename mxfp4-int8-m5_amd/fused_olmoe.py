@@ -127,9 +127,9 @@ class FusedOlmoe:
 
     def route(self, nw, xn, M):
         """mlx_lm's OlmoeSparseMoeBlock routing on the bf16 normalized rows (e2e/fused_olmoe.py:183-192): bf16 router
-        linear (an array op, as in the reference), then one kernel for the float32 softmax, the k largest probabilities
+        linear (an array op in the reference and beyond 16 rows), then one kernel for the float32 softmax, the k largest probabilities
         and the optional renormalisation."""
-        logits = xn[:M] @ nw["mlp.gate"].T
+        logits = S.linear_bf16(xn[:M], nw["mlp.gate"])
         return sc_moe.route(logits, self.args.num_experts_per_tok, renorm=self.args.norm_topk_prob)
 
     def _experts(self, xq, xs, inds, scores, h, nn, ex, L, quant=True):
@@ -187,7 +187,7 @@ class FusedOlmoe:
         return S.rmsnorm(h[:L], self.norm, self.eps)
 
     def logits(self, h):
-        return h @ self.lm_head.T
+        return S.linear_bf16(h, self.lm_head)
 
     def __call__(self, ids, cache=None):
         return self.logits(self.hidden(ids, cache))

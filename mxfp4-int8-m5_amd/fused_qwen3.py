@@ -207,7 +207,7 @@ class FusedQwen3:
         return S.rmsnorm(h[:L], self.norm, self.eps)
 
     def logits(self, h):
-        return h @ self.lm_head.T
+        return S.linear_bf16(h, self.lm_head)
 
     def __call__(self, ids, cache=None):
         """Logits for every position."""

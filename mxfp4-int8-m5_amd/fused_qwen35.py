@@ -39,9 +39,9 @@ class Qwen35MoeArgs:
 
 def route(gate_w, sg_w, xn, k):
     """Qwen3NextSparseMoeBlock routing on bf16 normalized rows xn [M, D] (e2e/fused_qwen35.py:171-180): the two bf16
-    linears are array ops as in the reference; one kernel does softmax (float32) -> k largest -> renormalise and
+    linears are array ops in the reference; one kernel does softmax (float32) -> k largest -> renormalise and
     appends the shared expert as slot k with index E and score sigmoid(xn . sg_w).  -> (inds int32, scores bf16) [M, k+1]."""
-    return sc_moe.route(xn @ gate_w.T, k, renorm=True, shared_logit=xn @ sg_w.T)
+    return sc_moe.route(S.linear_bf16(xn, gate_w), k, renorm=True, shared_logit=S.linear_bf16(xn, sg_w))
 
 
 def pack_experts(gate, up, down, fmt=None, fmt_name=None):
