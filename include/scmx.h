@@ -213,6 +213,12 @@ int scmx_attn_decode_qkv(const uint16_t* y, const uint16_t* qn, const uint16_t* 
 int scmx_attn_prefill(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, uint16_t* out, int L, int off,
                       int hq, int hk, int d, int cache_rows, float scale, void* stream);
 
+/* scmx_attn_prefill with the keys cut into up to `splits` (1..64) ranges, a workgroup per head, 128 queries and range, and
+ * a second launch that joins the ranges' float32 results out of `workspace`, float [splits * L * hq * (d + 2)], 16-byte
+ * aligned: for few new tokens behind a long cache.  splits == 1 needs no workspace (NULL) and is scmx_attn_prefill. */
+int scmx_attn_prefill_split(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, uint16_t* out, int L, int off,
+                            int hq, int hk, int d, int cache_rows, float scale, float* workspace, int splits, void* stream);
+
 /* OLMoE q/k/v split with RMSNorm over the full h*d width.  Replaces qkv_fullnorm_y, e2e/sc_kernels.py:390-423,
  * 629-637. */
 int scmx_qkv_fullnorm(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q,

@@ -352,17 +352,37 @@ def attn_decode(q, kcache, vcache, n, scale=None, splits=None):
     return out
 
 
-def attn_prefill(q, kcache, vcache, off, scale=None):
+def attn_prefill_splits(L, off, hq):
+    """Key ranges for the attention of L new tokens behind `off` cached ones.  Unsplit, a workgroup per head and 128 queries
+    walks all keys, 128 in 2 us.  Ranges help while all workgroups run at once (one a CU) and down to a range of 256 keys
+    (128 in short contexts); joining them costs a launch and the ranges' traffic, which grows with L hq.  Measured, us
+    whole / split, 16 heads, L behind off: 32 behind 300 11.4 / 10.6; 8 behind 500 13.2 / 10.8; 30 behind 2000 36 / 16; 100
+    behind 4000 73 / 23; 300 behind 3000 61 / 29; 600 behind 4000 82 / 43; 1000 behind 1000 41 / 33; and where the line is:
+    128 behind 256 (two steps of 128 keys fewer) 13.8 / 14.0; 300 behind 300 17.6 / 18.3 (three fewer); 300 behind 500
+    20.0 / 19.4 (five); 1000 alone 23.7 / 24.1 (four); 1500 alone, which fills more than half the CUs, 32 / 38."""
+    tiles, pairs = -(-L // 128) * hq, -(-(off + L) // 128)
+    if not 0 < tiles <= 128:
+        return 1
+    splits = min(64, 256 // tiles, pairs if pairs <= 4 else max(4, pairs // 2))
+    saved = pairs - -(-pairs // splits)
+    return splits if saved >= (2 if L * hq <= 1024 else 3 if L <= 128 else 5) else 1
+
+
+def attn_prefill(q, kcache, vcache, off, scale=None, splits=None):
     """Causal attention of L new tokens: q bf16 [hq, L, d], best as the view of [L, hq, d] storage that
     qkv_headnorm_rope returns with token_major=True (any other layout is copied into that one), caches [hk, rows, d]
-    whose rows off .. off+L-1 hold the new tokens' keys and values -> bf16 [L, hq * d].  Head dim 128."""
+    whose rows off .. off+L-1 hold the new tokens' keys and values -> bf16 [L, hq * d].  Head dim 128.
+    splits: ranges the keys are cut into (default: by the sizes)."""
     q = q.transpose(0, 1).contiguous()   # [L, hq, d] storage; no copy when q already is a view of it
     L, hq, d = q.shape
     hk, rows, _ = kcache.shape
     assert q.dtype == torch.bfloat16 and kcache.dtype == torch.bfloat16 and kcache.shape == vcache.shape
     out = _lib.native().empty_bf16(q, L, hq * d)
-    _lib.native().scmx_attn_prefill(q, kcache, vcache, out, L, int(off), hq, hk, d, rows,
-                                    float(scale if scale is not None else d ** -0.5))
+    if splits is None:
+        splits = attn_prefill_splits(L, int(off), hq)
+    work = _split_workspace(splits, L * hq, d, q)
+    _lib.native().scmx_attn_prefill_split(q, kcache, vcache, out, L, int(off), hq, hk, d, rows,
+                                          float(scale if scale is not None else d ** -0.5), work, splits)
     return out
 
 
