@@ -359,7 +359,7 @@ def attn_prefill_splits(L, off, hq):
     whole / split, 16 heads, L behind off: 32 behind 300 11.4 / 10.6; 8 behind 500 13.2 / 10.8; 30 behind 2000 36 / 16; 100
     behind 4000 73 / 23; 300 behind 3000 61 / 29; 600 behind 4000 82 / 43; 1000 behind 1000 41 / 33; and where the line is:
     128 behind 256 (two steps of 128 keys fewer) 13.8 / 14.0; 300 behind 300 17.6 / 18.3 (three fewer); 300 behind 500
-    20.0 / 19.4 (five); 1000 alone 23.7 / 24.1 (four); 1500 alone, which fills more than half the CUs, 32 / 38."""
+    20.0 / 19.4 (five); 1000 alone 23.6 / 23.5 (four); 1500 behind 1500, which fills more than half the CUs, 55 / 62."""
     tiles, pairs = -(-L // 128) * hq, -(-(off + L) // 128)
     if not 0 < tiles <= 128:
         return 1
