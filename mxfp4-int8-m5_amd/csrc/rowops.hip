@@ -785,6 +785,93 @@ __global__ __launch_bounds__(NT) void moe_combine_kernel(const uint16_t* __restr
     block_quant_row(nrow_s, K, xq + size_t(row) * K, xs + row, red);
 }
 
+// The same with a wave per row and the row in its registers from the first load to the codes: no LDS, no barriers, and the
+// rows' loads overlap freely.  Bound: HBM, top-k rows of y read per row written.  Same arithmetic, same order of sums, same bits.
+template <int CH>
+__global__ __launch_bounds__(256) void moe_combine_wave_kernel(const uint16_t* __restrict__ y, const int32_t* __restrict__ pos,
+                                                               const uint16_t* __restrict__ scores, const uint16_t* __restrict__ sscore,
+                                                               const uint16_t* __restrict__ res, const uint16_t* __restrict__ w,
+                                                               float eps, uint16_t* __restrict__ h, int8_t* __restrict__ xq,
+                                                               float* __restrict__ xs, int M, int Mp, int topk) {
+    constexpr int K = 512 * CH;
+    const int row = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
+    if (row >= Mp) return;   // wave-uniform
+    const int nsc = sscore ? topk - 1 : topk;
+    auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
+    auto hi = [](uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); };
+    u32x4 v[CH];
+    const u32x4* rrow = reinterpret_cast<const u32x4*>(res + size_t(row) * K) + lane;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) v[j] = rrow[64 * j];
+    if (row < M) {
+        float acc[CH][8];
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[j][i] = 0.0f;
+        for (int s0 = 0; s0 < topk; s0 += 2) {   // two slots' rows requested together, added in slot order
+            u32x4 yv[2][CH];
+            float sc[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int s = s0 + u;
+                if (s < topk) {
+                    sc[u] = bf16_to_f32((sscore && s == topk - 1) ? sscore[row] : scores[size_t(row) * nsc + s]);
+                    const u32x4* yrow = reinterpret_cast<const u32x4*>(y + size_t(pos[size_t(row) * topk + s]) * K) + lane;
+#pragma unroll
+                    for (int j = 0; j < CH; ++j) yv[u][j] = yrow[64 * j];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                if (s0 + u >= topk) break;
+#pragma unroll
+                for (int j = 0; j < CH; ++j)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float yf = i & 1 ? hi(yv[u][j][i >> 1]) : lo(yv[u][j][i >> 1]);
+                        acc[j][i] = round_bf16(__fadd_rn(round_bf16(__fmul_rn(yf, sc[u])), acc[j][i]));
+                    }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float a = __fadd_rn(lo(v[j][i]), acc[j][2 * i]), b = __fadd_rn(hi(v[j][i]), acc[j][2 * i + 1]);
+                v[j][i] = uint32_t(f32_to_bf16(a)) | (uint32_t(f32_to_bf16(b)) << 16);
+            }
+    }
+    u32x4* hrow = reinterpret_cast<u32x4*>(h + size_t(row) * K) + lane;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) hrow[64 * j] = v[j];
+    if (!xq) return;
+    const float inv = inv_rms(wave_row_sumsq(v), K, eps);
+    const u32x4* wrow = reinterpret_cast<const u32x4*>(w) + lane;
+    float amax = 0.0f;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        v[j] = norm8(v[j], wrow[64 * j], inv);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fmaxf(fabsf(lo(v[j][e])), fabsf(hi(v[j][e]))));
+    }
+    amax = wave_max(amax);
+    const float s = __fdiv_rn(amax, 127.0f);
+    const float qi = s > 0.0f ? __fdiv_rn(1.0f, s) : 0.0f;
+    u32x2* qrow = reinterpret_cast<u32x2*>(xq + size_t(row) * K) + lane;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        uint32_t o[2] = {0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[e >> 1] |= (uint32_t(quant_code(lo(v[j][e]), qi)) & 0xFFu) << (16 * (e & 1));
+            o[e >> 1] |= (uint32_t(quant_code(hi(v[j][e]), qi)) & 0xFFu) << (16 * (e & 1) + 8);
+        }
+        qrow[64 * j] = u32x2{o[0], o[1]};
+    }
+    if (lane == 0) xs[row] = s;
+}
+
 // fn(K / 512 as a compile-time constant), 1 ... 8: the kernels that keep a row in a wave's registers.
 template <typename Fn>
 static void by_chunks(int chunks, Fn&& fn) {
@@ -1133,6 +1220,21 @@ int scmx_moe_combine(const uint16_t* y, const int32_t* pos, const uint16_t* scor
         return SCMX_ERR_ARG;
     }
     if (Mp == 0) return SCMX_OK;
+    // A wave per row from 1024 rows on, where the waves fill the chip; below, a row's workgroup is the shorter chain.  Eight
+    // slots, us by workgroup / by wave: 1024 x 2048 13.8 / 11.2, 3000 x 2048 29.7 / 24.4, 8192 x 2048 76 / 74, without the
+    // codes 21.8 / 20.1 at 3000; at K = 4096 a lane's registers leave too few waves (1024 rows without codes 15.2 / 16.3).
+    if (Mp >= 1024 && K % 512 == 0 && K <= 2048 && (uintptr_t(y) | uintptr_t(res) | uintptr_t(h)) % 16 == 0 &&
+        (!xq || (uintptr_t(w) | uintptr_t(xq)) % 16 == 0)) {
+        auto go = [&](auto kernel) {
+            kernel<<<dim3((unsigned(Mp) + 3u) / 4u), dim3(256), 0, (hipStream_t)stream>>>(y, pos, scores, sscore, res, w, eps, h, xq,
+                                                                                         xs, M, Mp, topk);
+        };
+        if (K == 512) go(moe_combine_wave_kernel<1>);
+        else if (K == 1024) go(moe_combine_wave_kernel<2>);
+        else if (K == 1536) go(moe_combine_wave_kernel<3>);
+        else go(moe_combine_wave_kernel<4>);
+        return check_launch("moe_combine");
+    }
     if (K % 8 == 0 && (uintptr_t(y) | uintptr_t(res) | uintptr_t(h)) % 16 == 0)
         moe_combine_kernel<8><<<dim3(Mp), dim3(NT), size_t(K) * 4 + 72 * 4, (hipStream_t)stream>>>(y, pos, scores, sscore, res,
                                                                                                     w, eps, h, xq, xs, M, K, topk);
