@@ -277,8 +277,8 @@ __device__ __forceinline__ int family_index(const FamilyArgs& f, float x) {   //
     for (int i = 0; i < 7; ++i) idx += int(a > f.cut[i]);
     return idx;
 }
-__device__ __forceinline__ float family_level(const FamilyArgs& f, float a) {   // its magnitude, for a >= 0
-    float v = f.cb[0];
+__device__ __forceinline__ float family_level(const FamilyArgs& f, float a) {   // sign(a) times its magnitude, for a >= 0
+    float v = a > 0.0f ? f.cb[0] : 0.0f;   // (a zero has no sign: it costs nothing also where the smallest magnitude is not 0)
 #pragma unroll
     for (int i = 0; i < 7; ++i) v = a > f.cut[i] ? f.cb[i + 1] : v;
     return v;

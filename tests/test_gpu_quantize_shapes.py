@@ -62,3 +62,26 @@ def test_family(n, k, as_bf16, shift, name):
     dc, db, dw, _ = P.pack_matrix(_device(w, as_bf16, shift), name)
     assert np.array_equal(host(dw), ws) and np.array_equal(host(db), bc)
     assert np.array_equal(host(dc).view(np.uint32), codes)
+
+
+@pytest.mark.parametrize("block", [16, 32])
+@pytest.mark.parametrize("as_bf16", [False, True])
+def test_family_codebook_without_a_zero(monkeypatch, as_bf16, block):
+    """Smallest magnitude 1: a zero weight has no sign, costs nothing whatever the scale, and is stored as code 0."""
+    from mxfp4_int8_m5_amd import pack_format as P
+    monkeypatch.setitem(family.CODEBOOKS, "one", (1, 2, 3, 4, 5, 6, 7, 8))
+    fam = family.Family("one", block, tuple(range(1, 11)))
+    sf = fam.storage()
+    rng = np.random.default_rng(block)
+    w = llm_weights(rng, 24, 512).astype(F32)
+    w[rng.random(w.shape) < 0.4] = 0.0
+    w[0] = 0.0
+    if as_bf16:
+        w = bf16.from_bits(bf16.to_bits(w))
+    _, qi, base, scales = family.quantize(w, fam)
+    m = np.rint(scales / base[:, None]).astype(np.int64)
+    idx = np.searchsorted(sf.code_mag, np.abs(qi) // np.repeat(m, block, axis=1))
+    codes, bc, ws = layout.pack_rows((idx | (qi < 0) << 3).astype(np.uint8), np.searchsorted(sf.mult, m).astype(np.uint8), base, sf)
+    dc, db, dw, _ = P.pack_matrix(_device(w, as_bf16, 0), "one", product_format(sf))
+    assert np.array_equal(host(dw), ws) and np.array_equal(host(db), bc)
+    assert np.array_equal(host(dc).view(np.uint32), codes)
