@@ -166,9 +166,7 @@ class FusedOlmoe:
         S.set_format(self.fmt)
         a = self.args
         cache = cache if cache is not None else self.make_cache(max(4096, ids.numel()))
-        L = ids.numel()
-        Mp = S.pad_rows(L)
-        h = embed_rows(self.embed, ids, Mp)
+        h, L, Mp = embed_rows(self.embed, ids)
         nl = len(self.layers)
         xq, xs = S.rmsnorm_quant(h, self.layers[0][0]["input_layernorm"], self.eps, Mp)
         for i, (nw, ws, ex) in enumerate(self.layers):

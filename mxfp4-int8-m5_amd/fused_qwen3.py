@@ -60,14 +60,19 @@ class KVCache:
         return self.k[:, :self.offset], self.v[:, :self.offset]
 
 
-def embed_rows(embed, ids, Mp):
-    """The embeddings of ids [L] followed by zero rows up to Mp."""
+def embed_rows(embed, ids):
+    """(h, L, Mp): the embeddings of ids [L], which index rows as they do in embed[ids] (negative ones count from the
+    end), followed by zero rows up to Mp, a whole number of row tiles."""
     ids = ids.reshape(-1).to(embed.device)
+    if ids.dtype in (torch.bool, torch.uint8):   # to indexing these are masks
+        ids = ids.nonzero().reshape(-1)
+    L = ids.numel()
+    Mp = S.pad_rows(L)
     h = torch.empty((Mp, embed.shape[1]), dtype=embed.dtype, device=embed.device)
-    torch.index_select(embed, 0, ids, out=h[:ids.numel()])
-    if Mp > ids.numel():
-        h[ids.numel():].zero_()
-    return h
+    torch.ops.aten.index.Tensor_out(embed, [ids], out=h[:L])   # the indexing op, into place
+    if Mp > L:
+        h[L:].zero_()
+    return h, L, Mp
 
 
 class FusedQwen3:
@@ -146,11 +151,6 @@ class FusedQwen3:
         # this is a view; contiguous() copies only if a backend chose another layout
         return o[0].transpose(0, 1).reshape(L, -1).contiguous()
 
-    def _embed(self, ids):
-        L = ids.numel()
-        Mp = S.pad_rows(L)
-        return embed_rows(self.embed, ids, Mp), L, Mp
-
     # ---- prefill ------------------------------------------------------------------------------------------------
     def hidden(self, ids, cache=None):
         """Final normed hidden states [L, D] for prompt ids [L] (prefill into a fresh or offset cache)."""
@@ -161,7 +161,7 @@ class FusedQwen3:
     def _hidden_gemm_epi(self, ids, cache):
         a = self.args
         hq, hk, d = a.num_attention_heads, a.num_key_value_heads, a.head_dim
-        h, L, Mp = self._embed(ids)
+        h, L, Mp = embed_rows(self.embed, ids)
         nl = len(self.layers)
         # prefill-sized GEMMs on packed weights read their activations in 32x32 blocks (the quantizers write either layout)
         blk = {g: isinstance(w.unpack(), S.PackedWq) and S.prefers_blocked(Mp, w.N, w.K) for g, w in self.layers[0][1].items()}
@@ -185,7 +185,7 @@ class FusedQwen3:
     def _hidden_row_epi(self, ids, cache):
         a = self.args
         hq, hk, d = a.num_attention_heads, a.num_key_value_heads, a.head_dim
-        h, L, Mp = self._embed(ids)
+        h, L, Mp = embed_rows(self.embed, ids)
         nl = len(self.layers)
         xq, xs = S.rmsnorm_quant(h, self.layers[0][0]["input_layernorm"], self.eps, Mp)
         for i, (nw, ws) in enumerate(self.layers):
