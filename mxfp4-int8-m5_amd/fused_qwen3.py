@@ -69,7 +69,8 @@ def embed_rows(embed, ids):
     L = ids.numel()
     Mp = S.pad_rows(L)
     h = torch.empty((Mp, embed.shape[1]), dtype=embed.dtype, device=embed.device)
-    torch.ops.aten.index.Tensor_out(embed, [ids], out=h[:L])   # the indexing op, into place
+    # the indexing op, into place; out= takes no tensor that requires grad, and no gradient passes the kernels behind it
+    torch.ops.aten.index.Tensor_out(embed.detach(), [ids], out=h[:L])
     if Mp > L:
         h[L:].zero_()
     return h, L, Mp

@@ -31,3 +31,9 @@ def test_rows_on_the_gpu(dtype, where):
     ids = torch.arange(-150, 150, dtype=dtype)
     h, L, Mp = embed_rows(EMBED.cuda(), ids.to(where))
     assert (L, Mp) == (300, 384) and torch.equal(h[:L].cpu(), EMBED[ids.long()]) and not h[L:].any()
+
+
+def test_embedding_that_requires_grad():
+    """A model built from named_parameters(): the kernels behind the embedding cut the graph, so nothing is lost here."""
+    h, L, _ = embed_rows(EMBED.clone().requires_grad_(), torch.tensor([1, 2]))
+    assert torch.equal(h[:L], EMBED[1:3])
