@@ -228,10 +228,12 @@ def linear_bf16(x, w):
     16 rows the library's kernel, which reads w once at 5.5-6.3 TB/s (one row against 151936 x 2048: 112 us, the array op
     203; against 50304 x 2048: 33 / 31; a router of 64 x 2048: 7.4 / 18.7 a call) while the rows' fragments stay in
     registers: K up to 2048, beyond it for two rows (32000 x 4096: 41 us for one row, 60 for sixteen, the array op 41-43).
-    More rows, other types and layouts, and callers that differentiate, trace or cast the product get the array op."""
+    More rows, other types and layouts, tensors off the current device, and callers that differentiate, trace or cast the
+    product get the array op."""
     if (type(x) is type(w) is torch.Tensor and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= 16 and w.shape[0]
             and x.shape[1] == w.shape[1] and x.shape[1] and x.shape[1] % 64 == 0
             and (x.shape[1] <= 2048 or x.shape[0] <= 2) and x.is_cuda and x.device == w.device
+            and x.device.index == torch.cuda.current_device()   # where the binding launches
             and x.dtype == w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
             and not _transformed(x, w) and not (x.data_ptr() | w.data_ptr()) % 16):
         out = _lib.native().empty_bf16(x, x.shape[0], w.shape[0])
