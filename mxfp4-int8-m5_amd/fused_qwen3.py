@@ -25,6 +25,7 @@ from . import sc_kernels as S
 from .sc_weights import GROUPS, PackedWeight, pack_weights
 
 BF = torch.bfloat16
+rms_norm = S.rms_norm
 
 
 @dataclass

@@ -215,12 +215,20 @@ def rmsnorm_quant_n(x, w, eps, Mp=None, deps=(), blocked=False):
 
 
 def rmsnorm(x, w, eps):
-    """RMSNorm of bf16 rows x [M, K] -> bf16 [M, K]."""
-    M, K = x.shape
-    assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-    out = torch.empty_like(x)
-    _lib.native().scmx_rmsnorm(x, w, _eps(eps), out, M, K)
-    return out
+    """RMSNorm of bf16 rows x [M, K] -> bf16 [M, K] (K % 4 == 0, K <= 16384).  Other shapes, types and layouts, tensors off
+    the current device, and callers that differentiate, trace or cast the norm get the array op."""
+    if (_plain(x, w) and x.dim() == 2 and w.shape == x.shape[1:] and x.numel() and x.shape[1] % 4 == 0 and x.shape[1] <= 16384
+            and not (x.data_ptr() | w.data_ptr()) % 8):
+        out = _lib.native().empty_bf16(x, *x.shape)
+        _lib.native().scmx_rmsnorm(x, w, _eps(eps), out, *x.shape)
+        return out
+    return rms_norm(x, w, eps)
+
+
+def rms_norm(x, w, eps):
+    """RMSNorm as array ops, whatever the shape and type."""
+    v = x.float()
+    return (v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + eps)).to(x.dtype) * w
 
 
 def linear_bf16(x, w):
@@ -230,25 +238,26 @@ def linear_bf16(x, w):
     registers: K up to 2048, beyond it for two rows (32000 x 4096: 41 us for one row, 60 for sixteen, the array op 41-43).
     More rows, other types and layouts, tensors off the current device, and callers that differentiate, trace or cast the
     product get the array op."""
-    if (type(x) is type(w) is torch.Tensor and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= 16 and w.shape[0]
+    if (_plain(x, w) and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= 16 and w.shape[0]
             and x.shape[1] == w.shape[1] and x.shape[1] and x.shape[1] % 64 == 0
-            and (x.shape[1] <= 2048 or x.shape[0] <= 2) and x.is_cuda and x.device == w.device
-            and x.device.index == torch.cuda.current_device()   # where the binding launches
-            and x.dtype == w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
-            and not _transformed(x, w) and not (x.data_ptr() | w.data_ptr()) % 16):
+            and (x.shape[1] <= 2048 or x.shape[0] <= 2) and not (x.data_ptr() | w.data_ptr()) % 16):
         out = _lib.native().empty_bf16(x, x.shape[0], w.shape[0])
         _lib.native().scmx_linear_bf16(x, w, out, x.shape[0], w.shape[0], x.shape[1])
         return out
     return x @ w.T
 
 
-def _transformed(*ts):
-    """Whether torch would do more with an op on these tensors than run it: autograd (reverse or forward), functorch,
-    autocast, a dispatch or function mode, tracing or compilation."""
-    return (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch._C._functorch.maybe_current_level() is not None or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
-            or any(t.requires_grad for t in ts))
+def _plain(x, w):
+    """Whether a kernel may stand in for an array op on x and w: contiguous bf16 tensors on the current device (where the
+    binding launches) with which torch would do no more than run the op -- no subclass, autograd (reverse or forward),
+    functorch, autocast, dispatch or function mode, tracing or compilation."""
+    return (type(x) is type(w) is torch.Tensor and x.is_cuda and x.device == w.device
+            and x.device.index == torch.cuda.current_device() and x.dtype == w.dtype == torch.bfloat16
+            and x.is_contiguous() and w.is_contiguous()
+            and not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                     or torch._C._functorch.maybe_current_level() is not None
+                     or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0
+                     or torch._C._len_torch_function_stack() > 0 or x.requires_grad or w.requires_grad))
 
 
 def prefers_blocked(M, N, K):

@@ -51,3 +51,27 @@ def test_rmsnorm_rows(S, m, k):
     rng = np.random.default_rng(m * k)
     x, w = llm_acts(rng, m, k)[0], llm_acts(rng, 1, k)[0][0]
     assert np.array_equal(host(S.rmsnorm(dev(x), dev(w), 1e-6)), linear.rmsnorm(x, w, 1e-6))
+
+
+def test_rmsnorm_array_op(S, monkeypatch):
+    """Callers that differentiate or transform the norm, and tensors off the current device, get the array op."""
+    from mxfp4_int8_m5_amd.fused_qwen3 import rms_norm
+    x, w = torch.randn(5, 256, device="cuda").to(torch.bfloat16), torch.rand(256, device="cuda").to(torch.bfloat16)
+    ref = rms_norm(x, w, 1e-6)
+    for t in (x, w):
+        g = t.clone().requires_grad_()
+        a = (g, w) if t is x else (x, g)
+        S.rmsnorm(*a, 1e-6).float().sum().backward()
+        want = t.clone().requires_grad_()
+        rms_norm(*((want, w) if t is x else (x, want)), 1e-6).float().sum().backward()
+        assert torch.equal(g.grad, want.grad)
+        with torch.no_grad():
+            assert not S.rmsnorm(*a, 1e-6).requires_grad
+    assert torch.equal(torch.func.vmap(lambda r: S.rmsnorm(r[None], w, 1e-6)[0])(x), ref)
+    assert S.rmsnorm(x[:0], w, 1e-6).shape == (0, 256)
+    assert torch.equal(S.rmsnorm(x.t().contiguous().t(), w, 1e-6), ref)          # columns first
+    odd = torch.randn(3, 250, device="cuda").to(torch.bfloat16)
+    assert torch.equal(S.rmsnorm(odd, w[:250], 1e-6), rms_norm(odd, w[:250], 1e-6))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
+    monkeypatch.setattr(S._lib, "native", lambda: pytest.fail("launched on the current device"))
+    assert torch.equal(S.rmsnorm(x, w, 1e-6), ref)
