@@ -225,7 +225,7 @@ int scmx_qkv_fullnorm(const uint16_t* y, const uint16_t* qn, const uint16_t* kn,
                       uint16_t* k, uint16_t* v, int L, int h, int d, void* stream);
 
 /* scmx_qkv_fullnorm followed by the rotary embedding of q and k and the append to the KV cache; the remaining arguments as
- * in scmx_qkv_headnorm_rope (hq = hk = h; d <= 512).  Fuses what the model integration does with array ops after qkv_fullnorm_y
+ * in scmx_qkv_headnorm_rope (hq = hk = h).  Fuses what the model integration does with array ops after qkv_fullnorm_y
  * (e2e/fused_olmoe.py:197-203). */
 int scmx_qkv_fullnorm_rope(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q,
                            uint16_t* kcache, uint16_t* vcache, int L, int h, int d, const float* inv_freq,

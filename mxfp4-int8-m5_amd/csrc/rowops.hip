@@ -1119,8 +1119,11 @@ static int qkv_fullnorm(const char* who, const uint16_t* y, const uint16_t* qn, 
         };
         by_chunks(W / 512, go);
     } else {
-        qkv_fullnorm_kernel<<<dim3(L), dim3(NT), size_t(W) * 2 + (72 + (rope.inv_freq ? d : 0)) * 4, st>>>(
-            y, qn, kn, eps, q, k, v, L, h, d, rope);
+        const size_t smem = size_t(W) * 2 + (72 + (rope.inv_freq ? d : 0)) * 4;   // 96 KB and some at W = d = 16384
+        if (smem > 64 * 1024)
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(qkv_fullnorm_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      int(smem));
+        qkv_fullnorm_kernel<<<dim3(L), dim3(NT), smem, st>>>(y, qn, kn, eps, q, k, v, L, h, d, rope);
     }
     return check_launch(who);
 }
@@ -1134,8 +1137,8 @@ int scmx_qkv_fullnorm(const uint16_t* y, const uint16_t* qn, const uint16_t* kn,
 int scmx_qkv_fullnorm_rope(const uint16_t* y, const uint16_t* qn, const uint16_t* kn, float eps, uint16_t* q,
                            uint16_t* kcache, uint16_t* vcache, int L, int h, int d, const float* inv_freq,
                            const int64_t* pos_dev, int64_t pos0, int cache_rows, int q_token_major, void* stream) {
-    if (!inv_freq || d > 512) {
-        set_error("qkv_fullnorm_rope: null pointer argument or a head dim above 512 (d=%d)", d);
+    if (!inv_freq) {
+        set_error("qkv_fullnorm_rope: null pointer argument");
         return SCMX_ERR_ARG;
     }
     if (cache_rows < L || (!pos_dev && (pos0 < 0 || pos0 > int64_t(cache_rows) - L))) {

@@ -75,3 +75,9 @@ def test_rmsnorm_array_op(S, monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
     monkeypatch.setattr(S._lib, "native", lambda: pytest.fail("launched on the current device"))
     assert torch.equal(S.rmsnorm(x, w, 1e-6), ref)
+
+
+@pytest.mark.parametrize("h,d", [(1, 516), (2, 1024), (1, 16384)])
+@pytest.mark.parametrize("L,pos,on_device", [(1, 37, True), (7, 5, False)])
+def test_fullnorm_rope_long_heads(S, h, d, L, pos, on_device):
+    test_fullnorm_rope(S, h, d, L, pos, on_device)
