@@ -1,8 +1,11 @@
 """Access to libscmx.so (the C ABI declared in include/scmx.h): `native()` is what the wrappers call, tensors in, one native
-call per launch (csrc/torch_binding.cpp); `load()` the whole ABI through ctypes, for the queries and for foreign callers.
+call per launch (csrc/torch_binding.cpp); `load()` the whole ABI through ctypes, for the queries and for foreign callers,
+with `call`, `ptr` and `stream` to check a status and to make arguments of tensors.
 There is no fallback: a missing or incomplete library raises, and so does every call that returns a negative status."""
 import ctypes as C
 import os
+
+import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libscmx.so")
@@ -80,6 +83,31 @@ def load():
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+def call(name, *args):
+    """An entry point through ctypes, its status checked: call("scmx_act_quant", ptr(x), ptr(xq), ptr(xs), M, Mp, K, stream())."""
+    lib = load()
+    rc = getattr(lib, name)(*args)
+    if rc != 0:
+        msg = lib.scmx_last_error().decode()
+        raise (ValueError if rc in (-1, -2, -4) else RuntimeError)(f"{name} failed ({rc}): {msg}")
+
+
+def ptr(t):
+    """Device pointer of a contiguous CUDA tensor (None -> NULL)."""
+    if t is None:
+        return None
+    if not t.is_cuda:
+        raise ValueError("scmx kernels take CUDA (ROCm) tensors; got a CPU tensor")
+    if not t.is_contiguous():
+        raise ValueError("scmx kernels take contiguous tensors")
+    return t.data_ptr()
+
+
+def stream():
+    """The current stream's handle."""
+    return torch.cuda.current_stream().cuda_stream
 
 
 _native = None

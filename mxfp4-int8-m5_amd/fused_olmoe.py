@@ -104,6 +104,14 @@ class FusedOlmoe:
     def make_cache(self, max_len=4096):
         return [KVCache(self.args, max_len, self.device) for _ in self.layers]
 
+    def rope(self, x, offset):
+        """Rotary embedding of x [heads, L, d] at positions offset ..., as array ops (a prompt's runs in qkv_fullnorm_rope)."""
+        L = x.shape[1]
+        ang = torch.arange(offset, offset + L, device=x.device, dtype=torch.float32)[:, None] * self.inv_freq[None]
+        cos, sin = ang.cos()[None], ang.sin()[None]
+        x1, x2 = x.float().chunk(2, -1)
+        return torch.cat([x1 * cos - x2 * sin, x2 * cos + x1 * sin], -1).to(x.dtype)
+
     def _attention(self, c, nw, y, L):
         """q/k norm, rotary embedding and cache append of the q|k|v rows y, then attention -> bf16 [L, H * d]."""
         a, off = self.args, c.offset
