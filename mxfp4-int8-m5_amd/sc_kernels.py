@@ -251,8 +251,8 @@ def _plain(x, w):
     """Whether a kernel may stand in for an array op on x and w: contiguous bf16 tensors on the current device (where the
     binding launches) with which torch would do no more than run the op -- no subclass, autograd (reverse or forward),
     functorch, autocast, dispatch or function mode, tracing or compilation."""
-    return (type(x) is type(w) is torch.Tensor and x.is_cuda and x.device == w.device
-            and x.device.index == torch.cuda.current_device() and x.dtype == w.dtype == torch.bfloat16
+    return (type(x) is type(w) is torch.Tensor and x.is_cuda and w.is_cuda
+            and x.get_device() == w.get_device() == torch._C._cuda_getDevice() and x.dtype == w.dtype == torch.bfloat16
             and x.is_contiguous() and w.is_contiguous()
             and not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
                      or torch._C._functorch.maybe_current_level() is not None

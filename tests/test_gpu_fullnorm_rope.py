@@ -72,7 +72,7 @@ def test_rmsnorm_array_op(S, monkeypatch):
     assert torch.equal(S.rmsnorm(x.t().contiguous().t(), w, 1e-6), ref)          # columns first
     odd = torch.randn(3, 250, device="cuda").to(torch.bfloat16)
     assert torch.equal(S.rmsnorm(odd, w[:250], 1e-6), rms_norm(odd, w[:250], 1e-6))
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.device.index + 1)
     monkeypatch.setattr(S._lib, "native", lambda: pytest.fail("launched on the current device"))
     assert torch.equal(S.rmsnorm(x, w, 1e-6), ref)
 

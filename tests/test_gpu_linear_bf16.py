@@ -45,6 +45,6 @@ def test_linear_bf16_off_the_current_device(S, monkeypatch):
     """Kernels are launched on the current device: tensors of another GPU get the array op, which runs on theirs."""
     x, w = (torch.randn(r, 256, device="cuda").to(torch.bfloat16) for r in (4, 40))
     ref = x @ w.T
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.device.index + 1)
     monkeypatch.setattr(S._lib, "native", lambda: pytest.fail("launched on the current device"))
     assert torch.equal(S.linear_bf16(x, w), ref)
