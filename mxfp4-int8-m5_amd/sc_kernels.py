@@ -233,9 +233,12 @@ def rms_norm(x, w, eps):
 
 def linear_bf16(x, w):
     """x w^T of bf16 rows x [M, K] and a bf16 matrix w [N, K] (output head, router) -> bf16 [M, N], sums in float32.  Up to
-    16 rows the library's kernel, which reads w once at 5.5-6.3 TB/s (one row against 151936 x 2048: 112 us, the array op
-    203; against 50304 x 2048: 33 / 31; a router of 64 x 2048: 7.4 / 18.7 a call) while the rows' fragments stay in
-    registers: K up to 2048, beyond it for two rows (32000 x 4096: 41 us for one row, 60 for sixteen, the array op 41-43).
+    16 rows the library's kernel, which reads w once at 5.2-5.8 TB/s, beyond K = 2048 (where the rows' fragments no longer stay
+    in registers) for two rows.  The array op's time jumps with the shape.  One row, weights from HBM, calls in a row, us
+    kernel / array op: 151936 x 2048 108 / 201, x 2560 141 / 239; 50304 x 2048 38 / 48 (sixteen rows 42 / 48); 32000 x 4096 47 / 55;
+    128256 x 4096 174 / 183; a router of 64 x 2048 4.5 / 18.7.  Where it loses: 50304 x 2304 48 / 42, 65536 x 5120 123 / 111, 128256
+    x 5120 242 / 223, sixteen rows of 65536 x 1920 48 / 45; a single call waited for costs the array op 14 us more on top.
+    Sixteen rows beyond K = 2048: 32000 x 4096 66 / 56, 128256 x 4096 250 / 186.
     More rows, other types and layouts, tensors off the current device, and callers that differentiate, trace or cast the
     product get the array op."""
     if (_plain(x, w) and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= 16 and w.shape[0]

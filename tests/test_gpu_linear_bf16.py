@@ -48,3 +48,24 @@ def test_linear_bf16_off_the_current_device(S, monkeypatch):
     monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.device.index + 1)
     monkeypatch.setattr(S._lib, "native", lambda: pytest.fail("launched on the current device"))
     assert torch.equal(S.linear_bf16(x, w), ref)
+
+
+# every form of the kernel: one to four turns of a row, each full and not; several batches of three and of four, full and not,
+# with one tile and with several per workgroup (the next tile's first batch is requested behind this one's last)
+@pytest.mark.parametrize("m,n,k", [(3, 33, 576), (16, 40, 1024), (5, 16, 1088), (16, 9001, 1536), (4, 20, 1984), (1, 17000, 2112),
+                                   (2, 17000, 2560), (1, 9001, 4096), (2, 8200, 4608), (2, 9001, 3584), (16, 50, 6400), (1, 3, 8192)])
+def test_linear_bf16_forms(S, m, n, k):
+    test_linear_bf16_kernel(S, m, n, k)
+
+
+def test_linear_bf16_kernel(S, m=2, n=300, k=2048):
+    """The kernel itself, whichever op linear_bf16 chooses for the shape; nothing outside the rows reaches the sums."""
+    g = torch.Generator(device="cuda").manual_seed(m * n + k)
+    x, w = (torch.full((r * k + 128,), float("nan"), device="cuda", dtype=torch.bfloat16) for r in (m, n))
+    x, w = x[64:-64].view(m, k), w[64:-64].view(n, k)
+    x.copy_(torch.randn(m, k, device="cuda", generator=g)), w.copy_(torch.randn(n, k, device="cuda", generator=g))
+    y = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
+    S._lib.native().scmx_linear_bf16(x, w, y, m, n, k)
+    xd, wd = x.double(), w.double()
+    ref, mag = xd @ wd.T, xd.abs() @ wd.abs().T
+    assert ((y.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * k * 2.0 ** -24).all()
