@@ -145,6 +145,11 @@ struct Query<FN, R (*)(P...)> {
     }
 };
 
+struct NoGil {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // empty_<type>(like, dims...): an uninitialised tensor on the device of `like`.
 template <at::ScalarType TYPE>
 PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -154,7 +159,13 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (n > 5) fail(PyExc_TypeError, "at most four dimensions");
         for (Py_ssize_t i = 1; i < n; ++i) dims[i - 1] = as_int(args[i]);
         const at::Tensor& like = THPVariable_Unpack(args[0]);
-        return THPVariable_Wrap(at::empty(at::IntArrayRef(dims, size_t(n - 1)), at::TensorOptions().dtype(TYPE).device(like.device())));
+        const at::TensorOptions options = at::TensorOptions().dtype(TYPE).device(like.device());
+        at::Tensor t;
+        {
+            const NoGil released;   // the allocator may ask the driver, or wait for the GPU
+            t = at::empty(at::IntArrayRef(dims, size_t(n - 1)), options);
+        }
+        return THPVariable_Wrap(std::move(t));
     } catch (...) {
         return raised();
     }
