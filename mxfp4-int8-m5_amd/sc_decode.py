@@ -45,6 +45,8 @@ def gemv(xq, codes, bcodes, xscale, wscale, N, epi, dtype=torch.bfloat16, res=No
     nat = _lib.native()
     xscale = xscale if pro == 0 else None
     res = res if epi == 2 else None
+    if batch in (3, 5, 6, 7):   # counts between the kernels' sizes come from any layout
+        xq, xscale, res = (None if t is None else t.contiguous() for t in (xq, xscale, res))
     nw, eps = (nw, S._eps(eps)) if pro == 2 else (None, 0.0)
     if eidx is None:
         need = nat.scmx_gemv_rows_workspace(fmt.c, pro, batch, N, K) if batch > 1 else 0

@@ -54,3 +54,28 @@ def test_rows_equal_single_rows(rows, n, k, name):
             one = host(G.gemv(a[b], codes, bc, None if s is None else s[b:b + 1], ws, n, epi,
                               res=res[b] if epi == 2 else None, **kw))
             assert np.array_equal(y[b], one), (pro, epi, b)
+
+
+@pytest.mark.parametrize("rows", [3, 5, 6, 7, 11])
+def test_views_of_rows(rows):
+    """Row counts between the kernels' sizes have always been taken from any layout: columns of a wider matrix, every other row."""
+    from mxfp4_int8_m5_amd import sc_decode as G
+    rng = np.random.default_rng(rows)
+    n, k = 256, 512
+    codes, bc, ws, fmt = packed(rng, n, k, "published")
+    x = dev(llm_acts(rng, rows, 2 * k)[0])
+    xs = torch.from_numpy(rng.uniform(1e-3, 1e-2, 2 * rows).astype(F32)).cuda()
+    xq = torch.from_numpy(rng.integers(-127, 128, (rows, 2 * k)).astype(np.int8)).cuda()
+    res = dev(bf16.to_bits(rng.standard_normal((rows, 2 * n)).astype(F32)))
+    if rows > 8:   # eight rows and a rest of three: the first eight have to be contiguous
+        x, xq, xs, res = x[:, :k].contiguous(), xq[:, :k].contiguous(), xs[:rows], res[:, :n].contiguous()
+    else:
+        x, xq, xs, res = x[:, k:], xq[:, k:], xs[::2], res[:, n:]
+        assert not any(t.is_contiguous() for t in (x, xq, xs, res))
+    c = lambda t: t.contiguous()   # noqa: E731
+    for epi in (1, 2):
+        r = {"res": res} if epi == 2 else {}
+        rc = {"res": c(res)} if epi == 2 else {}
+        assert torch.equal(G.gemv(xq, codes, bc, xs, ws, n, epi, fmt=fmt, **r), G.gemv(c(xq), codes, bc, c(xs), ws, n, epi, fmt=fmt, **rc))
+        assert torch.equal(G.gemv(x, codes, bc, None, ws, n, epi, pro=1, fmt=fmt, **r),
+                           G.gemv(c(x), codes, bc, None, ws, n, epi, pro=1, fmt=fmt, **rc))
