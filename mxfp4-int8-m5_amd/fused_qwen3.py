@@ -244,10 +244,14 @@ class DecodeQwen3:
 
     def _logits(self, h):
         f = self.f
-        if self.head and self.packed_head is not None:   # the final norm in the GEMV's prologue
-            codes, bc, ws, n = self.packed_head
+        packed = self.packed_head if self.head else None
+        if packed is not None and f.norm.dtype == BF and f.norm.is_contiguous() and f.norm.data_ptr() % 16 == 0:
+            codes, bc, ws, n = packed   # the final norm in the GEMV's prologue
             return G.gemv(h, codes, bc, None, ws, n, 1, pro=2, nw=f.norm, eps=f.eps, fmt=self.head_fmt)[None]
         hn = S.rmsnorm(h, f.norm, f.eps)
+        if packed is not None:
+            codes, bc, ws, n = packed
+            return G.gemv(hn, codes, bc, None, ws, n, 1, pro=1, fmt=self.head_fmt)[None]
         return f.logits(hn) if self.head else hn
 
     def _pre(self, h, nw, w, c, pos):
