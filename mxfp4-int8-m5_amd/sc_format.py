@@ -49,6 +49,9 @@ class Format:
         """c_struct(), made once."""
         return self.c_struct()
 
+    def __getstate__(self):   # the fields alone, not the descriptor
+        return {k: v for k, v in self.__dict__.items() if k != "c"}
+
     def c_struct(self):
         """The scmx_format passed across the C ABI (a new one)."""
         if len(self.mult) > 16:

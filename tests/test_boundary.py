@@ -183,3 +183,14 @@ def test_host_code_under_address_and_undefined_behaviour_sanitizers():
         pytest.skip("a GPU is present")
     assert run.returncode == 0, run.stdout[-4000:]
     assert "0 failure(s)" in run.stdout and "runtime error" not in run.stdout and "AddressSanitizer" not in run.stdout
+
+
+def test_a_used_format_pickles_as_its_fields(pkg):
+    """The descriptor made for the kernels is not part of a Format's value: files and other processes get its fields."""
+    import copy
+    import pickle
+    fmt = pkg.sc_format.Format(block=16)
+    fresh = pickle.dumps(fmt)
+    assert fmt.c.block == 16
+    assert pickle.dumps(fmt) == fresh and vars(copy.copy(fmt)) == vars(pkg.sc_format.Format(block=16))
+    assert pickle.loads(fresh) == fmt and pickle.loads(fresh).c.block == 16
