@@ -1355,11 +1355,15 @@ extern "C" int scmx_gemv_rows(const scmx_format* fmt, const void* x, const float
                               const uint8_t* bcodes, const float* wscale, const uint16_t* res, uint16_t* out, int epi,
                               int pro, const uint16_t* nw, float eps, int rows, int N, int K, void* workspace,
                               size_t workspace_bytes, void* stream) {
-    if (workspace && wscale && epi >= 1 && N % 4 == 0 && (epi != SCMX_EPI_SWIGLU || N % 8 == 0) &&
+    // That route quantizes the rows before the GEMM's own checks: it is taken only with what those accept (the 32-bit
+    // offsets at the columns of a few-row shape: K <= 65536), and the rest is refused, or run, by the GEMV.
+    if (workspace && x && codes && bcodes && wscale && out && epi >= 1 && epi <= 3 && (epi != SCMX_EPI_RES || res) &&
+        N % 4 == 0 && (epi != SCMX_EPI_SWIGLU || N % 8 == 0) && K <= 65536 &&
         (uintptr_t(x) | uintptr_t(out) | uintptr_t(wscale) | uintptr_t(codes)) % 16 == 0 && uintptr_t(res) % 8 == 0 &&
         uintptr_t(workspace) % 256 == 0) {
         const size_t need = scmx_gemv_rows_workspace(fmt, pro, rows, N, K);
-        if (need && workspace_bytes >= need)
+        if (need && workspace_bytes >= need && K % fmt->block == 0 && (K / fmt->block * fmt->bc_bits) % 8 == 0 &&
+            (epi != SCMX_EPI_SWIGLU || silu_table_device()))
             return scmx_linear_w4a8(fmt, reinterpret_cast<const uint16_t*>(x), codes, bcodes, wscale, res, out, epi, rows, N, K,
                                     workspace, workspace_bytes, stream);
     }

@@ -185,6 +185,77 @@ int main() {
     expect(scmx_attn_prefill(h[0], h[1], h[2], oh[0], 60, 8, 4, 2, 128, 64, 0.1f, nullptr), SCMX_ERR_ARG,
            "attn_prefill rows past the cache");
     expect(scmx_qkv_fullnorm(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], nullptr, 4, 4, 64, nullptr), SCMX_ERR_ARG, "qkv_fullnorm null v");
+    for (int splits : {0, -1, 65, 2147483647})
+        expect(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], 8, 0, 4, 2, 128, 64, 0.1f, of, splits, nullptr), SCMX_ERR_ARG,
+               "attn_prefill_split ranges outside 1..64");
+    expect(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], 8, 0, 4, 2, 128, 64, 0.1f, nullptr, 2, nullptr), SCMX_ERR_ARG,
+           "attn_prefill_split without workspace");
+    expect(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], 8, 0, 4, 2, 128, 64, 0.1f, of + 1, 2, nullptr), SCMX_ERR_ARG,
+           "attn_prefill_split misaligned workspace");
+    expect(scmx_attn_prefill_split(h[0], nullptr, h[2], oh[0], 8, 0, 4, 2, 128, 64, 0.1f, of, 2, nullptr), SCMX_ERR_ARG,
+           "attn_prefill_split null cache");
+    expect(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], 60, 8, 4, 2, 128, 64, 0.1f, of, 2, nullptr), SCMX_ERR_ARG,
+           "attn_prefill_split rows past the cache");
+    expect(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 4, 4, 64, nullptr, pos, 0, 64, 1, nullptr), SCMX_ERR_ARG,
+           "qkv_fullnorm_rope null inv_freq");
+    expect(scmx_qkv_fullnorm_rope(nullptr, h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 4, 4, 64, f0, pos, 0, 64, 1, nullptr), SCMX_ERR_ARG,
+           "qkv_fullnorm_rope null y");
+    expect(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 4, 4, 64, f0, pos, 61, 64, 1, nullptr), SCMX_ERR_ARG,
+           "qkv_fullnorm_rope rows past the cache");
+    expect(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 4, 4, 64, f0, pos, -1, 64, 1, nullptr), SCMX_ERR_ARG,
+           "qkv_fullnorm_rope negative position");
+    expect(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 4, 4, 66, f0, pos, 0, 64, 1, nullptr), SCMX_ERR_ARG,
+           "qkv_fullnorm_rope head dim % 4");
+    expect(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 4, 257, 64, f0, pos, 0, 64, 1, nullptr), SCMX_ERR_ARG,
+           "qkv_fullnorm_rope width above 16384");
+    expect(scmx_rmsnorm(h[0], nullptr, 1e-6f, oh[0], 4, 128, nullptr), SCMX_ERR_ARG, "rmsnorm null weight");
+    expect(scmx_rmsnorm(h[0], h[1], 1e-6f, oh[0], 4, 130, nullptr), SCMX_ERR_ARG, "rmsnorm K % 4");
+    expect(scmx_rmsnorm(h[0], h[1], 1e-6f, oh[0], 4, 16388, nullptr), SCMX_ERR_ARG, "rmsnorm K > 16384");
+    expect(scmx_rmsnorm(h[0], h[1], 1e-6f, oh[0], -1, 128, nullptr), SCMX_ERR_ARG, "rmsnorm negative rows");
+    expect(scmx_linear_bf16(h[0], nullptr, oh[0], 4, 100, 128, nullptr), SCMX_ERR_ARG, "linear_bf16 null w");
+    expect(scmx_linear_bf16(h[0] + 4, h[1], oh[0], 4, 100, 128, nullptr), SCMX_ERR_ARG, "linear_bf16 misaligned x");
+    expect(scmx_linear_bf16(h[0], h[1] + 1, oh[0], 4, 100, 128, nullptr), SCMX_ERR_ARG, "linear_bf16 misaligned w");
+    expect(scmx_linear_bf16(h[0], h[1], oh[0], 17, 100, 128, nullptr), SCMX_ERR_ARG, "linear_bf16 M > 16");
+    expect(scmx_linear_bf16(h[0], h[1], oh[0], 4, 100, 96, nullptr), SCMX_ERR_ARG, "linear_bf16 K % 64");
+    expect(scmx_linear_bf16(h[0], h[1], oh[0], 4, 0, 128, nullptr), SCMX_ERR_ARG, "linear_bf16 N = 0");
+    expect(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 9, 8, 128, nullptr, 0, nullptr), SCMX_ERR_ARG,
+           "gemv_rows 9 rows");
+    expect(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 0, 8, 128, nullptr, 0, nullptr), SCMX_ERR_ARG,
+           "gemv_rows no rows");
+    expect(scmx_gemv_rows(&fmt, xq, nullptr, codes, bc, f1, nullptr, oh[0], 1, 0, nullptr, 0.0f, 3, 8, 128, nullptr, 0, nullptr), SCMX_ERR_ARG,
+           "gemv_rows prologue 0 without xscale");
+    expect(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 2, 1, nullptr, 0.0f, 4, 4096, 12288, wsp, 1 << 20, nullptr), SCMX_ERR_ARG,
+           "gemv_rows through the few-row GEMM, residual epilogue without res");
+    expect(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 4, 1, nullptr, 0.0f, 4, 4096, 12288, wsp, 1 << 20, nullptr), SCMX_ERR_ARG,
+           "gemv_rows through the few-row GEMM, unknown epilogue");
+    expect(scmx_gemv_rows(&fmt, h[0], nullptr, codes, nullptr, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 4, 4096, 12288, wsp, 1 << 20, nullptr),
+           SCMX_ERR_ARG, "gemv_rows through the few-row GEMM, null bcodes");
+    expect(scmx_gemv_rows(nullptr, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 4, 4096, 12288, wsp, 1 << 20, nullptr),
+           SCMX_ERR_ARG, "gemv_rows null format");
+    {
+        // a shape the half-precision kernels leave (4 rows of 12288 values): the GEMM's workspace; 0 wherever that is not a route
+        const size_t need = scmx_gemv_rows_workspace(&fmt, 1, 4, 4096, 12288);
+        scmx_format bad = fmt;
+        bad.bc_bits = 3;
+        if (need != scmx_linear_w4a8_workspace(4, 12288) || scmx_gemv_rows_workspace(&bad, 1, 4, 4096, 12288) ||
+            scmx_gemv_rows_workspace(nullptr, 1, 4, 4096, 12288) || scmx_gemv_rows_workspace(&fmt, 0, 4, 4096, 12288) ||
+            scmx_gemv_rows_workspace(&fmt, 2, 4, 4096, 12288) || scmx_gemv_rows_workspace(&fmt, 1, 1, 4096, 12288) ||
+            scmx_gemv_rows_workspace(&fmt, 1, 9, 4096, 12288) || scmx_gemv_rows_workspace(&fmt, 1, 4, 0, 12288) ||
+            scmx_gemv_rows_workspace(&fmt, 1, 4, 4096, -128) || scmx_gemv_rows_workspace(&fmt, 1, 4, 4096, 100) ||
+            scmx_gemv_rows_workspace(&fmt, 1, 4, 151936, 2048) || scmx_gemv_rows_workspace(&fmt, 1, 4, 2048, 2048)) {
+            printf("FAIL gemv_rows workspace sizes\n");
+            ++failures;
+        }
+        expect_valid(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 4, 4096, 12288, wsp, need, nullptr),
+                     "gemv_rows through the few-row GEMM");
+        // a smaller workspace, and none, leave the GEMV kernels, which take this shape as well
+        expect_valid(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 4, 4096, 12288, wsp, need - 1, nullptr),
+                     "gemv_rows with a small workspace");
+        expect_valid(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 4, 4096, 12288, nullptr, 0, nullptr),
+                     "gemv_rows without workspace");
+        expect(scmx_gemv_rows(&fmt, h[0], nullptr, codes, bc, f1, nullptr, oh[0], 1, 1, nullptr, 0.0f, 8, 2048, 16384, nullptr, 0, nullptr),
+               SCMX_ERR_ARG, "gemv_rows without workspace, more activations than a workgroup stages");
+    }
     expect(scmx_gemv(&fmt, xq, nullptr, codes, bc, f1, nullptr, oh[0], 1, 0, nullptr, 0.0f, 1, 8, 128, nullptr, 0, 0, -1, nullptr),
            SCMX_ERR_ARG, "gemv prologue 0 without xscale");
     expect(scmx_gemv(&fmt, xq, f0, codes, bc, f1, nullptr, oh[0], 1, 0, nullptr, 0.0f, 3, 8, 128, nullptr, 0, 0, -1, nullptr),
@@ -229,6 +300,11 @@ int main() {
     expect(scmx_moe_mm(&fmt, xq, f0, nullptr, 0, codes, bc, f1, ci, ci, 4, 64, 8, 128, 1, out, nullptr), SCMX_OK, "moe_mm R = 0");
     expect(scmx_route_topk(h[0], nullptr, 0, 64, 8, 1, oi[0], oh[0], nullptr), SCMX_OK, "route_topk M = 0");
     expect(scmx_qkv_fullnorm(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 0, 4, 64, nullptr), SCMX_OK, "qkv_fullnorm L = 0");
+    expect(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 0, 4, 64, f0, pos, 0, 64, 1, nullptr), SCMX_OK,
+           "qkv_fullnorm_rope L = 0");
+    expect(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], 0, 0, 4, 2, 128, 64, 0.1f, of, 3, nullptr), SCMX_OK, "attn_prefill_split L = 0");
+    expect(scmx_rmsnorm(h[0], h[1], 1e-6f, oh[0], 0, 128, nullptr), SCMX_OK, "rmsnorm M = 0");
+    expect(scmx_linear_bf16(h[0], h[1], oh[0], 0, 100, 128, nullptr), SCMX_OK, "linear_bf16 M = 0");
 
     // ---- plausible arguments: accepted, and stopped by the missing device at the earliest ---------------------------------
     expect_valid(scmx_unpack_i8(&fmt, codes, bc, oq, 4096, 2048, nullptr), "unpack_i8");
@@ -264,6 +340,21 @@ int main() {
                  "attn_decode_qkv");
     expect_valid(scmx_attn_prefill(h[0], h[1], h[2], oh[0], 2048, 0, 16, 8, 128, 2048, 0.088f, nullptr), "attn_prefill");
     expect_valid(scmx_qkv_fullnorm(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 100, 16, 128, nullptr), "qkv_fullnorm");
+    expect_valid(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], 100, 4000, 16, 8, 128, 4100, 0.088f, of, 16, nullptr), "attn_prefill_split");
+    expect_valid(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], 100, 20, 16, 8, 128, 4100, 0.088f, of, 64, nullptr),
+                 "attn_prefill_split more ranges than keys");
+    expect_valid(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 100, 16, 128, f0, pos, 300, 512, 1, nullptr),
+                 "qkv_fullnorm_rope");
+    expect_valid(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], 100, 1, 16384, f0, pos, 300, 512, 0, nullptr),
+                 "qkv_fullnorm_rope one long head");
+    for (int k : {4, 512, 1000, 4096, 16384}) expect_valid(scmx_rmsnorm(h[0], h[1], 1e-6f, oh[0], 300, k, nullptr), "rmsnorm");
+    for (int k : {64, 576, 1024, 1536, 2048, 2112, 2560, 1 << 26})
+        expect_valid(scmx_linear_bf16(h[0], h[1], oh[0], 16, 50304, k, nullptr), "linear_bf16");
+    for (int rows = 1; rows <= 8; ++rows)
+        for (int pro = 0; pro <= 2; ++pro)
+            expect_valid(scmx_gemv_rows(&fmt, pro ? (const void*)h[0] : (const void*)xq, pro ? nullptr : f0, codes, bc, f1, h[1], oh[0],
+                                        1 + pro % 2, pro, pro == 2 ? h[2] : nullptr, 1e-6f, rows, 151936, 2048, nullptr, 0, nullptr),
+                         "gemv_rows");
     for (int batch : {1, 2, 4, 8})
         for (int pro = 0; pro <= 2; ++pro)
             expect_valid(scmx_gemv(&fmt, pro ? (const void*)h[0] : (const void*)xq, pro ? nullptr : f0, codes, bc, f1, h[1], oh[0],
@@ -337,6 +428,23 @@ int main() {
                                 int(rng() % 5) - 1, (const uint16_t*)maybe(h[2]), 1e-6f, r(), r(), r(), (const int32_t*)maybe(ci), r(), r(),
                                 r(), nullptr),
                       "fuzz gemv");
+        expect_status(scmx_attn_prefill_split(h[0], h[1], h[2], oh[0], r(), r(), r(), r(), (rng() % 2) ? 128 : r(), r(), 0.1f, (float*)maybe(of),
+                                              r(), nullptr),
+                      "fuzz attn_prefill_split");
+        expect_status(scmx_qkv_fullnorm_rope(h[0], h[1], h[2], 1e-6f, oh[0], oh[1], oh[2], r(), r(), r(), (const float*)maybe(f0), pos,
+                                             int64_t(r()) * (rng() % 3), r(), int(rng() % 2), nullptr),
+                      "fuzz qkv_fullnorm_rope");
+        expect_status(scmx_rmsnorm(h[0], (const uint16_t*)maybe(h[1]), 1e-6f, oh[0], r(), r(), nullptr), "fuzz rmsnorm");
+        expect_status(scmx_linear_bf16(h[0], (const uint16_t*)maybe(h[1]), oh[0], (rng() % 2) ? int(rng() % 17) : r(), r(), r(), nullptr),
+                      "fuzz linear_bf16");
+        {
+            const int pro = int(rng() % 5) - 1, rows = (rng() % 2) ? int(rng() % 9) : r(), n = r(), k = r();
+            const size_t need = scmx_gemv_rows_workspace(&f, pro, rows, n, k);
+            expect_status(scmx_gemv_rows(&f, h[0], (const float*)maybe(f0), codes, bc, f1, (const uint16_t*)maybe(h[1]), oh[0],
+                                         int(rng() % 6) - 1, pro, (const uint16_t*)maybe(h[2]), 1e-6f, rows, n, k, (void*)maybe(wsp),
+                                         (rng() % 2) ? need : size_t(r()), nullptr),
+                          "fuzz gemv_rows");
+        }
         expect_status(scmx_route_topk(h[0], (const uint16_t*)maybe(h[1]), r(), r(), r(), int(rng() % 2), oi[0], oh[0], nullptr),
                       "fuzz route_topk");
         expect_status(scmx_route_sort(ci, r(), r(), r(), r(), oi[0], oi[1], oi[2], oi[3], oi[4], nullptr), "fuzz route_sort");
