@@ -1,5 +1,6 @@
 """Prefill attention with the keys cut into ranges, where that can go wrong: a query tile that ends in the first range beside
-one that does not, a range that some queries do not reach, one pair of tiles per range, more ranges than pairs."""
+one that does not, a range that some queries do not reach, one pair of tiles per range, more ranges than pairs, and head
+counts that are whole turns of the XCDs (the heads' order then differs) beside those that are not."""
 import pytest
 import torch
 
@@ -18,7 +19,8 @@ def test_ranges_stay_in_bounds():
 @pytest.mark.gpu
 @pytest.mark.parametrize("scale", [128 ** -0.5, 0.07, 0.031])
 @pytest.mark.parametrize("hq,hk,L,off,splits", [(2, 1, 1, 127, 2), (2, 2, 1, 128, 2), (4, 2, 32, 60, 1), (4, 2, 32, 1000, 8), (2, 1, 129, 1000, 3),
-                                                (2, 2, 300, 0, 2), (3, 3, 200, 120, 64), (1, 1, 2, 5000, 13)])
+                                                (2, 2, 300, 0, 2), (3, 3, 200, 120, 64), (1, 1, 2, 5000, 13),
+                                                (8, 2, 130, 700, 3), (16, 16, 40, 900, 8), (16, 8, 300, 200, 2), (24, 8, 1, 500, 4)])
 def test_attn_prefill_split(hq, hk, L, off, splits, scale):
     from mxfp4_int8_m5_amd import sc_kernels as S
     n, d = off + L, 128

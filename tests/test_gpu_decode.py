@@ -111,7 +111,7 @@ def test_gemv_fused_prologues(G, S, pro):
 @pytest.mark.parametrize("batch", [2, 3, 4, 5, 7, 8, 9, 19])
 def test_gemv_batch_equals_rows(G, batch):
     """B rows against one pass over the weights give the bits of B independent batch-1 GEMVs (3, 5, 6 and 7 rows run
-    padded to 4 / 8 by the Python surface, more than 8 rows eight at a time)."""
+    the four- and eight-row kernels without padding, more than 8 rows eight at a time)."""
     rng = np.random.default_rng(batch)
     n, k = 1024, 2048
     codes, bc, ws, q = random_packed(rng, n, k)
@@ -311,3 +311,20 @@ def test_gemv_block_codes_at_an_odd_address(G, n, k):
         ya = G.gemv(dx, dc, aligned, None, dw, n, 1, pro=1)
         yo = G.gemv(dx, dc, odd, None, dw, n, 1, pro=1)
         assert torch.equal(ya, yo), batch
+
+
+@pytest.mark.parametrize("name", ["published", "sixteen", "range", "high_range", "mxfp4"])
+@pytest.mark.parametrize("n,epi", [(64, 3), (16384, 1), (16388, 2)])
+@pytest.mark.parametrize("k", [2048, 2176, 3072, 4096, 4224])
+def test_gemv_norm_prologue_of_wide_layers(G, S, k, n, epi, name):
+    """One row with the RMSNorm in front, four weight rows per wave (SwiGLU, or 16384 rows and more): rows of up to 2048 values
+    in one register chunk per thread, up to 4096 in two, the second whole or in part, and beyond from memory.  The row's codes
+    are the oracle's, the product the bits of the GEMV on them."""
+    from tests.test_gpu_gemv_rows import packed
+    rng = np.random.default_rng(n + k)
+    codes, bc, ws, fmt = packed(rng, n, k, name)
+    x, nw = llm_acts(rng, 1, k)[0], llm_acts(rng, 1, k)[0][0]
+    rq, rs, _ = linear.rmsnorm_quant(x, nw, 1e-6)
+    res = {"res": dev(bf16.to_bits(rng.standard_normal(n).astype(F32)))} if epi == 2 else {}
+    y = G.gemv(dev(x)[0], codes, bc, None, ws, n, epi, pro=2, nw=dev(nw), eps=1e-6, fmt=fmt, **res)
+    assert torch.equal(y, G.gemv(dev(rq)[0], codes, bc, dev(rs), ws, n, epi, fmt=fmt, **res))
