@@ -277,20 +277,23 @@ __device__ __forceinline__ int family_index(const FamilyArgs& f, float x) {   //
     for (int i = 0; i < 7; ++i) idx += int(a > f.cut[i]);
     return idx;
 }
-__device__ __forceinline__ float family_level(const FamilyArgs& f, float a) {   // sign(a) times its magnitude, for a >= 0
-    float v = a > 0.0f ? f.cb[0] : 0.0f;   // (a zero has no sign: it costs nothing also where the smallest magnitude is not 0)
+// sign(a) times its magnitude, for a >= 0: a zero has no sign and costs nothing, also where the smallest magnitude is not 0
+// (in the E2M1 codebook it is).
+template <bool E2M1>
+__device__ __forceinline__ float family_level(const FamilyArgs& f, float a) {
+    float v = !E2M1 && a > 0.0f ? f.cb[0] : 0.0f;
 #pragma unroll
     for (int i = 0; i < 7; ++i) v = a > f.cut[i] ? f.cb[i + 1] : v;
     return v;
 }
 
 // Squared error of the block of magnitudes aw at scale sc, as the host evaluates it (float32, its order of sums).
-template <int BLOCK>
+template <int BLOCK, bool E2M1>
 __device__ __forceinline__ float family_sq_err(const FamilyArgs& f, const float (&aw)[BLOCK], float sc) {
     float r[8];
 #pragma unroll
     for (int i = 0; i < BLOCK; ++i) {
-        const float v = family_level(f, __fdiv_rn(aw[i], sc));
+        const float v = family_level<E2M1>(f, __fdiv_rn(aw[i], sc));
         const float d = __fsub_rn(__fmul_rn(v, sc), aw[i]);
         const float sq = __fmul_rn(d, d);
         r[i & 7] = i < 8 ? sq : __fadd_rn(r[i & 7], sq);
@@ -387,7 +390,7 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
                 float e = 0.0f;
                 // (a scale near the ends of the float32 range leaves its reciprocal no room)
                 if (E2M1 && sc > 1e-30f && sc < 1e30f) e = family_sq_err_e2m1<BLOCK>(aw, sc, &same);
-                if (!same) e = family_sq_err<BLOCK>(f, aw, sc);
+                if (!same) e = family_sq_err<BLOCK, E2M1>(f, aw, sc);
                 if (i == 0 || e < best) {
                     best = e;
                     best_i = i;
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
 #pragma unroll
             for (int i = 0; i < BLOCK; ++i) {
                 const float x = __fdiv_rn(v[i], sc);
-                const bool minus = x < 0.0f && family_level(f, fabsf(x)) > 0.0f;
+                const bool minus = x < 0.0f && family_level<E2M1>(f, fabsf(x)) > 0.0f;
                 c[i >> 3] |= (uint32_t(family_index(f, x)) | (minus ? 8u : 0u)) << (4 * (i & 7));
             }
         }
