@@ -279,8 +279,8 @@ __global__ __launch_bounds__(BLK ? 512 : 256, CH <= 12 ? 4 : CH <= 16 ? 3 : 1) v
 // xq as the large dense GEMM tiles take it: blocks of 32 rows x 32 k (1 KB), block (m / 32, k / 32) at
 // ((m / 32) * (K / 32) + k / 32) KB, and inside a block the 16 bytes of row r, k half h at (32 h + r) * 16 -- the order
 // in which the 64 lanes of a wave hold a 32x32x32 MFMA operand, so that a wave fetches one block with one coalesced load.
-// Rows of K <= 12288 go through act_quant_wave_kernel above, few rows through act_quant_row_kernel below; this is the kernel
-// for longer rows: one wave per row, eight rows per workgroup, the row read twice, every lane writing the 16 bytes of
+// Rows of K <= 12288 go through act_quant_wave_kernel above, few rows and those of up to 16384 through act_quant_row_kernel
+// below; this is the kernel for longer rows: one wave per row, eight rows per workgroup, the row read twice, every lane writing the 16 bytes of
 // its own 16 elements.  Same codes and scales as act_quant_kernel: the row maximum does not depend on the order it is
 // taken in.
 __global__ __launch_bounds__(512) void act_quant_blocked_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,

@@ -5,13 +5,16 @@
 // loads 16 bytes of codes (one run of 32 weights) per row per step, so a wave reads 1 KiB of contiguous weights
 // per load instruction.  With one activation row the codes go through the FP4 conversion instruction (two codes ->
 // two half-precision values, sign and block scale included) and v_dot2c_f32_f16 against the activations staged in
-// LDS as half precision: all values are small integers, so the FP32 partial sums are exact.  With several rows, or
-// another weight format, codes are decoded to INT8 four at a time with byte-permute lookups and accumulated with
+// LDS as half precision: all values are small integers, so the FP32 partial sums are exact.  A format that instruction
+// does not decode has its codes turned into INT8 four at a time with byte-permute lookups and accumulated with
 // v_dot4_i32_i8 against INT8 activations in LDS (bytes of every 8-group stored as elements 0,2,4,6,1,3,5,7 so the
-// decode needs no re-interleave).  Either way the totals are the GEMM's INT32 accumulators and the epilogues are
-// the GEMM's.  `BATCH` activation rows share one pass over the weights; for the published format they go through
-// gemv_mfma_kernel below, which hands the dot products to the 4x4x4 INT8 MFMA so that the vector work per weight
-// does not grow with the number of rows.
+// decode needs no re-interleave).
+//
+// Several activation rows share one pass over the weights.  In the formats of the FP4 conversion whole 16-row groups go
+// through gemv_hmfma_kernel (half-precision MFMA: the vector work per weight does not grow with the rows); published-format
+// layers outside its shapes through gemv_mfma_kernel (4x4x4 INT8 MFMA); what is left through the per-row kernel's byte
+// tables, or, given a workspace, through the few-row GEMM (scmx_gemv_rows).  However formed, the totals are the GEMM's INT32
+// accumulators and the epilogues are the GEMM's.
 #include "gemm_args.h"
 
 namespace scmx {

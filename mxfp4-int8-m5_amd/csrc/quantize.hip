@@ -115,9 +115,9 @@ __device__ __forceinline__ float fp4_sq_err(const float (&x)[BLOCK], float scale
     return r0 + r1;
 }
 
-// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: HBM (the weights are read once) and about 25 vector
-// instructions per weight.  12288 x 2048 bf16: 44.5 us (1.4 TB/s); 234 us with a lane per weight and every candidate in
-// float64 across lanes.
+// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: 37 vector instructions per weight, which keep the vector
+// ALU busy 63 % of the time with two waves a SIMD, and a wave's wait for its loads (39 % of its life) the rest; not HBM.
+// 12288 x 2048 bf16: 44.5 us (1.4 TB/s); 234 us with a lane per weight and every candidate in float64 across lanes.
 template <int BLOCK, bool BF16>
 __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                          uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
@@ -302,7 +302,7 @@ __device__ __forceinline__ float family_sq_err(const FamilyArgs& f, const float 
                      __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
 }
 
-// The same for the E2M1 codebook (0, 1, 2, 3, 4, 6, 8, 12 = twice the FP4 values) through the FP4 conversion: about 8
+// The same for the E2M1 codebook (0, 1, 2, 3, 4, 6, 8, 12 = twice the FP4 values) through the FP4 conversion: about 13
 // instructions per weight instead of 40.  The quotient is formed twice with an approximate reciprocal, 2^-20 too large
 // and 2^-20 too small: where both round to the same code so does the correctly rounded quotient, whose error lies
 // between; where they differ (a quotient next to a midpoint) *same is cleared and the caller takes the form above.
@@ -332,7 +332,7 @@ __device__ __forceinline__ float family_sq_err_e2m1(const float (&aw)[BLOCK], fl
 
 constexpr int FAM_ROWS = 4;   // rows per workgroup at most: more are needed only for K < 1024, and their tables cost LDS
 
-// Bound: vector ALU (8 bases x n_mult trials per weight).  2048 x 2048 bf16, ten multipliers: 130 us; 520 us with a lane
+// Bound: vector ALU (8 bases x n_mult trials per weight, 13 instructions each), 96 % busy.  2048 x 2048 bf16, ten multipliers: 130 us; 520 us with a lane
 // per weight, a correctly rounded division per trial and the sums across lanes.
 template <int BLOCK, bool BF16, bool E2M1>
 __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,

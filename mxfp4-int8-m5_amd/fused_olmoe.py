@@ -7,7 +7,7 @@ Per transformer block (e2e/fused_olmoe.py:1-16):
   o = attn_prefill / attn_decode                                   (array ops in the reference, as rope and the cache)
   h = mm_epi(act_quant(o), Wo, + h)                                residual add in the GEMM epilogue
   xq, xs, xn = rmsnorm_quant_n(h)                                  INT8 for the experts, bf16 for the router
-  router: bf16 linear (torch), softmax + top-k (+ renorm) kernel   route
+  router: linear_bf16, softmax + top-k (+ renorm) kernel           route; the linear is an array op beyond 16 rows
   route_sort; act = moe_mm(xq, gather=tok, Wg|Wu, SwiGLU)          token rows read through the sort, no xq[tok] copy
   y = moe_mm(act_quant(act), Wd); h, xq, xs = moe_combine(y, scores, + h) + next block's RMSNorm + INT8
 Expert weights stay packed; the grouped kernel decodes each expert's weight tile in LDS."""

@@ -101,6 +101,14 @@ int main() {
            "mm_w4a8 in-place MXFP4 without row scales");
     expect(scmx_mxfp4_to_sc(bc, nullptr, nullptr, oi[0], 8, 128, nullptr), SCMX_ERR_ARG, "mxfp4_to_sc null wscale");
 
+    expect_valid(scmx_init(), "init");
+    if (scmx_mm_w4a8_prefers_blocked(0, 4096, 2048) || scmx_mm_w4a8_prefers_blocked(40, -1, 2048) ||
+        scmx_mm_w4a8_prefers_blocked(40, 4096, 2000) || !scmx_mm_w4a8_prefers_blocked(40, 2048, 6144) ||
+        !scmx_mm_w4a8_prefers_blocked(4096, 12288, 2048)) {
+        printf("FAIL layout preference\n");
+        ++failures;
+    }
+
     // ---- refused arguments --------------------------------------------------------------------------------------------
     expect(scmx_unpack_i8(nullptr, codes, bc, oq, 8, 128, nullptr), SCMX_ERR_ARG, "unpack_i8 null format");
     expect(scmx_unpack_i8(&fmt, nullptr, bc, oq, 8, 128, nullptr), SCMX_ERR_ARG, "unpack_i8 null codes");
@@ -461,6 +469,7 @@ int main() {
         expect_status(scmx_quantize_sc(f0, int(rng() % 2), r(), r(), r(), ocodes, obc, of, nullptr), "fuzz quantize_sc");
         expect_status(scmx_quantize_family(&f, f0, int(rng() % 2), r(), r(), ocodes, obc, of, nullptr), "fuzz quantize_family");
         (void)scmx_linear_w4a8_workspace(r(), r());
+        (void)scmx_mm_w4a8_prefers_blocked(r(), r(), r());
     }
     printf("%ld calls, %d failure(s)\n", calls, failures);
     return failures ? 1 : 0;
