@@ -583,7 +583,8 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a) {
                         const BlockLut t = scaled_lut_shift(0x03020100u, 0x0C080604u, 0u);   // folds to constants
                         decode_word_split(wj, t, e, o);
                     } else {
-                        const uint32_t blk = uint32_t(32 * c + 8 * j) >> a.fmt.block_log2;
+                        // (lanes past the row end, whose activations are zero, take its last chunk's block codes)
+                        const uint32_t blk = uint32_t(32 * min(c, uint32_t(nchunk - 1)) + 8 * j) >> a.fmt.block_log2;
                         const uint32_t code = block_code(brow + r * a.bc_row_bytes, blk, a.fmt.bc_bits);
                         const BlockLut t = scaled_lut_mul(a.fmt.lut_lo, a.fmt.lut_hi, mult_of(a.fmt, code));
                         decode_word_split(wj, t, e, o);

@@ -5,8 +5,8 @@ import numpy as np
 import pytest
 import torch
 
-from oracle import bf16, layout
-from tests.util import dev, host, llm_acts, product_format
+from oracle import bf16, layout, linear
+from tests.util import dev, host, llm_acts, product_format, random_packed
 
 pytestmark = pytest.mark.gpu
 F32 = np.float32
@@ -79,3 +79,24 @@ def test_views_of_rows(rows):
         assert torch.equal(G.gemv(xq, codes, bc, xs, ws, n, epi, fmt=fmt, **r), G.gemv(c(xq), codes, bc, c(xs), ws, n, epi, fmt=fmt, **rc))
         assert torch.equal(G.gemv(x, codes, bc, None, ws, n, epi, pro=1, fmt=fmt, **r),
                            G.gemv(c(x), codes, bc, None, ws, n, epi, pro=1, fmt=fmt, **rc))
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 8])
+@pytest.mark.parametrize("k", [128, 896, 2176])
+@pytest.mark.parametrize("fmt", [layout.Format(block=16, mult=tuple(range(1, 11)), bc_bits=4), layout.Format(block=16),
+                                 layout.Format(code_mag=(0, 1, 2, 3, 4, 5, 6, 7), mult=(1, 3, 9, 15)),
+                                 layout.Format(block=8, code_mag=(0, 1, 2, 3, 4, 5, 6, 7), mult=(1, 3, 9, 15), bc_bits=8)])
+def test_block_codes_at_the_end_of_their_memory(fmt, k, rows):
+    """Rows that do not fill the lanes of a step: the lanes past the end read no block codes past the last row.  The block codes
+    are the last bytes of an allocation that is whole pages of its own (20 MiB)."""
+    from mxfp4_int8_m5_amd import sc_decode as G
+    rng = np.random.default_rng(k + rows)
+    n, pf = 1152, product_format(fmt)
+    c, b, w, q = random_packed(rng, n, k, fmt)
+    whole = torch.empty(20 << 20, dtype=torch.uint8, device="cuda")
+    bc = whole[-b.size:].view(b.shape)
+    bc.copy_(dev(b))
+    xq = rng.integers(-127, 128, (rows, k)).astype(np.int8)
+    xs = rng.uniform(1e-3, 1e-2, rows).astype(F32)
+    y = host(G.gemv(dev(xq), dev(c), bc, dev(xs), dev(w), n, 1, fmt=pf)).reshape(rows, n)
+    assert np.array_equal(y, linear.gemv(xq, xs, q, w, 1).reshape(rows, n))
