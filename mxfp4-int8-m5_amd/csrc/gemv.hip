@@ -15,6 +15,8 @@
 // layers outside its shapes through gemv_mfma_kernel (4x4x4 INT8 MFMA); what is left through the per-row kernel's byte
 // tables, or, given a workspace, through the few-row GEMM (scmx_gemv_rows).  However formed, the totals are the GEMM's INT32
 // accumulators and the epilogues are the GEMM's.
+#include <type_traits>
+
 #include "gemm_args.h"
 
 namespace scmx {
@@ -101,11 +103,11 @@ __device__ __forceinline__ bool block_prefetch_row(const GemvArgs& a, int row, R
 
 // Stage one activation row into LDS and return its scale: permuted INT8 (8 bytes per 8-group), or with F16 the codes
 // as half-precision values in element order (16 bytes per 8-group).  `red` holds 68 floats.
-// have_pre: the row is in `pre` and is read no more: two workgroup barriers before the last one (three times fewer trips
-// to memory and four barriers less than the loops below with the RMSNorm prologue: gate|up 12288 x 2048 8.45 -> 7.7 us,
-// q|k|v 4096 x 2048 5.7 -> 4.9).
+// have_pre: the row is in `pre` already; a row that fits is fetched into it otherwise.  It is then read no more: two workgroup
+// barriers before the last one (three times fewer trips to memory and four barriers less than the loops for longer rows
+// with the RMSNorm prologue: gate|up 12288 x 2048 8.45 -> 7.7 us, q|k|v 4096 x 2048 5.7 -> 4.9).
 template <int NT, int XMODE, int KEEP>
-__device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, const RowPre<KEEP>& pre, bool have_pre) {
+__device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, RowPre<KEEP>& pre, bool have_pre) {
     constexpr bool F16 = XMODE == X_HALF;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int K = a.K;
@@ -135,12 +137,14 @@ __device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, c
         return __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(tot, float(K)), a.eps)));
     };
     float inv = 1.0f;
-    // eight values of a chunk, normalised for pro 2
-    auto values = [&](const u32x4& p, const u32x4& q, float (&v)[8]) {
+    // Eight values of a chunk, normalised where NORM says so.  (The prologue is a compile-time choice around each sweep: tested
+    // per value, the compiler loaded the norm weight value by value under those tests, eight trips to memory one after
+    // the other: one row, 6144 x 4096 10.1 us and 13.1.)
+    auto values = [&](auto norm, const u32x4& p, const u32x4& q, float (&v)[8]) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const float xv = __uint_as_float(i & 1 ? (p[i >> 1] & 0xFFFF0000u) : (p[i >> 1] << 16));
-            if (a.pro == 2) {
+            if constexpr (decltype(norm)::value) {
                 const float wv = __uint_as_float(i & 1 ? (q[i >> 1] & 0xFFFF0000u) : (q[i >> 1] << 16));
                 v[i] = round_bf16(__fmul_rn(wv, round_bf16(__fmul_rn(xv, inv))));
             } else {
@@ -166,7 +170,7 @@ __device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, c
         else if (XMODE == X_PLAIN8) store_plain8(sx + 8 * c, q);
         else store_perm8(sx + 8 * c, q);
     };
-    if (have_pre) {
+    if (have_pre || block_prefetch_row<NT, KEEP>(a, row, pre)) {
         if (a.pro == 2) {
             // A chunk holds virtual threads 2 (c % 32) and 2 (c % 32) + 1 of group c / 32: their sums stay apart through
             // lane distances 16 ... 1 (32 ... 2 between virtual threads) and are added last (distance 1).
@@ -196,13 +200,16 @@ __device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, c
         }
         float kept[KEEP][8];
         float amax = 0.0f;
+        auto normalise = [&](auto norm) {
 #pragma unroll
-        for (int j = 0; j < KEEP; ++j) {
-            if (tid + j * NT >= K / 8) break;
-            values(pre.x[j], pre.w[j], kept[j]);
+            for (int j = 0; j < KEEP; ++j) {
+                if (tid + j * NT >= K / 8) break;
+                values(norm, pre.x[j], pre.w[j], kept[j]);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(kept[j][i]));
-        }
+                for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(kept[j][i]));
+            }
+        };
+        if (a.pro == 2) normalise(std::true_type{}); else normalise(std::false_type{});
         scale_of(amax);
 #pragma unroll
         for (int j = 0; j < KEEP; ++j)
@@ -227,23 +234,28 @@ __device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, c
             __syncthreads();
             inv = total_inv();
         }
-        auto load = [&](int c, float (&v)[8]) {
-            const u32x4 p = *reinterpret_cast<const u32x4*>(xr + 8 * c);
-            values(p, a.pro == 2 ? *reinterpret_cast<const u32x4*>(a.nw + 8 * c) : p, v);
-        };
-        float amax = 0.0f;
-        for (int c = tid; c < K / 8; c += NT) {
-            float v[8];
-            load(c, v);
+        auto sweeps = [&](auto norm) {
+            auto load = [&](int c, float (&v)[8]) {
+                const u32x4 p = *reinterpret_cast<const u32x4*>(xr + 8 * c);
+                u32x4 q = u32x4{0u, 0u, 0u, 0u};
+                if constexpr (decltype(norm)::value) q = *reinterpret_cast<const u32x4*>(a.nw + 8 * c);
+                values(norm, p, q, v);
+            };
+            float amax = 0.0f;
+            for (int c = tid; c < K / 8; c += NT) {
+                float v[8];
+                load(c, v);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-        }
-        scale_of(amax);
-        for (int c = tid; c < K / 8; c += NT) {
-            float v[8];
-            load(c, v);
-            emit(c, v);
-        }
+                for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+            }
+            scale_of(amax);
+            for (int c = tid; c < K / 8; c += NT) {
+                float v[8];
+                load(c, v);
+                emit(c, v);
+            }
+        };
+        if (a.pro == 2) sweeps(std::true_type{}); else sweeps(std::false_type{});
     }
     __syncthreads();   // `red` is reused by the next row
     return s;
