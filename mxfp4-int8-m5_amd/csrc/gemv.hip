@@ -103,10 +103,10 @@ __device__ __forceinline__ bool block_prefetch_row(const GemvArgs& a, int row, R
 
 // Stage one activation row into LDS and return its scale: permuted INT8 (8 bytes per 8-group), or with F16 the codes
 // as half-precision values in element order (16 bytes per 8-group).  `red` holds 68 floats.
-// have_pre: the row is in `pre` already; a row that fits is fetched into it otherwise.  It is then read no more: two workgroup
+// have_pre: the row is in `pre` already; with FETCH a row that fits is fetched into it.  It is then read no more: two workgroup
 // barriers before the last one (three times fewer trips to memory and four barriers less than the loops for longer rows
 // with the RMSNorm prologue: gate|up 12288 x 2048 8.45 -> 7.7 us, q|k|v 4096 x 2048 5.7 -> 4.9).
-template <int NT, int XMODE, int KEEP>
+template <int NT, int XMODE, int KEEP, bool FETCH>
 __device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, RowPre<KEEP>& pre, bool have_pre) {
     constexpr bool F16 = XMODE == X_HALF;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -170,7 +170,7 @@ __device__ float stage_row(const GemvArgs& a, int row, int8_t* sx, float* red, R
         else if (XMODE == X_PLAIN8) store_plain8(sx + 8 * c, q);
         else store_perm8(sx + 8 * c, q);
     };
-    if (have_pre || block_prefetch_row<NT, KEEP>(a, row, pre)) {
+    if (have_pre || (FETCH && block_prefetch_row<NT, KEEP>(a, row, pre))) {
         if (a.pro == 2) {
             // A chunk holds virtual threads 2 (c % 32) and 2 (c % 32) + 1 of group c / 32: their sums stay apart through
             // lane distances 16 ... 1 (32 ... 2 between virtual threads) and are added last (distance 1).
@@ -711,7 +711,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a) {
             for (int c = tid; c < Kp * XB / 4; c += NT) reinterpret_cast<uint32_t*>(sx + size_t(b) * Kp * XB)[c] = 0u;
             continue;
         }
-        const float s = stage_row<NT, FP4 ? X_HALF : X_PERM8, KEEP>(a, xrow0 + b, sx + size_t(b) * Kp * XB, red, xpre, have_pre && b == 0);
+        const float s = stage_row<NT, FP4 ? X_HALF : X_PERM8, KEEP, (BATCH > 1)>(a, xrow0 + b, sx + size_t(b) * Kp * XB, red, xpre, have_pre && b == 0);
         for (int c = K * XB / 4 + tid; c < Kp * XB / 4; c += NT) reinterpret_cast<uint32_t*>(sx + size_t(b) * Kp * XB)[c] = 0u;
         if (tid == 0) sxs[b] = s;
     }
@@ -1251,7 +1251,10 @@ static void launch_gemv_rows(const GemvArgs& a, int slots, int dflt, hipStream_t
     if constexpr (BATCH > 1) {
         if (dflt && bc4 && !a.eidx) {
             const bool wide = hmfma_wide(dflt, a.N, a.K);
-            if (wide || hmfma_narrow(dflt, BATCH, a.N, a.K)) {
+            // (the RMSNorm of eight long rows in each of very many workgroups costs the 16-block formats more than their byte
+            // tables: eight rows, 24576 x 4096 166 us against 146; 6144 x 4096 55 against 77)
+            const bool heavy = (dflt == 2 || dflt == 3) && a.pro == 2 && long(BATCH) * a.K * (a.N / 16) > 32000000;
+            if (wide || (hmfma_narrow(dflt, BATCH, a.N, a.K) && !heavy)) {
                 switch (dflt) {
                     case 1: return launch_gemv_hmfma<BATCH, H_SC>(a, !wide, s);
                     case 2: return launch_gemv_hmfma<BATCH, H_B16>(a, !wide, s);
@@ -1359,11 +1362,23 @@ extern "C" size_t scmx_gemv_rows_workspace(const scmx_format* fmt, int pro, int 
     DevFormat f;
     if (pro != 1 || rows < 2 || rows > 8 || N <= 0 || K <= 0 || K % 128 || make_dev_format(fmt, &f)) return 0;
     const int dflt = format_kind(f);
-    // The narrow form stages all rows in each of its N / 16 workgroups: up to about 10 M values in all (eight rows, 12288 x
-    // 2048: 12.6 M, 11.8 us against 9.8 this way; 24576 x 4096: 50 M, 48 against 22; four rows, 12288 x 2048: 6.3 M, 7.3
-    // against 9).
-    const bool narrow = hmfma_narrow(dflt, kernel_rows_of(rows), N, K) && long(kernel_rows_of(rows)) * K * (N / 16) <= 10000000;
-    if (hmfma_wide(dflt, N, K) || narrow || !skinny_fits(rows, N, K, -1)) return 0;
+    const int kr = kernel_rows_of(rows);
+    if (hmfma_wide(dflt, N, K) || 16L * N > 480000) return 0;
+    // The narrow form stages all rows in each of its N / 16 workgroups.  Values staged in all, and us this way / through the
+    // GEMM: two to four rows, K = 4096: 17 M 15.2 / 16.0, 29 M 23.4 / 25.6; K = 8192: 8.4 M 19.4 / 16.4; 2048 x 6144 3.1 M 7.7 / 8.5.
+    // Eight rows: 4096 x 2048 4.2 M 5.9 / 6.3, 4096 x 4096 8.4 M 8.7 / 8.3, 12288 x 2048 12.6 M 9.5 / 9.0, 6144 x 4096 12.6 M 15.5 / 10.5.
+    const long staged = long(kr) * K * (N / 16);
+    if (hmfma_narrow(dflt, kr, N, K) && staged <= (kr == 8 ? 8000000 : K <= 4096 ? 30000000 : 5000000)) return 0;
+    // Two rows without that form are cheap where they lie: table decode costs the GEMM's 16-row groups more than the GEMV (2048
+    // x 2048 5.9 / 9.2, 16384 x 8192 38 / 60), but for short reductions of wide layers (9728 x 896 with SwiGLU 11.1 / 7.7); and
+    // a small layer is over before a second launch has started (896 x 896 4.5 / 5.1, 896 x 4864 6.8 / 7.1, 16-block formats
+    // 896 x 1664 5.2 / 5.8; but 2304 x 896 5.1 / 5.0, 4864 x 896 with SwiGLU 8.0 / 5.2).
+    if (rows == 2 && K <= 32768) {   // (what the GEMV's workgroups can stage)
+        const long size = long(N) * K;
+        if (dflt == 0 && (K > 1024 || N < 4096)) return 0;
+        if ((dflt == 1 || dflt == 4) && (size <= 2000000 || (K > 1024 && size <= 5000000))) return 0;
+        if ((dflt == 2 || dflt == 3) && K > 1024 && size <= 2000000) return 0;
+    }
     return scmx_linear_w4a8_workspace(rows, K);
 }
 

@@ -160,6 +160,17 @@ def test_attention_split_policy_and_cache_names(pkg):
     assert (f.block, f.bc_bits, tuple(f.mult)) == (16, 4, tuple(range(1, 11)))
     f = PF.sc_format_of("e2m1/B32/pow2")
     assert (f.block, f.bc_bits, tuple(f.mult)) == (32, 2, (1, 2, 4, 8))
+    # activation layout by shape: the few-row kernel where it is the faster one (one turn of workgroups, or short reductions)
+    few = [(9, 896, 896), (64, 2048, 6144), (128, 2048, 2048), (96, 4096, 4096), (64, 4096, 12288), (40, 9728, 896), (16, 12288, 4096)]
+    many = [(64, 6144, 4096), (33, 6144, 4096), (16, 24576, 4096), (128, 2048, 4096), (96, 4096, 8192), (16, 6144, 8192)]
+    assert [S.prefers_blocked(*s) for s in few + many] == [True] * len(few) + [False] * len(many)
+    # several GEMV rows: which go through the few-row GEMM (a workspace) and which through the kernels of the GEMV
+    ws = lambda fmt, *a: pkg._lib.native().scmx_gemv_rows_workspace(fmt.c, 1, *a) > 0   # noqa: E731
+    sc, b16, gen = pkg.sc_format.DEFAULT, pkg.sc_format.Format(block=16), pkg.sc_format.Format(code_mag=tuple(range(8)), mult=(1, 3, 9, 15))
+    assert [ws(sc, *a) for a in ((2, 896, 896), (2, 24576, 4096), (4, 28672, 4096), (8, 2048, 2048), (2, 896, 4864))] == [False] * 5
+    assert [ws(sc, *a) for a in ((3, 896, 896), (2, 8192, 8192), (8, 6144, 4096), (2, 4096, 12288), (2, 9728, 896))] == [True] * 5
+    assert [ws(gen, *a) for a in ((2, 2048, 2048), (2, 24576, 4096), (3, 2048, 2048), (2, 9728, 896))] == [False, False, True, True]
+    assert [ws(b16, *a) for a in ((2, 896, 1664), (2, 896, 896))] == [False, True]
     # row tile of the grouped GEMM by rows per expert (64 experts: 512 tokens x 8 -> 64 rows each, 1024 -> 128)
     assert [pkg.sc_moe.row_tile(t * 8, 64) for t in (1, 512, 767, 768, 4096)] == [64, 64, 64, 256, 256]
 
