@@ -279,9 +279,9 @@ __global__ __launch_bounds__(BLK ? 512 : 256, CH <= 12 ? 4 : CH <= 16 ? 3 : 1) v
 // xq as the large dense GEMM tiles take it: blocks of 32 rows x 32 k (1 KB), block (m / 32, k / 32) at
 // ((m / 32) * (K / 32) + k / 32) KB, and inside a block the 16 bytes of row r, k half h at (32 h + r) * 16 -- the order
 // in which the 64 lanes of a wave hold a 32x32x32 MFMA operand, so that a wave fetches one block with one coalesced load.
-// Rows of K <= 12288 go through act_quant_wave_kernel above, few rows and those of up to 16384 through act_quant_row_kernel
-// below; this is the kernel for longer rows: one wave per row, eight rows per workgroup, the row read twice, every lane writing the 16 bytes of
-// its own 16 elements.  Same codes and scales as act_quant_kernel: the row maximum does not depend on the order it is
+// Rows of K <= 12288 go through act_quant_wave_kernel above, few rows (up to 16384 values) through act_quant_row_kernel below;
+// this is the kernel for longer rows and for many of more than 12288 values: one wave per row, eight rows per workgroup, the
+// row read twice, every lane writing the 16 bytes of its own 16 elements.  Same codes and scales as act_quant_kernel: the row maximum does not depend on the order it is
 // taken in.
 __global__ __launch_bounds__(512) void act_quant_blocked_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
                                                                 float* __restrict__ xs, int M, int Mp, int K) {
@@ -453,11 +453,12 @@ using namespace scmx;
 // A workgroup per row while the rows are few (by rows from 2049 values on: 8 rows x 2048 2.2 us with a wave per row, 2.4 with
 // a workgroup; 4096 2.6 and 2.4), and for rows beyond a wave's registers (4000 rows x 12288 by rows: 36 us read twice, 23).
 // Blocked, its 16-byte stores of a single row fill no line: the wave kernel then, up to 12288 values (4000
-// rows x 12288: 40 us read twice, 29).
+// rows x 12288: 40 us read twice, 29), and beyond, from 1024 rows on, the one that reads them twice (14336 values: 600 rows as
+// fast either way, 1500 21.6 us and 22.8 by row workgroups, 4000 47.8 and 55.6).
 static bool act_quant_rows_fit(int Mp, int K, bool blocked) {
     if (K % 32 || K > 16384) return false;
     if (K <= 2048) return blocked && Mp <= 128 && K > 512;
-    return Mp <= 256 || K > (blocked ? 12288 : 8192);
+    return Mp <= (blocked && K > 12288 ? 1024 : 256) || (!blocked && K > 8192);
 }
 template <bool BLK>
 static void launch_act_quant_rows(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int K, hipStream_t st) {
