@@ -49,6 +49,23 @@ __device__ double block_sq_err(W&& weight, int e) {
     return ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
 }
 
+// The same with a lane per weight b, the block's lanes side by side: the sum in the first of them, by the same additions.
+template <int BLOCK>
+__device__ double lane_sq_err(double b, int e) {
+    const double x = b * pow2_f64(-e);
+    const double q = e2m1_level(e2m1_index(x));
+    const double d = (x < 0.0 ? -q : q) * pow2_f64(e) - b;
+    const double sq = d * d;
+    double r = sq + __shfl_down(sq, 8, BLOCK);
+    if (BLOCK == 32) {
+        r = r + __shfl_down(sq, 16, BLOCK);
+        r = r + __shfl_down(sq, 24, BLOCK);
+    }
+    r = r + __shfl_xor(r, 1, BLOCK);
+    r = r + __shfl_xor(r, 2, BLOCK);
+    return r + __shfl_xor(r, 4, BLOCK);
+}
+
 // BLOCK consecutive weights into registers; vec: the address is 16-byte aligned.
 template <int BLOCK, bool BF16>
 __device__ __forceinline__ void load_block(const void* __restrict__ w, size_t at, bool vec, float (&v)[BLOCK]) {
@@ -134,59 +151,85 @@ __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict
 
     // ---- exponent of every block (sim/mx_int8.py:39-65, rule "search") --------------------------------------------
     float v[BLOCK];
-    for (int b = tid; b < total; b += QNT) {
+    for (int b0 = tid & ~63; b0 < total; b0 += QNT) {   // whole waves, for the ties
+        const int b = b0 + lane;
         const size_t at = base + size_t(b) * BLOCK;
-        load_block<BLOCK, BF16>(w, at, vec, v);
-        float amax = 0.0f;
+        int chosen = EMPTY, e0 = 0;
+        bool tie = false;
+        auto weight = [&](size_t i) -> float {
+            if (BF16) return bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[i]);
+            return reinterpret_cast<const float*>(w)[i];
+        };
+        if (b < total) {
+            load_block<BLOCK, BF16>(w, at, vec, v);
+            float amax = 0.0f;
 #pragma unroll
-        for (int i = 0; i < BLOCK; ++i) amax = fmaxf(amax, fabsf(v[i]));
-        int chosen = EMPTY;
-        if (amax > 0.0f) {
-            // floor(log2 amax) of a float32-born value is its binary exponent
-            const int e0 = int((__double_as_longlong(double(amax)) >> 52) & 0x7FF) - 1023 - 2;
-            float x[BLOCK];
+            for (int i = 0; i < BLOCK; ++i) amax = fmaxf(amax, fabsf(v[i]));
+            if (amax > 0.0f) {
+                // floor(log2 amax) of a float32-born value is its binary exponent
+                e0 = int((__double_as_longlong(double(amax)) >> 52) & 0x7FF) - 1023 - 2;
+                float x[BLOCK];
 #pragma unroll
-            for (int i = 0; i < BLOCK; ++i) x[i] = __builtin_amdgcn_ldexpf(v[i], -e0);
-            const float s0 = fp4_sq_err<BLOCK>(x, 1.0f), sm = fp4_sq_err<BLOCK>(x, 0.5f), sp = fp4_sq_err<BLOCK>(x, 2.0f);
-            // A float32 sum of 32 squares of exact differences is within 32 half-ulps (2e-6) of the exact one, the host's
-            // float64 sum within 1e-14: apart by more than 1e-5, the sums order alike.  (Below 1e-30 squares underflow.)
-            auto close = [](float a, float b) { return !(fabsf(a - b) > 1e-5f * fmaxf(a, b)) || fmaxf(a, b) < 1e-30f; };
-            const float s1 = sm < s0 ? sm : s0;
-            if (close(sm, s0) || close(sp, s1)) {
-                auto weight = [&](int i) -> float {
-                    if (BF16) return bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[at + i]);
-                    return reinterpret_cast<const float*>(w)[at + i];
-                };
-                double best = block_sq_err<BLOCK>(weight, e0);
-                chosen = e0;
-                double t = block_sq_err<BLOCK>(weight, e0 - 1);
-                if (t < best) {
-                    best = t;
-                    chosen = e0 - 1;
-                }
-                t = block_sq_err<BLOCK>(weight, e0 + 1);
-                if (t < best) chosen = e0 + 1;
-            } else {
+                for (int i = 0; i < BLOCK; ++i) x[i] = __builtin_amdgcn_ldexpf(v[i], -e0);
+                const float s0 = fp4_sq_err<BLOCK>(x, 1.0f), sm = fp4_sq_err<BLOCK>(x, 0.5f), sp = fp4_sq_err<BLOCK>(x, 2.0f);
+                // A float32 sum of 32 squares of exact differences is within 32 half-ulps (2e-6) of the exact one, the host's
+                // float64 sum within 1e-14: apart by more than 1e-5, the sums order alike.  (Below 1e-30 squares underflow.)
+                auto close = [](float a, float b) { return !(fabsf(a - b) > 1e-5f * fmaxf(a, b)) || fmaxf(a, b) < 1e-30f; };
+                const float s1 = sm < s0 ? sm : s0;
+                tie = close(sm, s0) || close(sp, s1);
                 chosen = sp < s1 ? e0 + 1 : sm < s0 ? e0 - 1 : e0;
             }
         }
-        s_e[b] = chosen;
+        // Near ties in float64.  A few of them the wave takes one after the other, a lane per weight (about 1.5 us each); where
+        // many lanes have one, each sums its own (15 us in all, as one does: a matrix of a few rows waited for its one tie).
+        uint64_t ties = __ballot(tie);
+        auto decide = [&](double t0, double tm, double tp) {
+            double best = t0;
+            int e = e0;
+            if (tm < best) {
+                best = tm;
+                e = e0 - 1;
+            }
+            return tp < best ? e0 + 1 : e;
+        };
+        if (__popcll(ties) > 8) {
+            if (tie) {
+                auto mine = [&](int i) { return weight(at + i); };
+                chosen = decide(block_sq_err<BLOCK>(mine, e0), block_sq_err<BLOCK>(mine, e0 - 1), block_sq_err<BLOCK>(mine, e0 + 1));
+            }
+        } else {
+            while (ties) {
+                const int src = __ffsll((unsigned long long)ties) - 1;
+                ties &= ties - 1;
+                const int e = __shfl(e0, src, WAVE), group = lane / BLOCK;
+                const double a = double(weight(base + size_t(b0 + src) * BLOCK + lane % BLOCK));
+                // lane group 0: exponent e, group 1: e - 1, the others e + 1 (of 32 lanes there are two groups: once more)
+                const double first = lane_sq_err<BLOCK>(a, group == 0 ? e : group == 1 ? e - 1 : e + 1);
+                const double third = BLOCK == 16 ? first : lane_sq_err<BLOCK>(a, e + 1);
+                const double t0 = __shfl(first, 0, WAVE), tm = __shfl(first, BLOCK, WAVE);
+                const double tp = __shfl(third, BLOCK == 16 ? 32 : 0, WAVE);
+                if (lane == src) chosen = decide(t0, tm, tp);
+            }
+        }
+        if (b < total) s_e[b] = chosen;
     }
     __syncthreads();
 
-    // ---- row constraint (sim/mx_int8.py:68-81) and the row's lowest exponent (sim/mx_int8.py:92-109): a wave per row ---
-    for (int r = tid >> 6; r < live; r += QNT / 64) {
+    // ---- row constraint (sim/mx_int8.py:68-81) and the row's lowest exponent (sim/mx_int8.py:92-109): as many lanes per row, a
+    // wave at most, as let the rows go side by side (a wave each, 64 rows took 16 turns: 64 x 128 13 us) ---------------------
+    int per = 64;
+    while (per * rows > QNT && per > 1) per >>= 1;
+    for (int r = tid / per; r < live; r += QNT / per) {
+        const int l = tid & (per - 1);
         int top = EMPTY;
-        for (int i = lane; i < nb; i += 64) top = max(top, s_e[r * nb + i]);
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) top = max(top, __shfl_xor(top, off, WAVE));
+        for (int i = l; i < nb; i += per) top = max(top, s_e[r * nb + i]);
+        for (int off = per >> 1; off >= 1; off >>= 1) top = max(top, __shfl_xor(top, off, WAVE));
         if (top == EMPTY) top = 0;   // all-zero row
         const int floor_e = top - MAX_SPREAD;
         int lo = INT_MAX;
-        for (int i = lane; i < nb; i += 64) lo = min(lo, max(s_e[r * nb + i], floor_e));
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) lo = min(lo, __shfl_xor(lo, off, WAVE));
-        if (lane == 0) {
+        for (int i = l; i < nb; i += per) lo = min(lo, max(s_e[r * nb + i], floor_e));
+        for (int off = per >> 1; off >= 1; off >>= 1) lo = min(lo, __shfl_xor(lo, off, WAVE));
+        if (l == 0) {
             s_floor[r] = floor_e;
             s_lo[r] = lo;
             wscale[row0 + r] = float(pow2_f64(lo - 1));   // 2^(E_lo - 1), sim/mx_int8.py:101
@@ -334,7 +377,9 @@ constexpr int FAM_ROWS = 4;   // rows per workgroup at most: more are needed onl
 
 // Bound: vector ALU (8 bases x n_mult trials per weight, 13 instructions each), 96 % busy.  2048 x 2048 bf16, ten multipliers: 130 us; 520 us with a lane
 // per weight, a correctly rounded division per trial and the sums across lanes.
-template <int BLOCK, bool BF16, bool E2M1>
+// SPREAD: a thread per block and base (fewer blocks than the chip has lanes: each would run all trials in one lane; 64 x 128,
+// ten multipliers 49 us).
+template <int BLOCK, bool BF16, bool E2M1, bool SPREAD>
 __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                              uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
                                                              int64_t N, int K, int rows, bool vec, const FamilyArgs f) {
@@ -371,15 +416,17 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
     };
 
     // ---- per candidate base and block: the best multiplier and its error ------------------------------------------
-    for (int b = tid; b < total; b += QNT) {
-        if (total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+    constexpr int BASES = SPREAD ? 1 : 8;   // bases per thread
+    for (int t = tid; t < total * (8 / BASES); t += QNT) {
+        const int b = t / (8 / BASES), j0 = SPREAD ? t % 8 : 0;
+        if (SPREAD || total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
         const int r = b / nb, kb = b - r * nb;
         const float top = row_top(r);
         float aw[BLOCK];
 #pragma unroll
         for (int i = 0; i < BLOCK; ++i) aw[i] = fabsf(v[i]);
 #pragma unroll 1
-        for (int j = 0; j < 8; ++j) {
+        for (int j = j0; j < j0 + BASES; ++j) {
             const float base = __fmul_rn(top, ladder[j]);
             float best = 0.0f;
             int best_i = 0;
@@ -418,7 +465,7 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
 
     // ---- codes ----------------------------------------------------------------------------------------------------
     for (int b = tid; b < total; b += QNT) {
-        if (total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+        if (SPREAD || total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
         const int r = b / nb, kb = b - r * nb, bj = s_best[r];
         const float base = __fmul_rn(row_top(r), ladder[bj]);
         const bool dead = base == 0.0f;   // a vanishing row underflows its base: it is exactly zero (e2e/pack_format.py:55-58)
@@ -501,7 +548,8 @@ extern "C" int scmx_quantize_family(const scmx_format* fmt, const void* w, int w
     f.bc_bits = fmt->bc_bits;
     if (N == 0) return SCMX_OK;
     const int nb = K / block;
-    const int rows = rows_per_group(nb, FAM_ROWS);
+    const bool spread = N * nb <= 65536;   // a wave per SIMD
+    const int rows = rows_per_group(spread ? 8 * nb : nb, FAM_ROWS);
     const size_t smem = size_t(rows) * 8 * nb * (sizeof(float) + 1);
     const dim3 grid((unsigned)((N + rows - 1) / rows)), wg(QNT);
     const bool vec = uintptr_t(w) % 16 == 0 && uintptr_t(codes) % 16 == 0;
@@ -512,8 +560,8 @@ extern "C" int scmx_quantize_family(const scmx_format* fmt, const void* w, int w
     auto typed = [&](auto blk, auto bf) {
         constexpr int B = decltype(blk)::value;
         constexpr bool BF = decltype(bf)::value;
-        if (e2m1) go(quantize_family_kernel<B, BF, true>);
-        else go(quantize_family_kernel<B, BF, false>);
+        if (e2m1) spread ? go(quantize_family_kernel<B, BF, true, true>) : go(quantize_family_kernel<B, BF, true, false>);
+        else spread ? go(quantize_family_kernel<B, BF, false, true>) : go(quantize_family_kernel<B, BF, false, false>);
     };
     by_block_and_type(block, w_is_bf16, typed);
     return check_launch("quantize_family");

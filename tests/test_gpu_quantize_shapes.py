@@ -64,6 +64,33 @@ def test_family(n, k, as_bf16, shift, name):
     assert np.array_equal(host(dc).view(np.uint32), codes)
 
 
+@pytest.mark.parametrize("name", ["e2m1/B16/M1..10", "int4/B16/M1..16"])
+def test_family_many_blocks(name):
+    """Enough blocks for a thread to take all bases of one (70400; the shapes above spread a block's bases over threads)."""
+    test_family(1100, 1024, True, 0, name)
+
+
+@pytest.mark.parametrize("block", [16, 32])
+@pytest.mark.parametrize("as_bf16", [False, True])
+@pytest.mark.parametrize("share", [0.002, 0.1, 1.0])
+def test_published_format_ties(share, as_bf16, block):
+    """Blocks of whole levels, whose sums tie or vanish at two exponents, among blocks that do not: none or a few of a wave's
+    lanes have one (the wave sums it), many or all (each lane its own)."""
+    from mxfp4_int8_m5_amd import sc_format as SF
+    rng = np.random.default_rng(int(1000 * share) + block)
+    n, k = 70, 1024
+    w = llm_weights(rng, n, k).astype(F32)
+    tied = np.repeat(rng.random((n, k // block)) < share, block, axis=1)
+    w[tied] = (rng.choice([0.0, 1.0, 2.0, 3.0, 4.0, 6.0], tied.sum()) * rng.choice([-1, 1], tied.sum()) * 2.0 ** -4).astype(F32)
+    if as_bf16:
+        w = bf16.from_bits(bf16.to_bits(w))
+    fmt = layout.Format(block=block)
+    codes, bc, ws, q = layout.quantize(w.astype(np.float64), fmt)
+    dc, db, dw, dq = SF.quantize(_device(w, as_bf16, 0), product_format(fmt))
+    assert np.array_equal(host(dc).view(np.uint32), codes)
+    assert np.array_equal(host(db), bc) and np.array_equal(host(dw), ws) and np.array_equal(host(dq), q)
+
+
 @pytest.mark.parametrize("block", [16, 32])
 @pytest.mark.parametrize("as_bf16", [False, True])
 def test_family_codebook_without_a_zero(monkeypatch, as_bf16, block):
