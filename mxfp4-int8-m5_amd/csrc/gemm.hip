@@ -858,9 +858,15 @@ static int packed_mode(const DevFormat& f) {
 // Dense: one launch, with the tile a cost model of the candidates below makes fastest.
 // Which tile a dense problem runs on: the index into the candidate table below.  blocked: the activations are in the
 // blocked layout, which four tiles read (their waves then load activation fragments straight from memory).
-static int dense_choice(long M, long N, long K, bool blocked) {
+// (Asked for on every call of a layer: shifts where the sizes are powers of two, no division for less than one wave.)
+struct TileChoice {
+    int index;
+    float us;   // its modelled time
+    int cus;
+};
+static TileChoice dense_choice(long M, long N, long K, bool blocked) {
     const long cus = device_cus();
-    auto tiles = [&](int bm, int bn) { return long((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    auto tiles = [&](int bm, int bn) { return ((M + bm - 1) >> __builtin_ctz(bm)) * ((N + bn - 1) >> __builtin_ctz(bn)); };
     // The tile is the one a small cost model makes fastest.  A launch runs its tiles in waves of (CUs x workgroups that
     // share a CU); a wave costs F + S per 128 of K and not less than W, all three measured per configuration and per
     // number of co-resident workgroups (four Qwen3-1.7B layer shapes and five others, K = 128 ... 6144, M = 64 ... 8192:
@@ -903,10 +909,10 @@ static int dense_choice(long M, long N, long K, bool blocked) {
         if (c == 5 && (n > cus || K % 256)) continue;
         if (c == 6 && (n > cus || K % 512)) continue;
         const long cap = cus * k.occ;
-        const long full = n / cap, rest = n % cap;
+        const long full = n < cap ? 0 : n / cap, rest = n - full * cap;
         float t = float(full) * fmaxf(k.f[k.occ - 1] + steps * k.s[k.occ - 1], k.w[k.occ - 1]);
         if (rest) {
-            const int r = int((rest + cus - 1) / cus);   // workgroups per CU in the last wave
+            const int r = rest <= cus ? 1 : int((rest + cus - 1) / cus);   // workgroups per CU in the last wave
             float w = fmaxf(k.f[r - 1] + steps * k.s[r - 1], k.w[r - 1]);
             if (r == 1) {   // CUs idle
                 const float fill = float(rest) / float(cus);
@@ -921,12 +927,30 @@ static int dense_choice(long M, long N, long K, bool blocked) {
             best = c;
         }
     }
-    return best;
+    return {best, best_t, int(cus)};
+}
+
+// Whether the few-row kernel is faster than the row-layout tiles (`tile`: the one of those that it would replace), by the two
+// models.  The table of the 64x32 tile was fitted to more rows: here it takes 1.27 times that, 1.35 where half of the CUs or more
+// have none (that does not make it faster here).  Formats whose codes are looked up: a tile's weights are decoded again by each
+// of its row groups, once by this kernel, which is worth half as much again.  On 4268 problems (16 ... 128 rows, widths 512 ...
+// 24576, reductions 512 ... 11008, both kernels timed) the choice costs 0.2 - 0.5 per cent over the faster one on average, by
+// format, and 11 - 30 per cent at most (one row tile of wide MXFP4 layers: 12288 x 8192 27.7 us for 21.2); the few-row kernel always
+// 3 - 4 (tables 0.6), the tiles always 20 (54).  us, few-row / tiles, whole linears: 2048 x 6144 at 80 rows 13.3 / 14.2, 4096 x
+// 8192 at 80 19.1 / 16.7, 896 x 5632 at 96 12.1 / 13.4, 6144 x 4096 at 64 15.5 / 11.6 (tables 24.6 / 19.4), 6144 x 4480 (no K groups
+// for the tiles) 15.0 / 17.0, 896 x 4864 at 112 13.2 / 15.4, 6144 x 4864 at 64 with tables 25.2 / 32.8.
+static bool few_rows(const scmx_format* fmt, int M, int N, int K, TileChoice tile) {
+    if (M < 1 || M > SKINNY_MAX_ROWS || N < 1 || K < 1 || long(M + 15) / 16 * 16 * N > 480000) return false;   // (beyond: not measured)
+    const float t = skinny_time(M, N, K, tile.cus);
+    const float more = tile.index != 6 ? 1.0f : long(M + 63) / 64 * ((N + 31) / 32) * 2 <= tile.cus ? 1.35f : 1.27f;
+    if (t < more * tile.us) return true;
+    DevFormat f;
+    return fmt && t < 1.5f * more * tile.us && make_dev_format(fmt, &f) == SCMX_OK && packed_mode(f) == B_PACKED_GENERIC;
 }
 
 static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
-    if (a.blocked && skinny_fits(a.M, a.N, a.K, bmode)) return launch_skinny(a, bmode, s);
-    const int best = dense_choice(a.M, a.N, a.K, a.blocked != 0);
+    if (a.blocked == FEW_ROWS) return launch_skinny(a, bmode, s);
+    const int best = dense_choice(a.M, a.N, a.K, a.blocked != 0).index;
     if (a.blocked) {
         switch (best) {
             case 0: return launch_tile<256, 256, 64, 4, 2, 1, 2, false, false, 1, true>(a, bmode, (a.M + 255) / 256, s);
@@ -1007,7 +1031,7 @@ int scmx_mm_i8_i32(const int8_t* xq, const int8_t* wq, int32_t* acc, int M, int 
 
 static int mm_w4a8(const scmx_format* fmt, const int8_t* xq, const float* xscale, const uint32_t* codes,
                    const uint8_t* bcodes, const float* wscale, const uint16_t* res, void* out, int epi, int M, int N,
-                   int K, bool blocked, void* stream) {
+                   int K, int blocked, void* stream) {
     DevFormat f;
     if (int rc = make_dev_format(fmt, &f)) return rc;
     if (int rc = check_gemm_common("mm_w4a8", M, N, K, epi, true, xq, xscale, wscale, res, out)) return rc;
@@ -1032,7 +1056,7 @@ static int mm_w4a8(const scmx_format* fmt, const int8_t* xq, const float* xscale
 int scmx_mm_w4a8(const scmx_format* fmt, const int8_t* xq, const float* xscale, const uint32_t* codes,
                  const uint8_t* bcodes, const float* wscale, const uint16_t* res, void* out, int epi, int M, int N,
                  int K, void* stream) {
-    return mm_w4a8(fmt, xq, xscale, codes, bcodes, wscale, res, out, epi, M, N, K, false, stream);
+    return mm_w4a8(fmt, xq, xscale, codes, bcodes, wscale, res, out, epi, M, N, K, 0, stream);
 }
 
 int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* xscale, const uint32_t* codes,
@@ -1046,12 +1070,14 @@ int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* 
         set_error("mm_w4a8_blocked: the activations' whole 32-row blocks lie beyond the 32-bit offsets of the kernel (M=%d K=%d)", M, K);
         return SCMX_ERR_ARG;
     }
-    return mm_w4a8(fmt, xq, xscale, codes, bcodes, wscale, res, out, epi, M, N, K, true, stream);
+    const bool few = M > 0 && N > 0 && K > 0 && few_rows(fmt, M, N, K, dense_choice(M, N, K, false));
+    return mm_w4a8(fmt, xq, xscale, codes, bcodes, wscale, res, out, epi, M, N, K, few ? FEW_ROWS : 1, stream);
 }
 
 int scmx_mm_w4a8_prefers_blocked(int M, int N, int K) {
-    return M > 0 && N > 0 && K > 0 && K % 128 == 0 &&
-           (skinny_fits(M, N, K, B_PACKED_DEFAULT) || dense_choice(M, N, K, false) <= 2);
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
+    const TileChoice tile = dense_choice(M, N, K, false);
+    return tile.index <= 2 || few_rows(nullptr, M, N, K, tile);
 }
 
 // The fused layer quantizes into whichever layout suits the shape: blocked where the row-layout model would run one of its
@@ -1060,8 +1086,11 @@ static int quantize_and_multiply(const scmx_format* fmt, const uint16_t* x, int8
                                  const uint32_t* codes, const uint8_t* bcodes, const float* wscale, const uint16_t* res,
                                  void* out, int epi, int M, int N, int K, void* stream) {
     const long long Mp = (static_cast<long long>(M) + 31) & ~31LL;
-    const bool blocked = room_for_blocks && Mp <= (1LL << 30) && uint64_t(Mp) * uint64_t(K > 0 ? K : 0) <= 0xFFFFFFFFull &&
-                         scmx_mm_w4a8_prefers_blocked(M, N, K);
+    int blocked = 0;
+    if (room_for_blocks && M > 0 && N > 0 && K > 0 && K % 128 == 0 && uint64_t(Mp) * uint64_t(K) <= 0xFFFFFFFFull) {
+        const TileChoice tile = dense_choice(M, N, K, false);
+        blocked = few_rows(fmt, M, N, K, tile) ? FEW_ROWS : tile.index <= 2;
+    }
     if (blocked) {
         if (int rc = scmx_act_quant_blocked(x, xq, xs, M, int(Mp), K, stream)) return rc;
     } else {

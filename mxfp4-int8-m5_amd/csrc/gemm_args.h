@@ -21,7 +21,7 @@ struct GemmArgs {
     const uint16_t* silu;    // SwiGLU epilogue: lookup table over bf16 gate values
     const int32_t* tstart;   // grouped: first row tile of each expert [E+1]
     int n_experts;
-    int blocked;             // dense: xq is in the blocked layout
+    int blocked;             // dense: xq is in the blocked layout (FEW_ROWS: and the few-row kernel takes it)
     DevFormat fmt;
 };
 
@@ -31,10 +31,12 @@ struct GemmArgs {
 // decode).
 // B_PACKED_E8M0: a standard MXFP4 tensor in place -- B_PACKED_DEFAULT's decode with the block's shift taken from its
 // E8M0 byte minus the row's lowest one (which the row scale carries).
+enum { FEW_ROWS = 2 };   // GemmArgs::blocked
 enum { B_INT8 = 0, B_PACKED_DEFAULT = 1, B_PACKED_GENERIC = 2, B_PACKED_B16 = 3, B_PACKED_B16M = 4, B_PACKED_E8M0 = 5 };
 
-// True when the few-row kernel takes this dense problem (activations in the blocked layout).
-bool skinny_fits(int M, int N, int K, int bmode);
+constexpr int SKINNY_MAX_ROWS = 128;
+// The few-row kernel's time (us) on a dense problem of up to SKINNY_MAX_ROWS rows, activations in the blocked layout.
+float skinny_time(int M, int N, int K, int cus);
 void launch_skinny(const GemmArgs& a, int bmode, hipStream_t s);
 
 }  // namespace scmx

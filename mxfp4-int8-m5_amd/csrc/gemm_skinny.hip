@@ -147,22 +147,14 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
     }
 }
 
-// Where it is the faster one.  A CU runs `turns` = ceil(N / 16 / CUs) workgroups, each of which reads all 16 ceil(M / 16) rows
-// of activations: from two turns on that costs what the tiled kernel's idle CUs cost it.  Whole linears, this / row-layout
-// tiles, us, one turn: 4096 x 2048 at M = 64 7.3 / 8.6, at 96 8.4 / 9.0, at 128 8.9 / 8.8; 4096 x 4096 at 64 10.4 / 11.3, at 96 12.2 /
-// 11.7 (formats with table decode 16.9 / 19.2), 2048 x 4096 at 112 12.3 / 11.0; 4096 x 6144 at 96 14.6 / 14.8, at 112 15.9 / 14.7;
-// 4096 x 12288 at 64 22.7 / 22.9, at 80 26 / 22.7.  More turns: K = 896 wins wherever M N <= 480 000; 6144 x 1536 at 64 8.3 / 8.3,
-// 9728 x 2048 at 32 10.0 / 10.0, at 48 10.9 / 10.1, 28672 x 2048 at 16 14.6 / 14.3; 6144 x 2304 at 48 9.9 / 10.5, at 64 11.3 / 10.6,
-// 16384 x 2304 at 16 12.0 / 11.3; 6144 x 3072 at 32 10.2 / 10.3, at 48 11.0 / 10.5; 12288 x 4096 at 16 13.7 / 14.0, 6144 x 4096 at
-// 32 12.2 / 11.2, at 64 15.5 / 11.6; 9728 x 6144 at 16 16.7 / 17.8; from K = 8192 on it loses (6144 x 8192 at 16 16.6 / 15.8).
-constexpr int SKINNY_MAX_ROWS = 128;
-bool skinny_fits(int M, int N, int K, int bmode) {
-    if (M > SKINNY_MAX_ROWS || bmode == B_INT8) return false;
-    const long rows = (M + 15) / 16 * 16, cus = device_cus(), turns = ((long(N) + 15) / 16 + cus - 1) / cus;
-    if (rows * N > 480000) return false;
-    if (turns == 1) return rows <= (K <= 3072 ? 128 : K <= 6144 ? 96 : 64);
-    const long most = K <= 1024 ? 160 : K <= 2048 ? 112 : K <= 2560 ? (turns == 2 ? 96 : 48) : K <= 3072 ? (turns == 2 ? 64 : 48) : K <= 6144 ? 48 : 0;
-    return turns * rows <= most;
+// Its time in us beside what any launch costs.  A CU runs `turns` = ceil(N / 16 / CUs) workgroups, each of which walks its
+// weights and all 16 ceil(M / 16) rows of activations (five row tiles run as six, seven as eight).  Fitted to 1002 problems (13
+// widths 896 ... 28672, 27 reductions 512 ... 14336, 16 ... 128 rows): within 5 per cent.
+float skinny_time(int M, int N, int K, int cus) {
+    const int tiles = (M + 15) / 16, columns = (N + 15) / 16, turns = columns <= cus ? 1 : (columns + cus - 1) / cus;
+    const float more = 16.0f * float((tiles == 5 ? 6 : tiles == 7 ? 8 : tiles) - 1), k = float(K);
+    return K <= 2048 ? 0.33f + 1.6e-5f * k + float(turns) * k * (5.6e-4f + 1.19e-5f * more)
+                     : 1.31e-4f * k - 0.3f + float(turns) * k * (6.8e-4f + 1.03e-5f * more);
 }
 
 void launch_skinny(const GemmArgs& args, int bmode, hipStream_t s) {

@@ -161,8 +161,9 @@ def test_attention_split_policy_and_cache_names(pkg):
     f = PF.sc_format_of("e2m1/B32/pow2")
     assert (f.block, f.bc_bits, tuple(f.mult)) == (32, 2, (1, 2, 4, 8))
     # activation layout by shape: the few-row kernel where it is the faster one (one turn of workgroups, or short reductions)
-    few = [(9, 896, 896), (64, 2048, 6144), (128, 2048, 2048), (96, 4096, 4096), (64, 4096, 12288), (40, 9728, 896), (16, 12288, 4096)]
-    many = [(64, 6144, 4096), (33, 6144, 4096), (16, 24576, 4096), (128, 2048, 4096), (96, 4096, 8192), (16, 6144, 8192)]
+    few = [(9, 896, 896), (64, 2048, 6144), (128, 2048, 2048), (96, 4096, 4096), (64, 4096, 12288), (40, 9728, 896), (16, 12288, 4096),
+           (112, 896, 4864), (64, 6144, 4480), (16, 6144, 8960), (80, 2048, 6144), (96, 896, 5632)]
+    many = [(64, 6144, 4096), (33, 6144, 4096), (16, 28672, 4096), (128, 2048, 4096), (96, 4096, 8192), (80, 4096, 8192)]
     assert [S.prefers_blocked(*s) for s in few + many] == [True] * len(few) + [False] * len(many)
     # several GEMV rows: which go through the few-row GEMM (a workspace) and which through the kernels of the GEMV
     ws = lambda fmt, *a: pkg._lib.native().scmx_gemv_rows_workspace(fmt.c, 1, *a) > 0   # noqa: E731
