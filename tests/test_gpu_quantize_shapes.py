@@ -66,7 +66,8 @@ def test_family(n, k, as_bf16, shift, name):
 
 @pytest.mark.parametrize("name", ["e2m1/B16/M1..10", "int4/B16/M1..16"])
 def test_family_many_blocks(name):
-    """Enough blocks for a thread to take all bases of one (70400; the shapes above spread a block's bases over threads)."""
+    """Enough blocks for a thread to take all bases of one (70400 and 35200; the shapes above spread a block's bases over threads)."""
+    test_family(1100, 512, True, 0, name)
     test_family(1100, 1024, True, 0, name)
 
 
