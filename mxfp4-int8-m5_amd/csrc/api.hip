@@ -211,8 +211,8 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
 // r, k 16 c ... at slot c * 8 + (r + c / 2) % 8 -- and are stored as whole 128-byte lines (8 rows x 16 bytes are adjacent
 // in a block).  The loads stay what they are by rows: 16 contiguous bytes per lane.
 // (Registers are held to what lets four waves share a SIMD up to 6144 values, three up to 8192: 4000 rows x 6144 blocked 16.6
-// us at three, 13.0 at four.  Whole rows of up to 6144 in the row layout fit without it and are given fewer registers then: 4096 values 76
-// for 82, six waves a SIMD for five, 3 - 6 per cent at 257 ... 1500 rows.)
+// us at three, 13.0 at four.  Whole rows of up to 6144 in the row layout fit without it and are given fewer registers then:
+// 4096 values 76 for 82, six waves a SIMD for five, 3 - 6 per cent at 257 ... 1500 rows.)
 template <int CH, bool BLK, bool WHOLE>
 __global__ __launch_bounds__(BLK ? 512 : 256, !BLK && WHOLE && CH <= 12 ? 1 : CH <= 12 ? 4 : CH <= 16 ? 3 : 1) void act_quant_wave_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
                                                                          float* __restrict__ xs, int M, int Mp, int K_any) {

@@ -132,9 +132,9 @@ __device__ __forceinline__ float fp4_sq_err(const float (&x)[BLOCK], float scale
     return r0 + r1;
 }
 
-// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: 37 vector instructions per weight, which keep the vector
-// ALU busy 63 % of the time with two waves a SIMD, and a wave's wait for its loads (39 % of its life) the rest; not HBM.
-// 12288 x 2048 bf16: 44.5 us (1.4 TB/s); 234 us with a lane per weight and every candidate in float64 across lanes.
+// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: vector ALU, 95 % busy with 39 instructions per weight
+// and 2.6 waves a SIMD.  12288 x 2048 bf16: 28.8 us (2.2 TB/s); 44 us with the near ties summed by one lane of the wave, 234 us
+// with a lane per weight and every candidate in float64 across lanes.
 template <int BLOCK, bool BF16>
 __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                          uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
