@@ -862,10 +862,8 @@ static int packed_mode(const DevFormat& f) {
 struct TileChoice {
     int index;
     float us;   // its modelled time
-    int cus;
 };
-static TileChoice dense_choice(long M, long N, long K, bool blocked) {
-    const long cus = device_cus();
+static TileChoice dense_choice(long M, long N, long K, bool blocked, long cus) {
     auto tiles = [&](int bm, int bn) { return ((M + bm - 1) >> __builtin_ctz(bm)) * ((N + bn - 1) >> __builtin_ctz(bn)); };
     // The tile is the one a small cost model makes fastest.  A launch runs its tiles in waves of (CUs x workgroups that
     // share a CU); a wave costs F + S per 128 of K and not less than W, all three measured per configuration and per
@@ -927,10 +925,10 @@ static TileChoice dense_choice(long M, long N, long K, bool blocked) {
             best = c;
         }
     }
-    return {best, best_t, int(cus)};
+    return {best, best_t};
 }
 
-// Whether the few-row kernel is faster than the row-layout tiles (`tile`: the one of those that it would replace), by the two
+// Whether the few-row kernel is faster than the row-layout tiles (the one that it would replace), by the two
 // models.  The table of the 64x32 tile was fitted to more rows: here it takes 1.27 times that, 1.35 where half of the CUs or more
 // have none (that does not make it faster here).  Formats whose codes are looked up: a tile's weights are decoded again by each
 // of its row groups, once by this kernel, which is worth half as much again.  On 4268 problems (16 ... 128 rows, widths 512 ...
@@ -939,18 +937,24 @@ static TileChoice dense_choice(long M, long N, long K, bool blocked) {
 // 3 - 4 (tables 0.6), the tiles always 20 (54).  us, few-row / tiles, whole linears: 2048 x 6144 at 80 rows 13.3 / 14.2, 4096 x
 // 8192 at 80 19.1 / 16.7, 896 x 5632 at 96 12.1 / 13.4, 6144 x 4096 at 64 15.5 / 11.6 (tables 24.6 / 19.4), 6144 x 4480 (no K groups
 // for the tiles) 15.0 / 17.0, 896 x 4864 at 112 13.2 / 15.4, 6144 x 4864 at 64 with tables 25.2 / 32.8.
-static bool few_rows(const scmx_format* fmt, int M, int N, int K, TileChoice tile) {
-    if (M < 1 || M > SKINNY_MAX_ROWS || N < 1 || K < 1 || long(M + 15) / 16 * 16 * N > 480000) return false;   // (beyond: not measured)
-    const float t = skinny_time(M, N, K, tile.cus);
-    const float more = tile.index != 6 ? 1.0f : long(M + 63) / 64 * ((N + 31) / 32) * 2 <= tile.cus ? 1.35f : 1.27f;
-    if (t < more * tile.us) return true;
+// *tile: that tile's choice, filled in where the answer is no.  No tile's table gives less than `least`, so the smallest calls,
+// which the host bounds, look no further: 0.05 us a call for 0.09.
+static bool few_rows(const scmx_format* fmt, int M, int N, int K, TileChoice* tile) {
+    const int cus = device_cus();
+    const bool candidate = M <= SKINNY_MAX_ROWS && long(M + 15) / 16 * 16 * N <= 480000;   // (beyond: not measured)
+    const float t = candidate ? skinny_time(M, N, K, cus) : 0.0f, least = 0.95f * fmaxf(1.9f, 1.26f + 0.14f / 128.0f * float(K));
+    if (candidate && t < least) return true;
+    *tile = dense_choice(M, N, K, false, cus);
+    if (!candidate) return false;
+    const float more = tile->index != 6 ? 1.0f : long(M + 63) / 64 * ((N + 31) / 32) * 2 <= cus ? 1.35f : 1.27f;
+    if (t < more * tile->us) return true;
     DevFormat f;
-    return fmt && t < 1.5f * more * tile.us && make_dev_format(fmt, &f) == SCMX_OK && packed_mode(f) == B_PACKED_GENERIC;
+    return fmt && t < 1.5f * more * tile->us && make_dev_format(fmt, &f) == SCMX_OK && packed_mode(f) == B_PACKED_GENERIC;
 }
 
 static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
     if (a.blocked == FEW_ROWS) return launch_skinny(a, bmode, s);
-    const int best = dense_choice(a.M, a.N, a.K, a.blocked != 0).index;
+    const int best = dense_choice(a.M, a.N, a.K, a.blocked != 0, device_cus()).index;
     if (a.blocked) {
         switch (best) {
             case 0: return launch_tile<256, 256, 64, 4, 2, 1, 2, false, false, 1, true>(a, bmode, (a.M + 255) / 256, s);
@@ -1070,14 +1074,15 @@ int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* 
         set_error("mm_w4a8_blocked: the activations' whole 32-row blocks lie beyond the 32-bit offsets of the kernel (M=%d K=%d)", M, K);
         return SCMX_ERR_ARG;
     }
-    const bool few = M > 0 && N > 0 && K > 0 && few_rows(fmt, M, N, K, dense_choice(M, N, K, false));
+    TileChoice tile;
+    const bool few = M > 0 && N > 0 && K > 0 && few_rows(fmt, M, N, K, &tile);
     return mm_w4a8(fmt, xq, xscale, codes, bcodes, wscale, res, out, epi, M, N, K, few ? FEW_ROWS : 1, stream);
 }
 
 int scmx_mm_w4a8_prefers_blocked(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    const TileChoice tile = dense_choice(M, N, K, false);
-    return tile.index <= 2 || few_rows(nullptr, M, N, K, tile);
+    TileChoice tile;
+    return few_rows(nullptr, M, N, K, &tile) || tile.index <= 2;
 }
 
 // The fused layer quantizes into whichever layout suits the shape: blocked where the row-layout model would run one of its
@@ -1088,8 +1093,8 @@ static int quantize_and_multiply(const scmx_format* fmt, const uint16_t* x, int8
     const long long Mp = (static_cast<long long>(M) + 31) & ~31LL;
     int blocked = 0;
     if (room_for_blocks && M > 0 && N > 0 && K > 0 && K % 128 == 0 && uint64_t(Mp) * uint64_t(K) <= 0xFFFFFFFFull) {
-        const TileChoice tile = dense_choice(M, N, K, false);
-        blocked = few_rows(fmt, M, N, K, tile) ? FEW_ROWS : tile.index <= 2;
+        TileChoice tile;
+        blocked = few_rows(fmt, M, N, K, &tile) ? FEW_ROWS : tile.index <= 2;
     }
     if (blocked) {
         if (int rc = scmx_act_quant_blocked(x, xq, xs, M, int(Mp), K, stream)) return rc;
