@@ -4,7 +4,7 @@
 // workgroup stages BM x BK activation bytes and BN x BK weight bytes in LDS; the weight bytes are produced in
 // registers from the packed 4-bit codes (16 bytes of codes = one run of 32 weights per thread) right before they
 // are written to LDS, so the INT8 form of the weights exists only there.  Waves then read 16-byte operand
-// fragments and issue v_mfma_i32_32x32x32_i8 with the weights as the row operand: each lane ends up with groups
+// fragments and issue v_mfma_i32_16x16x64_i8 with the weights as the row operand: each lane ends up with groups
 // of 4 consecutive output columns n of one token row m, which is the unit every epilogue works on.
 // LDS holds three stages of the K loop; global loads run four steps ahead in two register sets, and the decode and
 // LDS writes of step i+2 are issued between the MFMAs of step i, with one barrier per step.
@@ -15,27 +15,34 @@
 
 namespace scmx {
 
-// FD = number of fragment register buffers: fragments are fetched FD - 1 k slices ahead of their MFMAs.
-// SKIP (grouped launches): a row tile that ends inside its expert's segment multiplies only the 32-row blocks that hold
+// The 16x16x64 form of the instruction and not 32x32x32: the chip runs these kernels at its power limit (all-zero operands
+// run a third faster), and at that limit, on INT8 operands as they occur, a loop of MFMAs alone reaches 4420 TOP/s with
+// 16x16x64 and 3740 with 32x32x32 (half the accumulator traffic per multiply-add).  gate|up of 12288 x 2048 at 8192 rows, same
+// tile: 208 -> 199 us; the four layers of a 2048-wide model at 2048 rows 118 -> 108 with the tiles chosen below.
+//
+// FD = number of register buffers of the split operand's fragments: fetched FD - 1 phases (half k slices) ahead of their MFMAs.
+// SKIP (grouped launches): a row tile that ends inside its expert's segment multiplies only the 16-row blocks that hold
 // valid rows.  The two waves that share a SIMD then own the same columns and different row halves of the tile, so that
 // a half-empty tile halves the MFMA work of every SIMD instead of idling two of the four.
-// PK (B_PACKED_DEFAULT / B_PACKED_B16, K steps of 128): the weights stay packed in LDS -- 64 bytes of codes per row and
+// PK (the FP4-conversion formats, K steps of 128): the weights stay packed in LDS -- 64 bytes of codes per row and
 // K step plus the step's block-code bytes -- and every wave decodes its own fragments after reading them.  Half the
 // weight bytes through LDS in both directions, paid with one decode per wave row that shares the fragment.
 // KG > 1 (small problems: fewer tiles than CUs): KG groups of WGM x WGN waves share the tile, each multiplies its own
 // K / KG of the reduction out of LDS stages of its own, and the INT32 partial sums meet in LDS before the epilogue (exact:
 // integer addition is associative).  A CU then runs KG times the waves on the same tile count.
-// AD (dense, activations in the blocked layout): the activation tile does not pass through LDS; every wave loads the
-// fragments of its own rows from memory, one coalesced 1 KB load per 32-row x 32-k block, two K steps ahead.  Waves must
-// then not share rows (WGN = 1, or few column groups), and only the weight rows of a stage exist in LDS.
+// AD (ADM 1, dense: activations in the blocked layout; ADM 2, grouped: rows, gathered): the activation tile does not pass
+// through LDS; every wave loads the fragments of its own rows from memory, two K steps ahead: four runs of 256 bytes from
+// the blocked layout, sixteen of 64 from rows.  Waves must then not share rows (WGN = 1, or few column groups), and only the
+// weight rows of a stage exist in LDS.
 template <int BM, int BN, int BK, int WGM, int WGN, int BMODE, int OCC = 1, int FD = 2, bool SKIP = false, bool PK = false,
-          int KG = 1, bool AD = false>
+          int KG = 1, int ADM = 0>
 __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const GemmArgs a) {
+    constexpr bool AD = ADM != 0, ADR = ADM == 2;   // activation fragments straight from memory; from the row layout
     constexpr int NSTAGE = 3;   // LDS stages: one being read, one ready, one being written
     constexpr int NT = WGM * WGN * 64;   // threads of one K group
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
-    constexpr int MI = WTM / 32, NI = WTN / 32;
-    static_assert(WTM % 32 == 0 && WTN % 32 == 0 && (BK == 64 || BK == 128), "tile must be whole 32x32x32 MFMAs");
+    constexpr int MI = WTM / 16, NI = WTN / 16;   // 16-row / 16-column blocks of a wave's tile
+    static_assert(WTM % 32 == 0 && WTN % 32 == 0 && (BK == 64 || BK == 128), "tile must be whole pairs of 16x16x64 MFMAs");
     constexpr int CPR = BK / 16;             // 16-byte chunks per LDS row
     constexpr int RPB = 256 / BK;            // rows per 256 bytes, i.e. per sweep of the 64 LDS banks
     constexpr int A_CHUNKS = AD ? 0 : BM * CPR;   // 16-byte pieces of the activation tile
@@ -46,8 +53,10 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     constexpr int WPC = BN * BK / 32 >= NT ? 4 : 2;
     constexpr int B_CHUNKS = BMODE == B_INT8 ? BN * CPR : BN * BK / (8 * WPC);
     constexpr int B_PER = (B_CHUNKS + NT - 1) / NT;
-    constexpr int BCB = BMODE == B_PACKED_B16 ? 2 : 1;   // PK: block-code bytes per weight row and K step
-    static_assert(!PK || (BK == 128 && WPC == 4 && (BMODE == B_PACKED_DEFAULT || BMODE == B_PACKED_B16)),
+    // PK: block-code bytes per weight row and K step
+    constexpr int BCB = BMODE == B_PACKED_B16M || BMODE == B_PACKED_E8M0 ? 4 : BMODE == B_PACKED_B16 ? 2 : 1;
+    constexpr int BCR = BCB == 4 ? 2 : 1;   // registers for those of two steps
+    static_assert(!PK || (BK == 128 && WPC == 4 && BMODE != B_INT8 && BMODE != B_PACKED_GENERIC),
                   "packed weights in LDS: K steps of 128, 16-byte runs, FP4-conversion formats");
     // bytes per stage: BM activation rows, then BN weight rows (PK: 64 code bytes each)
     constexpr int STAGE = A_BYTES + (PK ? BN * (BK / 2) : BN * BK);
@@ -59,10 +68,10 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // need more than the stages and still fit the CU, the buffer is sized for them.
     constexpr int EPI_BYTES = WGM * WGN * WTM * (WTN * 2 + 16);
     static_assert(KG == 1 || (!PK && !SKIP), "K groups: staged dense tiles");
-    static_assert(!AD || (!PK && !SKIP && KG == 1), "activation fragments from memory: staged dense tiles");
+    static_assert(!AD || (!PK && KG == 1), "activation fragments from memory: staged tiles");
     constexpr int GROUP_BYTES = NSTAGE * STAGE;
     // after the K loop: group 0's output tiles (the widest epilogue's) from 0, then the other groups' partial sums
-    constexpr int PART_BYTES = NT * MI * NI * 64;
+    constexpr int PART_BYTES = NT * MI * NI * 16;
     constexpr int PART_BASE = WGM * WGN * WTM * (WTN * 4 + 16);
     constexpr int KG_BYTES = PART_BASE + (KG - 1) * PART_BYTES > KG * GROUP_BYTES ? PART_BASE + (KG - 1) * PART_BYTES : KG * GROUP_BYTES;
     static_assert(KG == 1 || KG_BYTES <= 160 * 1024, "stages and partial sums fit the CU's LDS");
@@ -86,20 +95,26 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     int m0, n0, row_end, expert = 0;
     if (a.tstart) {   // grouped: row tiles of BM inside expert segments
         // Workgroup b runs on XCD b % 8: inside every chunk of 8 row tiles each XCD takes one row tile with all of
-        // its column tiles, so an activation panel is fetched into one L2 only.
+        // its column tiles, so an activation panel is fetched into one L2 only.  The segments' row tiles (slots) may be
+        // taller than this kernel's: then a slot is 1 << sub_log2 of them.
         const int j = blockIdx.x % (8 * num_n);
-        const int slot = blockIdx.x / (8 * num_n) * 8 + (j & 7);
+        const int tile = blockIdx.x / (8 * num_n) * 8 + (j & 7), slot = tile >> a.sub_log2;
         n0 = (j >> 3) * BN;
         const int E = a.n_experts;
         if (slot >= a.tstart[E]) return;
-        int lo = 0, hi = E;   // largest e with tstart[e] <= slot
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (a.tstart[mid] <= slot) lo = mid; else hi = mid;
+        // largest e with tstart[e] <= slot: every lane probes one of up to 64 evenly spaced entries of the range, so 64 experts
+        // take one trip to memory and 4096 two (a binary search: six and twelve, in front of the first operand load)
+        int lo = 0, n = E;
+        while (n > 1) {
+            const int step = (n + 63) >> 6, at = int(threadIdx.x & 63) * step;
+            const int last = __popcll(__ballot(at < n && a.tstart[lo + min(at, n - 1)] <= slot)) - 1;   // entry 0 always is
+            lo += last * step;
+            n = min(step, n - last * step);
         }
-        expert = lo;
-        m0 = a.off[expert] + (slot - a.tstart[expert]) * BM;
+        expert = __builtin_amdgcn_readfirstlane(lo);
+        m0 = a.off[expert] + (((slot - a.tstart[expert]) << a.sub_log2) + (tile & ((1 << a.sub_log2) - 1))) * BM;
         row_end = a.off[expert + 1];
+        if (m0 >= row_end) return;   // the last slot's spare tiles
     } else {
         const int num_m = (a.M + BM - 1) / BM;
         int pid = blockIdx.x;
@@ -117,9 +132,9 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     const int K = a.K;
     const int KL = K / KG;         // length of this group's part of the reduction
     const int kbase = kg * KL;     // and its first k (a multiple of 128)
-    // 32-row blocks of this wave's tile that hold rows of the segment (wave-uniform)
+    // 16-row blocks of this wave's tile that hold rows of the segment (wave-uniform)
     const int mi_active =
-        SKIP ? __builtin_amdgcn_readfirstlane(min(MI, max(0, (row_end - (m0 + wm * WTM) + 31) / 32))) : MI;
+        SKIP ? __builtin_amdgcn_readfirstlane(min(MI, max(0, (row_end - (m0 + wm * WTM) + 15) / 16))) : MI;
     // The tile's scales are REQUESTED here, before the first operand loads, and stored to LDS after those have been
     // issued: memory returns a wave's loads in order, so scales requested first arrive first and their wait does not
     // cover the operand loads (fetched and stored up front they cost every tile two serial round trips to memory).
@@ -306,21 +321,20 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int q = 0; q < NKK; ++q) stage_slice(r, sm + stage * STAGE, k0, q, o);
     };
 
-    v16i acc[MI][NI];
+    v4i acc[MI][NI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+        for (int j = 0; j < NI; ++j) acc[i][j] = v4i{0, 0, 0, 0};
 
-    // fragment addresses: lane l supplies row l % 32 and the 16 k-bytes of half l / 32 of a 32-wide k slice; tile
-    // origins are multiples of 32 rows, so the swizzle term depends on the lane only
-    const int lr = lane & 31, half = lane >> 5;
+    // fragment addresses: lane l supplies row l % 16 and the 16 k-bytes of quarter l / 16 of a 64-wide k slice; block
+    // origins are multiples of 16 rows, so the swizzle term depends on the lane only
+    constexpr int KS = BK / 64;   // k slices of a step
+    const int lr = lane & 15, quad = lane >> 4;
     const int sw = (lr / RPB) & (CPR - 1);
-    int koff[NKK];
+    int koff[KS];
 #pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) koff[kk] = ((2 * kk + half) ^ sw) << 4;
+    for (int s = 0; s < KS; ++s) koff[s] = ((4 * s + quad) ^ sw) << 4;
     const int a_frag = (wm * WTM + lr) * BK;
     const int b_frag = A_BYTES + (wn * WTN + lr) * BK;
 
@@ -331,17 +345,63 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // after it was written, so the first fragments of step kt+1 are fetched at the end of iteration kt, ahead of the
     // barrier that opens kt+1.  The stage indices are compile-time constants (the loop is unrolled over the
     // 3 stages x 2 register sets), which keeps every LDS address an immediate offset from a fixed register.
-    [[maybe_unused]] uint32_t bcc[NI], bcn[NI];   // PK: block codes of the current / the next two K steps
+    // PK: block codes of the current / the next two K steps, one register per weight row (two in the formats with a byte
+    // or a 4-bit code per block: a register per step)
+    [[maybe_unused]] uint32_t bcc[NI][BCR], bcn[NI][BCR];
     [[maybe_unused]] int bc_src[NI];
 #pragma unroll
-    for (int j = 0; j < NI; ++j) bc_src[j] = min(n0 + wn * WTN + j * 32 + lr, a.N - 1) * a.bc_row_bytes;
+    for (int j = 0; j < NI; ++j) bc_src[j] = min(n0 + wn * WTN + j * 16 + lr, a.N - 1) * a.bc_row_bytes;
     // block codes of K steps s and s + 1 (s even); past the end the last pair of steps again (never consumed)
-    auto load_bc = [&](int s, uint32_t (&f)[NI]) {
+    auto load_bc = [&](int s, uint32_t (&f)[NI][BCR]) {
         const int so = min(s, (K / BK - 1) & ~1) * BCB;
 #pragma unroll
         for (int j = 0; j < NI; ++j)
-            f[j] = BCB == 2 ? uint32_t(__builtin_amdgcn_raw_buffer_load_b32(rbc, bc_src[j], so, 0))
-                            : uint32_t(__builtin_amdgcn_raw_buffer_load_b16(rbc, bc_src[j], so, 0));
+            if constexpr (BCR == 2) {
+                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rbc, bc_src[j], so, 0);
+                f[j][0] = v[0];
+                f[j][1] = v[1];
+            } else {
+                f[j][0] = BCB == 2 ? uint32_t(__builtin_amdgcn_raw_buffer_load_b32(rbc, bc_src[j], so, 0))
+                                   : uint32_t(__builtin_amdgcn_raw_buffer_load_b16(rbc, bc_src[j], so, 0));
+            }
+    };
+    // PK, E8M0: lowest exponent byte of the lane's weight rows
+    [[maybe_unused]] uint32_t w_rmin[NI];
+    if constexpr (PK && BMODE == B_PACKED_E8M0) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) w_rmin[j] = e8m0_row_min(a.wscale[erow + min(n0 + wn * WTN + j * 16 + lr, a.N - 1)]);
+    }
+    // AD: the activations come in 32-row x 32-k blocks of 1 KB, 16 bytes of a row per piece, piece (row % 32, k / 16 % 2) at
+    // (k / 16 % 2) * 512 + (row % 32) * 16, block (m / 32, k / 32) at ((m / 32) * (K / 32) + k / 32) KB.  A fragment (16
+    // rows x 64 k) is then four runs of 256 bytes.  Every wave loads the fragments of its own rows straight into registers,
+    // two K steps ahead, in three buffers that rotate with the LDS stages: the activation tile never passes through LDS.
+    constexpr int NAB = MI * NI > 16 ? 2 : NSTAGE;   // the largest wave tiles have registers for two buffers only (below)
+    [[maybe_unused]] v4i fad[NAB][KS][MI];
+    [[maybe_unused]] int ad_src[ADR ? MI : MI / 2];
+    if constexpr (ADR) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            int gr = min(m0 + wm * WTM + i * 16 + lr, row_end - 1);
+            if (a.gather) gr = a.gather[gr];
+            ad_src[i] = int(uint32_t(gr) * uint32_t(K) + uint32_t(quad) * 16u);
+        }
+    } else if constexpr (AD) {
+        const int last_block = (a.M + 31) / 32 - 1;
+#pragma unroll
+        for (int i = 0; i < MI / 2; ++i)
+            ad_src[i] = int(uint32_t(min((m0 + wm * WTM) / 32 + i, last_block)) * uint32_t(K >> 5) * 1024u +
+                            uint32_t(quad) * 512u + uint32_t(lr) * 16u + uint32_t(kbase) * 32u);
+    }
+    auto load_ad = [&](int buf, int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                if (SKIP && i >= mi_active) continue;
+                const u32x4 v = ADR ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR ? i : 0] + s * 64, k0, 0)
+                                    : __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR ? 0 : i / 2] + s * 2048 + (i & 1) * 256, k0 * 32, 0);
+                fad[buf][s][i] = v4i{int(v[0]), int(v[1]), int(v[2]), int(v[3])};
+            }
     };
     if constexpr (PK) load_bc(0, bcc);   // ahead of the operand loads, like the scales
     load_global(r0, 0);
@@ -354,70 +414,66 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int j = 0; j < WS_PER; ++j)
             if (tid + j * NT < BN) s_ws[tid + j * NT] = ws_reg[j];
     }
+    if constexpr (AD) load_ad(0, 0);
     store_lds(r0, 0, 0);
     store_lds(r1, 1, BK);
     load_global(r0, 2 * BK);
-    // the two sets' loads stay apart, in the order the K loop issues them: its first copy has two predecessors (this code
-    // and the loop's end) and waits for the fewer outstanding loads of the two -- interleaved here, that wait covered
-    // the younger set as well, in every trip
+    // The loads stay apart, in the order the K loop issues them (activations of a step, then the weights two steps ahead of
+    // them): the loop's first copy has two predecessors (this code and the loop's end) and waits for the fewer outstanding
+    // loads of the two -- interleaved here, that wait covered the younger set as well, in every trip
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (AD) {
+        load_ad(1, min(BK, KL - BK));
+        __builtin_amdgcn_sched_barrier(0);
+    }
     load_global(r1, 3 * BK);
     // ---- PK: fragments of packed weights ------------------------------------------------------------------------
-    // The k positions of a 64-wide pair of MFMA slices are dealt so that a lane's packed codes are one 16-byte read:
-    // lane half h supplies k = 64 kp + 32 h + 16 s + (0..15) to slice s of pair kp, i.e. 32 consecutive activation
-    // bytes (two 16-byte reads) and 32 consecutive codes (one), the latter one 32-block or two 16-blocks.
-    constexpr int NKP = NKK / 2;
-    // Three things are in flight per wave: the MFMAs of pair p, the decode of pair p + 1 (its codes were read during
-    // pair p - 1) and the LDS reads of pair p + 1's activations and pair p + 2's codes.
+    // A unit is one 64-wide k slice of one 16-column block: lane quarter q supplies k = 64 s + 16 q + (0..15) of a row, 8
+    // code bytes, which lie inside one block of 16 or 32 weights.  Three things are in flight per wave: the MFMAs of unit
+    // u, the decode of unit u + 1 (its codes were read during unit u - 1) and the LDS reads of the codes of unit u + 2 and
+    // of the next slice's activations.
     // The block codes do not pass through LDS: the lane that decodes row n reads the codes of two K steps of that row
     // (2 * BCB bytes) from memory every second step, two steps ahead.
-    [[maybe_unused]] v4i pa[2][2][MI];   // activation fragments [pair parity][slice][32-row block]
-    [[maybe_unused]] v4i pw[2][NI];      // 32 codes per weight row as read from LDS [pair parity]
-    [[maybe_unused]] v4i px[2][2][NI];   // decoded INT8 operands [pair parity][slice][32-column block]
-    [[maybe_unused]] int koff_pa[NKP][2], koff_pw[NKP];
+    constexpr int NU = KS * NI;          // units of a step
+    [[maybe_unused]] v4i pa[2][MI];      // activation fragments [slice parity][16-row block]
+    [[maybe_unused]] u32x2 pw[2];        // 16 codes of a weight row as read from LDS [unit parity]
+    [[maybe_unused]] v4i px[2];          // decoded INT8 operands [unit parity]
+    [[maybe_unused]] int koff_pw[KS];
 #pragma unroll
-    for (int kp = 0; kp < NKP; ++kp) {
-        koff_pa[kp][0] = ((4 * kp + 2 * half) ^ sw) << 4;
-        koff_pa[kp][1] = ((4 * kp + 2 * half + 1) ^ sw) << 4;
-        koff_pw[kp] = ((2 * kp + half) ^ ((lr >> 2) & 3)) << 4;
-    }
+    for (int s = 0; s < KS; ++s) koff_pw[s] = (((2 * s + (quad >> 1)) ^ ((lr >> 2) & 3)) << 4) + (quad & 1) * 8;
     [[maybe_unused]] const int w_frag = A_BYTES + (wn * WTN + lr) * (BK / 2);
-    auto load_pa = [&](const int8_t* src, int kp, v4i (&f)[2][MI]) {
+    auto load_pa = [&](const int8_t* src, int s, v4i (&f)[MI]) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
-            if (!SKIP || i < mi_active) {
-                f[0][i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + koff_pa[kp][0]);
-                f[1][i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + koff_pa[kp][1]);
-            }
+            if (!SKIP || (i & ~1) < mi_active) f[i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 16 * BK + koff[s]);
     };
-    auto load_pw = [&](const int8_t* src, int kp, v4i (&f)[NI]) {
-        if (SKIP && mi_active == 0) return;
-#pragma unroll
-        for (int j = 0; j < NI; ++j) f[j] = *reinterpret_cast<const v4i*>(src + w_frag + j * 32 * (BK / 2) + koff_pw[kp]);
+    auto load_pw = [&](const int8_t* src, int u, u32x2& f) {
+        f = *reinterpret_cast<const u32x2*>(src + w_frag + (u % NI) * 16 * (BK / 2) + koff_pw[u / NI]);
     };
-    // 32 codes -> the INT8 operands of the pair's two slices; `odd` = the K step's parity (which half of the block codes)
-    auto decode_pair = [&](const v4i (&f)[NI], const uint32_t (&bc)[NI], int odd, int kp, v4i (&x)[2][NI]) {
-        if (SKIP && mi_active == 0) return;
-#pragma unroll
-        for (int j = 0; j < NI; ++j) {
-            float s0, s1;
-            if (BMODE == B_PACKED_B16) {   // blocks 4 kp + 2 h and the next one of the step's 8
-                const uint32_t t = bc[j] >> (16 * odd + 8 * kp + 4 * half);
-                s0 = fp4_scale(t & 3u);
-                s1 = fp4_scale((t >> 2) & 3u);
-            } else {                       // block 2 kp + h of the step's 4
-                s0 = s1 = fp4_scale((bc[j] >> (8 * odd + 4 * kp + 2 * half)) & 3u);
-            }
-            uint32_t o[8];
-            decode_word_fp4(uint32_t(f[j][0]), s0, o[0], o[1]);
-            decode_word_fp4(uint32_t(f[j][1]), s0, o[2], o[3]);
-            decode_word_fp4(uint32_t(f[j][2]), s1, o[4], o[5]);
-            decode_word_fp4(uint32_t(f[j][3]), s1, o[6], o[7]);
-            x[0][j] = v4i{int(o[0]), int(o[1]), int(o[2]), int(o[3])};
-            x[1][j] = v4i{int(o[4]), int(o[5]), int(o[6]), int(o[7])};
+    // 16 codes -> the INT8 operand of unit u; `odd` = the K step's parity (which half of the block codes)
+    auto decode_unit = [&](const u32x2& f, const uint32_t (&bc)[NI][BCR], int odd, int u, v4i& x) {
+        const int s = u / NI, j = u % NI;
+        uint32_t o[4];
+        if constexpr (BMODE == B_PACKED_B16M) {   // block 4 s + q of the step's 8, 4 bits each
+            const uint32_t code = (bc[j][odd] >> (16 * s + 4 * quad)) & 15u;
+            const _Float16 m = _Float16(int(code + (a.fmt.mult[0] & 0xFFu)));
+            decode_word_fp4_mul(f[0], half2_t{m, m}, o[0], o[1]);
+            decode_word_fp4_mul(f[1], half2_t{m, m}, o[2], o[3]);
+        } else {
+            uint32_t shift;
+            if constexpr (BMODE == B_PACKED_B16)         // block 4 s + q of the step's 8
+                shift = (bc[j][0] >> (16 * odd + 8 * s + 2 * quad)) & 3u;
+            else if constexpr (BMODE == B_PACKED_E8M0)   // byte 2 s + q / 2 of the step's 4
+                shift = (((bc[j][odd] >> (16 * s + 8 * (quad >> 1))) & 0xFFu) - w_rmin[j]) & 0x7Fu;
+            else                                         // block 2 s + q / 2 of the step's 4
+                shift = (bc[j][0] >> (8 * odd + 4 * s + 2 * (quad >> 1))) & 3u;
+            const float sc = fp4_scale(shift);
+            decode_word_fp4(f[0], sc, o[0], o[1]);
+            decode_word_fp4(f[1], sc, o[2], o[3]);
         }
+        x = v4i{int(o[0]), int(o[1]), int(o[2]), int(o[3])};
     };
-    auto iteration_pk = [&](auto step_tag, auto parity_tag, Staged& r, int kt) {
+    auto iteration_pk = [&](auto step_tag, auto parity_tag, Staged& r, int kt) __attribute__((always_inline)) {
         constexpr int rd = decltype(step_tag)::value;
         constexpr int odd = decltype(parity_tag)::value;   // kt % 2
         constexpr int wr = (rd + 2) % NSTAGE;
@@ -431,94 +487,81 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         uint32_t o[B_PER][8];
         if (!odd) load_bc(kt + 2, bcn);
 #pragma unroll
-        for (int kp = 0; kp < NKP; ++kp) {
-            const int cur = kp % 2, oth = (kp + 1) % 2;   // NKP is even: pair 0 of every step has parity 0
-            if (kp + 1 < NKP) {
-                load_pa(src, kp + 1, pa[oth]);
-                decode_pair(pw[oth], bcc, odd, kp + 1, px[oth]);
-            } else {   // pair 0 of step kt + 1
-                load_pa(nxt, 0, pa[oth]);
+        for (int u = 0; u < NU; ++u) {
+            const int cur = u % 2, oth = (u + 1) % 2, s = u / NI;   // NU and KS are even: unit 0 of every step has parity 0
+            if (u % NI == 0) load_pa(s + 1 < KS ? src : nxt, (s + 1) % KS, pa[(s + 1) % 2]);
+            if (u + 1 < NU) {
+                decode_unit(pw[oth], bcc, odd, u + 1, px[oth]);
+            } else {   // unit 0 of step kt + 1
                 if (odd) {
 #pragma unroll
-                    for (int j = 0; j < NI; ++j) bcc[j] = bcn[j];
-                }
-                decode_pair(pw[oth], bcc, 1 - odd, 0, px[oth]);
-            }
-            load_pw(nxt, kp, pw[cur]);   // pair kp + 2 = pair kp of the next step; pw[cur] was decoded a pair ago
-#pragma unroll
-            for (int sl = 0; sl < 2; ++sl) {
-#pragma unroll
-                for (int i = 0; i < MI; ++i) {
-                    if (SKIP && i >= mi_active) continue;
-#pragma unroll
                     for (int j = 0; j < NI; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(px[cur][sl][j], pa[cur][sl][i], acc[i][j], 0, 0, 0);
+#pragma unroll
+                        for (int q = 0; q < BCR; ++q) bcc[j][q] = bcn[j][q];
                 }
-                stage_slice(r, dst, k2, 2 * kp + sl, o);
+                decode_unit(pw[oth], bcc, 1 - odd, 0, px[oth]);
             }
+            load_pw(u + 2 < NU ? src : nxt, (u + 2) % NU, pw[cur]);   // pw[cur] was decoded a unit ago
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                if (SKIP && (i & ~1) >= mi_active) continue;   // pairs of row blocks
+                acc[i][u % NI] = __builtin_amdgcn_mfma_i32_16x16x64_i8(px[cur], pa[s % 2][i], acc[i][u % NI], 0, 0, 0);
+            }
+            if (u < NKK) stage_slice(r, dst, k2, u, o);
         }
         load_global(r, k4);
     };
-    static_assert(!PK || NKP % 2 == 0, "the pair buffers return to phase 0 every K step");
+    static_assert(!PK || (KS == 2 && NU % 2 == 0 && NU >= NKK), "the buffers return to phase 0 every K step");
 
-    // Fragments are fetched FD - 1 k slices ahead of the MFMAs that use them, into FD rotating register buffers; the
-    // slices fetched at the end of an iteration belong to the next step's stage.
+    // A step runs in phases, two per 64-wide k slice: the operand with more 16-row blocks in the wave's tile is split, one
+    // half of its fragments per phase, and fetched FD - 1 phases ahead into FD rotating register buffers; the other
+    // operand's fragments are held for the slice and fetched one slice ahead, half of them in each phase.  The fragments
+    // fetched at the end of an iteration belong to the next step's stage.
+    constexpr bool SPLITN = AD || NI >= MI;                 // the split operand: weights (columns) or activations (rows)
+    constexpr int SF = (SPLITN ? NI : MI) / 2, HF = SPLITN ? MI : NI;
     constexpr int AHEAD = FD - 1;
     static_assert(AHEAD >= 1 && AHEAD <= NKK, "fragment prefetch distance");
-    [[maybe_unused]] v4i fa[FD][MI], fb[FD][NI];
-    auto load_frags = [&](const int8_t* src, int kk, v4i (&xa)[MI], v4i (&xb)[NI]) {
+    [[maybe_unused]] v4i fs[FD][SF], fh[2][HF];
+    auto load_split = [&](const int8_t* src, int phase, v4i (&x)[SF]) __attribute__((always_inline)) {
         if (SKIP && mi_active == 0) return;
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-            if (!AD && (!SKIP || i < mi_active)) xa[i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + koff[kk]);
-#pragma unroll
-        for (int j = 0; j < NI; ++j) xb[j] = *reinterpret_cast<const v4i*>(src + b_frag + j * 32 * BK + koff[kk]);
+        for (int f = 0; f < SF; ++f) {
+            const int blk = (phase & 1) * SF + f;
+            if (!SPLITN && SKIP && blk >= mi_active) continue;
+            x[f] = *reinterpret_cast<const v4i*>(src + (SPLITN ? b_frag : a_frag) + blk * 16 * BK + koff[phase >> 1]);
+        }
     };
-    // AD: the activations come in 32-row x 32-k blocks of 1 KB laid out as the MFMA takes them (lane l = row l % 32,
-    // k half l / 32, 16 bytes each), block (m / 32, k / 32) at ((m / 32) * (K / 32) + k / 32) KB.  Every wave loads the
-    // fragments of its own rows straight into registers, two K steps ahead, in three buffers that rotate with the LDS
-    // stages: the activation tile never passes through LDS.
-    [[maybe_unused]] v4i fad[NSTAGE][NKK][MI];
-    [[maybe_unused]] int ad_src[MI];
-    if constexpr (AD) {
-        const int last_block = (a.M + 31) / 32 - 1;
+    auto load_held = [&](const int8_t* src, int s, int part, v4i (&x)[HF]) __attribute__((always_inline)) {
+        if (AD || (SKIP && mi_active == 0)) return;
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-            ad_src[i] = int(uint32_t(min((m0 + wm * WTM) / 32 + i, last_block)) * uint32_t(K >> 5) * 1024u + uint32_t(lane) * 16u +
-                            uint32_t(kbase) * 32u);
-    }
-    auto load_ad = [&](int buf, int k0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int kk = 0; kk < NKK; ++kk)
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[i] + kk * 1024, k0 * 32, 0);
-                fad[buf][kk][i] = v4i{int(v[0]), int(v[1]), int(v[2]), int(v[3])};
-            }
+        for (int f = 0; f < HF; ++f) {
+            if (f / ((HF + 1) / 2) != part) continue;
+            if (SPLITN && SKIP && f >= mi_active) continue;
+            x[f] = *reinterpret_cast<const v4i*>(src + (SPLITN ? a_frag : b_frag) + f * 16 * BK + koff[s]);
+        }
     };
-    if constexpr (AD) {
-        load_ad(0, 0);
-        load_ad(1, min(BK, KL - BK));
-    }
     __syncthreads();
     if constexpr (PK) {
         load_pa(smem, 0, pa[0]);
         load_pw(smem, 0, pw[0]);
         load_pw(smem, 1, pw[1]);
-        decode_pair(pw[0], bcc, 0, 0, px[0]);
+        decode_unit(pw[0], bcc, 0, 0, px[0]);
     } else {
+        load_held(sm, 0, 0, fh[0]);
+        load_held(sm, 0, 1, fh[0]);
 #pragma unroll
-        for (int q = 0; q < AHEAD; ++q) load_frags(sm, q, fa[q], fb[q]);
+        for (int q = 0; q < AHEAD; ++q) load_split(sm, q, fs[q]);
     }
     // The k slices of an iteration are fenced against each other for the scheduler: left alone, the compiler sinks every
     // LDS write of the step to its end, in front of the barrier (M = 8192: 442 -> 429 us over the four layers with the
     // fences on the 256x256 tile; M = 128 ... 1024 on the small tiles: 2-3 %).
-    auto iteration_staged = [&](auto step_tag, auto stage_tag, Staged& r, int kt) __attribute__((always_inline)) {
+    auto iteration_staged = [&](auto step_tag, auto parity_tag, auto stage_tag, Staged& r, int kt) __attribute__((always_inline)) {
         constexpr int rd = decltype(step_tag)::value;        // kt % 3: stage of step kt
         constexpr bool ST = decltype(stage_tag)::value;      // false in the last two steps: nothing left to stage
         constexpr int wr = (rd + 2) % NSTAGE;                // stage of step kt + 2
         constexpr int nx = (rd + 1) % NSTAGE;                // stage of step kt + 1
-        constexpr int ph = (NKK * rd) % FD;                  // fragment buffer of slice 0 of this step (FD divides 6 * NKK)
+        constexpr int ph = (NKK * rd) % FD;                  // buffer of phase 0 of this step (FD divides 6 * NKK)
+        constexpr int hp = KS == 1 ? int(decltype(parity_tag)::value) : 0;   // held buffer of slice 0 (kt % 2 if odd counts)
         __syncthreads();
         const int8_t* src = sm + rd * STAGE;
         const int8_t* nxt = sm + nx * STAGE;
@@ -526,29 +569,34 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         const int k2 = min((kt + 2) * BK, KL - BK);      // past the end: rewrites a stage nobody reads again
         const int k4 = min((kt + 4) * BK, KL - BK);
         uint32_t o[B_PER][8];
-        if constexpr (AD && ST) load_ad(wr, k2);
+        constexpr int ab = NAB == 2 ? int(decltype(parity_tag)::value) : rd;   // activation buffer of this step
+        if constexpr (AD && ST && NAB == 3) load_ad(wr, k2);
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
-            if (kk + AHEAD < NKK)
-                load_frags(src, kk + AHEAD, fa[(ph + kk + AHEAD) % FD], fb[(ph + kk + AHEAD) % FD]);
-            else
-                load_frags(nxt, kk + AHEAD - NKK, fa[(ph + kk + AHEAD) % FD], fb[(ph + kk + AHEAD) % FD]);
+            const int s = kk >> 1, h = kk & 1;
+            load_split(kk + AHEAD < NKK ? src : nxt, (kk + AHEAD) % NKK, fs[(ph + kk + AHEAD) % FD]);
+            load_held(s + 1 < KS ? src : nxt, (s + 1) % KS, h, fh[(hp + s + 1) % 2]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
+            for (int x = 0; x < (SPLITN ? MI : SF); ++x) {
+                const int i = SPLITN ? x : h * SF + x;
                 if (SKIP && i >= mi_active) continue;
 #pragma unroll
-                for (int j = 0; j < NI; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[(ph + kk) % FD][j], AD ? fad[rd][kk][i] : fa[(ph + kk) % FD][i],
-                                                                      acc[i][j], 0, 0, 0);
+                for (int y = 0; y < (SPLITN ? SF : NI); ++y) {
+                    const int j = SPLITN ? h * SF + y : y;
+                    const v4i act = AD ? fad[ab][s][i] : SPLITN ? fh[(hp + s) % 2][i] : fs[(ph + kk) % FD][x];
+                    const v4i wgt = SPLITN ? fs[(ph + kk) % FD][y] : fh[(hp + s) % 2][j];
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wgt, act, acc[i][j], 0, 0, 0);
+                }
             }
             if constexpr (ST) stage_slice(r, dst, k2, kk, o);
             __builtin_amdgcn_sched_barrier(0);
         }
+        if constexpr (AD && ST && NAB == 2) load_ad(ab, k2);   // into the buffer just multiplied
         if constexpr (ST) load_global(r, k4);
     };
     auto iteration = [&](auto step_tag, auto parity_tag, Staged& r, int kt) __attribute__((always_inline)) {
-        if constexpr (PK) iteration_pk(step_tag, parity_tag, r, kt); else iteration_staged(step_tag, std::true_type{}, r, kt);
+        if constexpr (PK) iteration_pk(step_tag, parity_tag, r, kt); else iteration_staged(step_tag, parity_tag, std::true_type{}, r, kt);
     };
     using S0 = std::integral_constant<int, 0>;
     using S1 = std::integral_constant<int, 1>;
@@ -586,11 +634,12 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         // that work.  Small wave tiles append them at each exit of the staged steps (one predecessor each); larger
         // ones, with few registers to spare for the copies that so many joins cost, select them by the stage reached;
         // the largest (128 accumulators, 256x256) keeps every step alike and stages past the end.
-        constexpr bool INLINE_TAIL = MI * NI <= 2, NO_TAIL = MI * NI > 4;
+        constexpr bool INLINE_TAIL = MI * NI <= 8, NO_TAIL = MI * NI > 16;
+        static_assert(AD ? NAB == 3 || NO_TAIL : KS == 2 || NO_TAIL, "the copies without staging do not know their step's parity");
         const int KM = NO_TAIL ? KT : max(KT - 2, 0);   // steps that stage step kt + 2
         auto last_two = [&](auto s_first, auto s_second) __attribute__((always_inline)) {
-            iteration_staged(s_first, std::false_type{}, r0, 0);
-            if (KT >= 2) iteration_staged(s_second, std::false_type{}, r0, 0);
+            iteration_staged(s_first, Even{}, std::false_type{}, r0, 0);
+            if (KT >= 2) iteration_staged(s_second, Even{}, std::false_type{}, r0, 0);
         };
         auto tail = [&](auto s_first, auto s_second) __attribute__((always_inline)) {
             if constexpr (INLINE_TAIL) last_two(s_first, s_second);
@@ -639,7 +688,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     }
 
     // ---- epilogue ---------------------------------------------------------------------------------------------
-    // Lane holds acc[i][j][4g + r] = (m = i*32 + lane%32, n = j*32 + 8g + 4(lane/32) + r) of its wave tile: 4 consecutive
+    // Lane holds acc[i][j][r] = (m = i*16 + lane%16, n = j*16 + 4(lane/16) + r) of its wave tile: 4 consecutive
     // columns of one row, the unit every epilogue works on.  Results go through a per-wave LDS tile so that global
     // stores are 16 bytes per lane over whole contiguous row segments.
     const int N = a.N;
@@ -652,7 +701,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
                 for (int j = 0; j < NI; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) part[((i * NI + j) * 16 + r) * NT + tid] = acc[i][j][r];
+                    for (int r = 0; r < 4; ++r) part[((i * NI + j) * 4 + r) * NT + tid] = acc[i][j][r];
         }
         __syncthreads();
         if (kg > 0) return;
@@ -664,7 +713,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
                 for (int j = 0; j < NI; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] += other[((i * NI + j) * 16 + r) * NT + tid];
+                    for (int r = 0; r < 4; ++r) acc[i][j][r] += other[((i * NI + j) * 4 + r) * NT + tid];
         }
     }
     auto epilogue = [&](auto epi_tag) {
@@ -681,70 +730,64 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                       (epi != SCMX_EPI_RES || reinterpret_cast<uintptr_t>(a.res) % 16 == 0);
 
     float xsv[MI];
-    f32x4 wsv[NI][4];
+    f32x4 wsv[NI];
     if (epi != SCMX_EPI_I32) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) xsv[i] = s_xs[wm * WTM + i * 32 + lr];
+        for (int i = 0; i < MI; ++i) xsv[i] = s_xs[wm * WTM + i * 16 + lr];
 #pragma unroll
-        for (int j = 0; j < NI; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                wsv[j][g] = *reinterpret_cast<const f32x4*>(&s_ws[wn * WTN + j * 32 + 8 * g + 4 * half]);
+        for (int j = 0; j < NI; ++j) wsv[j] = *reinterpret_cast<const f32x4*>(&s_ws[wn * WTN + j * 16 + 4 * quad]);
     }
     auto emit = [&](auto wide_tag) __attribute__((always_inline)) {
     constexpr bool W = decltype(wide_tag)::value;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-        const int row = i * 32 + lr;
+        const int row = i * 16 + lr;
         const int m = wm0 + row;
         const float xs = epi != SCMX_EPI_I32 ? xsv[i] : 0.0f;
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
+            const int col = j * 16 + 4 * quad;
+            const int n = wn0 + col;
+            if (epi == SCMX_EPI_I32) {
+                const v4i v = acc[i][j];
+                if (W)
+                    *reinterpret_cast<v4i*>(wtile + row * rsb + col * 4) = v;
+                else if (m < row_end && n < N)
+                    *reinterpret_cast<v4i*>(reinterpret_cast<int32_t*>(a.out) + size_t(m) * N + n) = v;
+                continue;
+            }
+            const f32x4 w4 = wsv[j];
+            float y[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int col = j * 32 + 8 * g + 4 * half;
-                const int n = wn0 + col;
-                if (epi == SCMX_EPI_I32) {
-                    const v4i v = v4i{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-                    if (W)
-                        *reinterpret_cast<v4i*>(wtile + row * rsb + col * 4) = v;
-                    else if (m < row_end && n < N)
-                        *reinterpret_cast<v4i*>(reinterpret_cast<int32_t*>(a.out) + size_t(m) * N + n) = v;
-                    continue;
-                }
-                const f32x4 w4 = wsv[j][g];
-                float y[4];
+            for (int r = 0; r < 4; ++r)
+                y[r] = __fmul_rn(__fmul_rn(float(acc[i][j][r]), xs), w4[r]);
+            uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
+            if (epi == SCMX_EPI_SWIGLU) {   // (g, g, u, u) -> two outputs
+                const uint16_t s0 = swiglu_lut(a.silu, y[0], round_bf16(y[2]));
+                const uint16_t s1 = swiglu_lut(a.silu, y[1], round_bf16(y[3]));
+                const uint32_t o = uint32_t(s0) | (uint32_t(s1) << 16);
+                if (W)
+                    *reinterpret_cast<uint32_t*>(wtile + row * rsb + col) = o;
+                else if (m < row_end && n < N)
+                    *reinterpret_cast<uint32_t*>(out + size_t(m) * on + n / 2) = o;
+                continue;
+            }
+            u32x2 o;
+            o[0] = uint32_t(f32_to_bf16(y[0])) | (uint32_t(f32_to_bf16(y[1])) << 16);
+            o[1] = uint32_t(f32_to_bf16(y[2])) | (uint32_t(f32_to_bf16(y[3])) << 16);
+            if (W) {
+                *reinterpret_cast<u32x2*>(wtile + row * rsb + col * 2) = o;   // the residual is added on the way out
+            } else if (m < row_end && n < N) {
+                if (epi == SCMX_EPI_RES) {
+                    const u32x2 rr = *reinterpret_cast<const u32x2*>(a.res + size_t(m) * N + n);
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    y[r] = __fmul_rn(__fmul_rn(float(acc[i][j][4 * g + r]), xs), w4[r]);
-                uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
-                if (epi == SCMX_EPI_SWIGLU) {   // (g, g, u, u) -> two outputs
-                    const uint16_t s0 = swiglu_lut(a.silu, y[0], round_bf16(y[2]));
-                    const uint16_t s1 = swiglu_lut(a.silu, y[1], round_bf16(y[3]));
-                    const uint32_t o = uint32_t(s0) | (uint32_t(s1) << 16);
-                    if (W)
-                        *reinterpret_cast<uint32_t*>(wtile + row * rsb + col) = o;
-                    else if (m < row_end && n < N)
-                        *reinterpret_cast<uint32_t*>(out + size_t(m) * on + n / 2) = o;
-                    continue;
-                }
-                u32x2 o;
-                o[0] = uint32_t(f32_to_bf16(y[0])) | (uint32_t(f32_to_bf16(y[1])) << 16);
-                o[1] = uint32_t(f32_to_bf16(y[2])) | (uint32_t(f32_to_bf16(y[3])) << 16);
-                if (W) {
-                    *reinterpret_cast<u32x2*>(wtile + row * rsb + col * 2) = o;   // the residual is added on the way out
-                } else if (m < row_end && n < N) {
-                    if (epi == SCMX_EPI_RES) {
-                        const u32x2 rr = *reinterpret_cast<const u32x2*>(a.res + size_t(m) * N + n);
-#pragma unroll
-                        for (int r = 0; r < 2; ++r) {
-                            const float lo = __fadd_rn(__uint_as_float(rr[r] << 16), __uint_as_float(o[r] << 16));
-                            const float hi = __fadd_rn(__uint_as_float(rr[r] & 0xFFFF0000u), __uint_as_float(o[r] & 0xFFFF0000u));
-                            o[r] = uint32_t(f32_to_bf16(lo)) | (uint32_t(f32_to_bf16(hi)) << 16);
-                        }
+                    for (int r = 0; r < 2; ++r) {
+                        const float lo = __fadd_rn(__uint_as_float(rr[r] << 16), __uint_as_float(o[r] << 16));
+                        const float hi = __fadd_rn(__uint_as_float(rr[r] & 0xFFFF0000u), __uint_as_float(o[r] & 0xFFFF0000u));
+                        o[r] = uint32_t(f32_to_bf16(lo)) | (uint32_t(f32_to_bf16(hi)) << 16);
                     }
-                    *reinterpret_cast<u32x2*>(out + size_t(m) * N + n) = o;
                 }
+                *reinterpret_cast<u32x2*>(out + size_t(m) * N + n) = o;
             }
         }
     }
@@ -819,31 +862,35 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 // ---- host dispatch ---------------------------------------------------------------------------------------------
 
 template <int BM, int BN, int BK, int WGM, int WGN, int OCC = 1, int FD = 2, bool SKIP = false, bool PK = false, int KG = 1,
-          bool AD = false>
+          int ADM = 0>
 static void launch_tile(const GemmArgs& a_in, int bmode, int row_tiles, hipStream_t s) {
     GemmArgs a = a_in;
     if (a.epi == SCMX_EPI_SWIGLU) a.silu = silu_table_device();
     const int num_n = (a.N + BN - 1) / BN;
     if (a.tstart) row_tiles = (row_tiles + 7) & ~7;   // grouped: whole chunks of 8 row-tile slots (spare slots exit at once)
     const dim3 grid(unsigned(row_tiles) * unsigned(num_n)), block(WGM * WGN * KG * 64);
-    if constexpr (PK) {   // callers choose this tile for the two FP4-conversion formats only
+    if constexpr (PK) {   // callers choose this tile for the FP4-conversion formats only
         if (bmode == B_PACKED_DEFAULT)
             gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_DEFAULT, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
-        else
+        else if (bmode == B_PACKED_B16)
             gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
+        else if (bmode == B_PACKED_B16M)
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16M, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
+        else
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_E8M0, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
     } else {
         if (bmode == B_INT8)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_INT8, OCC, FD, SKIP, false, KG, AD><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_INT8, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_DEFAULT)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_DEFAULT, OCC, FD, SKIP, false, KG, AD><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_DEFAULT, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_B16)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16, OCC, FD, SKIP, false, KG, AD><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_B16M)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16M, OCC, FD, SKIP, false, KG, AD><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16M, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_E8M0)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_E8M0, OCC, FD, SKIP, false, KG, AD><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_E8M0, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
         else
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_GENERIC, OCC, FD, SKIP, false, KG, AD><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_GENERIC, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
     }
 }
 
@@ -855,57 +902,50 @@ static int packed_mode(const DevFormat& f) {
                                         : B_PACKED_GENERIC;
 }
 
-// Dense: one launch, with the tile a cost model of the candidates below makes fastest.
-// Which tile a dense problem runs on: the index into the candidate table below.  blocked: the activations are in the
-// blocked layout, which four tiles read (their waves then load activation fragments straight from memory).
-// (Asked for on every call of a layer: shifts where the sizes are powers of two, no division for less than one wave.)
+// Dense: one launch, with the tile a cost model makes fastest.  A launch runs its tiles in waves of (CUs x workgroups that
+// share a CU); a wave costs f + s per 128 of K and not less than w, all three by the number of co-resident workgroups, and a
+// last wave that leaves CUs idle costs a part of a full one.  Both tables are fitted to 334 problems (widths 896 ... 24576,
+// reductions 896 ... 12288, 33 ... 8192 rows, every tile timed): the choice costs 0.24 per cent over the fastest blocked tile
+// on average, 0.46 over the fastest row tile.
+struct Cand {
+    int bm, bn, occ;
+    float f[4], s[4], w[4];   // per wave, by co-resident workgroups 1..occ: fixed us, us per 128 of K, least us
+    float low, mid;           // a wave on half of the CUs or fewer / on three quarters of them costs this part of a full one
+};
+// Activations by rows, staged in LDS.  What the table encodes: 256x256 moves the fewest LDS bytes per MFMA; the small tiles share
+// a CU and lose less to a ragged tile count; with no more 64x64 tiles than CUs two K groups per tile put eight waves on
+// a CU, and with no more 64x32 tiles than CUs four K groups of two waves do.
+static const Cand ROW_TILES[7] = {
+    {256, 256, 1, {9.46f}, {1.772f}, {18.9f}, 0.78f, 0.86f},
+    {256, 128, 1, {5.97f}, {0.857f}, {11.5f}, 0.865f, 0.93f},
+    {128, 128, 1, {4.18f}, {0.513f}, {6.4f}, 0.98f, 1.04f},
+    {128, 64, 2, {3.9f, 2.64f}, {0.364f, 0.649f}, {2.26f, 8.32f}, 0.945f, 1.015f},
+    {64, 64, 3, {3.39f, 3.82f, 2.06f}, {0.322f, 0.462f, 0.607f}, {3.94f, 2.12f, 3.0f}, 0.975f, 1.01f},
+    {64, 64, 1, {2.51f}, {0.233f}, {4.81f}, 1.0f, 1.05f},    // two K groups
+    {64, 32, 1, {2.41f}, {0.157f}, {4.145f}, 1.0f, 1.05f},   // four K groups
+};
+// Blocked activations, read by the waves themselves.  Workgroups of four waves share a CU (two of 256x128, three of 128x64, four
+// of 64x64): their barriers and epilogues do not coincide, which eight waves of one workgroup cannot avoid.  Eight waves
+// on one tile are faster where the launch has no more than a tile per CU.
+static const Cand BLOCKED_TILES[5] = {
+    {256, 128, 2, {6.11f, 8.34f}, {0.966f, 1.498f}, {4.2f, 2.3f}, 0.914f, 0.96f},
+    {256, 128, 1, {5.51f}, {0.805f}, {11.5f}, 0.85f, 0.93f},   // eight waves
+    {256, 64, 1, {3.945f}, {0.416f}, {2.4f}, 0.98f, 1.05f},    // eight waves
+    {128, 64, 3, {3.78f, 4.09f, 2.62f}, {0.34f, 0.498f, 0.806f}, {3.83f, 5.3f, 3.0f}, 0.925f, 0.98f},
+    {64, 64, 4, {3.15f, 3.54f, 3.58f, 1.83f}, {0.294f, 0.419f, 0.618f, 0.782f}, {5.49f, 4.07f, 2.67f, 3.0f}, 0.95f, 1.0f},
+};
 struct TileChoice {
     int index;
-    float us;   // its modelled time
+    float us;   // its modelled time, a launch included
 };
-static TileChoice dense_choice(long M, long N, long K, bool blocked, long cus) {
-    auto tiles = [&](int bm, int bn) { return ((M + bm - 1) >> __builtin_ctz(bm)) * ((N + bn - 1) >> __builtin_ctz(bn)); };
-    // The tile is the one a small cost model makes fastest.  A launch runs its tiles in waves of (CUs x workgroups that
-    // share a CU); a wave costs F + S per 128 of K and not less than W, all three measured per configuration and per
-    // number of co-resident workgroups (four Qwen3-1.7B layer shapes and five others, K = 128 ... 6144, M = 64 ... 8192:
-    // the choice is within 2.5 % of the fastest configuration on all 118), and a last wave that leaves CUs idle runs
-    // faster (less contention for the L2s and HBM).  What the table encodes: 256x256 moves the fewest LDS bytes per MFMA
-    // and pays where it fills the chip or saves a round; a mostly empty last round costs more than a narrower tile's
-    // extra LDS traffic; the small tiles share a CU and lose less to a ragged tile count; with no more 64x64 tiles
-    // than CUs two K groups per tile put eight waves on a CU, and with no more 64x32 tiles than CUs four K groups of two
-    // waves do (a 2048-wide layer on up to 128 rows: 64 ... 128 tiles instead of 32 ... 64; down 14.4 -> 10.2-10.9 us).
-    // (A 256x64 tile was never the fastest and is gone.)
-    struct Cand {
-        int bm, bn, occ;
-        float f[3], s[3], w[3];   // per wave, by co-resident workgroups 1..occ: fixed us, us per 128 of K, least us
-        float low, mid;           // a wave on half of the CUs or fewer / on three quarters of them costs this part of a full one
-    };
-    static const Cand cand[7] = {
-        {256, 256, 1, {6.5f, 0, 0}, {1.9f, 0, 0}, {8.4f, 0, 0}, 0.70f, 0.835f},
-        {256, 128, 1, {4.2f, 0, 0}, {0.94f, 0, 0}, {5.5f, 0, 0}, 0.74f, 0.78f},
-        {128, 128, 1, {1.4f, 0, 0}, {0.62f, 0, 0}, {3.0f, 0, 0}, 0.86f, 0.97f},
-        {128, 64, 2, {1.4f, 1.2f, 0}, {0.39f, 0.77f, 0}, {2.2f, 3.0f, 0}, 0.91f, 1.0f},
-        {64, 64, 3, {0.85f, 0.6f, 0.6f}, {0.34f, 0.53f, 0.70f}, {1.9f, 2.3f, 2.7f}, 0.95f, 1.0f},
-        {64, 64, 1, {1.1f, 0, 0}, {0.26f, 0, 0}, {2.0f, 0, 0}, 0.97f, 1.0f},   // two K groups
-        {64, 32, 1, {1.26f, 0, 0}, {0.14f, 0, 0}, {2.0f, 0, 0}, 0.95f, 0.97f},  // four K groups
-    };
-    // the same tiles fed from blocked activations (fewer LDS bytes per MFMA: a shorter K step)
-    static const Cand cand_blocked[4] = {
-        {256, 256, 1, {6.8f, 0, 0}, {1.78f, 0, 0}, {8.4f, 0, 0}, 0.70f, 0.835f},
-        {256, 128, 1, {3.8f, 0, 0}, {0.92f, 0, 0}, {5.5f, 0, 0}, 0.74f, 0.78f},
-        {128, 128, 1, {2.8f, 0, 0}, {0.58f, 0, 0}, {3.0f, 0, 0}, 0.86f, 0.97f},
-        // eight waves stacked along M on 64 columns: half the weight staging of the 128x128 tile per MFMA, no activation
-        // row fetched twice (2048-wide layers at M = 1024 ... 2048: 13.7 -> 12.2 us, K = 6144: 30.8 -> 28.9)
-        {256, 64, 1, {2.2f, 0, 0}, {0.55f, 0, 0}, {3.0f, 0, 0}, 0.86f, 0.97f},
-    };
+// Asked for on every call of a layer: shifts where the sizes are powers of two, no division for less than one wave.
+static TileChoice fastest_tile(const Cand* cand, int first, int last, long M, long N, long K, long cus) {
     const float steps = float(K) / 128.0f;
-    int best = blocked ? 2 : 4;
-    float best_t = 1e30f;
-    for (int c = 0; c < (blocked ? 4 : 7); ++c) {
-        const Cand& k = blocked ? cand_blocked[c] : cand[c];
-        const long n = tiles(k.bm, k.bn);
-        if (c == 5 && (n > cus || K % 256)) continue;
-        if (c == 6 && (n > cus || K % 512)) continue;
+    TileChoice best = {-1, 1e30f};
+    for (int c = first; c <= last; ++c) {   // from the largest tile down: a tie goes to the larger one
+        const Cand& k = cand[c];
+        const long n = ((M + k.bm - 1) >> __builtin_ctz(k.bm)) * ((N + k.bn - 1) >> __builtin_ctz(k.bn));
+        if (cand == ROW_TILES && c >= 5 && (n > cus || K % (c == 5 ? 256 : 512))) continue;   // K groups
         const long cap = cus * k.occ;
         const long full = n < cap ? 0 : n / cap, rest = n - full * cap;
         float t = float(full) * fmaxf(k.f[k.occ - 1] + steps * k.s[k.occ - 1], k.w[k.occ - 1]);
@@ -920,57 +960,61 @@ static TileChoice dense_choice(long M, long N, long K, bool blocked, long cus) {
             }
             t += w;
         }
-        if (t < best_t * 0.98f) {   // candidates run from the largest tile down: a tie goes to the larger one
-            best_t = t;
-            best = c;
-        }
+        if (t < best.us) best = {c, t};
     }
-    return {best, best_t};
+    return best;
 }
 
-// Whether the few-row kernel is faster than the row-layout tiles (the one that it would replace), by the two
-// models.  The table of the 64x32 tile was fitted to more rows: here it takes 1.27 times that, 1.35 where half of the CUs or more
-// have none (that does not make it faster here).  Formats whose codes are looked up: a tile's weights are decoded again by each
-// of its row groups, once by this kernel, which is worth half as much again.  On 4268 problems (16 ... 128 rows, widths 512 ...
-// 24576, reductions 512 ... 11008, both kernels timed) the choice costs 0.2 - 0.5 per cent over the faster one on average, by
-// format, and 11 - 30 per cent at most (one row tile of wide MXFP4 layers: 12288 x 8192 27.7 us for 21.2); the few-row kernel always
-// 3 - 4 (tables 0.6), the tiles always 20 (54).  us, few-row / tiles, whole linears: 2048 x 6144 at 80 rows 13.3 / 14.2, 4096 x
-// 8192 at 80 19.1 / 16.7, 896 x 5632 at 96 12.1 / 13.4, 6144 x 4096 at 64 15.5 / 11.6 (tables 24.6 / 19.4), 6144 x 4480 (no K groups
-// for the tiles) 15.0 / 17.0, 896 x 4864 at 112 13.2 / 15.4, 6144 x 4864 at 64 with tables 25.2 / 32.8.
-// *tile: that tile's choice, filled in where the answer is no.  No tile's table gives less than `least`, so the smallest calls,
-// which the host bounds, look no further: 0.05 us a call for 0.09.
-static bool few_rows(const scmx_format* fmt, int M, int N, int K, TileChoice* tile) {
+// The layout a dense layer's activations are quantized into, and with it the kernel: the blocked tiles, the few-row kernel
+// (blocked as well) or the row tiles, by their models.  The quantizer takes 0.3 us longer for blocks.  Beyond the few-row
+// kernel's range only the row tiles with K groups were ever the fastest of all (up to 1.4 times, narrow layers); within it the
+// blocked tiles have to be a tenth faster (wide layers at 100 rows and more are: 128 x 12288 x 2048 9.3 us for 10.7).
+// The few-row kernel's model takes no launch in.  On the 61 problems of up to 128 rows the choice costs 0.1 per cent over the
+// fastest kernel on average.  Formats whose codes are looked up: a tile's weights are decoded again by each of its row groups,
+// once by the few-row kernel, which is worth half as much again.
+// No table gives less than `least`, so the smallest calls, which the host bounds, look no further.
+enum { BY_ROWS = 0, BLOCKED = 1 };   // and FEW_ROWS
+static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
     const int cus = device_cus();
-    const bool candidate = M <= SKINNY_MAX_ROWS && long(M + 15) / 16 * 16 * N <= 480000;   // (beyond: not measured)
-    const float t = candidate ? skinny_time(M, N, K, cus) : 0.0f, least = 0.95f * fmaxf(1.9f, 1.26f + 0.14f / 128.0f * float(K));
-    if (candidate && t < least) return true;
-    *tile = dense_choice(M, N, K, false, cus);
-    if (!candidate) return false;
-    const float more = tile->index != 6 ? 1.0f : long(M + 63) / 64 * ((N + 31) / 32) * 2 <= cus ? 1.35f : 1.27f;
-    if (t < more * tile->us) return true;
+    const bool small = M <= SKINNY_MAX_ROWS, candidate = small && long(M + 15) / 16 * 16 * N <= 480000;   // (beyond: not measured)
+    const float few = candidate ? 1.0f + 0.9f * skinny_time(M, N, K, cus) : 1e30f;
+    const float least = fmaxf(3.8f, 2.41f + 0.157f / 128.0f * float(K));
+    if (few < least) return FEW_ROWS;
+    const float rows = fastest_tile(ROW_TILES, small ? 0 : 5, 6, M, N, K, cus).us;
+    const float blocks = (0.3f + fastest_tile(BLOCKED_TILES, 0, 4, M, N, K, cus).us) * (small ? 1.1f : 1.0f);
+    const float tile = fminf(rows, blocks);
+    if (few < tile) return FEW_ROWS;
     DevFormat f;
-    return fmt && t < 1.5f * more * tile->us && make_dev_format(fmt, &f) == SCMX_OK && packed_mode(f) == B_PACKED_GENERIC;
+    if (fmt && few < 1.5f * tile && make_dev_format(fmt, &f) == SCMX_OK && packed_mode(f) == B_PACKED_GENERIC) return FEW_ROWS;
+    return blocks < rows ? BLOCKED : BY_ROWS;
 }
 
 static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
     if (a.blocked == FEW_ROWS) return launch_skinny(a, bmode, s);
-    const int best = dense_choice(a.M, a.N, a.K, a.blocked != 0, device_cus()).index;
+    const int rows256 = (a.M + 255) / 256, rows128 = (a.M + 127) / 128, rows64 = (a.M + 63) / 64;
     if (a.blocked) {
-        switch (best) {
-            case 0: return launch_tile<256, 256, 64, 4, 2, 1, 2, false, false, 1, true>(a, bmode, (a.M + 255) / 256, s);
-            case 1: return launch_tile<256, 128, 128, 8, 1, 1, 2, false, false, 1, true>(a, bmode, (a.M + 255) / 256, s);
-            case 3: return launch_tile<256, 64, 128, 8, 1, 1, 2, false, false, 1, true>(a, bmode, (a.M + 255) / 256, s);
-            default: return launch_tile<128, 128, 128, 4, 2, 1, 2, false, false, 1, true>(a, bmode, (a.M + 127) / 128, s);
+        // The four-wave 256x128 tile reads K in steps of 64.  With a byte per 32 weights and a row of those 128 bytes or longer it
+        // reads a cache line per weight row and step for two of them, and the vector L1 does not hold the lines until the next
+        // step: 6001 x 6144 x 4096 161 us against 152 of the eight waves (2-bit codes 144 / 148; K = 2048 66.6 / 68.8).  Table
+        // decode does not fit its registers.
+        const bool wide_codes = (bmode == B_PACKED_E8M0 || bmode == B_PACKED_B16M) && a.K >= 4096;
+        const int first = wide_codes || bmode == B_PACKED_GENERIC ? 1 : 0;
+        switch (fastest_tile(BLOCKED_TILES, first, 4, a.M, a.N, a.K, device_cus()).index) {
+            case 0: return launch_tile<256, 128, 64, 4, 1, 2, 2, false, false, 1, 1>(a, bmode, rows256, s);
+            case 1: return launch_tile<256, 128, 128, 8, 1, 1, 2, false, false, 1, 1>(a, bmode, rows256, s);
+            case 2: return launch_tile<256, 64, 128, 8, 1, 1, 2, false, false, 1, 1>(a, bmode, rows256, s);
+            case 3: return launch_tile<128, 64, 128, 4, 1, 2, 2, false, false, 1, 1>(a, bmode, rows128, s);
+            default: return launch_tile<64, 64, 128, 2, 2, 2, 2, false, false, 1, 1>(a, bmode, rows64, s);
         }
     }
-    switch (best) {
-        case 0: return launch_tile<256, 256, 64, 2, 4, 1, 2>(a, bmode, (a.M + 255) / 256, s);
-        case 1: return launch_tile<256, 128, 128, 4, 2, 1, 3>(a, bmode, (a.M + 255) / 256, s);
-        case 2: return launch_tile<128, 128, 128, 4, 2, 1, 3>(a, bmode, (a.M + 127) / 128, s);
-        case 3: return launch_tile<128, 64, 128, 4, 2>(a, bmode, (a.M + 127) / 128, s);
-        case 5: return launch_tile<64, 64, 128, 2, 2, 1, 2, false, false, 2>(a, bmode, (a.M + 63) / 64, s);
-        case 6: return launch_tile<64, 32, 128, 2, 1, 1, 2, false, false, 4>(a, bmode, (a.M + 63) / 64, s);
-        default: return launch_tile<64, 64, 128, 2, 2>(a, bmode, (a.M + 63) / 64, s);
+    switch (fastest_tile(ROW_TILES, 0, 6, a.M, a.N, a.K, device_cus()).index) {
+        case 0: return launch_tile<256, 256, 64, 2, 4, 1, 2>(a, bmode, rows256, s);
+        case 1: return launch_tile<256, 128, 128, 4, 2, 1, 3>(a, bmode, rows256, s);
+        case 2: return launch_tile<128, 128, 128, 4, 2, 1, 3>(a, bmode, rows128, s);
+        case 3: return launch_tile<128, 64, 128, 4, 2>(a, bmode, rows128, s);
+        case 5: return launch_tile<64, 64, 128, 2, 2, 1, 2, false, false, 2>(a, bmode, rows64, s);
+        case 6: return launch_tile<64, 32, 128, 2, 1, 1, 2, false, false, 4>(a, bmode, rows64, s);
+        default: return launch_tile<64, 64, 128, 2, 2>(a, bmode, rows64, s);
     }
 }
 
@@ -1074,28 +1118,23 @@ int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* 
         set_error("mm_w4a8_blocked: the activations' whole 32-row blocks lie beyond the 32-bit offsets of the kernel (M=%d K=%d)", M, K);
         return SCMX_ERR_ARG;
     }
-    TileChoice tile;
-    const bool few = M > 0 && N > 0 && K > 0 && few_rows(fmt, M, N, K, &tile);
-    return mm_w4a8(fmt, xq, xscale, codes, bcodes, wscale, res, out, epi, M, N, K, few ? FEW_ROWS : 1, stream);
+    const bool few = M > 0 && N > 0 && K > 0 && dense_layout(fmt, M, N, K) == FEW_ROWS;
+    return mm_w4a8(fmt, xq, xscale, codes, bcodes, wscale, res, out, epi, M, N, K, few ? FEW_ROWS : BLOCKED, stream);
 }
 
 int scmx_mm_w4a8_prefers_blocked(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    TileChoice tile;
-    return few_rows(nullptr, M, N, K, &tile) || tile.index <= 2;
+    return dense_layout(nullptr, M, N, K) != BY_ROWS;
 }
 
-// The fused layer quantizes into whichever layout suits the shape: blocked where the row-layout model would run one of its
-// three largest tiles (the blocked tiles then win), by rows otherwise.  Both layouts take (M rounded up to 32) x K bytes at most.
+// The fused layer quantizes into whichever layout suits the shape (dense_layout).  Both layouts take (M rounded up to 32) x K bytes at most.
 static int quantize_and_multiply(const scmx_format* fmt, const uint16_t* x, int8_t* xq, float* xs, bool room_for_blocks,
                                  const uint32_t* codes, const uint8_t* bcodes, const float* wscale, const uint16_t* res,
                                  void* out, int epi, int M, int N, int K, void* stream) {
     const long long Mp = (static_cast<long long>(M) + 31) & ~31LL;
-    int blocked = 0;
-    if (room_for_blocks && M > 0 && N > 0 && K > 0 && K % 128 == 0 && uint64_t(Mp) * uint64_t(K) <= 0xFFFFFFFFull) {
-        TileChoice tile;
-        blocked = few_rows(fmt, M, N, K, &tile) ? FEW_ROWS : tile.index <= 2;
-    }
+    int blocked = BY_ROWS;
+    if (room_for_blocks && M > 0 && N > 0 && K > 0 && K % 128 == 0 && uint64_t(Mp) * uint64_t(K) <= 0xFFFFFFFFull)
+        blocked = dense_layout(fmt, M, N, K);
     if (blocked) {
         if (int rc = scmx_act_quant_blocked(x, xq, xs, M, int(Mp), K, stream)) return rc;
     } else {
@@ -1217,19 +1256,26 @@ static int moe_common(const char* who, const int8_t* xq, const float* xscale, co
 
 static void launch_grouped(const GemmArgs& a, int bmode, int tm, hipStream_t s) {
     const int max_tiles = (a.M + tm - 1) / tm + a.n_experts;   // e2e/sc_moe.py:155
-    if (tm == 256 && (a.N % 256 == 0 || a.N >= 1024))   // 256-wide column tiles: fewer LDS bytes per MFMA
+    // 256-row tiles, activations staged in LDS, from 256 rows per expert on: the fewest LDS bytes per MFMA.  Below that 128-row
+    // ones (two to a slot where the segments are cut into 256): workgroups of four waves whose activation fragments come
+    // straight from the gathered rows, two of them on a CU.  64 experts of 2048 x 2048 / 2048 x 1024, 125 rows each: 67 + 37
+    // us for 86 + 51 (64-row tiles 74 + 41); 375 rows each 155 + 83 for 153 + 85.
+    if (tm == 256 && a.M / a.n_experts >= 256 && (a.N % 256 == 0 || a.N >= 1024))
         launch_tile<256, 256, 64, 2, 4, 1, 2, true>(a, bmode, max_tiles, s);
-    else if (tm == 256)
-        launch_tile<256, 128, 128, 4, 2, 1, 3>(a, bmode, max_tiles, s);
-    else if (tm == 128)
-        launch_tile<128, 128, 128, 4, 2, 1, 3>(a, bmode, max_tiles, s);
-    else if ((bmode == B_PACKED_DEFAULT || bmode == B_PACKED_B16) && a.K % 256 == 0 && a.N % 256 == 0 &&
-             reinterpret_cast<uintptr_t>(a.bcodes) % 4 == 0)
-        // few rows per expert: the pass streams the expert weights, and what it pays per weight is the staging.  The
-        // packed tile writes and reads half the weight bytes in LDS, its eight waves sit side by side along N (every
-        // fragment is decoded once) and two workgroups share a CU (128 registers).  Its lanes read the block codes of two
-        // K steps with one aligned 2- or 4-byte load, hence the conditions on K and on the pointer.
-        launch_tile<64, 256, 128, 1, 8, 4, 2, false, true>(a, bmode, max_tiles, s);
+    else if (tm >= 128) {
+        GemmArgs b = a;
+        b.sub_log2 = tm == 256 ? 1 : 0;
+        launch_tile<128, 128, 128, 4, 1, 2, 2, false, false, 1, 2>(b, bmode, max_tiles << b.sub_log2, s);
+    }
+    else if (bmode != B_INT8 && bmode != B_PACKED_GENERIC && a.K % 256 == 0 && a.N % 128 == 0 &&
+             reinterpret_cast<uintptr_t>(a.bcodes) % 8 == 0)
+        // Few rows per expert: the pass streams the expert weights, and what it pays per weight is the staging.  The packed
+        // tile writes and reads half the weight bytes in LDS, its four waves sit side by side along N (every fragment is
+        // decoded once) and three workgroups share a CU.  Its lanes read the block codes of two K steps with one aligned
+        // load of 2, 4 or 8 bytes, hence the conditions on K and on the pointer.  Bound by the vector ALU: 64 codes a lane
+        // and step to decode (10 instructions per 8) beside 16 MFMAs.  257 experts of 1024 x 2048 / 2048 x 512, 70 rows each,
+        // e2m1/B16/M1..10: 108 + 67 us, staged INT8 118 + 74.
+        launch_tile<64, 128, 128, 1, 4, 2, 2, false, true>(a, bmode, max_tiles, s);
     else
         launch_tile<64, 128, 128, 2, 4>(a, bmode, max_tiles, s);
 }

@@ -21,6 +21,7 @@ struct GemmArgs {
     const uint16_t* silu;    // SwiGLU epilogue: lookup table over bf16 gate values
     const int32_t* tstart;   // grouped: first row tile of each expert [E+1]
     int n_experts;
+    int sub_log2;            // grouped: a segment's row tile is 1 << sub_log2 of the kernel's
     int blocked;             // dense: xq is in the blocked layout (FEW_ROWS: and the few-row kernel takes it)
     DevFormat fmt;
 };

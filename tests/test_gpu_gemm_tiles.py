@@ -1,0 +1,74 @@
+"""The tiles of the blocked dense GEMM and of the grouped GEMM, INT32 against a float64 product of the decoded weights: ragged rows and
+columns, step counts that end in every tail of the unrolled K loops, each weight format."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import layout
+from tests.util import FORMATS, blocked_layout, dev, host, product_format, random_packed
+
+pytestmark = pytest.mark.gpu
+NAMES = {"published": FORMATS[0], "sixteen": FORMATS[1], "range": FORMATS[5], "table": FORMATS[4], "mxfp4": None}
+
+
+def weights(rng, n, k, name):
+    """(codes, block codes, row scales, product format, decoded INT8 [n, k]) on the device."""
+    from mxfp4_int8_m5_amd import sc_format as F
+    c, b, w, q = random_packed(rng, n, k, NAMES[name] or layout.DEFAULT)
+    if NAMES[name]:
+        return dev(c), dev(b), dev(w), product_format(NAMES[name]), dev(q)
+    nib, e8 = layout.to_mxfp4(c, b, w, n, k)
+    nib, e8 = dev(nib), dev(e8)
+    ws = F.mxfp4_row_scales(e8)
+    lift = torch.exp2(torch.log2(dev(w)) - torch.log2(ws))   # a row whose smallest shift is not 0 decodes to smaller integers
+    return F.mxfp4_codes(nib), e8, ws, F.MXFP4, (dev(q).double() * lift[:, None].double()).to(torch.int8)
+
+
+def product(xq, q):
+    return (xq.double() @ q.double().T).to(torch.int32)
+
+
+# one row of the list per tile of the blocked table (its order), more than one step count for those with a rotating loop
+@pytest.mark.parametrize("name", list(NAMES))
+@pytest.mark.parametrize("m,n,k", [(400, 12296, 384), (1030, 12296, 640), (385, 12288, 4224),   # 256x128, four waves (or, by format, the next)
+                                   (1000, 6152, 768), (1500, 4104, 2048),                        # 256x128, eight waves
+                                   (600, 4104, 2048), (1030, 2052, 1280),                        # 256x64
+                                   (515, 8200, 640), (1025, 8192, 384), (4099, 2052, 128),       # 128x64
+                                   (770, 1032, 1280), (129, 1028, 256), (300, 260, 896)])        # 64x64
+def test_blocked_tiles(m, n, k, name):
+    from mxfp4_int8_m5_amd import sc_kernels as S
+    rng = np.random.default_rng(m + n + k)
+    codes, bc, ws, fmt, q = weights(rng, n, k, name)
+    xq = rng.integers(-127, 128, (-(-m // 32) * 32, k)).astype(np.int8)
+    xb = S.BlockedXq(dev(blocked_layout(xq)), m, k)
+    assert torch.equal(S.mm_i8_i32(xb, S.PackedWq(codes, bc, n, k, fmt, ws))[:m], product(dev(xq)[:m], q))
+
+
+@pytest.mark.parametrize("name", list(NAMES))
+@pytest.mark.parametrize("tm", [64, 128, 256])
+@pytest.mark.parametrize("e,n,k", [(3, 1156, 512), (65, 256, 384), (130, 128, 256), (4100, 8, 128)])
+def test_grouped_tiles(e, n, k, tm, name):
+    """Segments of 0 to a little over 256 rows (a 256-row slot of which 128-row tiles use one or both halves, with and
+    without rows past the segment), expert counts either side of one and two levels of the tile's expert search; rows gathered."""
+    from mxfp4_int8_m5_amd import sc_moe as M
+    rng = np.random.default_rng(e + n + k)
+    counts = rng.choice([0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257], e) if e < 1000 else rng.choice([0, 0, 0, 1, 2], e)
+    counts[0] += 1
+    ex = np.repeat(np.arange(e), counts).astype(np.int32)
+    r = len(ex)
+    few = [weights(rng, n, k, name) for _ in range(min(e, 3))]
+    pick = [i % len(few) for i in range(e)]
+    codes, bc, ws, q = (torch.stack([few[i][f] for i in pick]) for f in (0, 1, 2, 4))
+    src = torch.from_numpy(rng.integers(-127, 128, (r + 9, k)).astype(np.int8)).cuda()
+    tok = torch.from_numpy(rng.permutation(r + 9)[:r].astype(np.int32)).cuda()
+    off, tstart, mt = M.segments(dev(ex), e, tm)
+    rows, idx = src[tok.long()], dev(ex).long()
+    want = torch.zeros((r, n), dtype=torch.int32, device="cuda")
+    for f in range(len(few)):
+        sel = (idx % len(few)) == f
+        want[sel] = product(rows[sel], few[f][4])
+    got = M.moe_mm(src, r, codes, bc, ws, off, tstart, mt, n, 0, tile=(tm, 64, 4), gather=tok, fmt=few[0][3])
+    assert torch.equal(got, want)
+    if name == "published":
+        got = M.moe_mm_i8(rows.contiguous(), r, q.reshape(e * n, k).contiguous(), ws, off, tstart, mt, n, 0, tile=(tm, 64, 4))
+        assert torch.equal(got, want)
