@@ -278,6 +278,7 @@ struct FamilyArgs {
     float cb[8];      // code magnitudes
     float cut[7];     // midpoints between neighbouring magnitudes
     float mult[16];
+    float half_inv[16];   // 0.5 / mult
     int n_mult, bc_bits;
 };
 
@@ -373,13 +374,48 @@ __device__ __forceinline__ float family_sq_err_e2m1(const float (&aw)[BLOCK], fl
                      __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
 }
 
+// That error to within the bound below, at 4 instructions per weight: one quotient, the conversion there and back, two fused
+// multiply-adds.
+template <int BLOCK>
+__device__ __forceinline__ float family_sq_err_near(const float (&aw)[BLOCK], float sc, float h) {   // h = 0.5 / sc
+    float r0 = 0.0f, r1 = 0.0f;
+    auto add = [&](int i, f32x2_t v) {
+        const float d0 = __builtin_fmaf(v[0], sc, -aw[i]), d1 = __builtin_fmaf(v[1], sc, -aw[i + 1]);
+        r0 = __builtin_fmaf(d0, d0, r0);
+        r1 = __builtin_fmaf(d1, d1, r1);
+    };
+#pragma unroll
+    for (int i = 0; i < BLOCK; i += 8) {   // the conversion writes one byte and keeps the others: four share a register
+        uint32_t c = 0u;
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, aw[i] * h, aw[i + 1] * h, 1.0f, 0);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, aw[i + 2] * h, aw[i + 3] * h, 1.0f, 1);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, aw[i + 4] * h, aw[i + 5] * h, 1.0f, 2);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, aw[i + 6] * h, aw[i + 7] * h, 1.0f, 3);
+        add(i, __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 2.0f, 0));
+        add(i + 2, __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 2.0f, 1));
+        add(i + 4, __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 2.0f, 2));
+        add(i + 6, __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 2.0f, 3));
+    }
+    return r0 + r1;
+}
+// How far the root of that sum can be from the root of the host's, twice (the two sides of a comparison), in parts of the norm of
+// the weights summed over.  With D_i the distance of weight i to the nearest level, D_i <= |w_i| (zero is a level): the level taken is
+// the nearest to a quotient 2^-21.4 off at most, so the difference to it exceeds D_i by 2^-20.4 |w_i| at most; seventeen additions
+// are 2^-20 of the sum, 2^-20.9 of its root.  The host's own roundings are 2^-21 of the norm.  By the triangle inequality 1.75 x 2^-20 in all,
+// twice 2^-18.2; for a row, whose sum of block errors rounds by 2^-20.4 of its root on either side, 2^-17.3.
+constexpr float NEAR = 7.62939453125e-6f;   // 2^-17
+
 constexpr int FAM_ROWS = 4;   // rows per workgroup at most: more are needed only for K < 1024, and their tables cost LDS
 
-// Bound: vector ALU (8 bases x n_mult trials per weight, 13 instructions each), 96 % busy.  2048 x 2048 bf16, ten multipliers: 130 us; 520 us with a lane
-// per weight, a correctly rounded division per trial and the sums across lanes.
-// SPREAD: a thread per block and base (fewer blocks than the chip has lanes: each would run all trials in one lane; 64 x 128,
-// ten multipliers 49 us).
-template <int BLOCK, bool BF16, bool E2M1, bool SPREAD>
+// Bound: vector ALU.  In the E2M1 codebook a trial is first evaluated to 2^-19 (family_sq_err_near): that settles nearly every
+// multiplier of a block and base, and all but one or two of a row's bases; only what it leaves open is evaluated as the host does.
+// Multipliers run from the largest down and end where clipping the block's largest weight alone costs more than the best so far, in every
+// lane.  2048 x 2048 bf16, ten multipliers: 67 us; 130 with every trial as the host evaluates it (13 instructions a weight), 520 with
+// a lane per weight, a correctly rounded division per trial and the sums across lanes.
+// BASES: 1 where there are fewer blocks than lanes, each of which would run all trials of one (64 x 128, ten multipliers 27 -> 11 us).
+// In the E2M1 codebook 4 beyond that: twice the waves to hide the conversions' latency and the uneven number of trials (600 x 2048
+// 44 us with all eight in a thread, 34 with four; 4096 x 2048 114 and 116).
+template <int BLOCK, bool BF16, bool E2M1, int BASES>   // bases per thread
 __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                              uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
                                                              int64_t N, int K, int rows, bool vec, const FamilyArgs f) {
@@ -387,6 +423,8 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
     __shared__ uint32_t s_peak[FAM_ROWS];
     __shared__ float s_tot[FAM_ROWS][8];
     __shared__ int s_best[FAM_ROWS];
+    __shared__ float s_norm[FAM_ROWS];     // sum of squares of the row
+    __shared__ uint32_t s_open[FAM_ROWS];  // bases whose totals have to be summed as the host does
     const int nb = K / BLOCK;
     float* s_err = s_f;
     uint8_t* s_mi = reinterpret_cast<uint8_t*>(s_f + size_t(rows) * 8 * nb);
@@ -395,7 +433,11 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
     const int total = live * nb, tid = threadIdx.x;
     const size_t wbase = row0 * K;
     // row peaks (bit patterns of non-negative floats order like the floats)
-    if (tid < FAM_ROWS) s_peak[tid] = 0u;
+    if (tid < FAM_ROWS) {
+        s_peak[tid] = 0u;
+        s_norm[tid] = 0.0f;
+        s_open[tid] = 0u;
+    }
     __syncthreads();
     float v[BLOCK];
     for (int b = tid; b < total; b += QNT) {
@@ -416,31 +458,75 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
     };
 
     // ---- per candidate base and block: the best multiplier and its error ------------------------------------------
-    constexpr int BASES = SPREAD ? 1 : 8;   // bases per thread
+    // The trial of one scale as the host evaluates it (a scale near the ends of the float32 range leaves its reciprocal no room).
+    auto in_range = [](float sc) { return sc > 1e-30f && sc < 1e30f; };
+    auto trial = [&](const float (&aw)[BLOCK], float sc) {
+        bool same = false;
+        float e = 0.0f;
+        if (E2M1 && in_range(sc)) e = family_sq_err_e2m1<BLOCK>(aw, sc, &same);
+        if (!same) e = family_sq_err<BLOCK, E2M1>(f, aw, sc);
+        return e;
+    };
     for (int t = tid; t < total * (8 / BASES); t += QNT) {
-        const int b = t / (8 / BASES), j0 = SPREAD ? t % 8 : 0;
-        if (SPREAD || total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+        const int b = t / (8 / BASES), j0 = t % (8 / BASES) * BASES;
+        if (BASES < 8 || total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
         const int r = b / nb, kb = b - r * nb;
         const float top = row_top(r);
-        float aw[BLOCK];
+        float aw[BLOCK], amax = 0.0f, norm2 = 0.0f;
 #pragma unroll
-        for (int i = 0; i < BLOCK; ++i) aw[i] = fabsf(v[i]);
+        for (int i = 0; i < BLOCK; ++i) {
+            aw[i] = fabsf(v[i]);
+            amax = fmaxf(amax, aw[i]);
+            norm2 = __builtin_fmaf(aw[i], aw[i], norm2);
+        }
+        // the bounds hold away from the ends of the float32 range; a block of zeros costs nothing at any scale
+        const bool near = E2M1 && ((norm2 > 1e-20f && norm2 < 1e20f) || (norm2 == 0.0f && amax == 0.0f)) &&
+                          in_range(top * ladder[7] * f.mult[0]) && in_range(top * f.mult[f.n_mult - 1]);
+        const float width = NEAR * __builtin_amdgcn_sqrtf(norm2);
+        if (E2M1) {
+            if (j0 == 0) atomicAdd(&s_norm[r], norm2);
+            if (!near) atomicOr(&s_open[r], 0xFFu);
+        }
 #pragma unroll 1
         for (int j = j0; j < j0 + BASES; ++j) {
             const float base = __fmul_rn(top, ladder[j]);
-            float best = 0.0f;
+            float best = __builtin_inff();
             int best_i = 0;
+            bool all = true;   // every multiplier as the host evaluates it
+            if (near) {
+                float second = __builtin_inff(), third = __builtin_inff();
+                int second_i = 0;
+                const float inv = __builtin_amdgcn_rcpf(base);
 #pragma unroll 1
-            for (int i = 0; i < f.n_mult; ++i) {
-                const float sc = __fmul_rn(base, f.mult[i]);
-                bool same = false;
-                float e = 0.0f;
-                // (a scale near the ends of the float32 range leaves its reciprocal no room)
-                if (E2M1 && sc > 1e-30f && sc < 1e30f) e = family_sq_err_e2m1<BLOCK>(aw, sc, &same);
-                if (!same) e = family_sq_err<BLOCK, E2M1>(f, aw, sc);
-                if (i == 0 || e < best) {
-                    best = e;
-                    best_i = i;
+                for (int i = f.n_mult - 1; i >= 0; --i) {
+                    const float sc = __fmul_rn(base, f.mult[i]);
+                    const float clip = amax - f.cb[7] * sc;
+                    if (!__any(!(clip * (1.0f - NEAR) > __builtin_amdgcn_sqrtf(best) + width))) break;   // of the lanes in the loop
+                    const float e = family_sq_err_near<BLOCK>(aw, sc, inv * f.half_inv[i]);
+                    const bool first = e < best, next = e < second;
+                    third = fminf(third, first ? second : fmaxf(e, second));
+                    second_i = first ? best_i : next ? i : second_i;
+                    second = first ? best : next ? e : second;
+                    best_i = first ? i : best_i;
+                    best = first ? e : best;
+                }
+                if (norm2 == 0.0f) best_i = 0;   // first of equals
+                const float limit = __builtin_amdgcn_sqrtf(best) + width;
+                all = norm2 != 0.0f && !(__builtin_amdgcn_sqrtf(third) > limit);
+                if (norm2 != 0.0f && !all && !(__builtin_amdgcn_sqrtf(second) > limit)) {   // one of two, the lower one of equals
+                    const int lo = min(best_i, second_i), hi = max(best_i, second_i);
+                    const float el = trial(aw, __fmul_rn(base, f.mult[lo])), eh = trial(aw, __fmul_rn(base, f.mult[hi]));
+                    best_i = eh < el ? hi : lo;
+                }
+            }
+            if (all) {
+#pragma unroll 1
+                for (int i = 0; i < f.n_mult; ++i) {
+                    const float e = trial(aw, __fmul_rn(base, f.mult[i]));
+                    if (i == 0 || e < best) {
+                        best = e;
+                        best_i = i;
+                    }
                 }
             }
             s_err[(r * 8 + j) * nb + kb] = best;
@@ -450,11 +536,46 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
     __syncthreads();
     if (tid < 8 * live) s_tot[tid >> 3][tid & 7] = np_pairwise_sum<4>(s_err + tid * nb, nb);
     __syncthreads();
+    if constexpr (E2M1) {   // the bases that these totals leave open: their blocks' errors once more, as the host sums them
+        if (tid < live) {
+            float least = __builtin_inff();
+            for (int j = 0; j < 8; ++j) least = fminf(least, s_tot[tid][j]);
+            const float limit = __builtin_amdgcn_sqrtf(least) + NEAR * __builtin_amdgcn_sqrtf(s_norm[tid]);
+            uint32_t open = s_open[tid];
+            for (int j = 0; j < 8; ++j)
+                if (!(__builtin_amdgcn_sqrtf(s_tot[tid][j]) > limit)) open |= 1u << j;
+            s_open[tid] = open;
+        }
+        __syncthreads();
+        for (int t = tid; t < total * (8 / BASES); t += QNT) {
+            const int b = t / (8 / BASES), j0 = t % (8 / BASES) * BASES, r = b / nb, kb = b - r * nb;
+            uint32_t open = s_open[r];
+            if ((open & (open - 1u)) == 0u) continue;   // settled
+            open &= ((1u << BASES) - 1u) << j0;
+            if (open == 0u) continue;
+            if (BASES < 8 || total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+            float aw[BLOCK];
+#pragma unroll
+            for (int i = 0; i < BLOCK; ++i) aw[i] = fabsf(v[i]);
+            for (; open; open &= open - 1u) {
+                const int j = __builtin_ctz(open);
+                const float sc = __fmul_rn(__fmul_rn(row_top(r), ladder[j]), f.mult[s_mi[(r * 8 + j) * nb + kb]]);
+                s_err[(r * 8 + j) * nb + kb] = trial(aw, sc);
+            }
+        }
+        __syncthreads();
+        if (tid < 8 * live) {
+            const uint32_t open = s_open[tid >> 3];
+            if ((open & (open - 1u)) != 0u && ((open >> (tid & 7)) & 1u))
+                s_tot[tid >> 3][tid & 7] = np_pairwise_sum<4>(s_err + tid * nb, nb);
+        }
+        __syncthreads();
+    }
     if (tid < live) {
         float best = __builtin_inff();
         int bj = 0;
         for (int j = 0; j < 8; ++j)
-            if (s_tot[tid][j] < best) {
+            if ((!E2M1 || ((s_open[tid] >> j) & 1u)) && s_tot[tid][j] < best) {
                 best = s_tot[tid][j];
                 bj = j;
             }
@@ -465,7 +586,7 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
 
     // ---- codes ----------------------------------------------------------------------------------------------------
     for (int b = tid; b < total; b += QNT) {
-        if (SPREAD || total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
+        if (BASES < 8 || total > QNT) load_block<BLOCK, BF16>(w, wbase + size_t(b) * BLOCK, vec, v);
         const int r = b / nb, kb = b - r * nb, bj = s_best[r];
         const float base = __fmul_rn(row_top(r), ladder[bj]);
         const bool dead = base == 0.0f;   // a vanishing row underflows its base: it is exactly zero (e2e/pack_format.py:55-58)
@@ -473,7 +594,31 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
         uint32_t c[BLOCK / 8];
 #pragma unroll
         for (int i = 0; i < BLOCK / 8; ++i) c[i] = 0u;
-        if (!dead) {
+        uint32_t open = 1u;   // quotients that two sides of a reciprocal round to different codes (as in family_sq_err_e2m1)
+        if (E2M1 && !dead && in_range(sc)) {
+            const float h = 0.5f * __builtin_amdgcn_rcpf(sc);
+            const float up = h * 1.00000095367431640625f, dn = h * 0.99999904632568359375f;
+            open = 0u;
+#pragma unroll
+            for (int q = 0; q < BLOCK / 8; ++q) {
+                const float* x = v + 8 * q;
+                auto code = [&](float g) {
+                    uint32_t o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[0] * g, x[1] * g, 1.0f, 0);
+                    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, x[2] * g, x[3] * g, 1.0f, 1);
+                    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, x[4] * g, x[5] * g, 1.0f, 2);
+                    return uint32_t(__builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, x[6] * g, x[7] * g, 1.0f, 3));
+                };
+                const uint32_t o = code(dn);
+                open |= o ^ code(up);
+                const uint32_t m = o & 0x77777777u;
+                c[q] = m | (o & (m + 0x77777777u) & 0x88888888u);   // a zero has no sign
+#pragma unroll
+                for (int i = 0; i < 8; ++i) open |= uint32_t(!(fabsf(x[i]) < 3e38f));   // infinities and NaN
+            }
+        }
+        if (!dead && open) {
+#pragma unroll
+            for (int i = 0; i < BLOCK / 8; ++i) c[i] = 0u;
 #pragma unroll
             for (int i = 0; i < BLOCK; ++i) {
                 const float x = __fdiv_rn(v[i], sc);
@@ -543,26 +688,27 @@ extern "C" int scmx_quantize_family(const scmx_format* fmt, const void* w, int w
             return SCMX_ERR_FORMAT;
         }
         f.mult[i] = float(fmt->mult[i]);
+        f.half_inv[i] = 0.5f / f.mult[i];
     }
     f.n_mult = fmt->n_mult;
     f.bc_bits = fmt->bc_bits;
     if (N == 0) return SCMX_OK;
     const int nb = K / block;
-    // Up to half a wave per SIMD.  (us, spread / not, bf16 in 16-blocks with ten multipliers: 269 x 896 42 / 56, 1000 x 896 66 / 56.)
-    const bool spread = long(N) * nb <= 32768;
-    const int rows = rows_per_group(spread ? 8 * nb : nb, FAM_ROWS);
+    // us, a thread per block and base / four bases a thread, bf16 in 16-blocks with ten multipliers: 640 x 896 22 / 26, 1000 x 896
+    // 25 / 28, 600 x 2048 35 / 33.  Other codebooks (a thread per base / per block): 269 x 896 42 / 56, 1000 x 896 66 / 56.
+    const bool e2m1 = df.lut_lo == 0x03020100u && df.lut_hi == 0x0C080604u, spread = long(N) * nb <= (e2m1 ? 65536 : 32768);
+    const int rows = rows_per_group(spread ? 8 * nb : e2m1 ? 2 * nb : nb, FAM_ROWS);
     const size_t smem = size_t(rows) * 8 * nb * (sizeof(float) + 1);
     const dim3 grid((unsigned)((N + rows - 1) / rows)), wg(QNT);
     const bool vec = uintptr_t(w) % 16 == 0 && uintptr_t(codes) % 16 == 0;
-    const bool e2m1 = df.lut_lo == 0x03020100u && df.lut_hi == 0x0C080604u;
     auto go = [&](auto kernel) {
         kernel<<<grid, wg, smem, (hipStream_t)stream>>>(w, codes, bcodes, wscale, N, K, rows, vec, f);
     };
     auto typed = [&](auto blk, auto bf) {
         constexpr int B = decltype(blk)::value;
         constexpr bool BF = decltype(bf)::value;
-        if (e2m1) spread ? go(quantize_family_kernel<B, BF, true, true>) : go(quantize_family_kernel<B, BF, true, false>);
-        else spread ? go(quantize_family_kernel<B, BF, false, true>) : go(quantize_family_kernel<B, BF, false, false>);
+        if (e2m1) spread ? go(quantize_family_kernel<B, BF, true, 1>) : go(quantize_family_kernel<B, BF, true, 4>);
+        else spread ? go(quantize_family_kernel<B, BF, false, 1>) : go(quantize_family_kernel<B, BF, false, 8>);
     };
     by_block_and_type(block, w_is_bf16, typed);
     return check_launch("quantize_family");
