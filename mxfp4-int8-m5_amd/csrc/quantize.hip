@@ -132,8 +132,24 @@ __device__ __forceinline__ float fp4_sq_err(const float (&x)[BLOCK], float scale
     return r0 + r1;
 }
 
-// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: vector ALU, 95 % busy with 39 instructions per weight
-// and 2.6 waves a SIMD.  12288 x 2048 bf16: 28.8 us (2.2 TB/s); 44 us with the near ties summed by one lane of the wave, 234 us
+// Eight weights' codes at a power-of-two scale, signs included: a word of the packed layout.
+__device__ __forceinline__ uint32_t fp4_word(const float* x, float scale) {
+    uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[0], x[1], scale, 0);
+    c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, x[2], x[3], scale, 1);
+    c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, x[4], x[5], scale, 2);
+    return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, x[6], x[7], scale, 3);
+}
+// A zero code has no sign.
+__device__ __forceinline__ uint32_t unsigned_zeros(uint32_t c) {
+    const uint32_t m = c & 0x77777777u;
+    return m | (c & (m + 0x77777777u) & 0x88888888u);
+}
+
+// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: vector ALU: three trial roundings with their error sums.
+// The codes come from the conversion, which takes a midpoint to the even code where the host takes the lower one.  bf16 weights have
+// eight bits: 2^-12 smaller, one on a midpoint lies below it and no other changes sides.  float32 weights are converted as they are and
+// 2^-23 smaller: where both agree so does the host (a midpoint whose even code is the lower one, or none near); the others' blocks
+// take the arithmetic.  12288 x 2048 bf16: 22.2 us; 28.8 with that arithmetic for every weight, 44 with the near ties summed by one lane of the wave, 234 us
 // with a lane per weight and every candidate in float64 across lanes.
 template <int BLOCK, bool BF16>
 __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
@@ -242,19 +258,37 @@ __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict
         const size_t at = base + size_t(b) * BLOCK;
         if (total > QNT) load_block<BLOCK, BF16>(w, at, vec, v);   // more than one block per thread: read them again
         const int e = max(s_e[b], s_floor[b / nb]);
-        uint32_t c[BLOCK / 8];
+        uint32_t c[BLOCK / 8], open = 1u;
+        if (e > -100 && e < 120) {   // (its scale is an ordinary float32)
+            const float scale = __uint_as_float(uint32_t(127 + e) << 23);
+            float y[BLOCK], sum = 0.0f;
 #pragma unroll
-        for (int i = 0; i < BLOCK / 8; ++i) c[i] = 0u;
+            for (int i = 0; i < BLOCK; ++i) {
+                y[i] = v[i] * (BF16 ? 1.0f - 0x1p-12f : 1.0f - 0x1p-23f);
+                sum += y[i];
+            }
+            open = uint32_t(!(fabsf(sum) < 3e38f));   // infinities and NaN
 #pragma unroll
-        for (int i = 0; i < BLOCK; ++i) {
-            // index of the E2M1 level nearest to a = |w| 2^-e, saturating at 7, a midpoint to the lower level
-            // (sim/mx_int8.py:23-25): levels are t / 2 apart from t = 2^max(floor(log2 a), 0) on, so the index is
-            // ceil(2 a / t - 1/2) plus two per octave above the first
-            const float a = fabsf(__builtin_amdgcn_ldexpf(v[i], -e));
-            const uint32_t t = max(__float_as_uint(a) & 0x7F800000u, 0x3F800000u);
-            const float m = ceilf(__builtin_fmaf(a, __uint_as_float(0x7F800000u - t), -0.5f));
-            const int idx = min(int(m) + 2 * (int(t >> 23) - 127), 7);
-            c[i >> 3] |= (uint32_t(idx) | ((v[i] < 0.0f && idx > 0) ? 8u : 0u)) << (4 * (i & 7));
+            for (int q = 0; q < BLOCK / 8; ++q) {
+                c[q] = fp4_word(y + 8 * q, scale);
+                if (!BF16) open |= c[q] ^ fp4_word(v + 8 * q, scale);
+                c[q] = unsigned_zeros(c[q]);
+            }
+        }
+        if (open) {
+#pragma unroll
+            for (int i = 0; i < BLOCK / 8; ++i) c[i] = 0u;
+#pragma unroll
+            for (int i = 0; i < BLOCK; ++i) {
+                // index of the E2M1 level nearest to a = |w| 2^-e, saturating at 7, a midpoint to the lower level
+                // (sim/mx_int8.py:23-25): levels are t / 2 apart from t = 2^max(floor(log2 a), 0) on, so the index is
+                // ceil(2 a / t - 1/2) plus two per octave above the first
+                const float a = fabsf(__builtin_amdgcn_ldexpf(v[i], -e));
+                const uint32_t t = max(__float_as_uint(a) & 0x7F800000u, 0x3F800000u);
+                const float m = ceilf(__builtin_fmaf(a, __uint_as_float(0x7F800000u - t), -0.5f));
+                const int idx = min(int(m) + 2 * (int(t >> 23) - 127), 7);
+                c[i >> 3] |= (uint32_t(idx) | ((v[i] < 0.0f && idx > 0) ? 8u : 0u)) << (4 * (i & 7));
+            }
         }
         store_codes<BLOCK>(codes + at / 8, vec, c);
     }
@@ -602,16 +636,15 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
 #pragma unroll
             for (int q = 0; q < BLOCK / 8; ++q) {
                 const float* x = v + 8 * q;
-                auto code = [&](float g) {
-                    uint32_t o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[0] * g, x[1] * g, 1.0f, 0);
-                    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, x[2] * g, x[3] * g, 1.0f, 1);
-                    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, x[4] * g, x[5] * g, 1.0f, 2);
-                    return uint32_t(__builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, x[6] * g, x[7] * g, 1.0f, 3));
-                };
-                const uint32_t o = code(dn);
-                open |= o ^ code(up);
-                const uint32_t m = o & 0x77777777u;
-                c[q] = m | (o & (m + 0x77777777u) & 0x88888888u);   // a zero has no sign
+                float below[8], above[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    below[i] = x[i] * dn;
+                    above[i] = x[i] * up;
+                }
+                c[q] = fp4_word(below, 1.0f);
+                open |= c[q] ^ fp4_word(above, 1.0f);
+                c[q] = unsigned_zeros(c[q]);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) open |= uint32_t(!(fabsf(x[i]) < 3e38f));   // infinities and NaN
             }
