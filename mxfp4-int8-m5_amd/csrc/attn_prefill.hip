@@ -60,7 +60,7 @@ __global__ __launch_bounds__(FA_NT) void attn_prefill_kernel(const uint16_t* __r
                                                              int L, int off, int hq, int hk, int rows, float scale_log2,
                                                              int range, float* __restrict__ part) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[2][2][FA_KBYTES + FA_VBYTES];   // [buffer][tile of the pair]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, h = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, h = lane >> 5;
     const int num_qt = (L + FA_BM - 1) / FA_BM;
     const int qt = num_qt - 1 - int(blockIdx.x / unsigned(hq)), turn = int(blockIdx.x % unsigned(hq));
     const int head = hq % XCDS ? turn : turn % XCDS * (hq / XCDS) + turn / XCDS, kvh = head / (hq / hk);
@@ -129,11 +129,24 @@ __global__ __launch_bounds__(FA_NT) void attn_prefill_kernel(const uint16_t* __r
         }
     };
 
+    // The queries are requested before any key and stay before them: loaded behind the first pair's, their wait inside the loop (of which
+    // this code is one predecessor) covered the loads of the pair after the next in every step.
+    __builtin_amdgcn_sched_barrier(0);
     load_pair(first);
+    __builtin_amdgcn_sched_barrier(0);
     store_pair(first & 1);
     if (first + 1 < npair) load_pair(first + 1);
     __syncthreads();
+    auto stage_next = [&](int i) {
+        if (i + 1 < npair) {   // the other buffer was last read one barrier ago
+            store_pair((i + 1) & 1);
+            if (i + 2 < npair) load_pair(i + 2);   // the registers are free again
+        }
+    };
     for (int i = first; i < npair; ++i) {
+        // The two waves of a SIMD (same queries, the two key halves) stage at opposite ends of the step, so that one's softmax
+        // runs beside the other's matrix products.
+        if (kh == 1) stage_next(i);
         const int t = 2 * i + kh;
         const int kv0 = t * FA_BN;
         if (kv0 <= off + qw0 + 31) {   // some key of the tile is visible to some query of this wave
@@ -202,10 +215,7 @@ __global__ __launch_bounds__(FA_NT) void attn_prefill_kernel(const uint16_t* __r
                     o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pb[s], o[db], 0, 0, 0);
                 }
         }
-        if (i + 1 < npair) {   // the other buffer was last read one barrier ago
-            store_pair((i + 1) & 1);
-            if (i + 2 < npair) load_pair(i + 2);   // the registers are free again
-        }
+        if (kh == 0) stage_next(i);
         __syncthreads();
     }
 
