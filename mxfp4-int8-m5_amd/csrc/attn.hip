@@ -13,7 +13,7 @@
 namespace scmx {
 
 constexpr int ANT = 512;
-constexpr int ATTN_SINGLE_MAX = 512;   // rows up to which a split launch falls back to one workgroup per head
+constexpr int ATTN_SINGLE_MAX = 128;   // rows up to which a split launch falls back to one workgroup per head: one turn of its loads
 
 // What the fused variant needs besides the attention operands: the token's q|k|v row as the qkv projection wrote it,
 // the per-head norm weights and the rotary frequencies.
@@ -56,7 +56,8 @@ __global__ __launch_bounds__(ANT) void attn_decode_kernel(const uint16_t* __rest
 
     // gridDim.y > 1: the valid rows are cut into gridDim.y equal ranges, one per workgroup of a head; every workgroup
     // leaves its unnormalised result, maximum and sum in `partial` and a second kernel merges them.
-    // A context of at most ATTN_SINGLE_MAX rows is read fastest by one workgroup per head: range 0 then takes all of
+    // A context of at most ATTN_SINGLE_MAX rows is read fastest by one workgroup per head (16 heads of a long cache, us, single /
+    // 16 ranges with the merge: 120 rows 6.9 / 7.4, 160 8.1 / 7.3, 300 9.5 / 7.5, 500 11.0 / 7.5): range 0 then takes all of
     // it and writes the output, the other workgroups leave at once and the merge kernel finds nothing to do.
     const bool single = gridDim.y == 1 || n <= ATTN_SINGLE_MAX;
     if (single && blockIdx.y > 0) return;
@@ -193,20 +194,43 @@ __global__ __launch_bounds__(ANT) void attn_decode_kernel(const uint16_t* __rest
 }
 
 // Merge of the per-range results of one head: out = sum_s w_s num_s / sum_s w_s den_s with w_s = exp(m_s - max m).
+// Bound: one trip to memory behind a launch.  All of up to 16 ranges is requested at once, and before the position is known: 16 heads, 3000 rows, 16 ranges, attention
+// and merge 13.9 -> 11.8 us, 12000 rows 29.5 -> 22.4 (range after range before).
 template <int D>
 __global__ __launch_bounds__(D) void attn_merge_kernel(const float* __restrict__ partial, uint16_t* __restrict__ out,
                                                      int splits, const int64_t* __restrict__ pos_dev, int n0, int rows) {
-    const int64_t n64 = pos_dev ? pos_dev[0] + 1 : int64_t(n0);
-    if (n64 <= ATTN_SINGLE_MAX || n64 > rows) return;   // range 0 wrote the output itself (zeros for a position outside the cache)
+    constexpr int AT_ONCE = 16;
     const int head = blockIdx.x, e = threadIdx.x;
     const float* pw = partial + size_t(head) * splits * (D + 2);
-    float mx = -3.0e38f;
-    for (int s = 0; s < splits; ++s) mx = fmaxf(mx, pw[s * (D + 2) + D]);
-    float num = 0.0f, den = 0.0f;
-    for (int s = 0; s < splits; ++s) {
-        const float w = __expf(pw[s * (D + 2) + D] - mx);
-        num += w * pw[s * (D + 2) + e];
-        den += w * pw[s * (D + 2) + D + 1];
+    float pm[AT_ONCE], pd[AT_ONCE], pn[AT_ONCE];
+    auto load = [&](int s0) {
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+            const float* p = pw + min(s0 + u, splits - 1) * (D + 2);
+            pm[u] = p[D];
+            pd[u] = p[D + 1];
+            pn[u] = p[e];
+        }
+    };
+    load(0);
+    const int64_t n64 = pos_dev ? pos_dev[0] + 1 : int64_t(n0);
+    if (n64 <= ATTN_SINGLE_MAX || n64 > rows) return;   // range 0 wrote the output itself (zeros for a position outside the cache)
+    float mx = -3.0e38f, num = 0.0f, den = 0.0f;
+    for (int s0 = 0; s0 < splits; s0 += AT_ONCE) {
+        if (s0 > 0) load(s0);
+        float m = mx;
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) m = fmaxf(m, pm[u]);
+        const float old = __expf(mx - m);
+        num *= old;
+        den *= old;
+        mx = m;
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+            const float w = s0 + u < splits ? __expf(pm[u] - mx) : 0.0f;
+            num += w * pn[u];
+            den += w * pd[u];
+        }
     }
     out[size_t(head) * D + e] = f32_to_bf16(num / den);
 }

@@ -338,12 +338,19 @@ def qkv_headnorm_rope(y, qn, kn, eps, L, hq, hk, d, kcache, vcache, pos, inv_fre
 
 
 def attn_splits(rows):
-    """Row ranges for the decode attention over up to `rows` cache rows: one workgroup per head reads a short context
-    fastest, longer ones are cut into 8 ranges, beyond 8192 rows into 16 (measured: 8.6 / 10.2 / 16.3 / 34 us at
-    1024 / 2048 / 4096 / 16000 rows against 23 / 43 / 86 / 354 us unsplit).  A split launch still serves contexts of
-    up to 512 rows with one workgroup per head (decided on the device), so a graph captured for a long cache does not
-    pay for the split while the context is short."""
+    """Row ranges for the decode attention over up to `rows` cache rows and many heads (more than 32): one workgroup per head
+    reads a short context fastest, longer ones are cut into 8 ranges, beyond 8192 rows into 16.  A split launch still serves
+    contexts of up to 128 rows with one workgroup per head (decided on the device)."""
     return 1 if rows <= 1024 else 8 if rows <= 8192 else 16
+
+
+def _decode_ranges(rows, hq):
+    """The same for any number of heads.  16 heads, us with 1 / 8 / 16 ranges: 513 rows 10.5 / 7.6 / 7.8, 1000 15.5 / 8.4 / 8.1, 1500
+    22.2 / 10.5 / 9.6, 3000 - / 12.7 / 11.8, 6000 - / 18.2 / 15.8, 12000 - / 27.2 / 22.4 (32 ranges 22.9); up to 512 rows the second
+    launch costs a host-bound loop more than it gives (300 rows 8.1 / 7.4 / 7.5)."""
+    if hq > 32:
+        return attn_splits(rows)
+    return 1 if rows <= 512 else 16
 
 
 def _split_workspace(splits, hq, d, like):
@@ -359,7 +366,7 @@ def attn_decode(q, kcache, vcache, n, scale=None, splits=None):
     out = _lib.native().empty_bf16(q, 1, hq * d)
     dev_pos = n if torch.is_tensor(n) else None
     if splits is None:
-        splits = attn_splits(rows if dev_pos is not None else int(n))
+        splits = _decode_ranges(rows if dev_pos is not None else int(n), hq)
     work = _split_workspace(splits, hq, d, q)
     _lib.native().scmx_attn_decode(q, kcache, vcache, dev_pos, 0 if dev_pos is not None else int(n), out, hq, hk, d, rows,
                                    float(scale if scale is not None else d ** -0.5), work, splits)
@@ -411,7 +418,7 @@ def attn_decode_qkv(y, qn, kn, eps, hq, hk, d, kcache, vcache, pos, inv_freq, sc
     dev_pos = pos if torch.is_tensor(pos) else None
     assert dev_pos is None or dev_pos.dtype == torch.int64
     if splits is None:
-        splits = attn_splits(kcache.shape[1] if dev_pos is not None else int(pos) + 1)
+        splits = _decode_ranges(kcache.shape[1] if dev_pos is not None else int(pos) + 1, hq)
     work = _split_workspace(splits, hq, d, y)
     _lib.native().scmx_attn_decode_qkv(y, qn, kn, _eps(eps), inv_freq, dev_pos, 0 if dev_pos is not None else int(pos),
                                        kcache, vcache, out, hq, hk, d, kcache.shape[1],
