@@ -277,6 +277,11 @@ int scmx_gemv_rows(const scmx_format* fmt, const void* x, const float* xscale, c
 int scmx_route_topk(const uint16_t* logits, const uint16_t* shared_logit, int M, int n_experts, int topk, int renorm,
                     int32_t* inds, uint16_t* scores, void* stream);
 
+/* One decode row: scmx_rmsnorm_quant with its bf16 row xn, and scmx_linear_bf16 of that row with a small matrix `mat` [N, K] (a router)
+ * -> out [N], in one launch, bit for bit.  K 512, 1024, 1536 or 2048, N up to 4096, operands 16-byte aligned. */
+int scmx_norm_linear(const uint16_t* x, const uint16_t* w, float eps, const uint16_t* mat, int K, int N, int8_t* xq, float* xs,
+                     uint16_t* xn, uint16_t* out, void* stream);
+
 /* Counting sort of the M*topk token-expert assignments by expert: pos [R], tok [R+tm], esorted [R], off [E+1],
  * tstart [E+1] (tile starts for row tiles of tm).  Replaces route_sort, e2e/sc_moe.py:114-155. */
 int scmx_route_sort(const int32_t* inds, int M, int topk, int n_experts, int tm, int32_t* pos, int32_t* tok,

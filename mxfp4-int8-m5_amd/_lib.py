@@ -57,6 +57,7 @@ SIGNATURES = {
     "scmx_gemv_rows_workspace": (_Z, [_FMT, _I, _I, _I, _I]),
     "scmx_gemv_rows": (_I, [_FMT, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _F, _I, _I, _I, _P, _Z, _P]),
     "scmx_route_topk": (_I, [_P, _P, _I, _I, _I, _I, _P, _P, _P]),
+    "scmx_norm_linear": (_I, [_P, _P, _F, _P, _I, _I, _P, _P, _P, _P, _P]),
     "scmx_route_sort": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P]),
     "scmx_moe_mm": (_I, [_FMT, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P]),
     "scmx_moe_mm_i8": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P]),

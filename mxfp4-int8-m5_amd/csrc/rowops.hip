@@ -1041,6 +1041,87 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const uint16_t* __restri
     }
 }
 
+// ---- one decode row: RMSNorm, its INT8 codes and a small bf16 linear (the router) on it, one launch ---------------------
+// What rmsnorm_quant with its bf16 row and linear_bf16 give, bit for bit (the same device functions, the same products by the same waves,
+// summed in the same order).  A workgroup per 16 rows of the matrix, whose loads are all requested before the norm, which
+// every workgroup takes for itself.  Bound: launch and two trips to memory; 64 x 2048 with the routing behind it 7.35 us against
+// 11.3 for three launches.  (With the
+// routing in it as well, in one workgroup, 256 KB came through one CU: 11.1 us, no less than three launches.)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+template <int CH>
+__global__ __launch_bounds__(512) void norm_linear_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, float eps,
+                                                          const uint16_t* __restrict__ mat, int N, int8_t* __restrict__ xq,
+                                                          float* __restrict__ xs, uint16_t* __restrict__ xn, uint16_t* __restrict__ out) {
+    constexpr int K = 512 * CH;
+    __shared__ u32x4 srow[K / 8];   // the normalised row
+    __shared__ f32x4 part[8][4];    // [wave][group of 4 matrix rows]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), r = lane & 15, g = lane >> 4;
+    const int n0 = int(blockIdx.x) * 16;
+    u32x4 v[CH], nw[CH], wv[2 * CH];
+    if (wave == 0) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) v[j] = reinterpret_cast<const u32x4*>(x)[lane + 64 * j];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) nw[j] = reinterpret_cast<const u32x4*>(w)[lane + 64 * j];
+    }
+    {   // wave w takes the chunks w, w + 8, ... of 64 columns
+        const uint16_t* row = mat + size_t(min(n0 + r, N - 1)) * K + wave * 64 + 8 * g;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            wv[2 * i] = *reinterpret_cast<const u32x4*>(row + i * 512);
+            wv[2 * i + 1] = *reinterpret_cast<const u32x4*>(row + i * 512 + 32);
+        }
+    }
+    if (wave == 0) {
+        const float inv = inv_rms(wave_row_sumsq(v), K, eps);
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            v[j] = norm8(v[j], nw[j], inv);
+            srow[lane + 64 * j] = v[j];
+        }
+    }
+    __syncthreads();
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[2 * i + s]),
+                                                          __builtin_bit_cast(bf16x8, srow[i * 64 + wave * 8 + 4 * s + g]), acc, 0, 0, 0);
+    if (r == 0) part[wave][g] = acc;
+    __syncthreads();
+    if (threadIdx.x >= 448) {   // the last wave: the others' sums
+        if (lane < 16 && n0 + lane < N) {
+            float s = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += part[u][lane >> 2][lane & 3];
+            out[n0 + lane] = f32_to_bf16(s);
+        }
+    } else if (wave == 0 && blockIdx.x == 0) {
+        float amax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            reinterpret_cast<u32x4*>(xn)[lane + 64 * j] = v[j];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                amax = fmaxf(amax, fmaxf(fabsf(__uint_as_float(v[j][e] << 16)), fabsf(__uint_as_float(v[j][e] & 0xFFFF0000u))));
+        }
+        amax = wave_max(amax);
+        const float s = __fdiv_rn(amax, 127.0f), qi = s > 0.0f ? __fdiv_rn(1.0f, s) : 0.0f;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            u32x2 o = {0u, 0u};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t u = v[j][e >> 1];
+                o[e >> 2] |= (uint32_t(quant_code(__uint_as_float(e & 1 ? (u & 0xFFFF0000u) : (u << 16)), qi)) & 0xFFu) << (8 * (e & 3));
+            }
+            reinterpret_cast<u32x2*>(xq)[lane + 64 * j] = o;
+        }
+        if (lane == 0) *xs = s;
+    }
+}
+
 }  // namespace scmx
 
 using namespace scmx;
@@ -1267,6 +1348,27 @@ int scmx_route_topk(const uint16_t* logits, const uint16_t* shared_logit, int M,
     else if (n_experts <= 512) launch(std::integral_constant<int, 8>{});
     else launch(std::integral_constant<int, 16>{});
     return check_launch("route_topk");
+}
+
+int scmx_norm_linear(const uint16_t* x, const uint16_t* w, float eps, const uint16_t* mat, int K, int N, int8_t* xq, float* xs,
+                     uint16_t* xn, uint16_t* out, void* stream) {
+    if (!x || !w || !mat || !xq || !xs || !xn || !out || (uintptr_t(x) | uintptr_t(w) | uintptr_t(mat) | uintptr_t(xn) | uintptr_t(xq)) % 16) {
+        set_error("norm_linear: null pointer, or x, w, mat, xq or xn not 16-byte aligned");
+        return SCMX_ERR_ARG;
+    }
+    if (K < 512 || K > 2048 || K % 512 || N < 1 || N > 4096) {
+        set_error("norm_linear: need K of 512, 1024, 1536 or 2048 (%d) and N (%d) in 1..4096", K, N);
+        return SCMX_ERR_ARG;
+    }
+    const auto go = [&](auto ch) {
+        norm_linear_kernel<decltype(ch)::value>
+            <<<dim3((unsigned(N) + 15u) / 16u), dim3(512), 0, (hipStream_t)stream>>>(x, w, eps, mat, N, xq, xs, xn, out);
+    };
+    if (K == 512) go(std::integral_constant<int, 1>{});
+    else if (K == 1024) go(std::integral_constant<int, 2>{});
+    else if (K == 1536) go(std::integral_constant<int, 3>{});
+    else go(std::integral_constant<int, 4>{});
+    return check_launch("norm_linear");
 }
 
 int scmx_route_sort(const int32_t* inds, int M, int topk, int n_experts, int tm, int32_t* pos, int32_t* tok,

@@ -214,6 +214,7 @@ class DecodeOlmoe:
         H, d, D, k = a.num_attention_heads, a.head_dim, a.hidden_size, a.num_experts_per_tok
         F2 = 2 * a.intermediate_size
         fp = self.fuse is True
+        own_route = getattr(f.route, "__func__", None) is FusedOlmoe.route   # (a caller's own routing is asked)
         h = f.embed[tok.reshape(-1)[:1]].contiguous()
         for i, (nw, ws, ex) in enumerate(f.layers):
             w = ws["qkv"]
@@ -230,8 +231,11 @@ class DecodeOlmoe:
             else:
                 xq, xs = S.act_quant(o, 1)
                 h = G.gemv(xq, wo.codes, wo.bcodes, xs, wo.wscale, D, 2, res=h, fmt=f.fmt)[None]
-            xq, xs, xn = S.rmsnorm_quant_n(h, nw["post_attention_layernorm"], f.eps, 1)
-            inds, scores = f.route(nw, xn, 1)
+            routed = sc_moe.norm_route(h, nw["post_attention_layernorm"], f.eps, nw["mlp.gate"], k, a.norm_topk_prob) if own_route else None
+            if routed is None:
+                xq, xs, xn = S.rmsnorm_quant_n(h, nw["post_attention_layernorm"], f.eps, 1)
+                routed = (xq, xs, xn, *f.route(nw, xn, 1))
+            xq, xs, _, inds, scores = routed
             e = inds.reshape(-1)
             cg, bg, sg = ex["gu"]
             cd, bd, sd = ex["down"]

@@ -30,6 +30,20 @@ def route(logits, k, renorm=True, shared_logit=None):
     return inds, scores
 
 
+def norm_route(x, w, eps, gate, k, renorm=True):
+    """rmsnorm_quant_n, linear_bf16 and route of one row, the first two in one launch: x bf16 [1, D], norm weight w [D], router gate
+    [E, D] -> (xq, xscale, xn, inds, scores) with the same bits.  None where that kernel does not take the shapes (D of 512 ... 2048) or
+    tensors that linear_bf16 would leave to the array op."""
+    D, E = x.shape[1], gate.shape[0]
+    if not (x.shape[0] == 1 and D % 512 == 0 and 512 <= D <= 2048 and 0 < k <= E <= 1024 and gate.shape[1] == D and tuple(w.shape) == (D,)
+            and S._plain(x, gate) and S._plain(x, w) and not (x.data_ptr() | w.data_ptr() | gate.data_ptr()) % 16):
+        return None
+    n = _lib.native()
+    xq, xs, xn, logits = n.empty_i8(x, 1, D), n.empty_f32(x, 1), n.empty_bf16(x, 1, D), n.empty_bf16(x, 1, E)
+    n.scmx_norm_linear(x, w, S._eps(eps), gate, D, E, xq, xs, xn, logits)
+    return xq, xs, xn, *route(logits, k, renorm)
+
+
 def route_sort(inds, n_experts, tm):
     """inds int [M, topk] -> (pos [R], tok [R + tm], e_sorted [R], off [E+1], tstart [E+1], max M-tiles)."""
     M, k = inds.shape
