@@ -4,8 +4,9 @@
 // workgroup stages BM x BK activation bytes and BN x BK weight bytes in LDS; the weight bytes are produced in
 // registers from the packed 4-bit codes (16 bytes of codes = one run of 32 weights per thread) right before they
 // are written to LDS, so the INT8 form of the weights exists only there.  Waves then read 16-byte operand
-// fragments and issue v_mfma_i32_16x16x64_i8 with the weights as the row operand: each lane ends up with groups
-// of 4 consecutive output columns n of one token row m, which is the unit every epilogue works on.
+// fragments and issue v_mfma_i32_16x16x64_i8 (MF = 16) or v_mfma_i32_32x32x32_i8 (MF = 32) with the weights as the row
+// operand: each lane ends up with groups of 4 consecutive output columns n of one token row m, which is the unit every
+// epilogue works on.
 // LDS holds three stages of the K loop; global loads run four steps ahead in two register sets, and the decode and
 // LDS writes of step i+2 are issued between the MFMAs of step i, with one barrier per step.
 #include <atomic>
@@ -15,10 +16,12 @@
 
 namespace scmx {
 
-// The 16x16x64 form of the instruction and not 32x32x32: the chip runs these kernels at its power limit (all-zero operands
-// run a third faster), and at that limit, on INT8 operands as they occur, a loop of MFMAs alone reaches 4420 TOP/s with
-// 16x16x64 and 3740 with 32x32x32 (half the accumulator traffic per multiply-add).  gate|up of 12288 x 2048 at 8192 rows, same
-// tile: 208 -> 199 us; the four layers of a 2048-wide model at 2048 rows 118 -> 108 with the tiles chosen below.
+// MF, the shape of the MFMA.  At the chip's power limit (all-zero operands run a third faster) and on INT8 operands as they
+// occur, a loop of MFMAs alone reaches 4420 TOP/s with 16x16x64 and 3740 with 32x32x32 (half the accumulator traffic per
+// multiply-add): gate|up of 12288 x 2048 at 8192 rows, same tile, 208 us with the latter and 199 with the former.  A launch
+// bound elsewhere is far from that limit, and 32x32x32 takes half the instructions: the packed tile (bound by the vector ALU
+// that decodes its weights) uses it, 16-block power-of-two format, 64 experts of 2048 x 2048 / 257 of 1024 x 2048, 70 rows
+// each: 50.2 -> 47.7 and 109 -> 104 us.
 //
 // FD = number of register buffers of the split operand's fragments: fetched FD - 1 phases (half k slices) ahead of their MFMAs.
 // SKIP (grouped launches): a row tile that ends inside its expert's segment multiplies only the 16-row blocks that hold
@@ -35,14 +38,16 @@ namespace scmx {
 // the blocked layout, sixteen of 64 from rows.  Waves must then not share rows (WGN = 1, or few column groups), and only the
 // weight rows of a stage exist in LDS.
 template <int BM, int BN, int BK, int WGM, int WGN, int BMODE, int OCC = 1, int FD = 2, bool SKIP = false, bool PK = false,
-          int KG = 1, int ADM = 0>
+          int KG = 1, int ADM = 0, int MF = 16>
 __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const GemmArgs a) {
     constexpr bool AD = ADM != 0, ADR = ADM == 2;   // activation fragments straight from memory; from the row layout
     constexpr int NSTAGE = 3;   // LDS stages: one being read, one ready, one being written
     constexpr int NT = WGM * WGN * 64;   // threads of one K group
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
-    constexpr int MI = WTM / 16, NI = WTN / 16;   // 16-row / 16-column blocks of a wave's tile
-    static_assert(WTM % 32 == 0 && WTN % 32 == 0 && (BK == 64 || BK == 128), "tile must be whole pairs of 16x16x64 MFMAs");
+    constexpr int MI = WTM / MF, NI = WTN / MF;   // MF-row / MF-column blocks of a wave's tile
+    constexpr int ACC16 = WTM * WTN / 256;        // its accumulators, in 16 x 16 blocks
+    static_assert(WTM % 32 == 0 && WTN % 32 == 0 && (BK == 64 || BK == 128), "tile must be whole 32x32 blocks");
+    static_assert(MF == (PK ? 32 : 16), "packed tiles multiply with 32x32x32, the others with 16x16x64");
     constexpr int CPR = BK / 16;             // 16-byte chunks per LDS row
     constexpr int RPB = 256 / BK;            // rows per 256 bytes, i.e. per sweep of the 64 LDS banks
     constexpr int A_CHUNKS = AD ? 0 : BM * CPR;   // 16-byte pieces of the activation tile
@@ -56,7 +61,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // PK: block-code bytes per weight row and K step
     constexpr int BCB = BMODE == B_PACKED_B16M || BMODE == B_PACKED_E8M0 ? 4 : BMODE == B_PACKED_B16 ? 2 : 1;
     constexpr int BCR = BCB == 4 ? 2 : 1;   // registers for those of two steps
-    static_assert(!PK || (BK == 128 && WPC == 4 && BMODE != B_INT8 && BMODE != B_PACKED_GENERIC),
+    static_assert(!PK || (BK == 128 && WPC == 4 && !SKIP && BMODE != B_INT8 && BMODE != B_PACKED_GENERIC),
                   "packed weights in LDS: K steps of 128, 16-byte runs, FP4-conversion formats");
     // bytes per stage: BM activation rows, then BN weight rows (PK: 64 code bytes each)
     constexpr int STAGE = A_BYTES + (PK ? BN * (BK / 2) : BN * BK);
@@ -71,7 +76,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     static_assert(!AD || (!PK && KG == 1), "activation fragments from memory: staged tiles");
     constexpr int GROUP_BYTES = NSTAGE * STAGE;
     // after the K loop: group 0's output tiles (the widest epilogue's) from 0, then the other groups' partial sums
-    constexpr int PART_BYTES = NT * MI * NI * 16;
+    constexpr int PART_BYTES = NT * ACC16 * 16;
     constexpr int PART_BASE = WGM * WGN * WTM * (WTN * 4 + 16);
     constexpr int KG_BYTES = PART_BASE + (KG - 1) * PART_BYTES > KG * GROUP_BYTES ? PART_BASE + (KG - 1) * PART_BYTES : KG * GROUP_BYTES;
     static_assert(KG == 1 || KG_BYTES <= 160 * 1024, "stages and partial sums fit the CU's LDS");
@@ -132,9 +137,9 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     const int K = a.K;
     const int KL = K / KG;         // length of this group's part of the reduction
     const int kbase = kg * KL;     // and its first k (a multiple of 128)
-    // 16-row blocks of this wave's tile that hold rows of the segment (wave-uniform)
+    // MF-row blocks of this wave's tile that hold rows of the segment (wave-uniform)
     const int mi_active =
-        SKIP ? __builtin_amdgcn_readfirstlane(min(MI, max(0, (row_end - (m0 + wm * WTM) + 15) / 16))) : MI;
+        SKIP ? __builtin_amdgcn_readfirstlane(min(MI, max(0, (row_end - (m0 + wm * WTM) + MF - 1) / MF))) : MI;
     // The tile's scales are REQUESTED here, before the first operand loads, and stored to LDS after those have been
     // issued: memory returns a wave's loads in order, so scales requested first arrive first and their wait does not
     // cover the operand loads (fetched and stored up front they cost every tile two serial round trips to memory).
@@ -321,20 +326,23 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int q = 0; q < NKK; ++q) stage_slice(r, sm + stage * STAGE, k0, q, o);
     };
 
-    v4i acc[MI][NI];
+    constexpr int AG = MF == 32 ? 4 : 1;   // groups of four columns of a row that a lane holds of a block
+    std::conditional_t<MF == 32, v16i, v4i> acc[MI][NI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+            for (int r = 0; r < 4 * AG; ++r) acc[i][j][r] = 0;
 
-    // fragment addresses: lane l supplies row l % 16 and the 16 k-bytes of quarter l / 16 of a 64-wide k slice; block
-    // origins are multiples of 16 rows, so the swizzle term depends on the lane only
-    constexpr int KS = BK / 64;   // k slices of a step
-    const int lr = lane & 15, quad = lane >> 4;
+    // fragment addresses: lane l supplies row l % MF and the 16 k-bytes of part l / MF of a k slice (64 wide in four parts, or
+    // 32 in two); block origins are multiples of MF rows, so the swizzle term depends on the lane only
+    constexpr int PARTS = 64 / MF, KS = BK / (16 * PARTS);   // k slices of a step
+    const int lr = lane % MF, part = lane / MF;
     const int sw = (lr / RPB) & (CPR - 1);
     int koff[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) koff[s] = ((4 * s + quad) ^ sw) << 4;
+    for (int s = 0; s < KS; ++s) koff[s] = ((PARTS * s + part) ^ sw) << 4;
     const int a_frag = (wm * WTM + lr) * BK;
     const int b_frag = A_BYTES + (wn * WTN + lr) * BK;
 
@@ -350,7 +358,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     [[maybe_unused]] uint32_t bcc[NI][BCR], bcn[NI][BCR];
     [[maybe_unused]] int bc_src[NI];
 #pragma unroll
-    for (int j = 0; j < NI; ++j) bc_src[j] = min(n0 + wn * WTN + j * 16 + lr, a.N - 1) * a.bc_row_bytes;
+    for (int j = 0; j < NI; ++j) bc_src[j] = min(n0 + wn * WTN + j * MF + lr, a.N - 1) * a.bc_row_bytes;
     // block codes of K steps s and s + 1 (s even); past the end the last pair of steps again (never consumed)
     auto load_bc = [&](int s, uint32_t (&f)[NI][BCR]) {
         const int so = min(s, (K / BK - 1) & ~1) * BCB;
@@ -369,28 +377,28 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     [[maybe_unused]] uint32_t w_rmin[NI];
     if constexpr (PK && BMODE == B_PACKED_E8M0) {
 #pragma unroll
-        for (int j = 0; j < NI; ++j) w_rmin[j] = e8m0_row_min(a.wscale[erow + min(n0 + wn * WTN + j * 16 + lr, a.N - 1)]);
+        for (int j = 0; j < NI; ++j) w_rmin[j] = e8m0_row_min(a.wscale[erow + min(n0 + wn * WTN + j * MF + lr, a.N - 1)]);
     }
     // AD: the activations come in 32-row x 32-k blocks of 1 KB, 16 bytes of a row per piece, piece (row % 32, k / 16 % 2) at
     // (k / 16 % 2) * 512 + (row % 32) * 16, block (m / 32, k / 32) at ((m / 32) * (K / 32) + k / 32) KB.  A fragment (16
     // rows x 64 k) is then four runs of 256 bytes.  Every wave loads the fragments of its own rows straight into registers,
     // two K steps ahead, in three buffers that rotate with the LDS stages: the activation tile never passes through LDS.
-    constexpr int NAB = MI * NI > 16 ? 2 : NSTAGE;   // the largest wave tiles have registers for two buffers only (below)
+    constexpr int NAB = MF == 16 && ACC16 > 16 ? 2 : NSTAGE;   // the largest wave tiles have registers for two buffers only (below)
     [[maybe_unused]] v4i fad[NAB][KS][MI];
-    [[maybe_unused]] int ad_src[ADR ? MI : MI / 2];
+    [[maybe_unused]] int ad_src[ADR ? MI : WTM / 32];
     if constexpr (ADR) {
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
             int gr = min(m0 + wm * WTM + i * 16 + lr, row_end - 1);
             if (a.gather) gr = a.gather[gr];
-            ad_src[i] = int(uint32_t(gr) * uint32_t(K) + uint32_t(quad) * 16u);
+            ad_src[i] = int(uint32_t(gr) * uint32_t(K) + uint32_t(part) * 16u);
         }
     } else if constexpr (AD) {
         const int last_block = (a.M + 31) / 32 - 1;
 #pragma unroll
-        for (int i = 0; i < MI / 2; ++i)
+        for (int i = 0; i < WTM / 32; ++i)
             ad_src[i] = int(uint32_t(min((m0 + wm * WTM) / 32 + i, last_block)) * uint32_t(K >> 5) * 1024u +
-                            uint32_t(quad) * 512u + uint32_t(lr) * 16u + uint32_t(kbase) * 32u);
+                            uint32_t(part) * 512u + uint32_t(lr) * 16u + uint32_t(kbase) * 32u);
     }
     auto load_ad = [&](int buf, int k0) __attribute__((always_inline)) {
 #pragma unroll
@@ -399,7 +407,8 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
             for (int i = 0; i < MI; ++i) {
                 if (SKIP && i >= mi_active) continue;
                 const u32x4 v = ADR ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR ? i : 0] + s * 64, k0, 0)
-                                    : __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR ? 0 : i / 2] + s * 2048 + (i & 1) * 256, k0 * 32, 0);
+                                : MF == 32 ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[MF == 32 ? i : 0] + s * 1024, k0 * 32, 0)
+                                    : __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR || MF == 32 ? 0 : i / 2] + s * 2048 + (i & 1) * 256, k0 * 32, 0);
                 fad[buf][s][i] = v4i{int(v[0]), int(v[1]), int(v[2]), int(v[3])};
             }
     };
@@ -428,50 +437,62 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     }
     load_global(r1, 3 * BK);
     // ---- PK: fragments of packed weights ------------------------------------------------------------------------
-    // A unit is one 64-wide k slice of one 16-column block: lane quarter q supplies k = 64 s + 16 q + (0..15) of a row, 8
-    // code bytes, which lie inside one block of 16 or 32 weights.  Three things are in flight per wave: the MFMAs of unit
-    // u, the decode of unit u + 1 (its codes were read during unit u - 1) and the LDS reads of the codes of unit u + 2 and
-    // of the next slice's activations.
+    // The k positions of a 64-wide pair of MFMA slices are dealt so that a lane's packed codes are one 16-byte read: lane
+    // half h supplies k = 64 p + 32 h + 16 s + (0..15) to slice s of pair p, i.e. 32 consecutive activation bytes (two
+    // 16-byte reads) and 32 consecutive codes (one), the latter one block of 32 or two of 16.
+    // Three things are in flight per wave: the MFMAs of pair p, the decode of pair p + 1 (its codes were read during pair
+    // p - 1) and the LDS reads of pair p + 1's activations and pair p + 2's codes.
     // The block codes do not pass through LDS: the lane that decodes row n reads the codes of two K steps of that row
     // (2 * BCB bytes) from memory every second step, two steps ahead.
-    constexpr int NU = KS * NI;          // units of a step
-    [[maybe_unused]] v4i pa[2][MI];      // activation fragments [slice parity][16-row block]
-    [[maybe_unused]] u32x2 pw[2];        // 16 codes of a weight row as read from LDS [unit parity]
-    [[maybe_unused]] v4i px[2];          // decoded INT8 operands [unit parity]
-    [[maybe_unused]] int koff_pw[KS];
-#pragma unroll
-    for (int s = 0; s < KS; ++s) koff_pw[s] = (((2 * s + (quad >> 1)) ^ ((lr >> 2) & 3)) << 4) + (quad & 1) * 8;
+    constexpr int NKP = NKK / 2, PMI = PK ? MI : 1, PNI = PK ? NI : 1;
+    [[maybe_unused]] v4i pa[2][2][PMI];   // activation fragments [pair parity][slice][row block]
+    [[maybe_unused]] v4i pw[2][PNI];      // 32 codes per weight row as read from LDS [pair parity]
+    [[maybe_unused]] v4i px[2][2][PNI];   // decoded INT8 operands [pair parity][slice][column block]
     [[maybe_unused]] const int w_frag = A_BYTES + (wn * WTN + lr) * (BK / 2);
-    auto load_pa = [&](const int8_t* src, int s, v4i (&f)[MI]) {
+    auto load_pa = [&](const int8_t* src, int kp, v4i (&f)[2][PMI]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-            if (!SKIP || (i & ~1) < mi_active) f[i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 16 * BK + koff[s]);
+        for (int i = 0; i < PMI; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                f[h][i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + (((4 * kp + 2 * part + h) ^ sw) << 4));
     };
-    auto load_pw = [&](const int8_t* src, int u, u32x2& f) {
-        f = *reinterpret_cast<const u32x2*>(src + w_frag + (u % NI) * 16 * (BK / 2) + koff_pw[u / NI]);
+    auto load_pw = [&](const int8_t* src, int kp, v4i (&f)[PNI]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < PNI; ++j)
+            f[j] = *reinterpret_cast<const v4i*>(src + w_frag + j * 32 * (BK / 2) + (((2 * kp + part) ^ ((lr >> 2) & 3)) << 4));
     };
-    // 16 codes -> the INT8 operand of unit u; `odd` = the K step's parity (which half of the block codes)
-    auto decode_unit = [&](const u32x2& f, const uint32_t (&bc)[NI][BCR], int odd, int u, v4i& x) {
-        const int s = u / NI, j = u % NI;
-        uint32_t o[4];
-        if constexpr (BMODE == B_PACKED_B16M) {   // block 4 s + q of the step's 8, 4 bits each
-            const uint32_t code = (bc[j][odd] >> (16 * s + 4 * quad)) & 15u;
-            const _Float16 m = _Float16(int(code + (a.fmt.mult[0] & 0xFFu)));
-            decode_word_fp4_mul(f[0], half2_t{m, m}, o[0], o[1]);
-            decode_word_fp4_mul(f[1], half2_t{m, m}, o[2], o[3]);
-        } else {
-            uint32_t shift;
-            if constexpr (BMODE == B_PACKED_B16)         // block 4 s + q of the step's 8
-                shift = (bc[j][0] >> (16 * odd + 8 * s + 2 * quad)) & 3u;
-            else if constexpr (BMODE == B_PACKED_E8M0)   // byte 2 s + q / 2 of the step's 4
-                shift = (((bc[j][odd] >> (16 * s + 8 * (quad >> 1))) & 0xFFu) - w_rmin[j]) & 0x7Fu;
-            else                                         // block 2 s + q / 2 of the step's 4
-                shift = (bc[j][0] >> (8 * odd + 4 * s + 2 * (quad >> 1))) & 3u;
-            const float sc = fp4_scale(shift);
-            decode_word_fp4(f[0], sc, o[0], o[1]);
-            decode_word_fp4(f[1], sc, o[2], o[3]);
+    // 32 codes -> the INT8 operands of the pair's two slices; `odd` = the K step's parity (which half of the block codes)
+    auto decode_pair = [&](const v4i (&f)[PNI], const uint32_t (&bc)[NI][BCR], int odd, int kp,
+                           v4i (&x)[2][PNI]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < PNI; ++j) {
+            uint32_t o[8];
+            if constexpr (BMODE == B_PACKED_B16M) {   // blocks 4 kp + 2 h and the next one of the step's 8, 4 bits each
+                const uint32_t t = bc[j][odd] >> (16 * kp + 8 * part);
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const _Float16 m = _Float16(int(((t >> (4 * (w >> 1))) & 15u) + (a.fmt.mult[0] & 0xFFu)));
+                    decode_word_fp4_mul(uint32_t(f[j][w]), half2_t{m, m}, o[2 * w], o[2 * w + 1]);
+                }
+            } else {
+                float s0, s1;
+                if constexpr (BMODE == B_PACKED_B16) {   // the same, 2 bits each
+                    const uint32_t t = bc[j][0] >> (16 * odd + 8 * kp + 4 * part);
+                    s0 = fp4_scale(t & 3u);
+                    s1 = fp4_scale((t >> 2) & 3u);
+                } else if constexpr (BMODE == B_PACKED_E8M0) {   // byte 2 kp + h of the step's 4
+                    s0 = s1 = fp4_scale((((bc[j][odd] >> (16 * kp + 8 * part)) & 0xFFu) - w_rmin[j]) & 0x7Fu);
+                } else {                                 // block 2 kp + h of the step's 4
+                    s0 = s1 = fp4_scale((bc[j][0] >> (8 * odd + 4 * kp + 2 * part)) & 3u);
+                }
+                decode_word_fp4(uint32_t(f[j][0]), s0, o[0], o[1]);
+                decode_word_fp4(uint32_t(f[j][1]), s0, o[2], o[3]);
+                decode_word_fp4(uint32_t(f[j][2]), s1, o[4], o[5]);
+                decode_word_fp4(uint32_t(f[j][3]), s1, o[6], o[7]);
+            }
+            x[0][j] = v4i{int(o[0]), int(o[1]), int(o[2]), int(o[3])};
+            x[1][j] = v4i{int(o[4]), int(o[5]), int(o[6]), int(o[7])};
         }
-        x = v4i{int(o[0]), int(o[1]), int(o[2]), int(o[3])};
     };
     auto iteration_pk = [&](auto step_tag, auto parity_tag, Staged& r, int kt) __attribute__((always_inline)) {
         constexpr int rd = decltype(step_tag)::value;
@@ -487,31 +508,30 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         uint32_t o[B_PER][8];
         if (!odd) load_bc(kt + 2, bcn);
 #pragma unroll
-        for (int u = 0; u < NU; ++u) {
-            const int cur = u % 2, oth = (u + 1) % 2, s = u / NI;   // NU and KS are even: unit 0 of every step has parity 0
-            if (u % NI == 0) load_pa(s + 1 < KS ? src : nxt, (s + 1) % KS, pa[(s + 1) % 2]);
-            if (u + 1 < NU) {
-                decode_unit(pw[oth], bcc, odd, u + 1, px[oth]);
-            } else {   // unit 0 of step kt + 1
-                if (odd) {
+        for (int kp = 0; kp < NKP; ++kp) {
+            const int cur = kp % 2, oth = (kp + 1) % 2;   // NKP is even: pair 0 of every step has parity 0
+            load_pa(kp + 1 < NKP ? src : nxt, (kp + 1) % NKP, pa[oth]);
+            if (kp + 1 == NKP && odd) {   // the next pair belongs to step kt + 1
 #pragma unroll
-                    for (int j = 0; j < NI; ++j)
+                for (int j = 0; j < NI; ++j)
 #pragma unroll
-                        for (int q = 0; q < BCR; ++q) bcc[j][q] = bcn[j][q];
-                }
-                decode_unit(pw[oth], bcc, 1 - odd, 0, px[oth]);
+                    for (int q = 0; q < BCR; ++q) bcc[j][q] = bcn[j][q];
             }
-            load_pw(u + 2 < NU ? src : nxt, (u + 2) % NU, pw[cur]);   // pw[cur] was decoded a unit ago
+            decode_pair(pw[oth], bcc, kp + 1 < NKP ? odd : 1 - odd, (kp + 1) % NKP, px[oth]);
+            load_pw(nxt, kp, pw[cur]);   // pair kp + 2 = pair kp of the next step; pw[cur] was decoded a pair ago
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                if (SKIP && (i & ~1) >= mi_active) continue;   // pairs of row blocks
-                acc[i][u % NI] = __builtin_amdgcn_mfma_i32_16x16x64_i8(px[cur], pa[s % 2][i], acc[i][u % NI], 0, 0, 0);
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int i = 0; i < PMI; ++i)
+#pragma unroll
+                    for (int j = 0; j < PNI; ++j)
+                        if constexpr (PK) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(px[cur][h][j], pa[cur][h][i], acc[i][j], 0, 0, 0);
+                stage_slice(r, dst, k2, 2 * kp + h, o);
             }
-            if (u < NKK) stage_slice(r, dst, k2, u, o);
         }
         load_global(r, k4);
     };
-    static_assert(!PK || (KS == 2 && NU % 2 == 0 && NU >= NKK), "the buffers return to phase 0 every K step");
+    static_assert(!PK || NKP == 2, "the pair buffers return to phase 0 every K step");
 
     // A step runs in phases, two per 64-wide k slice: the operand with more 16-row blocks in the wave's tile is split, one
     // half of its fragments per phase, and fetched FD - 1 phases ahead into FD rotating register buffers; the other
@@ -545,7 +565,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         load_pa(smem, 0, pa[0]);
         load_pw(smem, 0, pw[0]);
         load_pw(smem, 1, pw[1]);
-        decode_unit(pw[0], bcc, 0, 0, px[0]);
+        decode_pair(pw[0], bcc, 0, 0, px[0]);
     } else {
         load_held(sm, 0, 0, fh[0]);
         load_held(sm, 0, 1, fh[0]);
@@ -586,7 +606,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                     const int j = SPLITN ? h * SF + y : y;
                     const v4i act = AD ? fad[ab][s][i] : SPLITN ? fh[(hp + s) % 2][i] : fs[(ph + kk) % FD][x];
                     const v4i wgt = SPLITN ? fs[(ph + kk) % FD][y] : fh[(hp + s) % 2][j];
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wgt, act, acc[i][j], 0, 0, 0);
+                    if constexpr (MF == 16) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wgt, act, acc[i][j], 0, 0, 0);
                 }
             }
             if constexpr (ST) stage_slice(r, dst, k2, kk, o);
@@ -634,7 +654,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         // that work.  Small wave tiles append them at each exit of the staged steps (one predecessor each); larger
         // ones, with few registers to spare for the copies that so many joins cost, select them by the stage reached;
         // the largest (128 accumulators, 256x256) keeps every step alike and stages past the end.
-        constexpr bool INLINE_TAIL = MI * NI <= 8, NO_TAIL = MI * NI > 16;
+        constexpr bool INLINE_TAIL = ACC16 <= 8, NO_TAIL = ACC16 > 16;
         static_assert(AD ? NAB == 3 || NO_TAIL : KS == 2 || NO_TAIL, "the copies without staging do not know their step's parity");
         const int KM = NO_TAIL ? KT : max(KT - 2, 0);   // steps that stage step kt + 2
         auto last_two = [&](auto s_first, auto s_second) __attribute__((always_inline)) {
@@ -695,13 +715,13 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     __syncthreads();   // every wave is done reading the staging buffers
     if constexpr (KG > 1) {   // the groups' partial sums meet in group 0 (register r of thread t at word r * NT + t)
         if (kg > 0) {
-            int32_t* part = reinterpret_cast<int32_t*>(smem + PART_BASE + (kg - 1) * PART_BYTES);
+            int32_t* sums = reinterpret_cast<int32_t*>(smem + PART_BASE + (kg - 1) * PART_BYTES);
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int j = 0; j < NI; ++j)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) part[((i * NI + j) * 4 + r) * NT + tid] = acc[i][j][r];
+                    for (int r = 0; r < 4 * AG; ++r) sums[((i * NI + j) * 4 * AG + r) * NT + tid] = acc[i][j][r];
         }
         __syncthreads();
         if (kg > 0) return;
@@ -713,7 +733,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
                 for (int j = 0; j < NI; ++j)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[i][j][r] += other[((i * NI + j) * 4 + r) * NT + tid];
+                    for (int r = 0; r < 4 * AG; ++r) acc[i][j][r] += other[((i * NI + j) * 4 * AG + r) * NT + tid];
         }
     }
     auto epilogue = [&](auto epi_tag) {
@@ -730,37 +750,40 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                       (epi != SCMX_EPI_RES || reinterpret_cast<uintptr_t>(a.res) % 16 == 0);
 
     float xsv[MI];
-    f32x4 wsv[NI];
+    f32x4 wsv[NI][AG];
     if (epi != SCMX_EPI_I32) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) xsv[i] = s_xs[wm * WTM + i * 16 + lr];
+        for (int i = 0; i < MI; ++i) xsv[i] = s_xs[wm * WTM + i * MF + lr];
 #pragma unroll
-        for (int j = 0; j < NI; ++j) wsv[j] = *reinterpret_cast<const f32x4*>(&s_ws[wn * WTN + j * 16 + 4 * quad]);
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+            for (int g = 0; g < AG; ++g) wsv[j][g] = *reinterpret_cast<const f32x4*>(&s_ws[wn * WTN + j * MF + 8 * g + 4 * part]);
     }
     auto emit = [&](auto wide_tag) __attribute__((always_inline)) {
     constexpr bool W = decltype(wide_tag)::value;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-        const int row = i * 16 + lr;
+        const int row = i * MF + lr;
         const int m = wm0 + row;
         const float xs = epi != SCMX_EPI_I32 ? xsv[i] : 0.0f;
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-            const int col = j * 16 + 4 * quad;
+        for (int jg = 0; jg < NI * AG; ++jg) {
+            const int j = jg / AG, g = jg % AG;
+            const int col = j * MF + 8 * g + 4 * part;
             const int n = wn0 + col;
             if (epi == SCMX_EPI_I32) {
-                const v4i v = acc[i][j];
+                const v4i v = v4i{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
                 if (W)
                     *reinterpret_cast<v4i*>(wtile + row * rsb + col * 4) = v;
                 else if (m < row_end && n < N)
                     *reinterpret_cast<v4i*>(reinterpret_cast<int32_t*>(a.out) + size_t(m) * N + n) = v;
                 continue;
             }
-            const f32x4 w4 = wsv[j];
+            const f32x4 w4 = wsv[j][g];
             float y[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                y[r] = __fmul_rn(__fmul_rn(float(acc[i][j][r]), xs), w4[r]);
+                y[r] = __fmul_rn(__fmul_rn(float(acc[i][j][4 * g + r]), xs), w4[r]);
             uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
             if (epi == SCMX_EPI_SWIGLU) {   // (g, g, u, u) -> two outputs
                 const uint16_t s0 = swiglu_lut(a.silu, y[0], round_bf16(y[2]));
@@ -862,7 +885,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 // ---- host dispatch ---------------------------------------------------------------------------------------------
 
 template <int BM, int BN, int BK, int WGM, int WGN, int OCC = 1, int FD = 2, bool SKIP = false, bool PK = false, int KG = 1,
-          int ADM = 0>
+          int ADM = 0, int MF = 16>
 static void launch_tile(const GemmArgs& a_in, int bmode, int row_tiles, hipStream_t s) {
     GemmArgs a = a_in;
     if (a.epi == SCMX_EPI_SWIGLU) a.silu = silu_table_device();
@@ -871,26 +894,26 @@ static void launch_tile(const GemmArgs& a_in, int bmode, int row_tiles, hipStrea
     const dim3 grid(unsigned(row_tiles) * unsigned(num_n)), block(WGM * WGN * KG * 64);
     if constexpr (PK) {   // callers choose this tile for the FP4-conversion formats only
         if (bmode == B_PACKED_DEFAULT)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_DEFAULT, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_DEFAULT, OCC, FD, SKIP, true, 1, 0, MF><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_B16)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16, OCC, FD, SKIP, true, 1, 0, MF><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_B16M)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16M, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16M, OCC, FD, SKIP, true, 1, 0, MF><<<grid, block, 0, s>>>(a);
         else
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_E8M0, OCC, FD, SKIP, true><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_E8M0, OCC, FD, SKIP, true, 1, 0, MF><<<grid, block, 0, s>>>(a);
     } else {
         if (bmode == B_INT8)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_INT8, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_INT8, OCC, FD, SKIP, false, KG, ADM, MF><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_DEFAULT)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_DEFAULT, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_DEFAULT, OCC, FD, SKIP, false, KG, ADM, MF><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_B16)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16, OCC, FD, SKIP, false, KG, ADM, MF><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_B16M)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16M, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_B16M, OCC, FD, SKIP, false, KG, ADM, MF><<<grid, block, 0, s>>>(a);
         else if (bmode == B_PACKED_E8M0)
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_E8M0, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_E8M0, OCC, FD, SKIP, false, KG, ADM, MF><<<grid, block, 0, s>>>(a);
         else
-            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_GENERIC, OCC, FD, SKIP, false, KG, ADM><<<grid, block, 0, s>>>(a);
+            gemm_kernel<BM, BN, BK, WGM, WGN, B_PACKED_GENERIC, OCC, FD, SKIP, false, KG, ADM, MF><<<grid, block, 0, s>>>(a);
     }
 }
 
@@ -1268,15 +1291,22 @@ static void launch_grouped(const GemmArgs& a, int bmode, int tm, hipStream_t s) 
         launch_tile<128, 128, 128, 4, 1, 2, 2, false, false, 1, 2>(b, bmode, max_tiles << b.sub_log2, s);
     }
     else if (bmode != B_INT8 && bmode != B_PACKED_GENERIC && a.K % 256 == 0 && a.N % 128 == 0 &&
-             reinterpret_cast<uintptr_t>(a.bcodes) % 8 == 0)
+             reinterpret_cast<uintptr_t>(a.bcodes) % 8 == 0) {
         // Few rows per expert: the pass streams the expert weights, and what it pays per weight is the staging.  The packed
-        // tile writes and reads half the weight bytes in LDS, its four waves sit side by side along N (every fragment is
-        // decoded once) and three workgroups share a CU.  Its lanes read the block codes of two K steps with one aligned
+        // tile writes and reads half the weight bytes in LDS, its waves sit side by side along N (every fragment is decoded
+        // once) and two or three workgroups share a CU.  Its lanes read the block codes of two K steps with one aligned
         // load of 2, 4 or 8 bytes, hence the conditions on K and on the pointer.  Bound by the vector ALU: 64 codes a lane
-        // and step to decode (10 instructions per 8) beside 16 MFMAs.  257 experts of 1024 x 2048 / 2048 x 512, 70 rows each,
-        // e2m1/B16/M1..10: 108 + 67 us, staged INT8 118 + 74.
-        launch_tile<64, 128, 128, 1, 4, 2, 2, false, true>(a, bmode, max_tiles, s);
-    else
+        // and step to decode (10 instructions per 8) beside 8 MFMAs.  Skewed routing, 70 rows an expert on average, us packed
+        // / staged INT8: 257 experts of 1024 x 2048, published format 100.5 / 108, 16-blocks 104 / 117, MXFP4 105.5 / 114,
+        // e2m1/B16/M1..10 111 / 120; 64 of 2048 x 1024 30.4 / 31.2, 30.5 / 32.1, 30.9 / 32.0, 31.1 / 33.2.
+        // A reduction of four steps at most is mostly prologue and epilogue: eight waves on 256 columns, four a SIMD, share
+        // them.  257 experts of 2048 x 512, 70 rows, us 256 / 128 columns: 63.3 / 67.2, 61.6 / 69.9, 64.6 / 70.1, 64.9 / 71.0;
+        // 64 of 4096 x 256 23.5 / 24.6; K = 768 the other way round, 29.9 / 26.5.
+        if (a.K <= 512 && a.N % 256 == 0)
+            launch_tile<64, 256, 128, 1, 8, 4, 2, false, true, 1, 0, 32>(a, bmode, max_tiles, s);
+        else
+            launch_tile<64, 128, 128, 1, 4, 2, 2, false, true, 1, 0, 32>(a, bmode, max_tiles, s);
+    } else
         launch_tile<64, 128, 128, 2, 4>(a, bmode, max_tiles, s);
 }
 

@@ -44,16 +44,9 @@ def test_blocked_tiles(m, n, k, name):
     assert torch.equal(S.mm_i8_i32(xb, S.PackedWq(codes, bc, n, k, fmt, ws))[:m], product(dev(xq)[:m], q))
 
 
-@pytest.mark.parametrize("name", list(NAMES))
-@pytest.mark.parametrize("tm", [64, 128, 256])
-@pytest.mark.parametrize("e,n,k", [(3, 1156, 512), (65, 256, 384), (130, 128, 256), (4100, 8, 128)])
-def test_grouped_tiles(e, n, k, tm, name):
-    """Segments of 0 to a little over 256 rows (a 256-row slot of which 128-row tiles use one or both halves, with and
-    without rows past the segment), expert counts either side of one and two levels of the tile's expert search; rows gathered."""
+def grouped(e, n, k, tm, name, counts, rng):
+    """The grouped product of expert segments of `counts` gathered rows, INT32, against float64."""
     from mxfp4_int8_m5_amd import sc_moe as M
-    rng = np.random.default_rng(e + n + k)
-    counts = rng.choice([0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257], e) if e < 1000 else rng.choice([0, 0, 0, 1, 2], e)
-    counts[0] += 1
     ex = np.repeat(np.arange(e), counts).astype(np.int32)
     r = len(ex)
     few = [weights(rng, n, k, name) for _ in range(min(e, 3))]
@@ -72,3 +65,23 @@ def test_grouped_tiles(e, n, k, tm, name):
     if name == "published":
         got = M.moe_mm_i8(rows.contiguous(), r, q.reshape(e * n, k).contiguous(), ws, off, tstart, mt, n, 0, tile=(tm, 64, 4))
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("name", list(NAMES))
+@pytest.mark.parametrize("tm", [64, 128, 256])
+@pytest.mark.parametrize("e,n,k", [(3, 1156, 512), (65, 256, 384), (130, 128, 256), (4100, 8, 128)])
+def test_grouped_tiles(e, n, k, tm, name):
+    """Segments of 0 to a little over 256 rows (a 256-row slot of which 128-row tiles use one or both halves, with and
+    without rows past the segment), expert counts either side of one and two levels of the tile's expert search; rows gathered."""
+    rng = np.random.default_rng(e + n + k)
+    counts = rng.choice([0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257], e) if e < 1000 else rng.choice([0, 0, 0, 1, 2], e)
+    counts[0] += 1
+    grouped(e, n, k, tm, name, counts, rng)
+
+
+# 256 columns a workgroup up to 512 of K, 128 beyond or where the rows of weights do not divide; every tail of six steps
+@pytest.mark.parametrize("name", ["published", "sixteen", "range", "mxfp4"])
+@pytest.mark.parametrize("n,k", [(256, 256), (512, 512), (128, 512), (384, 256), (128, 768), (256, 1024), (256, 1280), (128, 1792)])
+def test_packed_tiles(n, k, name):
+    rng = np.random.default_rng(n + k)
+    grouped(9, n, k, 64, name, np.array([1, 0, 31, 32, 33, 63, 64, 65, 200]), rng)
