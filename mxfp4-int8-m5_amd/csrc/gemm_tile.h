@@ -48,7 +48,8 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     constexpr int MI = WTM / MF, NI = WTN / MF;   // MF-row / MF-column blocks of a wave's tile
     constexpr int ACC16 = WTM * WTN / 256;        // its accumulators, in 16 x 16 blocks
     static_assert(WTM % 32 == 0 && WTN % 32 == 0 && (BK == 64 || BK == 128), "tile must be whole 32x32 blocks");
-    static_assert(MF == (PK ? 32 : 16), "packed tiles multiply with 32x32x32, the others with 16x16x64");
+    static_assert(MF == 32 || (MF == 16 && !PK), "MFMA shapes 32x32x32 and, weights staged as INT8, 16x16x64");
+    static_assert(MF == 16 || ADM != 2, "activation fragments from gathered rows: 64-wide slices");
     constexpr int CPR = BK / 16;             // 16-byte chunks per LDS row
     constexpr int RPB = 256 / BK;            // rows per 256 bytes, i.e. per sweep of the 64 LDS banks
     constexpr int A_CHUNKS = AD ? 0 : BM * CPR;   // 16-byte pieces of the activation tile
@@ -534,12 +535,14 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     };
     static_assert(!PK || NKP == 2, "the pair buffers return to phase 0 every K step");
 
-    // A step runs in phases, two per 64-wide k slice: the operand with more 16-row blocks in the wave's tile is split, one
-    // half of its fragments per phase, and fetched FD - 1 phases ahead into FD rotating register buffers; the other
+    // MF = 16: a step runs in phases, two per 64-wide k slice: the operand with more 16-row blocks in the wave's tile is split,
+    // one half of its fragments per phase, and fetched FD - 1 phases ahead into FD rotating register buffers; the other
     // operand's fragments are held for the slice and fetched one slice ahead, half of them in each phase.  The fragments
     // fetched at the end of an iteration belong to the next step's stage.
+    // MF = 32: a phase is a 32-wide k slice with the fragments of all of the wave's rows and columns.
+    constexpr bool F16 = MF == 16;
     constexpr bool SPLITN = AD || NI >= MI;                 // the split operand: weights (columns) or activations (rows)
-    constexpr int SF = (SPLITN ? NI : MI) / 2, HF = SPLITN ? MI : NI;
+    constexpr int SF = F16 ? (SPLITN ? NI : MI) / 2 : 1, HF = F16 ? (SPLITN ? MI : NI) : 1;
     constexpr int AHEAD = FD - 1;
     static_assert(AHEAD >= 1 && AHEAD <= NKK, "fragment prefetch distance");
     [[maybe_unused]] v4i fs[FD][SF], fh[2][HF];
@@ -561,12 +564,25 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
             x[f] = *reinterpret_cast<const v4i*>(src + (SPLITN ? a_frag : b_frag) + f * 16 * BK + koff[s]);
         }
     };
+    constexpr int AI = F16 ? 1 : MI, BI = F16 ? 1 : NI;
+    [[maybe_unused]] v4i fa[FD][AI], fb[FD][BI];
+    auto load_frags = [&](const int8_t* src, int kk, v4i (&xa)[AI], v4i (&xb)[BI]) __attribute__((always_inline)) {
+        if (SKIP && mi_active == 0) return;
+#pragma unroll
+        for (int i = 0; i < AI; ++i)
+            if (!AD && (!SKIP || i < mi_active)) xa[i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + koff[kk]);
+#pragma unroll
+        for (int j = 0; j < BI; ++j) xb[j] = *reinterpret_cast<const v4i*>(src + b_frag + j * 32 * BK + koff[kk]);
+    };
     __syncthreads();
     if constexpr (PK) {
         load_pa(smem, 0, pa[0]);
         load_pw(smem, 0, pw[0]);
         load_pw(smem, 1, pw[1]);
         decode_pair(pw[0], bcc, 0, 0, px[0]);
+    } else if constexpr (!F16) {
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) load_frags(sm, q, fa[q], fb[q]);
     } else {
         load_held(sm, 0, 0, fh[0]);
         load_held(sm, 0, 1, fh[0]);
@@ -594,20 +610,28 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         if constexpr (AD && ST && NAB == 3) load_ad(wr, k2);
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
-            const int s = kk >> 1, h = kk & 1;
-            load_split(kk + AHEAD < NKK ? src : nxt, (kk + AHEAD) % NKK, fs[(ph + kk + AHEAD) % FD]);
-            load_held(s + 1 < KS ? src : nxt, (s + 1) % KS, h, fh[(hp + s + 1) % 2]);
+            const int s = F16 ? kk >> 1 : kk, h = kk & 1, now = (ph + kk) % FD, then = (ph + kk + AHEAD) % FD;
+            if constexpr (F16) {
+                load_split(kk + AHEAD < NKK ? src : nxt, (kk + AHEAD) % NKK, fs[then]);
+                load_held(s + 1 < KS ? src : nxt, (s + 1) % KS, h, fh[(hp + s + 1) % 2]);
+            } else {
+                load_frags(kk + AHEAD < NKK ? src : nxt, (kk + AHEAD) % NKK, fa[then], fb[then]);
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int x = 0; x < (SPLITN ? MI : SF); ++x) {
-                const int i = SPLITN ? x : h * SF + x;
+            for (int x = 0; x < (F16 && !SPLITN ? SF : MI); ++x) {
+                const int i = F16 && !SPLITN ? h * SF + x : x;
                 if (SKIP && i >= mi_active) continue;
 #pragma unroll
-                for (int y = 0; y < (SPLITN ? SF : NI); ++y) {
-                    const int j = SPLITN ? h * SF + y : y;
-                    const v4i act = AD ? fad[ab][s][i] : SPLITN ? fh[(hp + s) % 2][i] : fs[(ph + kk) % FD][x];
-                    const v4i wgt = SPLITN ? fs[(ph + kk) % FD][y] : fh[(hp + s) % 2][j];
-                    if constexpr (MF == 16) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wgt, act, acc[i][j], 0, 0, 0);
+                for (int y = 0; y < (F16 && SPLITN ? SF : NI); ++y) {
+                    const int j = F16 && SPLITN ? h * SF + y : y;
+                    if constexpr (F16) {
+                        const v4i act = AD ? fad[ab][s][i] : SPLITN ? fh[(hp + s) % 2][i] : fs[now][x];
+                        const v4i wgt = SPLITN ? fs[now][y] : fh[(hp + s) % 2][j];
+                        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wgt, act, acc[i][j], 0, 0, 0);
+                    } else {
+                        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[now][j], AD ? fad[ab][s][i] : fa[now][i], acc[i][j], 0, 0, 0);
+                    }
                 }
             }
             if constexpr (ST) stage_slice(r, dst, k2, kk, o);
@@ -656,7 +680,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         // ones, with few registers to spare for the copies that so many joins cost, select them by the stage reached;
         // the largest (128 accumulators, 256x256) keeps every step alike and stages past the end.
         constexpr bool INLINE_TAIL = ACC16 <= 8, NO_TAIL = ACC16 > 16;
-        static_assert(AD ? NAB == 3 || NO_TAIL : KS == 2 || NO_TAIL, "the copies without staging do not know their step's parity");
+        static_assert(!F16 || (AD ? NAB == 3 || NO_TAIL : KS == 2 || NO_TAIL), "the copies without staging do not know their step's parity");
         const int KM = NO_TAIL ? KT : max(KT - 2, 0);   // steps that stage step kt + 2
         auto last_two = [&](auto s_first, auto s_second) __attribute__((always_inline)) {
             iteration_staged(s_first, Even{}, std::false_type{}, r0, 0);

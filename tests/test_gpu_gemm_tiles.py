@@ -85,3 +85,13 @@ def test_grouped_tiles(e, n, k, tm, name):
 def test_packed_tiles(n, k, name):
     rng = np.random.default_rng(n + k)
     grouped(9, n, k, 64, name, np.array([1, 0, 31, 32, 33, 63, 64, 65, 200]), rng)
+
+
+# 256-row slots that hold more: whole and cut 256x256 tiles (one that fills the CUs among them), 256x128 ones for narrow
+# layers, an expert without rows, K loops of every length up to a trip and two more
+@pytest.mark.parametrize("name", list(NAMES))
+@pytest.mark.parametrize("counts", [(257, 300, 511), (512, 0, 300)])
+@pytest.mark.parametrize("n,k", [(256, 128), (1156, 256), (256, 384), (1156, 512), (256, 640), (22016, 128),
+                                 (128, 128), (132, 256), (128, 384), (128, 512), (128, 640), (128, 768), (128, 896)])
+def test_tall_segments(n, k, counts, name):
+    grouped(3, n, k, 256, name, np.array(counts), np.random.default_rng(n + k))
