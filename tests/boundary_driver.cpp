@@ -277,6 +277,11 @@ int main() {
     expect(scmx_route_topk(h[0], nullptr, 4, 2000, 8, 1, oi[0], oh[0], nullptr), SCMX_ERR_ARG, "route_topk 2000 experts");
     expect(scmx_route_topk(h[0], nullptr, 4, 4, 8, 1, oi[0], oh[0], nullptr), SCMX_ERR_ARG, "route_topk k > E");
     expect(scmx_route_topk(h[0], nullptr, 4, 128, 65, 1, oi[0], oh[0], nullptr), SCMX_ERR_ARG, "route_topk k > 64");
+    expect(scmx_norm_linear(h[0], nullptr, 1e-6f, h[1], 2048, 64, oq, of, oh[0], oh[1], nullptr), SCMX_ERR_ARG, "norm_linear null w");
+    expect(scmx_norm_linear(h[0], h[1], 1e-6f, h[2] + 4, 2048, 64, oq, of, oh[0], oh[1], nullptr), SCMX_ERR_ARG,
+           "norm_linear misaligned mat");
+    for (int k : {0, 576, 2560}) expect(scmx_norm_linear(h[0], h[1], 1e-6f, h[2], k, 64, oq, of, oh[0], oh[1], nullptr), SCMX_ERR_ARG, "norm_linear K");
+    for (int n : {0, 4097}) expect(scmx_norm_linear(h[0], h[1], 1e-6f, h[2], 2048, n, oq, of, oh[0], oh[1], nullptr), SCMX_ERR_ARG, "norm_linear N");
     expect(scmx_route_sort(ci, 4, 8, 2000, 64, oi[0], oi[1], oi[2], oi[3], oi[4], nullptr), SCMX_ERR_ARG, "route_sort 2000 experts");
     expect(scmx_route_sort(ci, 1 << 30, 8, 64, 64, oi[0], oi[1], oi[2], oi[3], oi[4], nullptr), SCMX_ERR_ARG,
            "route_sort M*topk beyond 32 bits");
@@ -371,6 +376,8 @@ int main() {
     expect_valid(scmx_gemv(&fmt, xq, f0, codes, bc, f1, nullptr, oh[0], 3, 0, nullptr, 0.0f, 1, 1024, 2048, ci, 8, 0, 256, nullptr),
                  "gemv expert slots");
     expect_valid(scmx_route_topk(h[0], h[1], 2048, 256, 8, 1, oi[0], oh[0], nullptr), "route_topk");
+    for (int k : {512, 1024, 1536, 2048})
+        for (int n : {1, 64, 4096}) expect_valid(scmx_norm_linear(h[0], h[1], 1e-6f, h[2], k, n, oq, of, oh[0], oh[1], nullptr), "norm_linear");
     expect_valid(scmx_route_sort(ci, 4096, 8, 64, 256, oi[0], oi[1], oi[2], oi[3], oi[4], nullptr), "route_sort");
     expect_valid(scmx_route_sort(ci, 10, 2, 8, 64, oi[0], oi[1], oi[2], oi[3], oi[4], nullptr), "route_sort small");
     for (int tm : {64, 128, 256})
@@ -455,6 +462,9 @@ int main() {
         }
         expect_status(scmx_route_topk(h[0], (const uint16_t*)maybe(h[1]), r(), r(), r(), int(rng() % 2), oi[0], oh[0], nullptr),
                       "fuzz route_topk");
+        expect_status(scmx_norm_linear(h[0], (const uint16_t*)maybe(h[1]), 1e-6f, (const uint16_t*)maybe(h[2]), r(), r(), (int8_t*)maybe(oq), of,
+                                       oh[0], oh[1], nullptr),
+                      "fuzz norm_linear");
         expect_status(scmx_route_sort(ci, r(), r(), r(), r(), oi[0], oi[1], oi[2], oi[3], oi[4], nullptr), "fuzz route_sort");
         expect_status(scmx_moe_mm(&f, xq, f0, (const int32_t*)maybe(ci), r(), codes, bc, f1, ci, ci, r(), r(), r(), r(), int(rng() % 6) - 1,
                                   out, nullptr),

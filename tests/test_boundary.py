@@ -176,6 +176,12 @@ def test_attention_split_policy_and_cache_names(pkg):
     assert [pkg.sc_moe.row_tile(t * 8, 64) for t in (1, 512, 767, 768, 4096)] == [64, 64, 64, 256, 256]
 
 
+def test_the_boundary_driver_calls_every_entry_point(pkg):
+    with open(os.path.join(ROOT, "tests", "boundary_driver.cpp")) as f:
+        calls = f.read()
+    assert [n for n in pkg._lib.SIGNATURES if n + "(" not in calls] == []
+
+
 @pytest.mark.skipif(shutil.which(os.environ.get("HIPCC", "hipcc")) is None, reason="needs hipcc to build the instrumented library")
 def test_host_code_under_address_and_undefined_behaviour_sanitizers():
     """The library's host code (argument checks, launch-shape arithmetic, dispatch) compiled with AddressSanitizer and
