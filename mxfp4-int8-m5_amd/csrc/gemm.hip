@@ -37,11 +37,15 @@ static const Cand ROW_TILES[7] = {
 };
 // Blocked activations, read by the waves themselves.  Workgroups of four waves share a CU (two of 256x128, three of 128x64, four
 // of 64x64): their barriers and epilogues do not coincide, which eight waves of one workgroup cannot avoid.  Eight waves
-// on one tile are faster where the launch has no more than a tile per CU.
-static const Cand BLOCKED_TILES[5] = {
+// on one tile are faster where the launch has no more than a tile per CU.  The entries of 256x256 and of eight waves on 256x128 are fitted
+// to 741 problems in which such launches are many (each tile timed; 200 of them with 120 ... 260 of those tiles, five times in turn): the
+// choice costs 0.37 per cent over the fastest tile on average there, 1.05 without 256x256 and with the entry that eight waves on
+// 256x128 had when launches of 129 ... 192 tiles were few (1024 x 6144 x 4096, MXFP4, 34.5 us for 28.6).
+static const Cand BLOCKED_TILES[6] = {
     {256, 128, 2, {6.11f, 8.34f}, {0.966f, 1.498f}, {4.2f, 2.3f}, 0.914f, 0.96f},
-    {256, 128, 1, {5.51f}, {0.805f}, {11.5f}, 0.85f, 0.93f},   // eight waves
-    {256, 64, 1, {3.945f}, {0.416f}, {2.4f}, 0.98f, 1.05f},    // eight waves
+    {256, 256, 1, {12.7f}, {1.46f}, {18.7f}, 0.813f, 0.856f},
+    {256, 128, 1, {6.96f}, {0.802f}, {11.5f}, 0.856f, 0.806f},   // eight waves
+    {256, 64, 1, {3.945f}, {0.416f}, {2.4f}, 0.98f, 1.05f},      // eight waves
     {128, 64, 3, {3.78f, 4.09f, 2.62f}, {0.34f, 0.498f, 0.806f}, {3.83f, 5.3f, 3.0f}, 0.925f, 0.98f},
     {64, 64, 4, {3.15f, 3.54f, 3.58f, 1.83f}, {0.294f, 0.419f, 0.618f, 0.782f}, {5.49f, 4.07f, 2.67f, 3.0f}, 0.95f, 1.0f},
 };
@@ -83,7 +87,8 @@ static TileChoice fastest_tile(const Cand* cand, int first, int last, long M, lo
 // The few-row kernel's model takes no launch in.  On the 61 problems of up to 128 rows the choice costs 0.1 per cent over the
 // fastest kernel on average.  Formats whose codes are looked up: a tile's weights are decoded again by each of its row groups,
 // once by the few-row kernel, which is worth half as much again.
-// No table gives less than `least`, so the smallest calls, which the host bounds, look no further.
+// No table gives less than `least`, so the smallest calls, which the host bounds, look no further.  The four-wave 256x128 tile,
+// which some formats do not take (launch_dense), never decides: the same layout with and without it on 250 000 drawn problems.
 enum { BY_ROWS = 0, BLOCKED = 1 };   // and FEW_ROWS
 static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
     const int cus = device_cus();
@@ -92,7 +97,7 @@ static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
     const float least = fmaxf(3.8f, 2.41f + 0.157f / 128.0f * float(K));
     if (few < least) return FEW_ROWS;
     const float rows = fastest_tile(ROW_TILES, small ? 0 : 5, 6, M, N, K, cus).us;
-    const float blocks = (0.3f + fastest_tile(BLOCKED_TILES, 0, 4, M, N, K, cus).us) * (small ? 1.1f : 1.0f);
+    const float blocks = (0.3f + fastest_tile(BLOCKED_TILES, 0, 5, M, N, K, cus).us) * (small ? 1.1f : 1.0f);
     const float tile = fminf(rows, blocks);
     if (few < tile) return FEW_ROWS;
     DevFormat f;
@@ -104,13 +109,16 @@ static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
     if (a.blocked == FEW_ROWS) return launch_skinny(a, bmode, s);
     const int rows256 = (a.M + 255) / 256, rows128 = (a.M + 127) / 128, rows64 = (a.M + 63) / 64;
     if (a.blocked) {
-        // The four-wave 256x128 tile reads K in steps of 64.  With a byte per 32 weights and a row of those 128 bytes or longer it
-        // reads a cache line per weight row and step for two of them, and the vector L1 does not hold the lines until the next
-        // step: 6001 x 6144 x 4096 161 us against 152 of the eight waves (2-bit codes 144 / 148; K = 2048 66.6 / 68.8).  Table
-        // decode does not fit its registers.
+        // The four-wave 256x128 tile and the 256x256 one read K in steps of 64.  With a byte per 32 weights and a row of those 128
+        // bytes or longer they read a cache line per weight row and step for two of them, and the vector L1 does not hold the lines
+        // until the next step: four waves on 6001 x 6144 x 4096 161 us against 152 of the eight waves (2-bit codes 144 / 148; K = 2048
+        // 66.6 / 68.8); 256x256 against the fastest other tile 0.98 times as fast with more than 192 tiles, 1.02 with fewer.  Table
+        // decode does not fit the registers of the four waves, and 256x256 is 1.07 times slower with it (40 problems; 12288 x
+        // 4096 at 896 rows 123 us, 108 on 256x64).
         const bool wide_codes = (bmode == B_PACKED_E8M0 || bmode == B_PACKED_B16M) && a.K >= 4096;
-        const int first = wide_codes || bmode == B_PACKED_GENERIC ? 1 : 0;
-        return launch_blocked(a, bmode, fastest_tile(BLOCKED_TILES, first, 4, a.M, a.N, a.K, device_cus()).index, s);
+        const bool many = 4LL * rows256 * ((a.N + 255) / 256) > 3 * device_cus();
+        const int first = bmode == B_PACKED_GENERIC || (wide_codes && many) ? 2 : wide_codes ? 1 : 0;
+        return launch_blocked(a, bmode, fastest_tile(BLOCKED_TILES, first, 5, a.M, a.N, a.K, device_cus()).index, s);
     }
     switch (fastest_tile(ROW_TILES, 0, 6, a.M, a.N, a.K, device_cus()).index) {
         case 0: return launch_tile<256, 256, 64, 2, 4, 1, 2>(a, bmode, rows256, s);

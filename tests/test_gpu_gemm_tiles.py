@@ -28,13 +28,21 @@ def product(xq, q):
     return (xq.double() @ q.double().T).to(torch.int32)
 
 
-# one row of the list per tile of the blocked table (its order), more than one step count for those with a rotating loop
+# (tile of the blocked table on 256 CUs, shapes): every tail of each tile's rotating loop (test_gemm_tile_choice.py checks the tiles)
+BLOCKED = [(0, [(1154, 10396, 128), (588, 10004, 384), (518, 10076, 640), (1030, 11864, 4224)]),   # 256x128, four waves (or, by format, another)
+           (1, [(935, 12296, 1536), (935, 12296, 1664), (772, 11664, 2176), (653, 11248, 4224)]),  # 256x256
+           (2, [(400, 9368, 4096), (588, 6584, 4224), (393, 8640, 5760), (393, 8640, 5888), (393, 8640, 6016), (393, 8640, 6144), (393, 8640, 6272),
+                (677, 8212, 512), (645, 8376, 640), (392, 12292, 768), (515, 10144, 896), (530, 9812, 1024),
+                (518, 10316, 1280)]),                                                              # 256x128, eight waves, both MFMA shapes
+           (3, [(216, 8564, 256), (146, 11004, 384), (148, 11192, 512), (134, 11848, 640), (130, 10900, 768), (137, 11804, 896)]),   # 256x64
+           (4, [(278, 180, 128), (319, 136, 256), (235, 136, 384), (154, 224, 512), (165, 340, 640), (133, 3888, 768),
+                (4133, 196, 896)]),                                                                # 128x64
+           (5, [(142, 7200, 128), (137, 6856, 256), (149, 8264, 384), (142, 8452, 512), (131, 8704, 640), (141, 144, 768),
+                (134, 316, 896)])]                                                                 # 64x64
+
+
 @pytest.mark.parametrize("name", list(NAMES))
-@pytest.mark.parametrize("m,n,k", [(400, 12296, 384), (1030, 12296, 640), (385, 12288, 4224),   # 256x128, four waves (or, by format, the next)
-                                   (1000, 6152, 768), (1500, 4104, 2048),                        # 256x128, eight waves
-                                   (600, 4104, 2048), (1030, 2052, 1280),                        # 256x64
-                                   (515, 8200, 640), (1025, 8192, 384), (4099, 2052, 128),       # 128x64
-                                   (770, 1032, 1280), (129, 1028, 256), (300, 260, 896)])        # 64x64
+@pytest.mark.parametrize("m,n,k", [s for _, shapes in BLOCKED for s in shapes])
 def test_blocked_tiles(m, n, k, name):
     from mxfp4_int8_m5_amd import sc_kernels as S
     rng = np.random.default_rng(m + n + k)
