@@ -10,7 +10,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libscmx.so")
 BINDING = os.path.join(HERE, "_binding.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-SOURCES = ["gemm.hip", "gemm_blocked.hip", "gemm_grouped.hip", "api.hip", "gemm_skinny.hip", "gemv.hip", "rowops.hip", "quantize.hip", "attn.hip", "attn_prefill.hip", "linear_bf16.hip", "silu_table.hip"]
+SOURCES = ["gemm_rows.hip", "gemm_blocked.hip", "gemm_grouped.hip", "gemm_rows_idle.hip", "gemm.hip", "api.hip",
+           "gemm_skinny.hip", "gemv.hip", "rowops.hip", "quantize.hip", "attn.hip", "attn_prefill.hip", "linear_bf16.hip", "silu_table.hip"]
 # packed FP32 instructions are kept off (they have misbehaved on this hardware pool); no FMA contraction, so the
 # FP32 epilogues and norms round exactly like a plain IEEE evaluation
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fhip-fp32-correctly-rounded-divide-sqrt", "-Wno-unused-command-line-argument", "-fconstexpr-steps=400000000",

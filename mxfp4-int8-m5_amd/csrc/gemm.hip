@@ -1,7 +1,7 @@
-// W4A8 GEMM: the C entry points, the choice of a dense problem's tile and the tiles that read activations by rows.
+// W4A8 GEMM: the C entry points and the choice of a dense problem's tile.
 #include <atomic>
 
-#include "gemm_tile.h"
+#include "gemm_args.h"
 
 namespace scmx {
 
@@ -107,7 +107,6 @@ static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
 
 static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
     if (a.blocked == FEW_ROWS) return launch_skinny(a, bmode, s);
-    const int rows256 = (a.M + 255) / 256, rows128 = (a.M + 127) / 128, rows64 = (a.M + 63) / 64;
     if (a.blocked) {
         // The four-wave 256x128 tile and the 256x256 one read K in steps of 64.  With a byte per 32 weights and a row of those 128
         // bytes or longer they read a cache line per weight row and step for two of them, and the vector L1 does not hold the lines
@@ -116,19 +115,11 @@ static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
         // decode does not fit the registers of the four waves, and 256x256 is 1.07 times slower with it (40 problems; 12288 x
         // 4096 at 896 rows 123 us, 108 on 256x64).
         const bool wide_codes = (bmode == B_PACKED_E8M0 || bmode == B_PACKED_B16M) && a.K >= 4096;
-        const bool many = 4LL * rows256 * ((a.N + 255) / 256) > 3 * device_cus();
+        const bool many = 4LL * ((a.M + 255) / 256) * ((a.N + 255) / 256) > 3 * device_cus();
         const int first = bmode == B_PACKED_GENERIC || (wide_codes && many) ? 2 : wide_codes ? 1 : 0;
         return launch_blocked(a, bmode, fastest_tile(BLOCKED_TILES, first, 5, a.M, a.N, a.K, device_cus()).index, s);
     }
-    switch (fastest_tile(ROW_TILES, 0, 6, a.M, a.N, a.K, device_cus()).index) {
-        case 0: return launch_tile<256, 256, 64, 2, 4, 1, 2>(a, bmode, rows256, s);
-        case 1: return launch_tile<256, 128, 128, 4, 2, 1, 3>(a, bmode, rows256, s);
-        case 2: return launch_tile<128, 128, 128, 4, 2, 1, 3>(a, bmode, rows128, s);
-        case 3: return launch_tile<128, 64, 128, 4, 2>(a, bmode, rows128, s);
-        case 5: return launch_tile<64, 64, 128, 2, 2, 1, 2, false, false, 2>(a, bmode, rows64, s);
-        case 6: return launch_tile<64, 32, 128, 2, 1, 1, 2, false, false, 4>(a, bmode, rows64, s);
-        default: return launch_tile<64, 64, 128, 2, 2>(a, bmode, rows64, s);
-    }
+    launch_rows(a, bmode, fastest_tile(ROW_TILES, 0, 6, a.M, a.N, a.K, device_cus()).index, s);
 }
 
 static int check_gemm_common(const char* who, int M, int N, int K, int epi, bool need_scales, const void* xq,

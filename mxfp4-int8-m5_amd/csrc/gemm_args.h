@@ -1,4 +1,4 @@
-// What the GEMM kernels are launched with: the dense and grouped tiles (gemm.hip) and the few-row kernel (gemm_skinny.hip).
+// What the GEMM kernels are launched with: the dense and grouped tiles (gemm_*.hip) and the few-row kernel (gemm_skinny.hip).
 #pragma once
 #include "scmx_common.h"
 
@@ -39,6 +39,8 @@ constexpr int SKINNY_MAX_ROWS = 128;
 // The few-row kernel's time (us) on a dense problem of up to SKINNY_MAX_ROWS rows, activations in the blocked layout.
 float skinny_time(int M, int N, int K, int cus);
 void launch_skinny(const GemmArgs& a, int bmode, hipStream_t s);
+void launch_rows(const GemmArgs& a, int bmode, int tile, hipStream_t s);
+void launch_rows_idle(const GemmArgs& a, int bmode, int tile, hipStream_t s);
 void launch_blocked(const GemmArgs& a, int bmode, int tile, hipStream_t s);
 void launch_grouped(const GemmArgs& a, int bmode, int tm, hipStream_t s);
 

@@ -1,4 +1,4 @@
-// W4A8 GEMM on CDNA4 INT8 MFMA: the tile kernel of dense prefill (gemm.hip, gemm_blocked.hip) and of grouped
+// W4A8 GEMM on CDNA4 INT8 MFMA: the tile kernel of dense prefill (gemm_rows*.hip, gemm_blocked.hip) and of grouped
 // mixture-of-experts (gemm_grouped.hip).
 //
 // One workgroup computes a BM x BN tile of  acc[m, n] = sum_k xq[m, k] * q[n, k]  in INT32.  Per K step of BK the

@@ -1,18 +1,18 @@
-"""The blocked tile that the GEMM's cost table chooses on 256 CUs, recomputed from the table in the source: the shapes of the GPU tile
-test reach the tiles that they are listed under, and 32x32x32 and 16x16x64 forms both."""
+"""The tile that the GEMM's cost tables choose on 256 CUs, recomputed from the tables in the source: the shapes of the GPU tile tests
+reach the tiles that they are listed under, and 32x32x32 and 16x16x64 forms both."""
 import os
 import re
 
 import pytest
 
-from tests.test_gpu_gemm_tiles import BLOCKED
+from tests.test_gpu_gemm_tiles import BLOCKED, ROWS
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mxfp4-int8-m5_amd", "csrc")
 
 
-def table():
+def table(name):
     with open(os.path.join(CSRC, "gemm.hip")) as f:
-        body = re.search(r"BLOCKED_TILES\[6\] = \{\n(.*?)\n\};", f.read(), re.S).group(1)
+        body = re.search(name + r"\[\d\] = \{\n(.*?)\n\};", f.read(), re.S).group(1)
     number = r"[\d.]+f?"
     rows = []
     for line in body.splitlines():
@@ -23,9 +23,11 @@ def table():
     return rows
 
 
-def chosen(m, n, k, cus=256):
+def chosen(name, m, n, k, cus=256):
     times = []
-    for bm, bn, occ, f, s, w, low, mid in table():
+    for i, (bm, bn, occ, f, s, w, low, mid) in enumerate(table(name)):
+        if name == "ROW_TILES" and i >= 5 and (-(-m // bm) * -(-n // bn) > cus or k % (256 if i == 5 else 512)):
+            continue   # K groups
         full, rest = divmod(-(-m // bm) * -(-n // bn), cus * occ)
         cost = lambda r: max(f[r - 1] + k / 128 * s[r - 1], w[r - 1])
         t = full * cost(occ)
@@ -38,11 +40,16 @@ def chosen(m, n, k, cus=256):
     return times.index(min(times))
 
 
-@pytest.mark.parametrize("tile,m,n,k", [(t, *s) for t, shapes in BLOCKED for s in shapes])
-def test_the_tile_test_reaches_its_tiles(tile, m, n, k):
-    assert chosen(m, n, k) == tile
+@pytest.mark.parametrize("name,tile,m,n,k", [(name, t, *s) for name, tiles in (("BLOCKED_TILES", BLOCKED), ("ROW_TILES", ROWS))
+                                             for t, shapes in tiles for s in shapes])
+def test_the_tile_tests_reach_their_tiles(name, tile, m, n, k):
+    assert chosen(name, m, n, k) == tile
 
 
 def test_both_mfma_shapes_are_reached():
-    tiles = [-(-m // 256) * -(-n // 128) for m, n, _ in BLOCKED[2][1]]
-    assert min(tiles) <= 160 < max(tiles)
+    count = lambda shapes, bm, bn: [-(-m // bm) * -(-n // bn) for m, n, _ in shapes]
+    blocked = count(BLOCKED[2][1], 256, 128)
+    assert min(blocked) <= 160 < max(blocked)
+    for (_, shapes), bm, bn in zip(ROWS, (256, 256, 128, 128), (256, 128, 128, 64)):
+        tiles = count(shapes, bm, bn)
+        assert min(tiles) <= 192 < max(tiles)

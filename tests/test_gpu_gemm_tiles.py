@@ -41,6 +41,28 @@ BLOCKED = [(0, [(1154, 10396, 128), (588, 10004, 384), (518, 10076, 640), (1030,
                 (134, 316, 896)])]                                                                 # 64x64
 
 
+# the same for the larger tiles by rows, which multiply with 32x32x32 up to three quarters of a tile per CU
+ROWS = [(0, [(706, 12476, 384), (705, 12352, 512), (642, 10944, 640), (661, 10996, 768), (968, 12392, 256), (796, 12556, 384)]),      # 256x256
+        (1, [(709, 5456, 512), (387, 8396, 640), (262, 11020, 768), (257, 11732, 896), (268, 10892, 1152), (265, 10984, 1536),
+             (326, 12380, 640)]),                                                                                # 256x128
+        (2, [(135, 10940, k) for k in (4096, 4224, 4352, 4480, 4608, 4736)] + [(206, 12332, 128), (196, 12416, 512)]),    # 128x128
+        (3, [(67, 8288, 128), (68, 8244, 256), (75, 8268, 384), (68, 9200, 512), (69, 8460, 640), (66, 9780, 768),
+             (65, 8416, 896), (68, 8296, 1024), (134, 6552, 256)])]                                              # 128x64
+
+
+@pytest.mark.parametrize("name", list(NAMES))
+@pytest.mark.parametrize("m,n,k", [s for _, shapes in ROWS for s in shapes])
+def test_row_tiles(m, n, k, name):
+    from mxfp4_int8_m5_amd import sc_kernels as S
+    rng = np.random.default_rng(m + n + k)
+    codes, bc, ws, fmt, q = weights(rng, n, k, name)
+    xq = torch.from_numpy(rng.integers(-127, 128, (m, k)).astype(np.int8)).cuda()
+    want = product(xq, q)
+    assert torch.equal(S.mm_i8_i32(xq, S.PackedWq(codes, bc, n, k, fmt, ws)), want)
+    if name == "published":
+        assert torch.equal(S.mm_i8_i32(xq, q), want)
+
+
 @pytest.mark.parametrize("name", list(NAMES))
 @pytest.mark.parametrize("m,n,k", [s for _, shapes in BLOCKED for s in shapes])
 def test_blocked_tiles(m, n, k, name):
