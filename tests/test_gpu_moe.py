@@ -30,7 +30,14 @@ def skewed_routing(rng, tokens, experts, topk):
 
 
 @pytest.mark.parametrize("m,topk,e,tm", [(75, 8, 8, 64), (4096, 8, 64, 128), (2048, 9, 257, 64), (1, 8, 64, 64),
-                                         (300, 1, 1024, 128), (1000, 5, 1024, 64), (515, 8, 300, 128)])
+                                         (300, 1, 1024, 128), (1000, 5, 1024, 64), (515, 8, 300, 128),
+                                         # one workgroup, then one launch of 2 and 3 of them, tails of all but one row
+                                         (2047, 1, 64, 64), (2048, 1, 64, 64), (3071, 1, 257, 64), (4095, 1, 64, 128),
+                                         # the last sort of one launch and the first of three, by rows and by rows an expert
+                                         (5120, 8, 64, 128), (40961, 1, 64, 64), (5120, 8, 257, 64), (40961, 1, 257, 64),
+                                         (3072, 8, 8, 64), (24577, 1, 8, 64),
+                                         # three launches, more than 64 workgroups: without a tail, with one, all experts
+                                         (8192, 9, 257, 256), (70001, 1, 64, 64), (16999, 8, 1024, 256)])
 def test_route_sort_contract(M, m, topk, e, tm):
     rng = np.random.default_rng(m + e)
     inds, _ = skewed_routing(rng, m, e, topk)
