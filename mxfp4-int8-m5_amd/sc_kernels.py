@@ -347,7 +347,11 @@ def attn_splits(rows):
 def _decode_ranges(rows, hq):
     """The same for any number of heads.  16 heads, us with 1 / 8 / 16 ranges: 513 rows 10.5 / 7.6 / 7.8, 1000 15.5 / 8.4 / 8.1, 1500
     22.2 / 10.5 / 9.6, 3000 - / 12.7 / 11.8, 6000 - / 18.2 / 15.8, 12000 - / 27.2 / 22.4 (32 ranges 22.9); up to 512 rows the second
-    launch costs a host-bound loop more than it gives (300 rows 8.1 / 7.4 / 7.5)."""
+    launch costs a host-bound loop more than it gives (300 rows 8.1 / 7.4 / 7.5).
+    With the position on the device `rows` is the cache's, and a short context in a longer cache pays for a merge that finds little
+    or nothing to do.  In a graph, cache of 1024 rows, us with 1 / 16 ranges by the context: 30 rows 4.1 / 5.7, 128 4.4 / 5.9, 160 5.5 /
+    6.4, 300 6.8 / 6.4, 500 8.2 / 6.5, 700 10.7 / 6.5, 1000 13.4 / 6.6: over a conversation that fills its cache the split gives more than
+    that costs from about 520 rows on."""
     if hq > 32:
         return attn_splits(rows)
     return 1 if rows <= 512 else 16
