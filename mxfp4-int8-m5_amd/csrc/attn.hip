@@ -55,10 +55,10 @@ __global__ __launch_bounds__(ANT) void attn_decode_kernel(const uint16_t* __rest
     const uint16_t* vbase = vc + size_t(kvh) * rows * D + 8 * c;
 
     // gridDim.y > 1: the valid rows are cut into gridDim.y equal ranges, one per workgroup of a head; every workgroup
-    // leaves its unnormalised result, maximum and sum in `partial` and a second kernel merges them.
-    // A context of at most ATTN_SINGLE_MAX rows is read fastest by one workgroup per head (16 heads of a long cache, us, single /
-    // 16 ranges with the merge: 120 rows 6.9 / 7.4, 160 8.1 / 7.3, 300 9.5 / 7.5, 500 11.0 / 7.5): range 0 then takes all of
-    // it and writes the output, the other workgroups leave at once and the merge kernel finds nothing to do.
+    // leaves its unnormalised result, maximum and sum in `partial` and a second kernel merges them. A context of at
+    // most ATTN_SINGLE_MAX rows is read fastest by one workgroup per head (16 heads of a long cache, us, single / 16
+    // ranges with the merge: 120 rows 6.9 / 7.4, 160 8.1 / 7.3, 300 9.5 / 7.5, 500 11.0 / 7.5): range 0 then takes all
+    // of it and writes the output, the other workgroups leave at once and the merge kernel finds nothing to do.
     const bool single = gridDim.y == 1 || n <= ATTN_SINGLE_MAX;
     if (single && blockIdx.y > 0) return;
     const int nsplit = single ? 1 : int(gridDim.y);
@@ -194,8 +194,9 @@ __global__ __launch_bounds__(ANT) void attn_decode_kernel(const uint16_t* __rest
 }
 
 // Merge of the per-range results of one head: out = sum_s w_s num_s / sum_s w_s den_s with w_s = exp(m_s - max m).
-// Bound: one trip to memory behind a launch.  All of up to 16 ranges is requested at once, and before the position is known: 16 heads, 3000 rows, 16 ranges, attention
-// and merge 13.9 -> 11.8 us, 12000 rows 29.5 -> 22.4 (range after range before).
+// Bound: one trip to memory behind a launch.  All of up to 16 ranges is requested at once, and before the position is
+// known: 16 heads, 3000 rows, 16 ranges, attention and merge 13.9 -> 11.8 us, 12000 rows 29.5 -> 22.4 (range after
+// range before).
 template <int D>
 __global__ __launch_bounds__(D) void attn_merge_kernel(const float* __restrict__ partial, uint16_t* __restrict__ out,
                                                      int splits, const int64_t* __restrict__ pos_dev, int n0, int rows) {

@@ -129,8 +129,8 @@ __global__ __launch_bounds__(FA_NT) void attn_prefill_kernel(const uint16_t* __r
         }
     };
 
-    // The queries are requested before any key and stay before them: loaded behind the first pair's, their wait inside the loop (of which
-    // this code is one predecessor) covered the loads of the pair after the next in every step.
+    // The queries are requested before any key and stay before them: loaded behind the first pair's, their wait inside
+    // the loop (of which this code is one predecessor) covered the loads of the pair after the next in every step.
     __builtin_amdgcn_sched_barrier(0);
     load_pair(first);
     __builtin_amdgcn_sched_barrier(0);

@@ -13,20 +13,21 @@ static int packed_mode(const DevFormat& f) {
                                         : B_PACKED_GENERIC;
 }
 
-// Dense: one launch, with the tile a cost model makes fastest.  A launch runs its tiles in waves of (CUs x workgroups that
-// share a CU); a wave costs f + s per 128 of K and not less than w, all three by the number of co-resident workgroups, and a
-// last wave that leaves CUs idle costs a part of a full one.  Both tables are fitted to 334 problems (widths 896 ... 24576,
-// reductions 896 ... 12288, 33 ... 8192 rows, every tile timed): the choice costs 0.24 per cent over the fastest blocked tile
-// on average, 0.46 over the fastest row tile.
+// Dense: one launch, with the tile a cost model makes fastest.  A launch runs its tiles in waves of (CUs x workgroups
+// that share a CU); a wave costs f + s per 128 of K and not less than w, all three by the number of co-resident
+// workgroups, and a last wave that leaves CUs idle costs a part of a full one.  Both tables are fitted to 334 problems
+// (widths 896 ... 24576, reductions 896 ... 12288, 33 ... 8192 rows, every tile timed): the choice costs 0.24 per cent
+// over the fastest blocked tile on average, 0.46 over the fastest row tile.
 struct Cand {
     int bm, bn, occ;
     float f[4], s[4], w[4];   // per wave, by co-resident workgroups 1..occ: fixed us, us per 128 of K, least us
     float low, mid;           // a wave on half of the CUs or fewer / on three quarters of them costs this part of a full one
 };
-// Activations by rows, staged in LDS.  What the table encodes: 256x256 moves the fewest LDS bytes per MFMA; the small tiles share
-// a CU and lose less to a ragged tile count; with no more 64x64 tiles than CUs two K groups per tile put eight waves on
-// a CU, and with no more 64x32 tiles than CUs four K groups of two waves do.  (Three 64x64 tiles on a CU: fitted apart to single waves of 513 ...
-// 768 of them, 2048 x 2048 at 1152 rows 14.3 us where the first fit gave 11.8 and 128x128 takes 12.9.)
+// Activations by rows, staged in LDS.  What the table encodes: 256x256 moves the fewest LDS bytes per MFMA; the small
+// tiles share a CU and lose less to a ragged tile count; with no more 64x64 tiles than CUs two K groups per tile put
+// eight waves on a CU, and with no more 64x32 tiles than CUs four K groups of two waves do.  (Three 64x64 tiles on a
+// CU: fitted apart to single waves of 513 ... 768 of them, 2048 x 2048 at 1152 rows 14.3 us where the first fit gave
+// 11.8 and 128x128 takes 12.9.)
 static const Cand ROW_TILES[7] = {
     {256, 256, 1, {9.46f}, {1.772f}, {18.9f}, 0.78f, 0.86f},
     {256, 128, 1, {5.97f}, {0.857f}, {11.5f}, 0.865f, 0.93f},
@@ -36,12 +37,13 @@ static const Cand ROW_TILES[7] = {
     {64, 64, 1, {2.51f}, {0.233f}, {4.81f}, 1.0f, 1.05f},    // two K groups
     {64, 32, 1, {2.41f}, {0.157f}, {4.145f}, 1.0f, 1.05f},   // four K groups
 };
-// Blocked activations, read by the waves themselves.  Workgroups of four waves share a CU (two of 256x128, three of 128x64, four
-// of 64x64): their barriers and epilogues do not coincide, which eight waves of one workgroup cannot avoid.  Eight waves
-// on one tile are faster where the launch has no more than a tile per CU.  The entries of 256x256 and of eight waves on 256x128 are fitted
-// to 741 problems in which such launches are many (each tile timed; 200 of them with 120 ... 260 of those tiles, five times in turn): the
-// choice costs 0.37 per cent over the fastest tile on average there, 1.05 without 256x256 and with the entry that eight waves on
-// 256x128 had when launches of 129 ... 192 tiles were few (1024 x 6144 x 4096, MXFP4, 34.5 us for 28.6).
+// Blocked activations, read by the waves themselves.  Workgroups of four waves share a CU (two of 256x128, three of
+// 128x64, four of 64x64): their barriers and epilogues do not coincide, which eight waves of one workgroup cannot
+// avoid.  Eight waves on one tile are faster where the launch has no more than a tile per CU.  The entries of 256x256
+// and of eight waves on 256x128 are fitted to 741 problems in which such launches are many (each tile timed; 200 of
+// them with 120 ... 260 of those tiles, five times in turn): the choice costs 0.37 per cent over the fastest tile on
+// average there, 1.05 without 256x256 and with the entry that eight waves on 256x128 had when launches of 129 ... 192
+// tiles were few (1024 x 6144 x 4096, MXFP4, 34.5 us for 28.6).
 static const Cand BLOCKED_TILES[6] = {
     {256, 128, 2, {6.11f, 8.34f}, {0.966f, 1.498f}, {4.2f, 2.3f}, 0.914f, 0.96f},
     {256, 256, 1, {12.7f}, {1.46f}, {18.7f}, 0.813f, 0.856f},
@@ -81,15 +83,16 @@ static TileChoice fastest_tile(const Cand* cand, int first, int last, long M, lo
     return best;
 }
 
-// The layout a dense layer's activations are quantized into, and with it the kernel: the blocked tiles, the few-row kernel
-// (blocked as well) or the row tiles, by their models.  The quantizer takes 0.3 us longer for blocks.  Beyond the few-row
-// kernel's range only the row tiles with K groups were ever the fastest of all (up to 1.4 times, narrow layers); within it the
-// blocked tiles have to be a tenth faster (wide layers at 100 rows and more are: 128 x 12288 x 2048 9.3 us for 10.7).
-// The few-row kernel's model takes no launch in.  On the 61 problems of up to 128 rows the choice costs 0.1 per cent over the
-// fastest kernel on average.  Formats whose codes are looked up: a tile's weights are decoded again by each of its row groups,
-// once by the few-row kernel, which is worth half as much again.
-// No table gives less than `least`, so the smallest calls, which the host bounds, look no further.  The four-wave 256x128 tile,
-// which some formats do not take (launch_dense), never decides: the same layout with and without it on 250 000 drawn problems.
+// The layout a dense layer's activations are quantized into, and with it the kernel: the blocked tiles, the few-row
+// kernel (blocked as well) or the row tiles, by their models.  The quantizer takes 0.3 us longer for blocks.  Beyond
+// the few-row kernel's range only the row tiles with K groups were ever the fastest of all (up to 1.4 times, narrow
+// layers); within it the blocked tiles have to be a tenth faster (wide layers at 100 rows and more are: 128 x 12288 x
+// 2048 9.3 us for 10.7). The few-row kernel's model takes no launch in.  On the 61 problems of up to 128 rows the
+// choice costs 0.1 per cent over the fastest kernel on average.  Formats whose codes are looked up: a tile's weights
+// are decoded again by each of its row groups, once by the few-row kernel, which is worth half as much again. No table
+// gives less than `least`, so the smallest calls, which the host bounds, look no further.  The four-wave 256x128 tile,
+// which some formats do not take (launch_dense), never decides: the same layout with and without it on 250 000 drawn
+// problems.
 enum { BY_ROWS = 0, BLOCKED = 1 };   // and FEW_ROWS
 static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
     const int cus = device_cus();
@@ -109,12 +112,13 @@ static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
 static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
     if (a.blocked == FEW_ROWS) return launch_skinny(a, bmode, s);
     if (a.blocked) {
-        // The four-wave 256x128 tile and the 256x256 one read K in steps of 64.  With a byte per 32 weights and a row of those 128
-        // bytes or longer they read a cache line per weight row and step for two of them, and the vector L1 does not hold the lines
-        // until the next step: four waves on 6001 x 6144 x 4096 161 us against 152 of the eight waves (2-bit codes 144 / 148; K = 2048
-        // 66.6 / 68.8); 256x256 against the fastest other tile 0.98 times as fast with more than 192 tiles, 1.02 with fewer.  Table
-        // decode does not fit the registers of the four waves, and 256x256 is 1.07 times slower with it (40 problems; 12288 x
-        // 4096 at 896 rows 123 us, 108 on 256x64).
+        // The four-wave 256x128 tile and the 256x256 one read K in steps of 64.  With a byte per 32 weights and a row
+        // of those 128 bytes or longer they read a cache line per weight row and step for two of them, and the vector
+        // L1 does not hold the lines until the next step: four waves on 6001 x 6144 x 4096 161 us against 152 of the
+        // eight waves (2-bit codes 144 / 148; K = 2048 66.6 / 68.8); 256x256 against the fastest other tile 0.98 times
+        // as fast with more than 192 tiles, 1.02 with fewer.  Table decode does not fit the registers of the four
+        // waves, and 256x256 is 1.07 times slower with it (40 problems; 12288 x 4096 at 896 rows 123 us, 108 on
+        // 256x64).
         const bool wide_codes = (bmode == B_PACKED_E8M0 || bmode == B_PACKED_B16M) && a.K >= 4096;
         const bool many = 4LL * ((a.M + 255) / 256) * ((a.N + 255) / 256) > 3 * device_cus();
         const int first = bmode == B_PACKED_GENERIC || (wide_codes && many) ? 2 : wide_codes ? 1 : 0;
@@ -232,7 +236,8 @@ int scmx_mm_w4a8_prefers_blocked(int M, int N, int K) {
     return dense_layout(nullptr, M, N, K) != BY_ROWS;
 }
 
-// The fused layer quantizes into whichever layout suits the shape (dense_layout).  Both layouts take (M rounded up to 32) x K bytes at most.
+// The fused layer quantizes into whichever layout suits the shape (dense_layout).  Both layouts take (M rounded up to
+// 32) x K bytes at most.
 static int quantize_and_multiply(const scmx_format* fmt, const uint16_t* x, int8_t* xq, float* xs, bool room_for_blocks,
                                  const uint32_t* codes, const uint8_t* bcodes, const float* wscale, const uint16_t* res,
                                  void* out, int epi, int M, int N, int K, void* stream) {
@@ -335,7 +340,8 @@ int scmx_linear_w4a8_static(const scmx_format* fmt, const uint16_t* x, const uin
     int8_t* xq = reinterpret_cast<int8_t*>(base);
     float* xs = reinterpret_cast<float*>(base + STATIC_XQ_BYTES);
     // every byte of xq and xs[M] that the GEMM reads is written by the quantization first (in the blocked layout: the
-    // whole last 32-row block, rows past M as zeros): nothing has to start at zero, whatever the previous call left behind
+    // whole last 32-row block, rows past M as zeros): nothing has to start at zero, whatever the previous call left
+    // behind
     const size_t Mp = (size_t(M) + 31) & ~size_t(31);
     const bool room = Mp * size_t(K) <= STATIC_XQ_BYTES && Mp <= size_t(STATIC_MAX_ROWS);
     return quantize_and_multiply(fmt, x, xq, xs, room, codes, bcodes, wscale, res, out, epi, M, N, K, stream);

@@ -17,27 +17,28 @@
 
 namespace scmx {
 
-// MF, the shape of the MFMA.  At the chip's power limit (all-zero operands run a third faster) and on INT8 operands as they
-// occur, a loop of MFMAs alone reaches 4420 TOP/s with 16x16x64 and 3740 with 32x32x32 (half the accumulator traffic per
-// multiply-add): gate|up of 12288 x 2048 at 8192 rows, same tile, 208 us with the latter and 199 with the former.  A launch
-// bound elsewhere is far from that limit, and 32x32x32 takes half the instructions: the packed tile (bound by the vector ALU
-// that decodes its weights) uses it, 16-block power-of-two format, 64 experts of 2048 x 2048 / 257 of 1024 x 2048, 70 rows
-// each: 50.2 -> 47.7 and 109 -> 104 us.
+// MF, the shape of the MFMA.  At the chip's power limit (all-zero operands run a third faster) and on INT8 operands as
+// they occur, a loop of MFMAs alone reaches 4420 TOP/s with 16x16x64 and 3740 with 32x32x32 (half the accumulator
+// traffic per multiply-add): gate|up of 12288 x 2048 at 8192 rows, same tile, 208 us with the latter and 199 with the
+// former.  A launch bound elsewhere is far from that limit, and 32x32x32 takes half the instructions: the packed tile
+// (bound by the vector ALU that decodes its weights) uses it, 16-block power-of-two format, 64 experts of 2048 x 2048 /
+// 257 of 1024 x 2048, 70 rows each: 50.2 -> 47.7 and 109 -> 104 us.
 //
-// FD = number of register buffers of the split operand's fragments: fetched FD - 1 phases (half k slices) ahead of their MFMAs.
+// FD = number of register buffers of the split operand's fragments: fetched FD - 1 phases (half k slices) ahead of
+// their MFMAs.
 // SKIP (grouped launches): a row tile that ends inside its expert's segment multiplies only the 16-row blocks that hold
 // valid rows.  The two waves that share a SIMD then own the same columns and different row halves of the tile, so that
 // a half-empty tile halves the MFMA work of every SIMD instead of idling two of the four.
-// PK (the FP4-conversion formats, K steps of 128): the weights stay packed in LDS -- 64 bytes of codes per row and
-// K step plus the step's block-code bytes -- and every wave decodes its own fragments after reading them.  Half the
+// PK (the FP4-conversion formats, K steps of 128): the weights stay packed in LDS -- 64 bytes of codes per row and K
+// step plus the step's block-code bytes -- and every wave decodes its own fragments after reading them.  Half the
 // weight bytes through LDS in both directions, paid with one decode per wave row that shares the fragment.
-// KG > 1 (small problems: fewer tiles than CUs): KG groups of WGM x WGN waves share the tile, each multiplies its own
-// K / KG of the reduction out of LDS stages of its own, and the INT32 partial sums meet in LDS before the epilogue (exact:
-// integer addition is associative).  A CU then runs KG times the waves on the same tile count.
-// AD (ADM 1, dense: activations in the blocked layout; ADM 2, grouped: rows, gathered): the activation tile does not pass
-// through LDS; every wave loads the fragments of its own rows from memory, two K steps ahead: four runs of 256 bytes from
-// the blocked layout, sixteen of 64 from rows.  Waves must then not share rows (WGN = 1, or few column groups), and only the
-// weight rows of a stage exist in LDS.
+// KG > 1 (small problems: fewer tiles than CUs): KG groups of WGM x WGN waves share the tile, each multiplies its own K
+// / KG of the reduction out of LDS stages of its own, and the INT32 partial sums meet in LDS before the epilogue
+// (exact: integer addition is associative).  A CU then runs KG times the waves on the same tile count.
+// AD (ADM 1, dense: activations in the blocked layout; ADM 2, grouped: rows, gathered): the activation tile does not
+// pass through LDS; every wave loads the fragments of its own rows from memory, two K steps ahead: four runs of 256
+// bytes from the blocked layout, sixteen of 64 from rows.  Waves must then not share rows (WGN = 1, or few column
+// groups), and only the weight rows of a stage exist in LDS.
 template <int BM, int BN, int BK, int WGM, int WGN, int BMODE, int OCC = 1, int FD = 2, bool SKIP = false, bool PK = false,
           int KG = 1, int ADM = 0, int MF = 16>
 __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const GemmArgs a) {
@@ -109,8 +110,9 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         n0 = (j >> 3) * BN;
         const int E = a.n_experts;
         if (slot >= a.tstart[E]) return;
-        // largest e with tstart[e] <= slot: every lane probes one of up to 64 evenly spaced entries of the range, so 64 experts
-        // take one trip to memory and 4096 two (a binary search: six and twelve, in front of the first operand load)
+        // largest e with tstart[e] <= slot: every lane probes one of up to 64 evenly spaced entries of the range, so 64
+        // experts take one trip to memory and 4096 two (a binary search: six and twelve, in front of the first operand
+        // load)
         int lo = 0, n = E;
         while (n > 1) {
             const int step = (n + 63) >> 6, at = int(threadIdx.x & 63) * step;
@@ -127,8 +129,9 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         int pid = blockIdx.x;
         const int total = num_m * num_n;
         if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);   // neighbours in tile order share an XCD
-        // Tile order: bands of 4 row tiles, inside a band column by column.  The 32 workgroups an XCD runs at once
-        // then share 4 activation panels and 8 weight panels (what its L2 holds) however large M is.
+        // Tile order: bands of 4 row tiles, inside a band column by column.  The 32 to 128 workgroups
+        // an XCD runs at once (one to four a CU) then share 4 activation panels and 8 to 32 weight panels however large
+        // M is.  (Four was measured with one workgroup a CU.)
         constexpr int GM = 4;
         const int band = pid / (GM * num_n), r = pid % (GM * num_n);
         const int rows_in_band = min(GM, num_m - band * GM);
@@ -337,8 +340,8 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
             for (int r = 0; r < 4 * AG; ++r) acc[i][j][r] = 0;
 
-    // fragment addresses: lane l supplies row l % MF and the 16 k-bytes of part l / MF of a k slice (64 wide in four parts, or
-    // 32 in two); block origins are multiples of MF rows, so the swizzle term depends on the lane only
+    // fragment addresses: lane l supplies row l % MF and the 16 k-bytes of part l / MF of a k slice (64 wide in four
+    // parts, or 32 in two); block origins are multiples of MF rows, so the swizzle term depends on the lane only
     constexpr int PARTS = 64 / MF, KS = BK / (16 * PARTS);   // k slices of a step
     const int lr = lane % MF, part = lane / MF;
     const int sw = (lr / RPB) & (CPR - 1);
@@ -381,10 +384,11 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
         for (int j = 0; j < NI; ++j) w_rmin[j] = e8m0_row_min(a.wscale[erow + min(n0 + wn * WTN + j * MF + lr, a.N - 1)]);
     }
-    // AD: the activations come in 32-row x 32-k blocks of 1 KB, 16 bytes of a row per piece, piece (row % 32, k / 16 % 2) at
-    // (k / 16 % 2) * 512 + (row % 32) * 16, block (m / 32, k / 32) at ((m / 32) * (K / 32) + k / 32) KB.  A fragment (16
-    // rows x 64 k) is then four runs of 256 bytes.  Every wave loads the fragments of its own rows straight into registers,
-    // two K steps ahead, in three buffers that rotate with the LDS stages: the activation tile never passes through LDS.
+    // AD: the activations come in 32-row x 32-k blocks of 1 KB, 16 bytes of a row per piece, piece (row % 32, k / 16 %
+    // 2) at (k / 16 % 2) * 512 + (row % 32) * 16, block (m / 32, k / 32) at ((m / 32) * (K / 32) + k / 32) KB.  A
+    // fragment (16 rows x 64 k) is then four runs of 256 bytes.  Every wave loads the fragments of its own rows
+    // straight into registers, two K steps ahead, in three buffers that rotate with the LDS stages (two where the largest
+    // wave tile leaves no registers for a third): the activation tile never passes through LDS.
     constexpr int NAB = MF == 16 && ACC16 > 16 ? 2 : NSTAGE;   // the largest wave tiles have registers for two buffers only (below)
     [[maybe_unused]] v4i fad[NAB][KS][MI];
     [[maybe_unused]] int ad_src[ADR ? MI : WTM / 32];
@@ -429,9 +433,9 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     store_lds(r0, 0, 0);
     store_lds(r1, 1, BK);
     load_global(r0, 2 * BK);
-    // The loads stay apart, in the order the K loop issues them (activations of a step, then the weights two steps ahead of
-    // them): the loop's first copy has two predecessors (this code and the loop's end) and waits for the fewer outstanding
-    // loads of the two -- interleaved here, that wait covered the younger set as well, in every trip
+    // The loads stay apart, in the order the K loop issues them (activations of a step, then the weights two steps
+    // ahead of them): the loop's first copy has two predecessors (this code and the loop's end) and waits for the fewer
+    // outstanding loads of the two -- interleaved here, that wait covered the younger set as well, in every trip
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (AD) {
         load_ad(1, min(BK, KL - BK));
@@ -535,10 +539,10 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     };
     static_assert(!PK || NKP == 2, "the pair buffers return to phase 0 every K step");
 
-    // MF = 16: a step runs in phases, two per 64-wide k slice: the operand with more 16-row blocks in the wave's tile is split,
-    // one half of its fragments per phase, and fetched FD - 1 phases ahead into FD rotating register buffers; the other
-    // operand's fragments are held for the slice and fetched one slice ahead, half of them in each phase.  The fragments
-    // fetched at the end of an iteration belong to the next step's stage.
+    // MF = 16: a step runs in phases, two per 64-wide k slice: the operand with more 16-row blocks in the wave's tile
+    // is split, one half of its fragments per phase, and fetched FD - 1 phases ahead into FD rotating register buffers;
+    // the other operand's fragments are held for the slice and fetched one slice ahead, half of them in each phase.
+    // The fragments fetched at the end of an iteration belong to the next step's stage.
     // MF = 32: a phase is a 32-wide k slice with the fragments of all of the wave's rows and columns.
     constexpr bool F16 = MF == 16;
     constexpr bool SPLITN = AD || NI >= MI;                 // the split operand: weights (columns) or activations (rows)
@@ -590,8 +594,8 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int q = 0; q < AHEAD; ++q) load_split(sm, q, fs[q]);
     }
     // The k slices of an iteration are fenced against each other for the scheduler: left alone, the compiler sinks every
-    // LDS write of the step to its end, in front of the barrier (M = 8192: 442 -> 429 us over the four layers with the
-    // fences on the 256x256 tile; M = 128 ... 1024 on the small tiles: 2-3 %).
+    // LDS write of the step to its end, in front of the barrier (32x32x32 MFMAs, M = 8192: 442 -> 429 us over the four
+    // layers with the fences on the 256x256 tile; M = 128 ... 1024 on the small tiles: 2-3 %).
     auto iteration_staged = [&](auto step_tag, auto parity_tag, auto stage_tag, Staged& r, int kt) __attribute__((always_inline)) {
         constexpr int rd = decltype(step_tag)::value;        // kt % 3: stage of step kt
         constexpr bool ST = decltype(stage_tag)::value;      // false in the last two steps: nothing left to stage

@@ -145,12 +145,13 @@ __device__ __forceinline__ uint32_t unsigned_zeros(uint32_t c) {
     return m | (c & (m + 0x77777777u) & 0x88888888u);
 }
 
-// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: vector ALU: three trial roundings with their error sums.
-// The codes come from the conversion, which takes a midpoint to the even code where the host takes the lower one.  bf16 weights have
-// eight bits: 2^-12 smaller, one on a midpoint lies below it and no other changes sides.  float32 weights are converted as they are and
-// 2^-23 smaller: where both agree so does the host (a midpoint whose even code is the lower one, or none near); the others' blocks
-// take the arithmetic.  12288 x 2048 bf16: 22.2 us; 28.8 with that arithmetic for every weight, 44 with the near ties summed by one lane of the wave, 234 us
-// with a lane per weight and every candidate in float64 across lanes.
+// nb = K / BLOCK blocks per row, `rows` rows per workgroup.  Bound: vector ALU: three trial roundings with their error
+// sums. The codes come from the conversion, which takes a midpoint to the even code where the host takes the lower one.
+// bf16 weights have eight bits: 2^-12 smaller, one on a midpoint lies below it and no other changes sides.  float32
+// weights are converted as they are and 2^-23 smaller: where both agree so does the host (a midpoint whose even code is
+// the lower one, or none near); the others' blocks take the arithmetic.  12288 x 2048 bf16: 22.2 us; 28.8 with that
+// arithmetic for every weight, 44 with the near ties summed by one lane of the wave, 234 us with a lane per weight and
+// every candidate in float64 across lanes.
 template <int BLOCK, bool BF16>
 __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                          uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
@@ -188,16 +189,18 @@ __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict
 #pragma unroll
                 for (int i = 0; i < BLOCK; ++i) x[i] = __builtin_amdgcn_ldexpf(v[i], -e0);
                 const float s0 = fp4_sq_err<BLOCK>(x, 1.0f), sm = fp4_sq_err<BLOCK>(x, 0.5f), sp = fp4_sq_err<BLOCK>(x, 2.0f);
-                // A float32 sum of 32 squares of exact differences is within 32 half-ulps (2e-6) of the exact one, the host's
-                // float64 sum within 1e-14: apart by more than 1e-5, the sums order alike.  (Below 1e-30 squares underflow.)
+                // A float32 sum of 32 squares of exact differences is within 32 half-ulps (2e-6) of the exact one, the
+                // host's float64 sum within 1e-14: apart by more than 1e-5, the sums order alike.  (Below 1e-30 squares
+                // underflow.)
                 auto close = [](float a, float b) { return !(fabsf(a - b) > 1e-5f * fmaxf(a, b)) || fmaxf(a, b) < 1e-30f; };
                 const float s1 = sm < s0 ? sm : s0;
                 tie = close(sm, s0) || close(sp, s1);
                 chosen = sp < s1 ? e0 + 1 : sm < s0 ? e0 - 1 : e0;
             }
         }
-        // Near ties in float64.  A few of them the wave takes one after the other, a lane per weight (about 1.5 us each); where
-        // many lanes have one, each sums its own (15 us in all, as one does: a matrix of a few rows waited for its one tie).
+        // Near ties in float64.  A few of them the wave takes one after the other, a lane per weight (about 1.5 us
+        // each); where many lanes have one, each sums its own (15 us in all, as one does: a matrix of a few rows waited
+        // for its one tie).
         uint64_t ties = __ballot(tie);
         auto decide = [&](double t0, double tm, double tp) {
             double best = t0;
@@ -219,7 +222,8 @@ __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict
                 ties &= ties - 1;
                 const int e = __shfl(e0, src, WAVE), group = lane / BLOCK;
                 const double a = double(weight(base + size_t(b0 + src) * BLOCK + lane % BLOCK));
-                // lane group 0: exponent e, group 1: e - 1, the others e + 1 (of 32 lanes there are two groups: once more)
+                // lane group 0: exponent e, group 1: e - 1, the others e + 1 (of 32 lanes there are two groups: once
+                // more)
                 const double first = lane_sq_err<BLOCK>(a, group == 0 ? e : group == 1 ? e - 1 : e + 1);
                 const double third = BLOCK == 16 ? first : lane_sq_err<BLOCK>(a, e + 1);
                 const double t0 = __shfl(first, 0, WAVE), tm = __shfl(first, BLOCK, WAVE);
@@ -355,8 +359,8 @@ __device__ __forceinline__ int family_index(const FamilyArgs& f, float x) {   //
     for (int i = 0; i < 7; ++i) idx += int(a > f.cut[i]);
     return idx;
 }
-// sign(a) times its magnitude, for a >= 0: a zero has no sign and costs nothing, also where the smallest magnitude is not 0
-// (in the E2M1 codebook it is).
+// sign(a) times its magnitude, for a >= 0: a zero has no sign and costs nothing, also where the smallest magnitude is
+// not 0 (in the E2M1 codebook it is).
 template <bool E2M1>
 __device__ __forceinline__ float family_level(const FamilyArgs& f, float a) {
     float v = !E2M1 && a > 0.0f ? f.cb[0] : 0.0f;
@@ -408,8 +412,8 @@ __device__ __forceinline__ float family_sq_err_e2m1(const float (&aw)[BLOCK], fl
                      __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
 }
 
-// That error to within the bound below, at 4 instructions per weight: one quotient, the conversion there and back, two fused
-// multiply-adds.
+// That error to within the bound below, at 4 instructions per weight: one quotient, the conversion there and back, two
+// fused multiply-adds.
 template <int BLOCK>
 __device__ __forceinline__ float family_sq_err_near(const float (&aw)[BLOCK], float sc, float h) {   // h = 0.5 / sc
     float r0 = 0.0f, r1 = 0.0f;
@@ -432,23 +436,25 @@ __device__ __forceinline__ float family_sq_err_near(const float (&aw)[BLOCK], fl
     }
     return r0 + r1;
 }
-// How far the root of that sum can be from the root of the host's, twice (the two sides of a comparison), in parts of the norm of
-// the weights summed over.  With D_i the distance of weight i to the nearest level, D_i <= |w_i| (zero is a level): the level taken is
-// the nearest to a quotient 2^-21.4 off at most, so the difference to it exceeds D_i by 2^-20.4 |w_i| at most; seventeen additions
-// are 2^-20 of the sum, 2^-20.9 of its root.  The host's own roundings are 2^-21 of the norm.  By the triangle inequality 1.75 x 2^-20 in all,
-// twice 2^-18.2; for a row, whose sum of block errors rounds by 2^-20.4 of its root on either side, 2^-17.3.
+// How far the root of that sum can be from the root of the host's, twice (the two sides of a comparison), in parts of
+// the norm of the weights summed over.  With D_i the distance of weight i to the nearest level, D_i <= |w_i| (zero is a
+// level): the level taken is the nearest to a quotient 2^-21.4 off at most, so the difference to it exceeds D_i by
+// 2^-20.4 |w_i| at most; seventeen additions are 2^-20 of the sum, 2^-20.9 of its root.  The host's own roundings are
+// 2^-21 of the norm.  By the triangle inequality 1.75 x 2^-20 in all, twice 2^-18.2; for a row, whose sum of block
+// errors rounds by 2^-20.4 of its root on either side, 2^-17.3.
 constexpr float NEAR = 7.62939453125e-6f;   // 2^-17
 
 constexpr int FAM_ROWS = 4;   // rows per workgroup at most: more are needed only for K < 1024, and their tables cost LDS
 
-// Bound: vector ALU.  In the E2M1 codebook a trial is first evaluated to 2^-19 (family_sq_err_near): that settles nearly every
-// multiplier of a block and base, and all but one or two of a row's bases; only what it leaves open is evaluated as the host does.
-// Multipliers run from the largest down and end where clipping the block's largest weight alone costs more than the best so far, in every
-// lane.  2048 x 2048 bf16, ten multipliers: 67 us; 130 with every trial as the host evaluates it (13 instructions a weight), 520 with
-// a lane per weight, a correctly rounded division per trial and the sums across lanes.
-// BASES: 1 where there are fewer blocks than lanes, each of which would run all trials of one (64 x 128, ten multipliers 27 -> 11 us).
-// In the E2M1 codebook 4 beyond that: twice the waves to hide the conversions' latency and the uneven number of trials (600 x 2048
-// 44 us with all eight in a thread, 34 with four; 4096 x 2048 114 and 116).
+// Bound: vector ALU.  In the E2M1 codebook a trial is first evaluated to 2^-19 (family_sq_err_near): that settles
+// nearly every multiplier of a block and base, and all but one or two of a row's bases; only what it leaves open is
+// evaluated as the host does. Multipliers run from the largest down and end where clipping the block's largest weight
+// alone costs more than the best so far, in every lane.  2048 x 2048 bf16, ten multipliers: 67 us; 130 with every trial
+// as the host evaluates it (13 instructions a weight), 520 with a lane per weight, a correctly rounded division per
+// trial and the sums across lanes.
+// BASES: 1 where there are fewer blocks than lanes, each of which would run all trials of one (64 x 128, ten
+// multipliers 27 -> 11 us). In the E2M1 codebook 4 beyond that: twice the waves to hide the conversions' latency and
+// the uneven number of trials (600 x 2048 44 us with all eight in a thread, 34 with four; 4096 x 2048 114 and 116).
 template <int BLOCK, bool BF16, bool E2M1, int BASES>   // bases per thread
 __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
                                                              uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
@@ -492,7 +498,8 @@ __global__ __launch_bounds__(QNT) void quantize_family_kernel(const void* __rest
     };
 
     // ---- per candidate base and block: the best multiplier and its error ------------------------------------------
-    // The trial of one scale as the host evaluates it (a scale near the ends of the float32 range leaves its reciprocal no room).
+    // The trial of one scale as the host evaluates it (a scale near the ends of the float32 range leaves its reciprocal
+    // no room).
     auto in_range = [](float sc) { return sc > 1e-30f && sc < 1e30f; };
     auto trial = [&](const float (&aw)[BLOCK], float sc) {
         bool same = false;
@@ -727,8 +734,9 @@ extern "C" int scmx_quantize_family(const scmx_format* fmt, const void* w, int w
     f.bc_bits = fmt->bc_bits;
     if (N == 0) return SCMX_OK;
     const int nb = K / block;
-    // us, a thread per block and base / four bases a thread, bf16 in 16-blocks with ten multipliers: 640 x 896 22 / 26, 1000 x 896
-    // 25 / 28, 600 x 2048 35 / 33.  Other codebooks (a thread per base / per block): 269 x 896 42 / 56, 1000 x 896 66 / 56.
+    // us, a thread per block and base / four bases a thread, bf16 in 16-blocks with ten multipliers: 640 x 896 22 / 26,
+    // 1000 x 896 25 / 28, 600 x 2048 35 / 33.  Other codebooks (a thread per base / per block): 269 x 896 42 / 56, 1000
+    // x 896 66 / 56.
     const bool e2m1 = df.lut_lo == 0x03020100u && df.lut_hi == 0x0C080604u, spread = long(N) * nb <= (e2m1 ? 65536 : 32768);
     const int rows = rows_per_group(spread ? 8 * nb : e2m1 ? 2 * nb : nb, FAM_ROWS);
     const size_t smem = size_t(rows) * 8 * nb * (sizeof(float) + 1);

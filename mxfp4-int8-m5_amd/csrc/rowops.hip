@@ -482,8 +482,8 @@ __global__ __launch_bounds__(NT) void qkv_headnorm128_kernel(const uint16_t* __r
 }
 
 // ---- OLMoE q/k/v split with RMSNorm over the full h*d width ------------------------------------------------------
-// ROPE: also the rotary embedding of q and k and the append to the caches (RopeArgs, as above).  (Tested in the loops instead,
-// the plain form took 7 % longer: seven heads of 96, 1000 rows 6.1 us against 5.7.)
+// ROPE: also the rotary embedding of q and k and the append to the caches (RopeArgs, as above).  (Tested in the loops
+// instead, the plain form took 7 % longer: seven heads of 96, 1000 rows 6.1 us against 5.7.)
 template <bool ROPE>
 __global__ __launch_bounds__(NT) void qkv_fullnorm_kernel(const uint16_t* __restrict__ y, const uint16_t* __restrict__ qn,
                                                           const uint16_t* __restrict__ kn, float eps, uint16_t* __restrict__ q,
@@ -529,10 +529,10 @@ __global__ __launch_bounds__(NT) void qkv_fullnorm_kernel(const uint16_t* __rest
     }
 }
 
-// The same for W = 512 * CH and head dims of 16 ... 512 that are powers of two: a wave per part (q, k, v) of a row, the part
-// in registers, 16-byte accesses, and a rotation partner d / 16 lanes away.  Same bits (wave_row_sumsq).  Bound: HBM
-// (read 3 W, write 3 W bf16 per row).  The array operations it replaces after a norm kernel of its own were 22 launches a
-// block: two blocks of an OLMoE prompt of 3000 tokens 1591 -> 1130 us, of a decode step 752 -> 319 us.
+// The same for W = 512 * CH and head dims of 16 ... 512 that are powers of two: a wave per part (q, k, v) of a row, the
+// part in registers, 16-byte accesses, and a rotation partner d / 16 lanes away.  Same bits (wave_row_sumsq).  Bound:
+// HBM (read 3 W, write 3 W bf16 per row).  The array operations it replaces after a norm kernel of its own were 22
+// launches a block: two blocks of an OLMoE prompt of 3000 tokens 1591 -> 1130 us, of a decode step 752 -> 319 us.
 template <int CH>
 __global__ __launch_bounds__(192) void qkv_fullnorm_wave_kernel(const uint16_t* __restrict__ y, const uint16_t* __restrict__ qn,
                                                                 const uint16_t* __restrict__ kn, float eps,
@@ -638,10 +638,11 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const int32_t* __restr
 }
 
 // ---- MoE: the same counting sort over several workgroups, one launch -----------------------------------------------
-// Workgroup g owns assignments [g * 1024, (g + 1) * 1024), the last one also the tail of fewer than 1024.  Every workgroup counts
-// ALL assignments (they lie in the L2), those before its own apart, so that it knows its experts' first rows without hearing from
-// the others.  That costs R / 1024 LDS atomics a thread and saves two dependent launches: 24000 assignments over 64 experts 8.2
-// us against 11.7 with counting, scanning and placing launched one after the other.
+// Workgroup g owns assignments [g * 1024, (g + 1) * 1024), the last one also the tail of fewer than 1024.  Every
+// workgroup counts ALL assignments (they lie in the L2), those before its own apart, so that it knows its experts'
+// first rows without hearing from the others.  That costs R / 1024 LDS atomics a thread and saves two dependent
+// launches: 24000 assignments over 64 experts 8.2 us against 11.7 with counting, scanning and placing launched one
+// after the other.
 constexpr int RS_CHUNK = 1024;
 
 // Inclusive prefix sums of a and b over the workgroup's 1024 threads.
@@ -717,9 +718,9 @@ __global__ __launch_bounds__(RS_CHUNK) void route_sort_wide_kernel(const int32_t
 }
 
 // ---- and over more, three launches ---------------------------------------------------------------------------------
-// A workgroup's per-expert counts, and later its per-expert first rows, are parked in pos[g * 1024 + e] (E <= 1024), i.e. inside the
-// part of `pos` that only this workgroup writes in the last pass, so no extra memory is needed and no workgroup reads
-// what another one may already have overwritten.
+// A workgroup's per-expert counts, and later its per-expert first rows, are parked in pos[g * 1024 + e] (E <= 1024),
+// i.e. inside the part of `pos` that only this workgroup writes in the last pass, so no extra memory is needed and no
+// workgroup reads what another one may already have overwritten.
 __global__ __launch_bounds__(RS_CHUNK) void route_count_kernel(const int32_t* __restrict__ inds, int R, int E,
                                                                int32_t* __restrict__ pos) {
     __shared__ uint32_t cnt[1024];
@@ -863,8 +864,9 @@ __global__ __launch_bounds__(NT) void moe_combine_kernel(const uint16_t* __restr
     block_quant_row(nrow_s, K, xq + size_t(row) * K, xs + row, red);
 }
 
-// The same with a wave per row and the row in its registers from the first load to the codes: no LDS, no barriers, and the
-// rows' loads overlap freely.  Bound: HBM, top-k rows of y read per row written.  Same arithmetic, same order of sums, same bits.
+// The same with a wave per row and the row in its registers from the first load to the codes: no LDS, no barriers, and
+// the rows' loads overlap freely.  Bound: HBM, top-k rows of y read per row written.  Same arithmetic, same order of
+// sums, same bits.
 template <int CH>
 __global__ __launch_bounds__(256) void moe_combine_wave_kernel(const uint16_t* __restrict__ y, const int32_t* __restrict__ pos,
                                                                const uint16_t* __restrict__ scores, const uint16_t* __restrict__ sscore,
@@ -979,8 +981,8 @@ static bool row_shape_ok(const char* who, int rows, int K, int max_k) {
 // taken per lane in rising j and then by the butterfly wave_sum.  The k winners are found by k wave-wide maxima over
 // the key (probability bits << 16 | 65535 - j): largest probability first, equal ones by rising expert index.
 constexpr int ROUTE_MAX_E = 1024;
-// PER = experts per lane the kernel is built for (64 * PER >= E): slots past E cost what live ones do, so the launch picks
-// the smallest of 1, 2, 4, 8, 16 that covers E.  The arithmetic of the live slots does not depend on PER.
+// PER = experts per lane the kernel is built for (64 * PER >= E): slots past E cost what live ones do, so the launch
+// picks the smallest of 1, 2, 4, 8, 16 that covers E.  The arithmetic of the live slots does not depend on PER.
 template <int PER>
 __global__ __launch_bounds__(NT) void route_topk_kernel(const uint16_t* __restrict__ logits,
                                                         const uint16_t* __restrict__ shared_logit, int M, int E, int topk,
@@ -1042,11 +1044,11 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const uint16_t* __restri
 }
 
 // ---- one decode row: RMSNorm, its INT8 codes and a small bf16 linear (the router) on it, one launch ---------------------
-// What rmsnorm_quant with its bf16 row and linear_bf16 give, bit for bit (the same device functions, the same products by the same waves,
-// summed in the same order).  A workgroup per 16 rows of the matrix, whose loads are all requested before the norm, which
-// every workgroup takes for itself.  Bound: launch and two trips to memory; 64 x 2048 with the routing behind it 7.35 us against
-// 11.3 for three launches.  (With the
-// routing in it as well, in one workgroup, 256 KB came through one CU: 11.1 us, no less than three launches.)
+// What rmsnorm_quant with its bf16 row and linear_bf16 give, bit for bit (the same device functions, the same products
+// by the same waves, summed in the same order).  A workgroup per 16 rows of the matrix, whose loads are all requested
+// before the norm, which every workgroup takes for itself.  Bound: launch and two trips to memory; 64 x 2048 with the
+// routing behind it 7.35 us against 11.3 for three launches.  (With the routing in it as well, in one workgroup, 256 KB
+// came through one CU: 11.1 us, no less than three launches.)
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 template <int CH>
 __global__ __launch_bounds__(512) void norm_linear_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, float eps,
@@ -1201,8 +1203,8 @@ static dim3 headnorm_grid(int L, int heads) {
     return dim3(L, L >= 256 ? 1 : groups);
 }
 
-// Many rows of bf16 input with head dim 128 and 16-byte aligned operands take the kernel with 16-byte accesses (a few rows
-// are spread over more workgroups by the general one).
+// Many rows of bf16 input with head dim 128 and 16-byte aligned operands take the kernel with 16-byte accesses (a few
+// rows are spread over more workgroups by the general one).
 static bool headnorm128_fits(const int32_t* acc, const uint16_t* y, const uint16_t* qn, const uint16_t* kn, const uint16_t* q,
                              const uint16_t* k, const uint16_t* v, int L, int d) {
     return !acc && d == 128 && L >= 16 &&
@@ -1389,8 +1391,8 @@ int scmx_route_sort(const int32_t* inds, int M, int topk, int n_experts, int tm,
         route_sort_kernel<<<dim3(1), dim3(1024), 0, st>>>(inds, int(R), topk, n_experts, tm, pos, tok, esorted, off, tstart);
         return check_launch("route_sort");
     }
-    // us, one launch / three: 16000 assignments 7.2 / 11.4, 36864 10.6 / 11.7, 54000 13.2 / 12.8; the atomics of few experts meet:
-    // 8 experts 16000 9.0 / 10.7, 24000 11.1 / 11.1, 40000 16.6 / 11.4
+    // us, one launch / three: 16000 assignments 7.2 / 11.4, 36864 10.6 / 11.7, 54000 13.2 / 12.8; the atomics of few
+    // experts meet: 8 experts 16000 9.0 / 10.7, 24000 11.1 / 11.1, 40000 16.6 / 11.4
     if (R <= 40960 && R <= 3072LL * n_experts) {
         route_sort_wide_kernel<<<dim3(G), dim3(RS_CHUNK), 0, st>>>(inds, int(R), topk, n_experts, tm, pos, tok, esorted, off, tstart);
         return check_launch("route_sort");
@@ -1411,9 +1413,10 @@ int scmx_moe_combine(const uint16_t* y, const int32_t* pos, const uint16_t* scor
         return SCMX_ERR_ARG;
     }
     if (Mp == 0) return SCMX_OK;
-    // A wave per row from 1024 rows on, where the waves fill the chip; below, a row's workgroup is the shorter chain.  Eight
-    // slots, us by workgroup / by wave: 1024 x 2048 13.8 / 11.2, 3000 x 2048 29.7 / 24.4, 8192 x 2048 76 / 74, without the
-    // codes 21.8 / 20.1 at 3000; at K = 4096 a lane's registers leave too few waves (1024 rows without codes 15.2 / 16.3).
+    // A wave per row from 1024 rows on, where the waves fill the chip; below, a row's workgroup is the shorter chain.
+    // Eight slots, us by workgroup / by wave: 1024 x 2048 13.8 / 11.2, 3000 x 2048 29.7 / 24.4, 8192 x 2048 76 / 74,
+    // without the codes 21.8 / 20.1 at 3000; at K = 4096 a lane's registers leave too few waves (1024 rows without
+    // codes 15.2 / 16.3).
     if (Mp >= 1024 && K % 512 == 0 && K <= 2048 && (uintptr_t(y) | uintptr_t(res) | uintptr_t(h)) % 16 == 0 &&
         (!xq || (uintptr_t(w) | uintptr_t(xq)) % 16 == 0)) {
         auto go = [&](auto kernel) {
