@@ -22,7 +22,9 @@ struct Cand {
     int bm, bn, occ;
     float f[4], s[4], w[4];   // per wave, by co-resident workgroups 1..occ: fixed us, us per 128 of K, least us
     float low, mid;           // a wave on half of the CUs or fewer / on three quarters of them costs this part of a full one
+    int waves;                // ONE, SEVERAL: only for launches of that many
 };
+enum { ONE = 1, SEVERAL = 2 };
 // Activations by rows, staged in LDS.  What the table encodes: 256x256 moves the fewest LDS bytes per MFMA; the small
 // tiles share a CU and lose less to a ragged tile count; with no more 64x64 tiles than CUs two K groups per tile put
 // eight waves on a CU, and with no more 64x32 tiles than CUs four K groups of two waves do.  (Three 64x64 tiles on a
@@ -39,16 +41,16 @@ static const Cand ROW_TILES[7] = {
 };
 // Blocked activations, read by the waves themselves.  Workgroups of four waves share a CU (two of 256x128, three of
 // 128x64, four of 64x64): their barriers and epilogues do not coincide, which eight waves of one workgroup cannot
-// avoid.  Eight waves on one tile are faster where the launch has no more than a tile per CU.  The entries of 256x256
-// and of eight waves on 256x128 are fitted to 741 problems in which such launches are many (each tile timed; 200 of
-// them with 120 ... 260 of those tiles, five times in turn): the choice costs 0.37 per cent over the fastest tile on
-// average there, 1.05 without 256x256 and with the entry that eight waves on 256x128 had when launches of 129 ... 192
-// tiles were few (1024 x 6144 x 4096, MXFP4, 34.5 us for 28.6).
-static const Cand BLOCKED_TILES[6] = {
+// avoid.  Eight waves on one tile are faster where the launch has no more than a tile per CU.  The one-wave entries are
+// fitted to 741 problems in which such launches are many (each tile timed; 200 of them with 120 ... 260 tiles, five
+// times in turn): the choice costs 0.37 per cent over the fastest tile on average there, 1.05 without 256x256 and with
+// the entry for several waves (1024 x 6144 x 4096, MXFP4, 34.5 us for 28.6).
+static const Cand BLOCKED_TILES[7] = {
     {256, 128, 2, {6.11f, 8.34f}, {0.966f, 1.498f}, {4.2f, 2.3f}, 0.914f, 0.96f},
-    {256, 256, 1, {12.7f}, {1.46f}, {18.7f}, 0.813f, 0.856f},
-    {256, 128, 1, {6.96f}, {0.802f}, {11.5f}, 0.856f, 0.806f},   // eight waves
-    {256, 64, 1, {3.945f}, {0.416f}, {2.4f}, 0.98f, 1.05f},      // eight waves
+    {256, 256, 1, {12.7f}, {1.46f}, {18.7f}, 0.813f, 0.856f, ONE},
+    {256, 128, 1, {5.51f}, {0.805f}, {11.5f}, 0.9f, 0.85f, ONE},       // eight waves
+    {256, 128, 1, {5.51f}, {0.805f}, {11.5f}, 0.85f, 0.93f, SEVERAL},  // eight waves
+    {256, 64, 1, {3.945f}, {0.416f}, {2.4f}, 0.98f, 1.05f},            // eight waves
     {128, 64, 3, {3.78f, 4.09f, 2.62f}, {0.34f, 0.498f, 0.806f}, {3.83f, 5.3f, 3.0f}, 0.925f, 0.98f},
     {64, 64, 4, {3.15f, 3.54f, 3.58f, 1.83f}, {0.294f, 0.419f, 0.618f, 0.782f}, {5.49f, 4.07f, 2.67f, 3.0f}, 0.95f, 1.0f},
 };
@@ -65,6 +67,7 @@ static TileChoice fastest_tile(const Cand* cand, int first, int last, long M, lo
         const long n = ((M + k.bm - 1) >> __builtin_ctz(k.bm)) * ((N + k.bn - 1) >> __builtin_ctz(k.bn));
         if (cand == ROW_TILES && c >= 5 && (n > cus || K % (c == 5 ? 256 : 512))) continue;   // K groups
         const long cap = cus * k.occ;
+        if (k.waves && (n <= cap) != (k.waves == ONE)) continue;
         const long full = n < cap ? 0 : n / cap, rest = n - full * cap;
         float t = float(full) * fmaxf(k.f[k.occ - 1] + steps * k.s[k.occ - 1], k.w[k.occ - 1]);
         if (rest) {
@@ -101,7 +104,7 @@ static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
     const float least = fmaxf(3.8f, 2.41f + 0.157f / 128.0f * float(K));
     if (few < least) return FEW_ROWS;
     const float rows = fastest_tile(ROW_TILES, small ? 0 : 5, 6, M, N, K, cus).us;
-    const float blocks = (0.3f + fastest_tile(BLOCKED_TILES, 0, 5, M, N, K, cus).us) * (small ? 1.1f : 1.0f);
+    const float blocks = (0.3f + fastest_tile(BLOCKED_TILES, 0, 6, M, N, K, cus).us) * (small ? 1.1f : 1.0f);
     const float tile = fminf(rows, blocks);
     if (few < tile) return FEW_ROWS;
     DevFormat f;
@@ -122,7 +125,7 @@ static void launch_dense(const GemmArgs& a, int bmode, hipStream_t s) {
         const bool wide_codes = (bmode == B_PACKED_E8M0 || bmode == B_PACKED_B16M) && a.K >= 4096;
         const bool many = 4LL * ((a.M + 255) / 256) * ((a.N + 255) / 256) > 3 * device_cus();
         const int first = bmode == B_PACKED_GENERIC || (wide_codes && many) ? 2 : wide_codes ? 1 : 0;
-        return launch_blocked(a, bmode, fastest_tile(BLOCKED_TILES, first, 5, a.M, a.N, a.K, device_cus()).index, s);
+        return launch_blocked(a, bmode, fastest_tile(BLOCKED_TILES, first, 6, a.M, a.N, a.K, device_cus()).index, s);
     }
     launch_rows(a, bmode, fastest_tile(ROW_TILES, 0, 6, a.M, a.N, a.K, device_cus()).index, s);
 }

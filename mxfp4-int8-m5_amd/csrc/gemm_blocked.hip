@@ -15,11 +15,12 @@ void launch_blocked(const GemmArgs& a, int bmode, int tile, hipStream_t s) {
         case 0: return launch_tile<256, 128, 64, 4, 1, 2, 2, false, false, 1, 1, 16, FP4_MODES>(a, bmode, rows256, s);
         case 1: return launch_tile<256, 256, 64, 4, 2, 1, 2, false, false, 1, 1, 32, FP4_MODES>(a, bmode, rows256, s);
         case 2:
+        case 3:
             if (bmode == B_PACKED_GENERIC || 8LL * rows256 * ((a.N + 127) / 128) <= 5 * cus)
                 return launch_tile<256, 128, 128, 8, 1, 1, 2, false, false, 1, 1, 32, PACKED_MODES>(a, bmode, rows256, s);
             return launch_tile<256, 128, 128, 8, 1, 1, 2, false, false, 1, 1, 16, FP4_MODES>(a, bmode, rows256, s);
-        case 3: return launch_tile<256, 64, 128, 8, 1, 1, 2, false, false, 1, 1, 16, PACKED_MODES>(a, bmode, rows256, s);
-        case 4: return launch_tile<128, 64, 128, 4, 1, 2, 2, false, false, 1, 1, 16, PACKED_MODES>(a, bmode, (a.M + 127) / 128, s);
+        case 4: return launch_tile<256, 64, 128, 8, 1, 1, 2, false, false, 1, 1, 16, PACKED_MODES>(a, bmode, rows256, s);
+        case 5: return launch_tile<128, 64, 128, 4, 1, 2, 2, false, false, 1, 1, 16, PACKED_MODES>(a, bmode, (a.M + 127) / 128, s);
         default: return launch_tile<64, 64, 128, 2, 2, 2, 2, false, false, 1, 1, 16, PACKED_MODES>(a, bmode, (a.M + 63) / 64, s);
     }
 }

@@ -18,16 +18,18 @@ def table(name):
     for line in body.splitlines():
         head = [int(x) for x in re.match(r"\s*\{(\d+), (\d+), (\d+),", line).groups()]
         lists = [[float(x.rstrip("f")) for x in re.findall(number, l)] for l in re.findall(r"\{([^{}]*)\}", line[line.index("{") + 1:])]
-        low, mid = (float(x) for x in re.search(r"\}, ([\d.]+)f, ([\d.]+)f\}", line).groups())
-        rows.append((*head, *lists, low, mid))
+        low, mid, waves = re.search(r"\}, ([\d.]+)f, ([\d.]+)f(?:, (ONE|SEVERAL))?\}", line).groups()
+        rows.append((*head, *lists, float(low), float(mid), waves))
     return rows
 
 
 def chosen(name, m, n, k, cus=256):
-    times = []
-    for i, (bm, bn, occ, f, s, w, low, mid) in enumerate(table(name)):
+    times = {}
+    for i, (bm, bn, occ, f, s, w, low, mid, waves) in enumerate(table(name)):
         if name == "ROW_TILES" and i >= 5 and (-(-m // bm) * -(-n // bn) > cus or k % (256 if i == 5 else 512)):
             continue   # K groups
+        if waves and (-(-m // bm) * -(-n // bn) <= cus * occ) != (waves == "ONE"):
+            continue
         full, rest = divmod(-(-m // bm) * -(-n // bn), cus * occ)
         cost = lambda r: max(f[r - 1] + k / 128 * s[r - 1], w[r - 1])
         t = full * cost(occ)
@@ -36,8 +38,8 @@ def chosen(name, m, n, k, cus=256):
         elif rest:
             fill = rest / cus
             t += cost(1) * (low if fill <= 0.5 else low + (mid - low) * (fill - 0.5) * 4 if fill <= 0.75 else mid + (1 - mid) * (fill - 0.75) * 4)
-        times.append(t)
-    return times.index(min(times))
+        times[i] = t
+    return min(times, key=times.get)
 
 
 @pytest.mark.parametrize("name,tile,m,n,k", [(name, t, *s) for name, tiles in (("BLOCKED_TILES", BLOCKED), ("ROW_TILES", ROWS))

@@ -31,13 +31,14 @@ def product(xq, q):
 # (tile of the blocked table on 256 CUs, shapes): every tail of each tile's rotating loop (test_gemm_tile_choice.py checks the tiles)
 BLOCKED = [(0, [(1154, 10396, 128), (588, 10004, 384), (518, 10076, 640), (1030, 11864, 4224)]),   # 256x128, four waves (or, by format, another)
            (1, [(935, 12296, 1536), (935, 12296, 1664), (772, 11664, 2176), (653, 11248, 4224)]),  # 256x256
-           (2, [(400, 9368, 4096), (588, 6584, 4224), (393, 8640, 5760), (393, 8640, 5888), (393, 8640, 6016), (393, 8640, 6144), (393, 8640, 6272),
-                (677, 8212, 512), (645, 8376, 640), (392, 12292, 768), (515, 10144, 896), (530, 9812, 1024),
-                (518, 10316, 1280)]),                                                              # 256x128, eight waves, both MFMA shapes
-           (3, [(216, 8564, 256), (146, 11004, 384), (148, 11192, 512), (134, 11848, 640), (130, 10900, 768), (137, 11804, 896)]),   # 256x64
-           (4, [(278, 180, 128), (319, 136, 256), (235, 136, 384), (154, 224, 512), (165, 340, 640), (133, 3888, 768),
+           (2, [(400, 9368, 4096), (588, 6584, 4224), (455, 8240, 4352), (454, 8284, 4480), (387, 9476, 4608), (391, 9536, 4736),
+                (645, 8376, 640), (392, 12292, 768), (515, 10144, 896), (530, 9812, 1024), (518, 10316, 1280),
+                (273, 11488, 4224)]),                                                              # 256x128, eight waves, both MFMA shapes
+           (3, [(1581, 11764, 4224)]),                                                             # the same, several waves of tiles
+           (4, [(216, 8564, 256), (146, 11004, 384), (148, 11192, 512), (134, 11848, 640), (130, 10900, 768), (137, 11804, 896)]),   # 256x64
+           (5, [(278, 180, 128), (319, 136, 256), (235, 136, 384), (154, 224, 512), (165, 340, 640), (133, 3888, 768),
                 (4133, 196, 896)]),                                                                # 128x64
-           (5, [(142, 7200, 128), (137, 6856, 256), (149, 8264, 384), (142, 8452, 512), (131, 8704, 640), (141, 144, 768),
+           (6, [(142, 7200, 128), (137, 6856, 256), (149, 8264, 384), (142, 8452, 512), (131, 8704, 640), (141, 144, 768),
                 (134, 316, 896)])]                                                                 # 64x64
 
 
