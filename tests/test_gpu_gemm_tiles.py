@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from oracle import layout
+from oracle import bf16, layout, linear
 from tests.util import FORMATS, blocked_layout, dev, host, product_format, random_packed
 
 pytestmark = pytest.mark.gpu
@@ -42,6 +42,10 @@ BLOCKED = [(0, [(1154, 10396, 128), (588, 10004, 384), (518, 10076, 640), (1030,
                 (134, 316, 896)])]                                                                 # 64x64
 
 
+# whichever tile they take
+MORE = [(400, 12296, 384), (1030, 12296, 640), (385, 12288, 4224), (1000, 6152, 768), (1500, 4104, 2048), (600, 4104, 2048),
+        (1030, 2052, 1280), (515, 8200, 640), (1025, 8192, 384), (4099, 2052, 128), (770, 1032, 1280), (129, 1028, 256), (300, 260, 896)]
+
 # the same for the larger tiles by rows, which multiply with 32x32x32 up to three quarters of a tile per CU
 ROWS = [(0, [(706, 12476, 384), (705, 12352, 512), (642, 10944, 640), (661, 10996, 768), (968, 12392, 256), (796, 12556, 384)]),      # 256x256
         (1, [(709, 5456, 512), (387, 8396, 640), (262, 11020, 768), (257, 11732, 896), (268, 10892, 1152), (265, 10984, 1536),
@@ -65,7 +69,7 @@ def test_row_tiles(m, n, k, name):
 
 
 @pytest.mark.parametrize("name", list(NAMES))
-@pytest.mark.parametrize("m,n,k", [s for _, shapes in BLOCKED for s in shapes])
+@pytest.mark.parametrize("m,n,k", [s for _, shapes in BLOCKED for s in shapes] + MORE)
 def test_blocked_tiles(m, n, k, name):
     from mxfp4_int8_m5_amd import sc_kernels as S
     rng = np.random.default_rng(m + n + k)
@@ -73,6 +77,24 @@ def test_blocked_tiles(m, n, k, name):
     xq = rng.integers(-127, 128, (-(-m // 32) * 32, k)).astype(np.int8)
     xb = S.BlockedXq(dev(blocked_layout(xq)), m, k)
     assert torch.equal(S.mm_i8_i32(xb, S.PackedWq(codes, bc, n, k, fmt, ws))[:m], product(dev(xq)[:m], q))
+
+
+# a shape per tile that multiplies with 32x32x32, by layout
+@pytest.mark.parametrize("epi", [1, 2, 3])
+@pytest.mark.parametrize("m,n,k,blocked", [(935, 12296, 1536, True), (400, 9368, 4096, True), (706, 12480, 384, False), (709, 5456, 512, False),
+                                           (135, 10944, 4096, False), (67, 8288, 128, False)])
+def test_epilogues_of_launches_that_leave_cus_idle(m, n, k, blocked, epi):
+    """Bit for bit against the oracle's epilogue of the exact sums, output rows that are whole 16-byte pieces and not."""
+    from mxfp4_int8_m5_amd import sc_kernels as S
+    rng = np.random.default_rng(m + n + epi)
+    c, b, w, q = random_packed(rng, n, k, FORMATS[0])
+    xq = rng.integers(-127, 128, (-(-m // 32) * 32, k)).astype(np.int8)
+    xs = (2.0 ** -7 * (0.5 + rng.random(m))).astype(np.float32)
+    res = bf16.to_bits(rng.standard_normal((m, n)).astype(np.float32)) if epi == 2 else None
+    x = S.BlockedXq(dev(blocked_layout(xq)), m, k) if blocked else dev(xq[:m])
+    got = S.mm_epi(x, S.PackedWq(dev(c), dev(b), n, k, product_format(FORMATS[0]), dev(w)), dev(xs), dev(w), epi,
+                   res=dev(res) if epi == 2 else None)
+    assert np.array_equal(host(got), linear.epilogue(host(product(dev(xq)[:m], dev(q))), xs, w, epi, res))
 
 
 def grouped(e, n, k, tm, name, counts, rng):
