@@ -18,7 +18,7 @@ struct GemmArgs {
     int bc_row_bytes;
     int epi;
     const int32_t* off;      // grouped: expert segment offsets [E+1]; dense: NULL
-    const uint16_t* silu;    // SwiGLU epilogue: lookup table over bf16 gate values
+    const uint16_t* silu;    // SwiGLU epilogue: the table of the rounded sigmoid
     const int32_t* tstart;   // grouped: first row tile of each expert [E+1]
     int n_experts;
     int sub_log2;            // grouped: a segment's row tile is 1 << sub_log2 of the kernel's

@@ -129,8 +129,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
         for (int i = 0; i < 4; ++i) y[i] = __fmul_rn(__fmul_rn(float(tot[i]), xs), ws[i]);
         uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
         if (a.epi == SCMX_EPI_SWIGLU) {   // rows (g, g, u, u)
-            const uint32_t lo = swiglu_lut(a.silu, y[0], round_bf16(y[2])), hi = swiglu_lut(a.silu, y[1], round_bf16(y[3]));
-            *reinterpret_cast<uint32_t*>(out + size_t(m) * (N / 2) + n / 2) = lo | (hi << 16);
+            *reinterpret_cast<uint32_t*>(out + size_t(m) * (N / 2) + n / 2) = swiglu_lut2(a.silu, y[0], y[1], y[2], y[3]);
             continue;
         }
         if (a.epi == SCMX_EPI_RES) {

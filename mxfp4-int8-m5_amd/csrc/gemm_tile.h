@@ -89,6 +89,14 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // scales of the tile's rows and columns, fetched before the K loop so that the epilogue does not start with a
     // round trip to memory
     __shared__ __attribute__((aligned(16))) float s_xs[BM], s_ws[BN];
+    // SwiGLU: the sigmoid's table (8 KB), copied to LDS while the first operands are on their way, where it costs the CU
+    // no workgroup (all but the packed expert tiles); the lookups go to memory otherwise.  A wave's 64 gates lie in some
+    // 30 cache lines, which the vector L1 serves one after the other.  With the 65536-entry table of silu(g) in memory,
+    // two conversions and one lookup at a time instead of two, 12288 x 2048 at 2048 rows took 57.3 us for 53.0, at 1500
+    // 51.1 for 49.4, at 256 12.0 for 11.1; 6144 x 4096 at 6000 rows 152.5 for 148.4.
+    constexpr int CU_WGS = OCC * 4 * 64 / (NT * KG) > 1 ? OCC * 4 * 64 / (NT * KG) : 1;
+    constexpr bool SIG = !PK && SMEM_BYTES + (BM + BN) * 4 + int(sizeof(uint16_t)) * 2 * int(SIGMOID_ENTRIES) <= 160 * 1024 / CU_WGS;
+    __shared__ __attribute__((aligned(16))) uint16_t s_sig[SIG ? 2 * SIGMOID_ENTRIES : 8];
     auto swz = [](int row, int chunk) { return row * BK + ((chunk ^ ((row / RPB) & (CPR - 1))) << 4); };
     // packed weight rows (64 bytes, 4 chunks): 4 rows per sweep of the banks, chunk c of row r at c ^ ((r / 4) % 4)
     auto swzp = [](int row, int chunk) { return row * (BK / 2) + ((chunk ^ ((row >> 2) & 3)) << 4); };
@@ -224,6 +232,15 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     for (int j = 0; j < WS_PER; ++j) {
         const int c = tid + j * NT;
         ws_reg[j] = (a.xscale && c < BN && n0 + c < a.N) ? a.wscale[size_t(expert) * a.N + n0 + c] : 0.0f;
+    }
+
+    constexpr int SIG_PER = (2 * int(SIGMOID_ENTRIES) / 8 + NT * KG - 1) / (NT * KG);   // 16-byte pieces of the table a thread copies
+    [[maybe_unused]] u32x4 sig_reg[SIG_PER];
+    const bool sig_copy = SIG && a.epi == SCMX_EPI_SWIGLU;
+    if (sig_copy) {
+#pragma unroll
+        for (int j = 0; j < SIG_PER; ++j)
+            sig_reg[j] = reinterpret_cast<const u32x4*>(a.silu)[min(int(threadIdx.x) + j * NT * KG, 2 * int(SIGMOID_ENTRIES) / 8 - 1)];
     }
 
     // Two register sets hold the global loads of two K steps in flight.
@@ -428,6 +445,11 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
         for (int j = 0; j < WS_PER; ++j)
             if (tid + j * NT < BN) s_ws[tid + j * NT] = ws_reg[j];
+    }
+    if (sig_copy) {
+#pragma unroll
+        for (int j = 0; j < SIG_PER; ++j)
+            if (int(threadIdx.x) + j * NT * KG < 2 * int(SIGMOID_ENTRIES) / 8) reinterpret_cast<u32x4*>(s_sig)[int(threadIdx.x) + j * NT * KG] = sig_reg[j];
     }
     if constexpr (AD) load_ad(0, 0);
     store_lds(r0, 0, 0);
@@ -815,9 +837,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                 y[r] = __fmul_rn(__fmul_rn(float(acc[i][j][4 * g + r]), xs), w4[r]);
             uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
             if (epi == SCMX_EPI_SWIGLU) {   // (g, g, u, u) -> two outputs
-                const uint16_t s0 = swiglu_lut(a.silu, y[0], round_bf16(y[2]));
-                const uint16_t s1 = swiglu_lut(a.silu, y[1], round_bf16(y[3]));
-                const uint32_t o = uint32_t(s0) | (uint32_t(s1) << 16);
+                const uint32_t o = swiglu_lut2(SIG ? s_sig : a.silu, y[0], y[1], y[2], y[3]);
                 if (W)
                     *reinterpret_cast<uint32_t*>(wtile + row * rsb + col) = o;
                 else if (m < row_end && n < N)
@@ -825,8 +845,8 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                 continue;
             }
             u32x2 o;
-            o[0] = uint32_t(f32_to_bf16(y[0])) | (uint32_t(f32_to_bf16(y[1])) << 16);
-            o[1] = uint32_t(f32_to_bf16(y[2])) | (uint32_t(f32_to_bf16(y[3])) << 16);
+            o[0] = f32_to_bf16x2(y[0], y[1]);
+            o[1] = f32_to_bf16x2(y[2], y[3]);
             if (W) {
                 *reinterpret_cast<u32x2*>(wtile + row * rsb + col * 2) = o;   // the residual is added on the way out
             } else if (m < row_end && n < N) {
@@ -836,7 +856,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                     for (int r = 0; r < 2; ++r) {
                         const float lo = __fadd_rn(__uint_as_float(rr[r] << 16), __uint_as_float(o[r] << 16));
                         const float hi = __fadd_rn(__uint_as_float(rr[r] & 0xFFFF0000u), __uint_as_float(o[r] & 0xFFFF0000u));
-                        o[r] = uint32_t(f32_to_bf16(lo)) | (uint32_t(f32_to_bf16(hi)) << 16);
+                        o[r] = f32_to_bf16x2(lo, hi);
                     }
                 }
                 *reinterpret_cast<u32x2*>(out + size_t(m) * N + n) = o;
@@ -891,7 +911,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                 for (int r = 0; r < 4; ++r) {
                     const float lo = __fadd_rn(__uint_as_float(rr[i][r] << 16), __uint_as_float(v[i][r] << 16));
                     const float hi = __fadd_rn(__uint_as_float(rr[i][r] & 0xFFFF0000u), __uint_as_float(v[i][r] & 0xFFFF0000u));
-                    v[i][r] = uint32_t(f32_to_bf16(lo)) | (uint32_t(f32_to_bf16(hi)) << 16);
+                    v[i][r] = f32_to_bf16x2(lo, hi);
                 }
             }
             if (full[i])

@@ -314,15 +314,13 @@ __global__ __launch_bounds__(NT) void swiglu_quant_kernel(const int32_t* __restr
         const v4i u4 = *reinterpret_cast<const v4i*>(ar + F + 4 * c);
         const f32x4 wg = *reinterpret_cast<const f32x4*>(wscale + 4 * c);
         const f32x4 wu = *reinterpret_cast<const f32x4*>(wscale + F + 4 * c);
-        uint16_t o[4];
+        float g[4], u[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float g = __fmul_rn(__fmul_rn(float(g4[i]), xsr), wg[i]);
-            const float u = round_bf16(__fmul_rn(__fmul_rn(float(u4[i]), xsr), wu[i]));
-            o[i] = swiglu_lut(silu, g, u);   // table over the bf16 value of the gate
+            g[i] = __fmul_rn(__fmul_rn(float(g4[i]), xsr), wg[i]);
+            u[i] = __fmul_rn(__fmul_rn(float(u4[i]), xsr), wu[i]);
         }
-        *reinterpret_cast<u32x2*>(srow + 4 * c) =
-            u32x2{uint32_t(o[0]) | (uint32_t(o[1]) << 16), uint32_t(o[2]) | (uint32_t(o[3]) << 16)};
+        *reinterpret_cast<u32x2*>(srow + 4 * c) = u32x2{swiglu_lut2(silu, g[0], g[1], u[0], u[1]), swiglu_lut2(silu, g[2], g[3], u[2], u[3])};
     }
     __syncthreads();
     block_quant_row(srow, F, xq + size_t(row) * F, xs + row, red);

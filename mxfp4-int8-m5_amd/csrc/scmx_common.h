@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "../../include/scmx.h"
+#include "silu_table.h"
 
 namespace scmx {
 
@@ -70,6 +71,13 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {   // round to nearest
     __bf16 h = (__bf16)f;
     return __builtin_bit_cast(uint16_t, h);
 }
+__device__ __forceinline__ uint32_t f32_to_bf16x2(float lo, float hi) {   // two at once: one instruction
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+}
+__device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
 __device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 
 // ---- deterministic FP32 exp for a >= 0: IEEE multiply / add / rint only (no FMA contraction) ------------------
@@ -100,11 +108,22 @@ __device__ __forceinline__ uint16_t swiglu_bf16(float g, float u) {
     return f32_to_bf16(__fmul_rn(silu, u));
 }
 
-// Device address (current device) of the 65536-entry table silu[g] = bf16(g * sigmoid(g)) over bf16 gate bit patterns,
-// built at compile time from the same operation sequence as swiglu_bf16; NULL if the symbol cannot be resolved.
+// Device address (current device) of the table of the rounded sigmoid (silu_table.h: 2 x 2048 entries, built at compile
+// time from the same operation sequence as swiglu_bf16); NULL if the symbol cannot be resolved.
 const uint16_t* silu_table_device();
-__device__ __forceinline__ uint16_t swiglu_lut(const uint16_t* __restrict__ table, float g, float u) {
-    return f32_to_bf16(__fmul_rn(bf16_to_f32(table[f32_to_bf16(g)]), u));
+// Two outputs from unrounded gates and ups: conversions and the table's entries two at a time, packed.  The entries are
+// computed as byte offsets: 2 |g| less the first entry's, clamped, and the gate's sign in bit 12.
+__device__ __forceinline__ uint32_t swiglu_lut2(const uint16_t* __restrict__ table, float g0, float g1, float u0, float u1) {
+    static_assert(SIGMOID_ENTRIES == 2048, "the sign lands on bit 12");
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const uint32_t g = f32_to_bf16x2(g0, g1), u = f32_to_bf16x2(u0, u1);
+    const u16x2 twice = __builtin_bit_cast(u16x2, g) << u16x2{1, 1};
+    const u16x2 from = __builtin_elementwise_sub_sat(twice, u16x2{2 * SIGMOID_FIRST, 2 * SIGMOID_FIRST});
+    const u16x2 at = __builtin_elementwise_min(from, u16x2{2 * SIGMOID_ENTRIES - 2, 2 * SIGMOID_ENTRIES - 2});
+    const uint32_t e = __builtin_bit_cast(uint32_t, at) | ((g >> 3) & 0x10001000u);
+    const auto entry = [&](uint32_t byte) { return bf16_to_f32(*reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(table) + byte)); };
+    const uint32_t silu = f32_to_bf16x2(__fmul_rn(bf16_lo(g), entry(e & 0xFFFFu)), __fmul_rn(bf16_hi(g), entry(e >> 16)));
+    return f32_to_bf16x2(__fmul_rn(bf16_lo(silu), bf16_lo(u)), __fmul_rn(bf16_hi(silu), bf16_hi(u)));
 }
 
 // ---- 4-bit code decode -----------------------------------------------------------------------------------------

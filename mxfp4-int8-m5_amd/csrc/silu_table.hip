@@ -1,8 +1,7 @@
-// The SiLU lookup table as a device constant, and the host accessor that hands kernels its device address.
+// The table of the rounded sigmoid as a device constant, and the host accessor that hands kernels its device address.
 #include <atomic>
 
 #include "scmx_common.h"
-#include "silu_table.h"
 
 namespace scmx {
 

@@ -215,7 +215,7 @@ def test_linear_one_call(S, m, n, k):
 
 
 def test_swiglu_epilogue_every_gate_value(S):
-    """The SwiGLU epilogue looks silu(g) up in a 65536-entry table built at compile time.  Drive every bf16 bit
+    """The SwiGLU epilogue looks the sigmoid up in a table built at compile time.  Drive every bf16 bit
     pattern through it as the gate (acc = +-1, xscale = 1, wscale = the value itself) with two different up values
     and compare with the oracle's operation-by-operation bf16 evaluation: bit-exact for every finite gate, NaN where
     the oracle gives NaN."""
