@@ -297,6 +297,23 @@ int scmx_moe_mm(const scmx_format* fmt, const int8_t* xq, const float* xscale, c
                 const uint32_t* codes, const uint8_t* bcodes, const float* wscale, const int32_t* off,
                 const int32_t* tstart, int n_experts, int tm, int N, int K, int epi, void* out, void* stream);
 
+/* scmx_moe_mm on activations in SLOTS of 256 rows: off / tstart built for row tiles of 256, segment e's rows in slots
+ * tstart[e], tstart[e] + 1, ..., each slot 256 rows in the blocked layout of scmx_act_quant_blocked ((ceil(R / 256) + E) *
+ * 256 * K bytes at most, below 2^32; rows past a segment are not read into any result), xscale [R] by sorted row.  Same
+ * results.  Formats that decode with the FP4 conversion (the published one, its 16-block variant, 16-blocks with
+ * consecutive multipliers, standard MXFP4), K % 128 == 0.  The two kernels that fill the slots: the gather of quantized
+ * rows, out[slot row] = xq[gather[sorted row]] and out_scale [R] = xscale[gather[.]] (gather [R]), and the quantization of
+ * sorted bf16 rows x [R, K], K <= 12288 (scmx_act_quant's codes and scales).  All tensors 16-byte aligned.  No counterpart in
+ * the reference (its GEMM takes row-major operands). */
+int scmx_moe_gather_blocked(const int8_t* xq, const float* xscale, const int32_t* gather, const int32_t* off, const int32_t* tstart,
+                            int n_experts, int R, int K, int8_t* out, float* out_scale, void* stream);
+int scmx_act_quant_sorted(const uint16_t* x, const int32_t* off, const int32_t* tstart, int n_experts, int R, int K, int8_t* xq, float* xs,
+                          void* stream);
+int scmx_moe_mm_takes_slots(const scmx_format* fmt, int R, int n_experts, int K);   /* 1: all three do; 0 */
+int scmx_moe_mm_blocked(const scmx_format* fmt, const int8_t* xq, const float* xscale, int R, const uint32_t* codes,
+                        const uint8_t* bcodes, const float* wscale, const int32_t* off, const int32_t* tstart, int n_experts,
+                        int N, int K, int epi, void* out, void* stream);
+
 /* The two-pass variant on pre-unpacked INT8 weights [E*N, K].  Replaces moe_mm_i8, e2e/sc_moe.py:95-107,188-200. */
 int scmx_moe_mm_i8(const int8_t* xq, const float* xscale, const int32_t* gather, int R, const int8_t* wq,
                    const float* wscale, const int32_t* off, const int32_t* tstart, int n_experts, int tm, int N,

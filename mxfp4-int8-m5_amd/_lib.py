@@ -60,6 +60,10 @@ SIGNATURES = {
     "scmx_norm_linear": (_I, [_P, _P, _F, _P, _I, _I, _P, _P, _P, _P, _P]),
     "scmx_route_sort": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P]),
     "scmx_moe_mm": (_I, [_FMT, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P]),
+    "scmx_moe_gather_blocked": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
+    "scmx_act_quant_sorted": (_I, [_P, _P, _P, _I, _I, _I, _P, _P, _P]),
+    "scmx_moe_mm_takes_slots": (_I, [_FMT, _I, _I, _I]),
+    "scmx_moe_mm_blocked": (_I, [_FMT, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P]),
     "scmx_moe_mm_i8": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P]),
     "scmx_moe_combine": (_I, [_P, _P, _P, _P, _P, _P, _F, _P, _P, _P, _I, _I, _I, _I, _P]),
     "scmx_rot_quant": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),

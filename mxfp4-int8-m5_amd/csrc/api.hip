@@ -213,14 +213,39 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
 // (Registers are held to what lets four waves share a SIMD up to 6144 values, three up to 8192: 4000 rows x 6144 blocked 16.6
 // us at three, 13.0 at four.  Whole rows of up to 6144 in the row layout fit without it and are given fewer registers then:
 // 4096 values 76 for 82, six waves a SIMD for five, 3 - 6 per cent at 257 ... 1500 rows.)
-template <int CH, bool BLK, bool WHOLE>
+// SORT (BLK): the rows of x are sorted by expert and those of xq are the slots of the grouped GEMM, 256 rows each: row p of
+// a slot holds row p of that slot's part of the segment.  Of the rows past a segment only those of its last eight are
+// written (as zeros).
+struct SortedRows {
+    const int32_t *off, *tstart;   // as for the grouped GEMM
+    int n_experts;
+    // Workgroup b's 2^LOG rows, aligned in their slot: the first one and the segment's end among the sorted rows, and the
+    // first one's place in the slots; false: none.  Expert e's groups start at off[e] / 2^LOG + e, room enough for a cut one
+    // each, so R / 2^LOG + E workgroups cover every segment.  (A grid over the rows of all slots idles where experts have
+    // few: 8000 x 1024 over 64 experts 8.5 us for 5.9, 54000 x 512 over 257 30.5 for 20.4.)
+    template <int LOG>
+    __device__ bool rows(int b, int* first, int* end, int* place) const {
+        const int e = last_started(n_experts, b, [&](int i) { return (off[i] >> LOG) + i; });
+        const int o = off[e], r = (b - (o >> LOG) - e) << LOG;
+        *first = o + r;
+        *end = off[e + 1];
+        *place = (tstart[e] << 8) + r;
+        return *first < *end;
+    }
+};
+template <int CH, bool BLK, bool WHOLE, bool SORT = false>
 __global__ __launch_bounds__(BLK ? 512 : 256, !BLK && WHOLE && CH <= 12 ? 1 : CH <= 12 ? 4 : CH <= 16 ? 3 : 1) void act_quant_wave_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
-                                                                         float* __restrict__ xs, int M, int Mp, int K_any) {
+                                                                         float* __restrict__ xs, int M, int Mp, int K_any, SortedRows sort) {
     const int K = WHOLE ? 512 * CH : K_any;   // WHOLE: every lane has all of its CH pieces
     constexpr int RPW = BLK ? 8 : 4;
     constexpr int TURN = CH > 16 ? CH / 2 : CH;   // pieces whose codes are in LDS at once (at most 64 KB)
     __shared__ u32x2 tile[BLK ? TURN * 64 * 8 : 1];
-    const int wid = threadIdx.x >> 6, row0 = blockIdx.x * RPW, row = row0 + wid, lane = threadIdx.x & 63;
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int row0 = blockIdx.x * RPW, row = row0 + wid;   // of xq; of x and xs
+    if constexpr (SORT) {
+        if (!sort.rows<3>(blockIdx.x, &row, &M, &row0)) return;
+        row += wid;
+    }
     auto gather_store = [&](int j0) {   // BLK: the codes of pieces j0 .. j0 + TURN - 1 of every row, after all are in LDS
         __syncthreads();
         int8_t* const blk = xq + (size_t(row0 >> 5) * size_t(K >> 5)) * 1024;
@@ -249,7 +274,7 @@ __global__ __launch_bounds__(BLK ? 512 : 256, !BLK && WHOLE && CH <= 12 ? 1 : CH
                 }
             if (BLK) gather_store(j0);
         }
-        if (lane == 0) xs[row] = 0.0f;
+        if (!SORT && lane == 0) xs[row] = 0.0f;
         return;
     }
     const u32x4* xrow = reinterpret_cast<const u32x4*>(x + size_t(row) * K);
@@ -353,6 +378,43 @@ __global__ __launch_bounds__(WAVES * 64) void act_quant_row_kernel(const uint16_
         *at(c) = u32x4{lo[0], lo[1], hi[0], hi[1]};
     }
     if (tid == 0) xs[row] = s;
+}
+
+// ---- rows of xq, sorted by expert, into the grouped GEMM's blocked slots -------------------------------------------
+// A workgroup per 32-row block of a slot, its waves in turn on 512 of K: loads of 128 contiguous bytes of each of 8 rows,
+// stored as pieces of 8 rows x 16 bytes, whole 128-byte lines of the blocks.  Bound by the stores: 24000 rows of 2048
+// (every row eight times), 49 MB written, 16.8 us, the launch and four dependent trips to memory in it.
+__global__ __launch_bounds__(256) void moe_gather_blocked_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xscale,
+                                                                 const int32_t* __restrict__ gather, SortedRows sort, int K,
+                                                                 int8_t* __restrict__ out, float* __restrict__ out_scale) {
+    const int lane = threadIdx.x & 63;
+    int first, end, place;
+    if (!sort.rows<5>(blockIdx.x, &first, &end, &place)) return;
+    const int r8 = lane >> 3, c = lane & 7;   // row within eight, 16-byte piece within 128 bytes
+    const int8_t* src[4];
+    bool live[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const int r = first + 8 * g + r8;
+        live[g] = r < end;
+        const int from = gather[min(r, end - 1)];
+        src[g] = xq + size_t(from) * K + c * 16;
+        if (threadIdx.x < 64 && c == 0 && live[g]) out_scale[r] = xscale[from];
+    }
+    int8_t* const dst = out + size_t(place >> 5) * size_t(K >> 5) * 1024 + (c >> 1) * 1024 + (c & 1) * 512 + r8 * 16;
+    for (int k = (threadIdx.x >> 6) * 512; k < K; k += 2048) {
+        u32x4 v[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                if (k + 128 * q < K) v[q][g] = *reinterpret_cast<const u32x4*>(src[g] + k + 128 * q);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                if (k + 128 * q < K && live[g]) *reinterpret_cast<u32x4*>(dst + size_t((k >> 5) + 4 * q) * 1024 + g * 128) = v[q][g];
+    }
 }
 
 // ---- rot_quant: randomized Hadamard rotation of every 32-wide block, then per-token INT8 ---------------------------
@@ -469,14 +531,14 @@ static void launch_act_quant_rows(const uint16_t* x, int8_t* xq, float* xs, int 
     else act_quant_row_kernel<8, 2, BLK><<<dim3(Mp), dim3(512), 0, st>>>(x, xq, xs, M, K);
 }
 // A wave per row: the smallest number of register pieces that holds it.  False: the row is too long (or K % 32 != 0).
-template <bool BLK>
-static bool launch_act_quant_waves(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int K, hipStream_t st) {
+template <bool BLK, bool SORT = false>
+static bool launch_act_quant_waves(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int K, hipStream_t st, SortedRows sort = {}) {
     if (K % 32 || K > (BLK ? 12288 : 8192)) return false;
-    const dim3 grid(BLK ? unsigned(Mp) / 8u : (unsigned(Mp) + 3u) / 4u), block(BLK ? 512 : 256);
+    const dim3 grid(SORT ? unsigned(M) / 8u + unsigned(sort.n_experts) : BLK ? unsigned(Mp) / 8u : (unsigned(Mp) + 3u) / 4u), block(BLK ? 512 : 256);
     auto go = [&](auto ch) {
         constexpr int CH = decltype(ch)::value;
-        if (K == 512 * CH) act_quant_wave_kernel<CH, BLK, true><<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K);
-        else act_quant_wave_kernel<CH, BLK, false><<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K);
+        if (K == 512 * CH) act_quant_wave_kernel<CH, BLK, true, SORT><<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K, sort);
+        else act_quant_wave_kernel<CH, BLK, false, SORT><<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K, sort);
     };
     const int ch = (K + 511) / 512;
     if (ch <= 1) go(std::integral_constant<int, 1>{});
@@ -580,6 +642,44 @@ int scmx_act_quant(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int 
     else if (!launch_act_quant_waves<false>(x, xq, xs, M, Mp, K, st))
         act_quant_kernel<<<dim3(Mp), dim3(256), 0, st>>>(x, xq, xs, M, K);
     return check_launch("act_quant");
+}
+
+static int check_sorted(const char* who, const int32_t* off, const int32_t* tstart, int n_experts, int R, int K, SortedRows* s) {
+    if (!off || !tstart || n_experts < 1 || n_experts > (1 << 20) || R < 0 || K <= 0 || K % 128 ||
+        (uint64_t(R) / 256 + 1 + uint64_t(n_experts)) * 256 * uint64_t(K) > 0xFFFFFFFFull) {
+        set_error("%s: need off / tstart, 1 <= n_experts <= 2^20 (%d), K %% 128 == 0 (K = %d) and slots within 2^32 bytes (R = %d)", who,
+                  n_experts, K, R);
+        return SCMX_ERR_ARG;
+    }
+    *s = SortedRows{off, tstart, n_experts};
+    return SCMX_OK;
+}
+
+int scmx_moe_gather_blocked(const int8_t* xq, const float* xscale, const int32_t* gather, const int32_t* off, const int32_t* tstart,
+                            int n_experts, int R, int K, int8_t* out, float* out_scale, void* stream) {
+    SortedRows s;
+    if (int rc = check_sorted("moe_gather_blocked", off, tstart, n_experts, R, K, &s)) return rc;
+    if (!xq || !xscale || !gather || !out || !out_scale || uintptr_t(xq) % 16 || uintptr_t(out) % 16) {
+        set_error("moe_gather_blocked: null pointer argument, or xq / out not 16-byte aligned");
+        return SCMX_ERR_ARG;
+    }
+    if (R == 0) return SCMX_OK;
+    moe_gather_blocked_kernel<<<dim3(unsigned(R) / 32u + unsigned(n_experts)), dim3(256), 0, (hipStream_t)stream>>>(xq, xscale, gather, s, K,
+                                                                                                                out, out_scale);
+    return check_launch("moe_gather_blocked");
+}
+
+int scmx_act_quant_sorted(const uint16_t* x, const int32_t* off, const int32_t* tstart, int n_experts, int R, int K, int8_t* xq, float* xs,
+                          void* stream) {
+    SortedRows s;
+    if (int rc = check_sorted("act_quant_sorted", off, tstart, n_experts, R, K, &s)) return rc;
+    if (!x || !xq || !xs || uintptr_t(x) % 16 || uintptr_t(xq) % 16 || K > 12288) {
+        set_error("act_quant_sorted: need x, xq and xs, x and xq 16-byte aligned, K <= 12288 (K = %d)", K);
+        return SCMX_ERR_ARG;
+    }
+    if (R == 0) return SCMX_OK;
+    launch_act_quant_waves<true, true>(x, xq, xs, R, R, K, (hipStream_t)stream, s);
+    return check_launch("act_quant_sorted");
 }
 
 int scmx_rot_quant(const uint16_t* x, const float* signs, int8_t* xq, float* xs, int M, int Mp, int K, void* stream) {

@@ -368,9 +368,9 @@ static int moe_common(const char* who, const int8_t* xq, const float* xscale, co
     return SCMX_OK;
 }
 
-int scmx_moe_mm(const scmx_format* fmt, const int8_t* xq, const float* xscale, const int32_t* gather, int R,
-                const uint32_t* codes, const uint8_t* bcodes, const float* wscale, const int32_t* off,
-                const int32_t* tstart, int n_experts, int tm, int N, int K, int epi, void* out, void* stream) {
+static int moe_mm(const scmx_format* fmt, const int8_t* xq, const float* xscale, const int32_t* gather, int R,
+                  const uint32_t* codes, const uint8_t* bcodes, const float* wscale, const int32_t* off, const int32_t* tstart,
+                  int n_experts, int tm, int N, int K, int epi, void* out, int blocked, void* stream) {
     DevFormat f;
     if (int rc = make_dev_format(fmt, &f)) return rc;
     GemmArgs a;
@@ -387,8 +387,35 @@ int scmx_moe_mm(const scmx_format* fmt, const int8_t* xq, const float* xscale, c
     if (R == 0) return SCMX_OK;
     a.codes = codes; a.bcodes = bcodes; a.fmt = f;
     a.bc_row_bytes = K / f.block * f.bc_bits / 8;
+    a.blocked = blocked;
     launch_grouped(a, packed_mode(f), tm, (hipStream_t)stream);
     return check_launch("moe_mm");
+}
+
+int scmx_moe_mm(const scmx_format* fmt, const int8_t* xq, const float* xscale, const int32_t* gather, int R,
+                const uint32_t* codes, const uint8_t* bcodes, const float* wscale, const int32_t* off,
+                const int32_t* tstart, int n_experts, int tm, int N, int K, int epi, void* out, void* stream) {
+    return moe_mm(fmt, xq, xscale, gather, R, codes, bcodes, wscale, off, tstart, n_experts, tm, N, K, epi, out, 0, stream);
+}
+
+int scmx_moe_mm_takes_slots(const scmx_format* fmt, int R, int n_experts, int K) {
+    DevFormat f;
+    return R >= 0 && n_experts >= 1 && n_experts <= (1 << 20) && K > 0 && K % 128 == 0 && K <= 12288 &&
+           (uint64_t(R) / 256 + 1 + uint64_t(n_experts)) * 256 * uint64_t(K) <= 0xFFFFFFFFull &&
+           make_dev_format(fmt, &f) == SCMX_OK && packed_mode(f) != B_PACKED_GENERIC;
+}
+
+int scmx_moe_mm_blocked(const scmx_format* fmt, const int8_t* xq, const float* xscale, int R, const uint32_t* codes,
+                        const uint8_t* bcodes, const float* wscale, const int32_t* off, const int32_t* tstart, int n_experts,
+                        int N, int K, int epi, void* out, void* stream) {
+    DevFormat f;
+    if (int rc = make_dev_format(fmt, &f)) return rc;
+    if (!scmx_moe_mm_takes_slots(fmt, R, n_experts, K)) {
+        set_error("moe_mm_blocked: need a format that decodes with the FP4 conversion, 1 <= n_experts <= 2^20, K a multiple of 128 up to "
+                  "12288 and slots within 2^32 bytes (R=%d K=%d, %d experts)", R, K, n_experts);
+        return packed_mode(f) == B_PACKED_GENERIC ? SCMX_ERR_FORMAT : SCMX_ERR_ARG;
+    }
+    return moe_mm(fmt, xq, xscale, nullptr, R, codes, bcodes, wscale, off, tstart, n_experts, 256, N, K, epi, out, 1, stream);
 }
 
 int scmx_moe_mm_i8(const int8_t* xq, const float* xscale, const int32_t* gather, int R, const int8_t* wq,

@@ -60,6 +60,13 @@ static void launch_256(const GemmArgs& a, int bmode, int slots, hipStream_t s) {
 
 void launch_grouped(const GemmArgs& a, int bmode, int tm, hipStream_t s) {
     const int max_tiles = (a.M + tm - 1) / tm + a.n_experts;   // e2e/sc_moe.py:155
+    if (a.blocked)
+        // Slots of blocked activations: the dense GEMM's 256x128 tile of four waves, two workgroups a CU, whose waves take
+        // the tile's 16-row blocks in turn, so that a slot's missing rows are missing from all four SIMDs.  Bound like the
+        // dense tile (matrix pipe 39 per cent busy, vector ALU 36, LDS 46) and by what a tile costs beyond its K loop.
+        // Published format, skewed routing, us by rows (launch_256) / from slots: 64 experts of 2048 x 2048, 8000 rows 76.5
+        // / 64.7, 24000 159.3 / 131.7; of 2048 x 1024 43.0 / 37.5, 88.2 / 73.5; 257 of 1024 x 2048, 54000 rows 197 / 192.5.
+        return launch_tile<256, 128, 64, 4, 1, 2, 2, true, false, 1, 1, 16, FP4_MODES>(a, bmode, max_tiles, s);
     const bool fp4 = bmode != B_INT8 && bmode != B_PACKED_GENERIC;
     if (tm == 256) {
         launch_256(a, bmode, max_tiles, s);

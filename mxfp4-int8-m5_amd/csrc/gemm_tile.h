@@ -43,6 +43,7 @@ template <int BM, int BN, int BK, int WGM, int WGN, int BMODE, int OCC = 1, int 
           int KG = 1, int ADM = 0, int MF = 16>
 __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const GemmArgs a) {
     constexpr bool AD = ADM != 0, ADR = ADM == 2;   // activation fragments straight from memory; from the row layout
+    constexpr bool DEAL = SKIP && AD;   // the tile's MF-row blocks are dealt to the waves in turn
     constexpr int NSTAGE = 3;   // LDS stages: one being read, one ready, one being written
     constexpr int NT = WGM * WGN * 64;   // threads of one K group
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
@@ -106,9 +107,13 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     int8_t* const sm = smem + kg * GROUP_BYTES;   // this group's stages
     const int wm = SKIP ? wave / WGN : wave % WGM, wn = SKIP ? wave % WGN : wave / WGM;
 
+    // tile row of row r of this wave's tile (r counts whole MF-row blocks of the wave)
+    auto tile_row = [&](int r) { return DEAL ? (r / MF * WGM + wm) * MF + r % MF : wm * WTM + r; };
+
     // ---- which tile ------------------------------------------------------------------------------------------
     const int num_n = (a.N + BN - 1) / BN;
     int m0, n0, row_end, expert = 0;
+    [[maybe_unused]] int ablk0;   // first 32-row block of the tile's activations in the blocked layout
     if (a.tstart) {   // grouped: row tiles of BM inside expert segments
         // Workgroup b runs on XCD b % 8: inside every chunk of 8 row tiles each XCD takes one row tile with all of
         // its column tiles, so an activation panel is fetched into one L2 only.  The segments' row tiles (slots) may be
@@ -118,20 +123,11 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         n0 = (j >> 3) * BN;
         const int E = a.n_experts;
         if (slot >= a.tstart[E]) return;
-        // largest e with tstart[e] <= slot: every lane probes one of up to 64 evenly spaced entries of the range, so 64
-        // experts take one trip to memory and 4096 two (a binary search: six and twelve, in front of the first operand
-        // load)
-        int lo = 0, n = E;
-        while (n > 1) {
-            const int step = (n + 63) >> 6, at = int(threadIdx.x & 63) * step;
-            const int last = __popcll(__ballot(at < n && a.tstart[lo + min(at, n - 1)] <= slot)) - 1;   // entry 0 always is
-            lo += last * step;
-            n = min(step, n - last * step);
-        }
-        expert = __builtin_amdgcn_readfirstlane(lo);
+        expert = last_started(E, slot, [&](int e) { return a.tstart[e]; });   // the expert the slot belongs to
         m0 = a.off[expert] + (((slot - a.tstart[expert]) << a.sub_log2) + (tile & ((1 << a.sub_log2) - 1))) * BM;
         row_end = a.off[expert + 1];
         if (m0 >= row_end) return;   // the last slot's spare tiles
+        ablk0 = tile * (BM / 32);    // blocked: slots are whole, one after the other
     } else {
         const int num_m = (a.M + BM - 1) / BM;
         int pid = blockIdx.x;
@@ -146,13 +142,16 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         n0 = (r / rows_in_band) * BN;
         m0 = (band * GM + r % rows_in_band) * BM;
         row_end = a.M;
+        ablk0 = m0 / 32;
     }
     const int K = a.K;
     const int KL = K / KG;         // length of this group's part of the reduction
     const int kbase = kg * KL;     // and its first k (a multiple of 128)
     // MF-row blocks of this wave's tile that hold rows of the segment (wave-uniform)
     const int mi_active =
-        SKIP ? __builtin_amdgcn_readfirstlane(min(MI, max(0, (row_end - (m0 + wm * WTM) + MF - 1) / MF))) : MI;
+        DEAL   ? __builtin_amdgcn_readfirstlane(min(MI, max(0, ((row_end - m0 + MF - 1) / MF - wm + WGM - 1) / WGM)))
+        : SKIP ? __builtin_amdgcn_readfirstlane(min(MI, max(0, (row_end - (m0 + wm * WTM) + MF - 1) / MF)))
+               : MI;
     // The tile's scales are REQUESTED here, before the first operand loads, and stored to LDS after those have been
     // issued: memory returns a wave's loads in order, so scales requested first arrive first and their wait does not
     // cover the operand loads (fetched and stored up front they cost every tile two serial round trips to memory).
@@ -408,13 +407,20 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // wave tile leaves no registers for a third): the activation tile never passes through LDS.
     constexpr int NAB = MF == 16 && ACC16 > 16 ? 2 : NSTAGE;   // the largest wave tiles have registers for two buffers only (below)
     [[maybe_unused]] v4i fad[NAB][KS][MI];
-    [[maybe_unused]] int ad_src[ADR ? MI : WTM / 32];
+    [[maybe_unused]] int ad_src[ADR || DEAL ? MI : WTM / 32];
     if constexpr (ADR) {
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-            int gr = min(m0 + wm * WTM + i * 16 + lr, row_end - 1);
+            int gr = min(m0 + tile_row(i * 16 + lr), row_end - 1);
             if (a.gather) gr = a.gather[gr];
             ad_src[i] = int(uint32_t(gr) * uint32_t(K) + uint32_t(part) * 16u);
+        }
+    } else if constexpr (DEAL) {   // blocks past the segment: the wave's last one (or the tile's first) again
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const int b = mi_active ? min(i, mi_active - 1) * WGM + wm : 0;   // MF-row block of the tile
+            ad_src[i] = int(uint32_t(ablk0 + (MF == 32 ? b : b >> 1)) * uint32_t(K >> 5) * 1024u + uint32_t(MF == 32 ? 0 : b & 1) * 256u +
+                            uint32_t(part) * 512u + uint32_t(lr) * 16u);
         }
     } else if constexpr (AD) {
         const int last_block = (a.M + 31) / 32 - 1;
@@ -428,9 +434,9 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int s = 0; s < KS; ++s)
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
-                if (SKIP && i >= mi_active) continue;
                 const u32x4 v = ADR ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR ? i : 0] + s * 64, k0, 0)
-                                : MF == 32 ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[MF == 32 ? i : 0] + s * 1024, k0 * 32, 0)
+                                : DEAL ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[DEAL ? i : 0] + s * (MF == 32 ? 1024 : 2048), k0 * 32, 0)
+                                : MF == 32 ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[MF == 32 && !DEAL ? i : 0] + s * 1024, k0 * 32, 0)
                                     : __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR || MF == 32 ? 0 : i / 2] + s * 2048 + (i & 1) * 256, k0 * 32, 0);
                 fad[buf][s][i] = v4i{int(v[0]), int(v[1]), int(v[2]), int(v[3])};
             }
@@ -796,7 +802,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     constexpr int rsb = rowb + 16;                                     // padded LDS row stride
     constexpr bool fits = WGM * WGN * WTM * rsb <= SMEM_BYTES;   // per-wave tiles reuse the staging LDS
     int8_t* wtile = smem + (fits ? wave * (WTM * rsb) : 0);
-    const int wm0 = m0 + wm * WTM, wn0 = n0 + wn * WTN;            // wave tile origin (input column index)
+    const int wn0 = n0 + wn * WTN;            // wave tile origin (input column index)
     const bool wide = fits && (size_t(on) * esize) % 16 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0 &&
                       (epi != SCMX_EPI_RES || reinterpret_cast<uintptr_t>(a.res) % 16 == 0);
 
@@ -804,7 +810,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     f32x4 wsv[NI][AG];
     if (epi != SCMX_EPI_I32) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) xsv[i] = s_xs[wm * WTM + i * MF + lr];
+        for (int i = 0; i < MI; ++i) xsv[i] = s_xs[tile_row(i * MF + lr)];
 #pragma unroll
         for (int j = 0; j < NI; ++j)
 #pragma unroll
@@ -815,7 +821,8 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int row = i * MF + lr;
-        const int m = wm0 + row;
+        const int m = m0 + tile_row(row);
+        if (SKIP && i >= mi_active) break;
         const float xs = epi != SCMX_EPI_I32 ? xsv[i] : 0.0f;
 #pragma unroll
         for (int jg = 0; jg < NI * AG; ++jg) {
@@ -877,7 +884,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     constexpr int NP = WTM * ppr / 64, NB = NP < 8 ? NP : 8;
     static_assert(WTM * ppr % 64 == 0 && NP % NB == 0, "whole batches of pieces per lane");
 #pragma unroll 1
-    for (int p0 = lane; p0 < WTM * ppr; p0 += 64 * NB) {
+    for (int p0 = lane; p0 < (SKIP ? mi_active * MF : WTM) * ppr; p0 += 64 * NB) {
         u32x4 v[NB], rr[NB];
         bool ok[NB], full[NB];
         int8_t* dst[NB];
@@ -885,7 +892,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int i = 0; i < NB; ++i) {
             const int p = p0 + 64 * i;
             const int row = p / ppr, pc = p % ppr;
-            const int m = wm0 + row, c = ocol0 + pc * epp;
+            const int m = m0 + tile_row(row), c = ocol0 + pc * epp;
             ok[i] = m < row_end && c < on;
             full[i] = c + epp <= on;
             dst[i] = reinterpret_cast<int8_t*>(a.out) + (size_t(m) * on + c) * esize;

@@ -277,6 +277,21 @@ __device__ __forceinline__ void head_norm_rope(const float* yv, float ss, int pe
     head_rope(nv, per, lane, d, sn, cs, emit);
 }
 
+// The largest e of 0 .. E - 1 with start(e) <= at, start rising and start(0) <= at (wave-uniform, the whole wave present).
+// Every lane probes one of up to 64 evenly spaced entries of the range, so 64 experts take one trip to memory and 4096
+// two (a binary search: six and twelve, in front of the first operand load).
+template <typename Start>
+__device__ __forceinline__ int last_started(int E, int at, Start&& start) {
+    int lo = 0, n = E;
+    while (n > 1) {
+        const int step = (n + 63) >> 6, i = int(threadIdx.x & 63) * step;
+        const int last = __popcll(__ballot(i < n && start(lo + min(i, n - 1)) <= at)) - 1;   // entry 0 always is
+        lo += last * step;
+        n = min(step, n - last * step);
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
 // Symmetric INT8 code of v at inverse scale qi: clamp(rint(v * qi), +-127).
 __device__ __forceinline__ int quant_code(float v, float qi) {
     float r = rintf(__fmul_rn(v, qi));

@@ -1,5 +1,5 @@
 // Python binding of the C ABI for torch tensors: `_binding`, a module whose functions are the entry points of
-// include/scmx.h that enqueue work (and three of its queries), under the same names and with the same arguments except the last.  A pointer argument
+// include/scmx.h that enqueue work (and four of its queries), under the same names and with the same arguments except the last.  A pointer argument
 // takes a tensor (contiguous, on the GPU), None or an integer address; a format argument an object whose buffer is the
 // scmx_format; the stream is the caller's current one and is not passed.  A negative status raises.
 //
@@ -189,9 +189,9 @@ PyMODINIT_FUNC PyInit__binding() {
         ENTRY(scmx_swiglu_quant), ENTRY(scmx_qkv_headnorm), ENTRY(scmx_qkv_headnorm_rope), ENTRY(scmx_qkv_fullnorm),
         ENTRY(scmx_qkv_fullnorm_rope), ENTRY(scmx_attn_decode), ENTRY(scmx_attn_decode_qkv), ENTRY(scmx_attn_prefill), ENTRY(scmx_attn_prefill_split),
         ENTRY(scmx_gemv), ENTRY(scmx_gemv_rows), ENTRY(scmx_route_topk), ENTRY(scmx_norm_linear), ENTRY(scmx_route_sort), ENTRY(scmx_moe_mm),
-        ENTRY(scmx_moe_mm_i8), ENTRY(scmx_moe_combine), ENTRY(scmx_rot_quant), ENTRY(scmx_mxfp4_to_sc),
+        ENTRY(scmx_moe_mm_i8), ENTRY(scmx_moe_mm_blocked), ENTRY(scmx_moe_gather_blocked), ENTRY(scmx_act_quant_sorted), ENTRY(scmx_moe_combine), ENTRY(scmx_rot_quant), ENTRY(scmx_mxfp4_to_sc),
         ENTRY(scmx_quantize_sc), ENTRY(scmx_quantize_family),
-        QUERY(scmx_linear_w4a8_workspace), QUERY(scmx_gemv_rows_workspace), QUERY(scmx_mm_w4a8_prefers_blocked),
+        QUERY(scmx_linear_w4a8_workspace), QUERY(scmx_gemv_rows_workspace), QUERY(scmx_mm_w4a8_prefers_blocked), QUERY(scmx_moe_mm_takes_slots),
         EMPTY(bf16, BFloat16), EMPTY(i8, Char), EMPTY(u8, Byte), EMPTY(i32, Int), EMPTY(f32, Float),
         {nullptr, nullptr, 0, nullptr}};
     module_def.m_methods = methods;

@@ -156,17 +156,14 @@ class FusedOlmoe:
                              torch.zeros(tm, dtype=torch.int32, device=inds.device)])
         cg, bg, sg = ex["gu"]
         cd, bd, sd = ex["down"]
-        t = (tm, 64, 4)
         if self.two_pass:
+            t = (tm, 64, 4)
             act = sc_moe.moe_mm_i8(xq, R, sc_moe.unpack_experts(cg, bg, F2, D), sg, off, tstart, maxt, F2, 3, xs, tile=t,
                                    gather=tok)
-        else:
-            act = sc_moe.moe_mm(xq, R, cg, bg, sg, off, tstart, maxt, F2, 3, xs, tile=t, gather=tok, fmt=self.fmt)
-        xq2, xs2 = S.act_quant(act, R)
-        if self.two_pass:
+            xq2, xs2 = S.act_quant(act, R)
             yd = sc_moe.moe_mm_i8(xq2, R, sc_moe.unpack_experts(cd, bd, D, F2 // 2), sd, off, tstart, maxt, D, 1, xs2, tile=t)
         else:
-            yd = sc_moe.moe_mm(xq2, R, cd, bd, sd, off, tstart, maxt, D, 1, xs2, tile=t, fmt=self.fmt)
+            yd = sc_moe.expert_mlp(xq, xs, R, ex["gu"], ex["down"], tok, off, tstart, maxt, tm, self.fmt)
         return sc_moe.moe_combine(yd, pos, scores, h, nn, self.eps, L, quant=quant)
 
     def hidden(self, ids, cache=None):

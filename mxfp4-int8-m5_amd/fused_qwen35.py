@@ -121,17 +121,14 @@ class Qwen35Moe:
         xq, xs, xn = S.rmsnorm_quant_n(h, self.pn, self.eps)
         inds9, scores9 = self._route(xn[:L])
         pos, tok, _, off, tstart, maxt = sc_moe.route_sort(inds9, E1, tm)
-        (cg, bg, sg), (cd, bd, sd), t = self.gu, self.down, (tm, 64, 4)
         if two_pass:
+            (cg, bg, sg), (cd, bd, sd), t = self.gu, self.down, (tm, 64, 4)
             act = sc_moe.moe_mm_i8(xq, R, sc_moe.unpack_experts(cg, bg, F2, D), sg, off, tstart, maxt, F2, 3, xs, tile=t,
                                    gather=tok)
-        else:
-            act = sc_moe.moe_mm(xq, R, cg, bg, sg, off, tstart, maxt, F2, 3, xs, tile=t, gather=tok, fmt=self.fmt)
-        xq2, xs2 = S.act_quant(act, R)
-        if two_pass:
+            xq2, xs2 = S.act_quant(act, R)
             yd = sc_moe.moe_mm_i8(xq2, R, sc_moe.unpack_experts(cd, bd, D, F2 // 2), sd, off, tstart, maxt, D, 1, xs2, tile=t)
         else:
-            yd = sc_moe.moe_mm(xq2, R, cd, bd, sd, off, tstart, maxt, D, 1, xs2, tile=t, fmt=self.fmt)
+            yd = sc_moe.expert_mlp(xq, xs, R, self.gu, self.down, tok, off, tstart, maxt, tm, self.fmt)
         return sc_moe.moe_combine(yd, pos, scores9, h, self.pn, self.eps, L, quant=False)[0]
 
     def decode(self, h, lean=True):

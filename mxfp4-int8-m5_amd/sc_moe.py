@@ -62,7 +62,8 @@ def row_tile(R, n_experts):
     """Row tile of the grouped GEMM for R assignments over n_experts: 256-row tiles (the fewest LDS bytes per MFMA) from
     about 96 rows per expert on, below that 64-row tiles (less padding, packed weights in LDS).  Measured on 64 experts
     of 2048 x 2048 / 2048 x 1024 with top-8 routing: 512 tokens 149 us with 64-row tiles against 169 with 256-row ones,
-    1024 tokens 205 against 180."""
+    1024 tokens 205 against 180.  (With the 256-row tiles reading slots, below, the line is nearer 80 rows: 5600 over 64
+    experts 115 us either way.)"""
     return 256 if R >= 96 * n_experts else 64
 
 
@@ -94,6 +95,59 @@ def moe_mm(xq, R, codes, bcodes, wscale, off, tstart, max_tiles, N, epi, xscale=
     out = _out(R, N, epi, xq)
     _lib.native().scmx_moe_mm(fmt.c, xq, xscale, gather, R, codes, bcodes, wscale, off, tstart, E, tile[0], N, K, epi, out)
     return out
+
+
+def gather_blocked(xq, xscale, tok, R, off, tstart):
+    """The sorted rows xq[tok] (and their scales) in the 256-row slots of moe_mm_blocked -> (slots, xscale f32 [R])."""
+    K, E = xq.shape[1], off.shape[0] - 1
+    out, xs = _lib.native().empty_i8(xq, (-(-R // 256) + E) * 256 * K), _lib.native().empty_f32(xq, R)
+    _lib.native().scmx_moe_gather_blocked(xq, xscale, tok, off, tstart, E, R, K, out, xs)
+    return out, xs
+
+
+def act_quant_sorted(x, R, off, tstart):
+    """act_quant of sorted rows x bf16 [R, K] into the same slots -> (slots, xscale f32 [R])."""
+    K, E = x.shape[1], off.shape[0] - 1
+    assert x.dtype == torch.bfloat16
+    xq, xs = _lib.native().empty_i8(x, (-(-R // 256) + E) * 256 * K), _lib.native().empty_f32(x, R)
+    _lib.native().scmx_act_quant_sorted(x, off, tstart, E, R, K, xq, xs)
+    return xq, xs
+
+
+def moe_mm_blocked(slots, xscale, R, K, codes, bcodes, wscale, off, tstart, N, epi, fmt=None):
+    """moe_mm on rows in slots (gather_blocked, act_quant_sorted; off / tstart of 256-row tiles)."""
+    fmt = fmt or F.DEFAULT
+    out = _out(R, N, epi, slots)
+    _lib.native().scmx_moe_mm_blocked(fmt.c, slots, xscale, R, codes, bcodes, wscale, off, tstart, wscale.shape[0], N, K, epi, out)
+    return out
+
+
+def takes_slots(R, n_experts, K, tm, fmt):
+    """Whether a grouped GEMM with reduction K and row tile tm can read its activations from slots."""
+    return tm == 256 and bool(_lib.native().scmx_moe_mm_takes_slots(fmt.c, R, n_experts, K))
+
+
+def expert_mlp(xq, xs, R, gate_up, down, tok, off, tstart, max_tiles, tm, fmt):
+    """Gate|up with SwiGLU, INT8, down of the routed experts on packed weights: xq int8 [M, D] with the token of each sorted row in tok,
+    gate_up / down = (codes, bcodes, wscale) stacked over the experts -> bf16 [R, D] by sorted row.  With 256-row tiles the activations
+    go through slots in the blocked layout where that pays: always for down, whose quantization writes them, for gate|up from
+    2048 columns on (the copy costs R * D bytes, what it gains grows with R * D * columns).  Both GEMMs, quantization and copy, us
+    without / with slots, 64 experts of 2048 x 2048 and 2048 x 1024, skewed routing: 8000 rows 126 / 117, 12000 169 / 149, 24000
+    260 / 236, 48000 425 / 416, 24000 in e2m1/B16/M1..10 261 / 247; 16 of 4096 x 4096 264 / 225; 257 of 1024 x 2048, 54000
+    rows: gate|up 197 / 229 with the copy, down 145 / 136."""
+    (cg, bg, sg), (cd, bd, sd) = gate_up, down
+    E, F2 = sg.shape
+    D, K2, tile = sd.shape[1], F2 // 2, (tm, 64, 4)
+    if F2 >= 2048 and takes_slots(R, E, D, tm, fmt):
+        slots, xs = gather_blocked(xq, xs, tok, R, off, tstart)
+        act = moe_mm_blocked(slots, xs, R, D, cg, bg, sg, off, tstart, F2, 3, fmt)
+    else:
+        act = moe_mm(xq, R, cg, bg, sg, off, tstart, max_tiles, F2, 3, xs, tile=tile, gather=tok, fmt=fmt)
+    if takes_slots(R, E, K2, tm, fmt):
+        slots, xs = act_quant_sorted(act, R, off, tstart)
+        return moe_mm_blocked(slots, xs, R, K2, cd, bd, sd, off, tstart, D, 1, fmt)
+    xq, xs = S.act_quant(act, R)
+    return moe_mm(xq, R, cd, bd, sd, off, tstart, max_tiles, D, 1, xs, tile=tile, fmt=fmt)
 
 
 def moe_mm_i8(xq, R, wq, wscale, off, tstart, max_tiles, N, epi, xscale=None, dtype=torch.bfloat16, tile=(64, 64, 4),

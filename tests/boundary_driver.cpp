@@ -291,6 +291,17 @@ int main() {
            "moe_mm residual epilogue");
     expect(scmx_moe_mm(&fmt, xq, f0, nullptr, 100, codes, bc, f1, nullptr, ci, 4, 64, 8, 128, 1, out, nullptr), SCMX_ERR_ARG,
            "moe_mm null off");
+    expect(scmx_moe_mm_blocked(&fmt, xq, f0, 100, codes, bc, f1, nullptr, ci, 4, 8, 128, 1, out, nullptr), SCMX_ERR_ARG, "moe_mm_blocked null off");
+    expect(scmx_moe_mm_blocked(&fmt, xq, f0, 1 << 20, codes, bc, f1, ci, ci, 4, 8, 8192, 1, out, nullptr), SCMX_ERR_ARG, "moe_mm_blocked slots beyond 2^32 bytes");
+    expect(scmx_moe_mm_blocked(&fmt, xq, f0, 100, codes, bc, f1, ci, ci, 4, 8, 64, 1, out, nullptr), SCMX_ERR_ARG, "moe_mm_blocked K % 128");
+    expect(scmx_moe_gather_blocked(xq, f0, nullptr, ci, ci, 4, 100, 128, oq, of, nullptr), SCMX_ERR_ARG, "moe_gather_blocked null gather");
+    expect(scmx_moe_gather_blocked(xq, f0, ci, ci, ci, 4, 100, 192, oq, of, nullptr), SCMX_ERR_ARG, "moe_gather_blocked K % 128");
+    expect(scmx_moe_gather_blocked(xq, f0, ci, ci, ci, 1 << 21, 100, 128, oq, of, nullptr), SCMX_ERR_ARG, "moe_gather_blocked experts");
+    expect(scmx_act_quant_sorted(h[0], ci, nullptr, 4, 100, 128, oq, of, nullptr), SCMX_ERR_ARG, "act_quant_sorted null tstart");
+    expect(scmx_act_quant_sorted(h[0] + 4, ci, ci, 4, 100, 128, oq, of, nullptr), SCMX_ERR_ARG, "act_quant_sorted misaligned x");
+    expect(scmx_act_quant_sorted(h[0], ci, ci, 4, 100, 12416, oq, of, nullptr), SCMX_ERR_ARG, "act_quant_sorted K > 12288");
+    expect(scmx_moe_mm_takes_slots(&fmt, 100, 4, 2048), 1, "moe_mm_takes_slots");
+    expect(scmx_moe_mm_takes_slots(&fmt, 100, 4, 2000), 0, "moe_mm_takes_slots K % 128");
     expect(scmx_moe_mm_i8(xq, f0, nullptr, 100, nullptr, f1, ci, ci, 4, 64, 8, 128, 1, out, nullptr), SCMX_ERR_ARG, "moe_mm_i8 null wq");
     expect(scmx_moe_combine(h[0], ci, h[1], nullptr, h[2], nullptr, 0.0f, oh[0], oq, of, 4, 4, 128, 8, nullptr), SCMX_ERR_ARG,
            "moe_combine quantization without norm weight");
@@ -382,6 +393,11 @@ int main() {
     expect_valid(scmx_route_sort(ci, 10, 2, 8, 64, oi[0], oi[1], oi[2], oi[3], oi[4], nullptr), "route_sort small");
     for (int tm : {64, 128, 256})
         expect_valid(scmx_moe_mm(&fmt, xq, f0, ci, 32768, codes, bc, f1, ci, ci, 64, tm, 2048, 2048, 3, out, nullptr), "moe_mm");
+    for (int k : {128, 1024, 2048, 12288}) {
+        expect_valid(scmx_moe_gather_blocked(xq, f0, ci, ci, ci, 64, 4096, k, oq, of, nullptr), "moe_gather_blocked");
+        expect_valid(scmx_act_quant_sorted(h[0], ci, ci, 64, 4096, k, oq, of, nullptr), "act_quant_sorted");
+        expect_valid(scmx_moe_mm_blocked(&fmt, xq, f0, 4096, codes, bc, f1, ci, ci, 64, 2048, k, 3, out, nullptr), "moe_mm_blocked");
+    }
     expect_valid(scmx_moe_mm_i8(xq, f0, nullptr, 600, xq, f1, ci, ci, 8, 64, 256, 512, 0, out, nullptr), "moe_mm_i8");
     expect_valid(scmx_moe_combine(h[0], ci, h[1], nullptr, h[2], h[3], 1e-5f, oh[0], oq, of, 200, 256, 2048, 8, nullptr), "moe_combine");
     expect_valid(scmx_rot_quant(h[0], f0, oq, of, 17, 128, 1536, nullptr), "rot_quant");
@@ -469,6 +485,10 @@ int main() {
         expect_status(scmx_moe_mm(&f, xq, f0, (const int32_t*)maybe(ci), r(), codes, bc, f1, ci, ci, r(), r(), r(), r(), int(rng() % 6) - 1,
                                   out, nullptr),
                       "fuzz moe_mm");
+        expect_status(scmx_moe_gather_blocked(xq, f0, (const int32_t*)maybe(ci), ci, ci, r(), r(), r(), oq, of, nullptr), "fuzz moe_gather_blocked");
+        expect_status(scmx_act_quant_sorted((const uint16_t*)maybe(h[0]), ci, ci, r(), r(), r(), oq, of, nullptr), "fuzz act_quant_sorted");
+        expect_status(scmx_moe_mm_blocked(&f, xq, (const float*)maybe(f0), r(), codes, bc, f1, ci, ci, r(), r(), r(), int(rng() % 6) - 1, out, nullptr),
+                      "fuzz moe_mm_blocked");
         expect_status(scmx_moe_mm_i8(xq, f0, nullptr, r(), xq, f1, ci, ci, r(), r(), r(), r(), int(rng() % 6) - 1, out, nullptr),
                       "fuzz moe_mm_i8");
         expect_status(scmx_moe_combine(h[0], ci, h[1], (const uint16_t*)maybe(h[4]), h[2], (const uint16_t*)maybe(h[3]), 1e-5f, oh[0],
