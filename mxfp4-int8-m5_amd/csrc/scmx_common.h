@@ -242,13 +242,14 @@ __device__ __forceinline__ int wave_sum_i32(int v) {
 }
 
 // Per-head RMSNorm of one q or k head held by one wave: the lane holds the bf16-valued elements per*lane ..
-// per*lane + per - 1 of the head in yv and their sum of squares in ss; nv receives the normalised values (bf16-valued).
-__device__ __forceinline__ void head_norm(const float* yv, float ss, int per, int lane, int d,
-                                          const uint16_t* __restrict__ w, float eps, float* nv) {
+// per*lane + per - 1 of the head in yv and their sum of squares in ss, weight(i) is the norm weight of its element i; nv
+// receives the normalised values (bf16-valued).
+template <typename Weight>
+__device__ __forceinline__ void head_norm(const float* yv, float ss, int per, int d, Weight&& weight, float eps, float* nv) {
     ss = wave_sum(ss);
     const float inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, float(d)), eps)));
     for (int i = 0; i < per; ++i)
-        nv[i] = round_bf16(__fmul_rn(bf16_to_f32(w[per * lane + i]), round_bf16(__fmul_rn(yv[i], inv))));
+        nv[i] = round_bf16(__fmul_rn(weight(i), round_bf16(__fmul_rn(yv[i], inv))));
 }
 // The rotary embedding of such a head (sn / cs: the d / 2 sines and cosines of the row's position; sn == nullptr: no
 // rotation).  emit(i, value) receives the bf16 result of element per*lane + i.
@@ -273,7 +274,7 @@ __device__ __forceinline__ void head_norm_rope(const float* yv, float ss, int pe
                                                const uint16_t* __restrict__ w, float eps, const float* sn,
                                                const float* cs, Emit&& emit) {
     float nv[8];
-    head_norm(yv, ss, per, lane, d, w, eps, nv);
+    head_norm(yv, ss, per, d, [&](int i) { return bf16_to_f32(w[per * lane + i]); }, eps, nv);
     head_rope(nv, per, lane, d, sn, cs, emit);
 }
 

@@ -344,17 +344,17 @@ def attn_splits(rows):
     return 1 if rows <= 1024 else 8 if rows <= 8192 else 16
 
 
-def _decode_ranges(rows, hq):
-    """The same for any number of heads.  16 heads, us with 1 / 8 / 16 ranges: 513 rows 10.5 / 7.6 / 7.8, 1000 15.5 / 8.4 / 8.1, 1500
-    22.2 / 10.5 / 9.6, 3000 - / 12.7 / 11.8, 6000 - / 18.2 / 15.8, 12000 - / 27.2 / 22.4 (32 ranges 22.9); up to 512 rows the second
-    launch costs a host-bound loop more than it gives (300 rows 8.1 / 7.4 / 7.5).
+def _decode_ranges(rows, hq, hk):
+    """The same for any number of heads.  16 heads, us with 8 / 16 ranges: 160 rows 6.2 / 6.3, 500 6.4 / 6.3, 1000 7.3 / 6.8, 3000 10.5 /
+    9.5, 6000 15.0 / 13.7, 12000 26.6 / 23.4 (32 ranges 22.2); up to 512 rows the second launch costs a host-bound loop more than it gives
+    (300 rows 6.2 with one).  32 ranges let the kernel serve two query heads of a KV head from one reading of the cache, which it does
+    beyond 3072 rows (8 KV heads: 6000 rows 12.0, 12000 15.2; up to there it cuts them into 16).
     With the position on the device `rows` is the cache's, and a short context in a longer cache pays for a merge that finds little
-    or nothing to do.  In a graph, cache of 1024 rows, us with 1 / 16 ranges by the context: 30 rows 4.1 / 5.7, 128 4.4 / 5.9, 160 5.5 /
-    6.4, 300 6.8 / 6.4, 500 8.2 / 6.5, 700 10.7 / 6.5, 1000 13.4 / 6.6: over a conversation that fills its cache the split gives more than
-    that costs from about 520 rows on."""
+    or nothing to do: in a graph, with 1 range / in a longer cache, 30 rows 4.2 / 5.7, 128 4.7 / 6.2, 300 6.2 / 6.4; from about 300 rows on
+    the ranges win."""
     if hq > 32:
         return attn_splits(rows)
-    return 1 if rows <= 512 else 16
+    return 1 if rows <= 512 else 16 if rows <= 3072 or hq // hk % 2 else 32
 
 
 def _split_workspace(splits, hq, d, like):
@@ -370,7 +370,7 @@ def attn_decode(q, kcache, vcache, n, scale=None, splits=None):
     out = _lib.native().empty_bf16(q, 1, hq * d)
     dev_pos = n if torch.is_tensor(n) else None
     if splits is None:
-        splits = _decode_ranges(rows if dev_pos is not None else int(n), hq)
+        splits = _decode_ranges(rows if dev_pos is not None else int(n), hq, hk)
     work = _split_workspace(splits, hq, d, q)
     _lib.native().scmx_attn_decode(q, kcache, vcache, dev_pos, 0 if dev_pos is not None else int(n), out, hq, hk, d, rows,
                                    float(scale if scale is not None else d ** -0.5), work, splits)
@@ -422,7 +422,7 @@ def attn_decode_qkv(y, qn, kn, eps, hq, hk, d, kcache, vcache, pos, inv_freq, sc
     dev_pos = pos if torch.is_tensor(pos) else None
     assert dev_pos is None or dev_pos.dtype == torch.int64
     if splits is None:
-        splits = _decode_ranges(kcache.shape[1] if dev_pos is not None else int(pos) + 1, hq)
+        splits = _decode_ranges(kcache.shape[1] if dev_pos is not None else int(pos) + 1, hq, hk)
     work = _split_workspace(splits, hq, d, y)
     _lib.native().scmx_attn_decode_qkv(y, qn, kn, _eps(eps), inv_freq, dev_pos, 0 if dev_pos is not None else int(pos),
                                        kcache, vcache, out, hq, hk, d, kcache.shape[1],
