@@ -171,6 +171,70 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
 }
 
+// A contiguous tensor on the GPU, and if `type` is given of that type; NULL: something else.
+const at::Tensor* plain(PyObject* o, at::ScalarType type = at::ScalarType::Undefined) {
+    if (!THPVariable_Check(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    return t.is_cuda() && t.is_contiguous() && (type == at::ScalarType::Undefined || t.scalar_type() == type) ? &t : nullptr;
+}
+
+// gemv(format, xq, xscale, codes, bcodes, wscale, N, epi, res, eidx, xstride, shared, pro, nw, eps): sc_decode.gemv for the operands of
+// every decode step -- plain tensors, up to eight rows -- in one call: output (and workspace) allocated, the kernel launched.  None
+// where an operand is anything else: the caller's general way converts or refuses it.  With both in Python a call on one row of
+// 2048 x 2048 took the host 5.0 us, in its kernel's 4.0.
+PyObject* gemv(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    try {
+        if (n != 15) fail(PyExc_TypeError, "gemv takes 15 arguments");
+        for (int i : {6, 7, 10, 12})
+            if (!PyLong_Check(args[i])) Py_RETURN_NONE;
+        if (args[11] != Py_None && !PyLong_Check(args[11])) Py_RETURN_NONE;
+        const int N = convert<int>(args[6]), epi = convert<int>(args[7]), xstride = convert<int>(args[10]), pro = convert<int>(args[12]);
+        const at::Tensor* x = plain(args[1], pro == 0 ? at::ScalarType::Char : at::ScalarType::BFloat16);
+        const at::Tensor *codes = plain(args[3]), *bcodes = plain(args[4]), *wscale = plain(args[5]);
+        const at::Tensor* xscale = pro == 0 ? plain(args[2]) : x;
+        const at::Tensor* res = epi == SCMX_EPI_RES ? plain(args[8]) : x;
+        const at::Tensor* nw = pro == 2 ? plain(args[13]) : x;
+        if (!x || !codes || !bcodes || !wscale || !xscale || !res || !nw || x->dim() < 1 || x->dim() > 2 || (pro == 2 && !PyFloat_Check(args[14])))
+            Py_RETURN_NONE;
+        const at::Tensor* eidx = args[9] == Py_None ? nullptr : plain(args[9], at::ScalarType::Int);
+        const int64_t rows = x->dim() == 2 ? x->size(0) : 1, K64 = x->size(-1), slots64 = eidx ? eidx->numel() : 0;
+        if ((args[9] != Py_None && !eidx) || N < 0 || K64 > INT32_MAX || slots64 > INT32_MAX - 1 || (!eidx && rows > 8)) Py_RETURN_NONE;
+        const scmx_format* fmt = convert<const scmx_format*>(args[0]);
+        const int K = int(K64), shared = args[11] == Py_None ? -1 : convert<int>(args[11]);
+        const float eps = pro == 2 ? convert<float>(args[14]) : 0.0f;
+        const int batch = !eidx && rows > 1 ? int(rows) : 1, slots = int(slots64) + (args[11] != Py_None);
+        const int64_t width = epi == SCMX_EPI_SWIGLU ? N / 2 : N;
+        const auto ptr = [](const at::Tensor* t) { return t->data_ptr(); };
+        at::Tensor out;
+        int rc;
+        {
+            const NoGil released;   // the allocator may ask the driver, or wait for the GPU
+            const at::TensorOptions options = at::TensorOptions().dtype(at::ScalarType::BFloat16).device(x->device());
+            out = eidx ? at::empty({slots, width}, options) : batch > 1 ? at::empty({batch, width}, options) : at::empty({width}, options);
+            const auto *xs = pro == 0 ? static_cast<const float*>(ptr(xscale)) : nullptr;
+            const auto *rs = epi == SCMX_EPI_RES ? static_cast<const uint16_t*>(ptr(res)) : nullptr;
+            const auto *w = pro == 2 ? static_cast<const uint16_t*>(ptr(nw)) : nullptr;
+            const auto *c = static_cast<const uint32_t*>(ptr(codes));
+            const auto *b = static_cast<const uint8_t*>(ptr(bcodes));
+            const auto *s = static_cast<const float*>(ptr(wscale));
+            auto* o = static_cast<uint16_t*>(out.data_ptr());
+            if (eidx) {
+                rc = scmx_gemv(fmt, ptr(x), xs, c, b, s, rs, o, epi, pro, w, eps, batch, N, K, static_cast<const int32_t*>(ptr(eidx)), int(slots64),
+                               xstride, shared, c10::hip::getCurrentHIPStream().stream());
+            } else {
+                const size_t need = batch > 1 ? scmx_gemv_rows_workspace(fmt, pro, batch, N, K) : 0;
+                const at::Tensor work = need ? at::empty({int64_t(need)}, options.dtype(at::ScalarType::Byte)) : at::Tensor();
+                rc = scmx_gemv_rows(fmt, ptr(x), xs, c, b, s, rs, o, epi, pro, w, eps, batch, N, K, need ? work.data_ptr() : nullptr, need,
+                                    c10::hip::getCurrentHIPStream().stream());
+            }
+        }
+        if (rc != SCMX_OK) return status(eidx ? "scmx_gemv" : "scmx_gemv_rows", rc);
+        return THPVariable_Wrap(std::move(out));
+    } catch (...) {
+        return raised();
+    }
+}
+
 #define ENTRY(fn) \
     {#fn, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(((Call<&fn>::name = #fn), &Call<&fn>::call))), METH_FASTCALL, nullptr}
 #define QUERY(fn) {#fn, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Query<&fn>::call)), METH_FASTCALL, nullptr}
@@ -192,6 +256,7 @@ PyMODINIT_FUNC PyInit__binding() {
         ENTRY(scmx_moe_mm_i8), ENTRY(scmx_moe_mm_blocked), ENTRY(scmx_moe_gather_blocked), ENTRY(scmx_act_quant_sorted), ENTRY(scmx_moe_combine), ENTRY(scmx_rot_quant), ENTRY(scmx_mxfp4_to_sc),
         ENTRY(scmx_quantize_sc), ENTRY(scmx_quantize_family),
         QUERY(scmx_linear_w4a8_workspace), QUERY(scmx_gemv_rows_workspace), QUERY(scmx_mm_w4a8_prefers_blocked), QUERY(scmx_moe_mm_takes_slots),
+        {"gemv", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&gemv)), METH_FASTCALL, nullptr},
         EMPTY(bf16, BFloat16), EMPTY(i8, Char), EMPTY(u8, Byte), EMPTY(i32, Int), EMPTY(f32, Float),
         {nullptr, nullptr, 0, nullptr}};
     module_def.m_methods = methods;

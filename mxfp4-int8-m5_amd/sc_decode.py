@@ -21,8 +21,13 @@ def gemv(xq, codes, bcodes, xscale, wscale, N, epi, dtype=torch.bfloat16, res=No
     dozen rows on the dense GEMM is the faster path).
     MoE (eidx int32 [S]): codes [E, ..], wscale [E, N]; slot j uses expert eidx[j] and input row j if xstride=1;
     shared=e adds one slot for expert e -> [S(+1), N or N/2]."""
-    S._check_dtype(dtype)
+    if dtype is not torch.bfloat16:
+        S._check_dtype(dtype)
     fmt = fmt or F.DEFAULT
+    # one native call where every operand is a plain tensor; None: what follows converts or refuses what is not
+    out = _lib.native().gemv(fmt.c, xq, xscale, codes, bcodes, wscale, N, epi, res, eidx, xstride, shared, pro, nw, eps)
+    if out is not None:
+        return out
     K = xq.shape[-1]
     no = N // 2 if epi == 3 else N
     batch, nslot = 1, 0
