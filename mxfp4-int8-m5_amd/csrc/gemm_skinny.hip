@@ -1,7 +1,8 @@
 // Dense W4A8 GEMM for few activation rows (a short prompt, sequences decoding together): M up to 128.
 //
 // Such a problem streams the weights once and is over: what it needs is every CU loading at once, not operand reuse.  A
-// workgroup owns 16 weight rows and all M activation rows; its waves split K (wave w of NW takes the 128-wide steps w,
+// workgroup owns 16 weight rows and all M activation rows (or, on layers of so few columns that CUs would idle, some of the
+// 16-row tiles of them: row_groups); its waves split K (wave w of NW takes the 128-wide steps w,
 // w + NW, ...), decode the weights in registers and multiply with v_mfma_i32_16x16x64_i8, weights as the row operand.
 // Nothing passes through LDS but the waves' INT32 partial sums at the end, which add up exactly in any order.
 //
@@ -25,6 +26,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int K = a.K, N = a.N, M = a.M, steps = K / 128, n0 = int(blockIdx.x) * 16;
+    const int tile0 = int(blockIdx.y) * TILES;   // first 16-row tile of this workgroup's activation rows
     const size_t wrow = size_t(min(n0 + r, N - 1));
     const uint8_t* cp = reinterpret_cast<const uint8_t*>(a.codes) + wrow * (K / 2) + 16 * g;
     const uint8_t* bp = a.bcodes + wrow * a.bc_row_bytes;
@@ -33,7 +35,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
     const int8_t* ap[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t)
-        ap[t] = a.xq + (size_t(min(t, (M - 1) / 16) >> 1) * (K / 32) + g) * 1024 + (16 * (t & 1) + r) * 16;   // (a tile past M: any block)
+        ap[t] = a.xq + (size_t(min(tile0 + t, (M - 1) / 16) >> 1) * (K / 32) + g) * 1024 + (16 * ((tile0 + t) & 1) + r) * 16;   // (a tile past M: any block)
 
     struct Weights {
         u32x4 w;
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
     __syncthreads();
     for (int e = threadIdx.x; e < TILES * 64; e += NW * 64) {
         const int t = e >> 6, l = e & 63;
-        const int m = 16 * t + (l & 15), n = n0 + 4 * (l >> 4);
+        const int m = 16 * (tile0 + t) + (l & 15), n = n0 + 4 * (l >> 4);
         if (m >= M || n >= N) continue;   // N % 4 == 0
         v4i tot = part[0][t][l];
 #pragma unroll
@@ -140,17 +142,27 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
                 y[i] = __fadd_rn(rv, round_bf16(y[i]));
             }
         }
-        *reinterpret_cast<u32x2*>(out + size_t(m) * N + n) =
-            u32x2{uint32_t(f32_to_bf16(y[0])) | (uint32_t(f32_to_bf16(y[1])) << 16),
-                  uint32_t(f32_to_bf16(y[2])) | (uint32_t(f32_to_bf16(y[3])) << 16)};
+        *reinterpret_cast<u32x2*>(out + size_t(m) * N + n) = u32x2{f32_to_bf16x2(y[0], y[1]), f32_to_bf16x2(y[2], y[3])};
     }
 }
 
+// Groups that the 16-row tiles are cut into, a workgroup each: as many as the CUs that a workgroup per 16 columns leaves idle
+// allow.  What a workgroup takes beyond the latency of its loads is its activations through the vector L1 (48 rows of 6144:
+// 295 KB at 64 bytes a clock); the weights that several then decode come from the L2.  us with one group / several: 2048 x
+// 6144 at 40 rows 7.5 / 6.8 (two), 64 8.3 / 6.9, 128 11.3 / 8.5; 896 x 4864 at 40 rows 6.4 / 5.3 (three), 128 9.6 / 5.9
+// (four); 2048 x 2048 at 128 5.6 / 4.5.  Groups beyond that share CUs: 4096 x 4096 at 40 rows 6.6 / 9.1, 2048 x 6144 in
+// three 9.5.
+static int row_groups(int tiles, int columns, int cus) {
+    const int room = max(1, cus / columns), per = (tiles + room - 1) / room;
+    return (tiles + per - 1) / per;
+}
+
 // Its time in us beside what any launch costs.  A CU runs `turns` = ceil(N / 16 / CUs) workgroups, each of which walks its
-// weights and all 16 ceil(M / 16) rows of activations (five row tiles run as six, seven as eight).  Fitted to 1002 problems (13
+// weights and the rows of activations of its group (five row tiles run as six, seven as eight).  Fitted to 1002 problems (13
 // widths 896 ... 28672, 27 reductions 512 ... 14336, 16 ... 128 rows): within 5 per cent.
 float skinny_time(int M, int N, int K, int cus) {
-    const int tiles = (M + 15) / 16, columns = (N + 15) / 16, turns = columns <= cus ? 1 : (columns + cus - 1) / cus;
+    const int columns = (N + 15) / 16, turns = columns <= cus ? 1 : (columns + cus - 1) / cus;
+    const int rows16 = (M + 15) / 16, groups = row_groups(rows16, columns, cus), tiles = (rows16 + groups - 1) / groups;
     const float more = 16.0f * float((tiles == 5 ? 6 : tiles == 7 ? 8 : tiles) - 1), k = float(K);
     return K <= 2048 ? 0.33f + 1.6e-5f * k + float(turns) * k * (5.6e-4f + 1.19e-5f * more)
                      : 1.31e-4f * k - 0.3f + float(turns) * k * (6.8e-4f + 1.03e-5f * more);
@@ -159,7 +171,8 @@ float skinny_time(int M, int N, int K, int cus) {
 void launch_skinny(const GemmArgs& args, int bmode, hipStream_t s) {
     GemmArgs a = args;
     if (a.epi == SCMX_EPI_SWIGLU) a.silu = silu_table_device();   // (the argument check has seen that it is there)
-    const dim3 grid((a.N + 15) / 16);
+    const int columns = (a.N + 15) / 16, rows16 = (a.M + 15) / 16, groups = row_groups(rows16, columns, device_cus());
+    const dim3 grid(columns, groups);
     // Waves per workgroup: four with four steps each where that is all of K (fewer partial sums to add: 2048 x 2048 at M = 40
     // 4.3 against 4.4 us, 12288 x 2048 at 32 7.9 against 10), else eight with six steps in flight (2048 x 6144 7.6 against 9.9).
     auto tiles = [&](auto bm) {
@@ -169,7 +182,7 @@ void launch_skinny(const GemmArgs& args, int bmode, hipStream_t s) {
             if (a.K <= 2048) skinny_kernel<T, BM, 4, 4><<<grid, dim3(256), 0, s>>>(a);
             else skinny_kernel<T, BM, 8, 6><<<grid, dim3(512), 0, s>>>(a);
         };
-        switch ((a.M + 15) / 16) {
+        switch ((rows16 + groups - 1) / groups) {   // (several groups: of at most four tiles)
             case 1: return go(std::integral_constant<int, 1>{});
             case 2: return go(std::integral_constant<int, 2>{});
             case 3: return go(std::integral_constant<int, 3>{});
