@@ -84,10 +84,13 @@ void launch_grouped(const GemmArgs& a, int bmode, int tm, hipStream_t s) {
         // 31.1 / 33.2.  A reduction of four steps at most is mostly prologue and epilogue: eight waves on 256 columns,
         // four a SIMD, share them.  257 experts of 2048 x 512, 70 rows, us 256 / 128 columns: 63.3 / 67.2, 61.6 / 69.9,
         // 64.6 / 70.1, 64.9 / 71.0; 64 of 4096 x 256 23.5 / 24.6; K = 768 the other way round, 29.9 / 26.5.
+        // The four-wave tile leaves out the MFMAs and LDS traffic of a half without rows: 257 experts of 1024 x 2048, 70
+        // rows each 115 -> 113 us (e2m1/B16/M1..10), 104 -> 102 (published), 25 rows 67.6 -> 64.3, 4 rows 54.3 -> 51.0;
+        // level at K = 1024.  Eight waves have no registers for it (63 -> 73).
         if (a.K <= 512 && a.N % 256 == 0)
             launch_tile<64, 256, 128, 1, 8, 4, 2, false, true, 1, 0, 32, FP4_MODES>(a, bmode, max_tiles, s);
         else
-            launch_tile<64, 128, 128, 1, 4, 2, 2, false, true, 1, 0, 32, FP4_MODES>(a, bmode, max_tiles, s);
+            launch_tile<64, 128, 128, 1, 4, 2, 2, true, true, 1, 0, 32, FP4_MODES>(a, bmode, max_tiles, s);
     } else
         launch_tile<64, 128, 128, 2, 4>(a, bmode, max_tiles, s);
 }

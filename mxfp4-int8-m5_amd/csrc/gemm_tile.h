@@ -29,6 +29,7 @@ namespace scmx {
 // SKIP (grouped launches): a row tile that ends inside its expert's segment multiplies only the 16-row blocks that hold
 // valid rows.  The two waves that share a SIMD then own the same columns and different row halves of the tile, so that
 // a half-empty tile halves the MFMA work of every SIMD instead of idling two of the four.
+// (PK: the halves of 32 rows; the waves sit side by side along the columns and skip alike.)
 // PK (the FP4-conversion formats, K steps of 128): the weights stay packed in LDS -- 64 bytes of codes per row and K
 // step plus the step's block-code bytes -- and every wave decodes its own fragments after reading them.  Half the
 // weight bytes through LDS in both directions, paid with one decode per wave row that shares the fragment.
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // PK: block-code bytes per weight row and K step
     constexpr int BCB = BMODE == B_PACKED_B16M || BMODE == B_PACKED_E8M0 ? 4 : BMODE == B_PACKED_B16 ? 2 : 1;
     constexpr int BCR = BCB == 4 ? 2 : 1;   // registers for those of two steps
-    static_assert(!PK || (BK == 128 && WPC == 4 && !SKIP && BMODE != B_INT8 && BMODE != B_PACKED_GENERIC),
+    static_assert(!PK || (BK == 128 && WPC == 4 && BMODE != B_INT8 && BMODE != B_PACKED_GENERIC),
                   "packed weights in LDS: K steps of 128, 16-byte runs, FP4-conversion formats");
     // bytes per stage: BM activation rows, then BN weight rows (PK: 64 code bytes each)
     constexpr int STAGE = A_BYTES + (PK ? BN * (BK / 2) : BN * BK);
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int i = 0; i < PMI; ++i)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                f[h][i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + (((4 * kp + 2 * part + h) ^ sw) << 4));
+                if (!SKIP || i < mi_active) f[h][i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + (((4 * kp + 2 * part + h) ^ sw) << 4));
     };
     auto load_pw = [&](const int8_t* src, int kp, v4i (&f)[PNI]) __attribute__((always_inline)) {
 #pragma unroll
@@ -556,10 +557,12 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
 #pragma unroll
-                for (int i = 0; i < PMI; ++i)
+                for (int i = 0; i < PMI; ++i) {
+                    if (SKIP && i >= mi_active) break;
 #pragma unroll
                     for (int j = 0; j < PNI; ++j)
                         if constexpr (PK) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(px[cur][h][j], pa[cur][h][i], acc[i][j], 0, 0, 0);
+                }
                 stage_slice(r, dst, k2, 2 * kp + h, o);
             }
         }
