@@ -327,6 +327,12 @@ int scmx_moe_combine(const uint16_t* y, const int32_t* pos, const uint16_t* scor
                      const uint16_t* res, const uint16_t* w, float eps, uint16_t* h, int8_t* xq, float* xs, int M,
                      int Mp, int K, int topk, void* stream);
 
+/* scmx_moe_combine with xq in the blocked layout of scmx_act_quant_blocked, for a q|k|v projection through scmx_mm_w4a8_blocked: Mp %
+ * 32 == 0, K % 512 == 0, K <= 2048, everything 16-byte aligned and, but for sscore, given. */
+int scmx_moe_combine_blocked(const uint16_t* y, const int32_t* pos, const uint16_t* scores, const uint16_t* sscore, const uint16_t* res,
+                             const uint16_t* w, float eps, uint16_t* h, int8_t* xq, float* xs, int M, int Mp, int K, int topk,
+                             void* stream);
+
 /* Randomized Hadamard rotation of every 32-wide block of x T[M, K] (signs f32 [K], +-1; FP32 butterflies, result times
  * 1/sqrt(32) rounded to T), then per-token INT8 as scmx_act_quant.  K % 32 == 0, K <= 8192.
  * Replaces rot_quant, e2e/sc_kernels.py:231-275,571-582. */

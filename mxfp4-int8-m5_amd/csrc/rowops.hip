@@ -865,15 +865,16 @@ __global__ __launch_bounds__(NT) void moe_combine_kernel(const uint16_t* __restr
 // The same with a wave per row and the row in its registers from the first load to the codes: no LDS, no barriers, and
 // the rows' loads overlap freely.  Bound: HBM, top-k rows of y read per row written.  Same arithmetic, same order of
 // sums, same bits.
-template <int CH>
-__global__ __launch_bounds__(256) void moe_combine_wave_kernel(const uint16_t* __restrict__ y, const int32_t* __restrict__ pos,
+// BLK: xq leaves in the blocked layout of the dense GEMM (Mp % 32 == 0), eight rows a workgroup, as in rmsnorm_quant_wave_kernel.
+template <int CH, bool BLK = false>
+__global__ __launch_bounds__(BLK ? 512 : 256) void moe_combine_wave_kernel(const uint16_t* __restrict__ y, const int32_t* __restrict__ pos,
                                                                const uint16_t* __restrict__ scores, const uint16_t* __restrict__ sscore,
                                                                const uint16_t* __restrict__ res, const uint16_t* __restrict__ w,
                                                                float eps, uint16_t* __restrict__ h, int8_t* __restrict__ xq,
                                                                float* __restrict__ xs, int M, int Mp, int topk) {
     constexpr int K = 512 * CH;
-    const int row = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
-    if (row >= Mp) return;   // wave-uniform
+    const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), row = int(blockIdx.x) * (BLK ? 8 : 4) + wid, lane = threadIdx.x & 63;
+    if (row >= Mp) return;   // wave-uniform (BLK: never)
     const int nsc = sscore ? topk - 1 : topk;
     auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
     auto hi = [](uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); };
@@ -937,6 +938,7 @@ __global__ __launch_bounds__(256) void moe_combine_wave_kernel(const uint16_t* _
     const float s = __fdiv_rn(amax, 127.0f);
     const float qi = s > 0.0f ? __fdiv_rn(1.0f, s) : 0.0f;
     u32x2* qrow = reinterpret_cast<u32x2*>(xq + size_t(row) * K) + lane;
+    __shared__ u32x2 tile[BLK ? CH * 64 * 8 : 1];
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
         uint32_t o[2] = {0u, 0u};
@@ -945,9 +947,22 @@ __global__ __launch_bounds__(256) void moe_combine_wave_kernel(const uint16_t* _
             o[e >> 1] |= (uint32_t(quant_code(lo(v[j][e]), qi)) & 0xFFu) << (16 * (e & 1));
             o[e >> 1] |= (uint32_t(quant_code(hi(v[j][e]), qi)) & 0xFFu) << (16 * (e & 1) + 8);
         }
-        qrow[64 * j] = u32x2{o[0], o[1]};
+        const int p = lane + 64 * j;   // piece of 8 codes: half p % 2 of the 16-byte slot of chunk p / 2
+        if (BLK) tile[((p >> 1) * 8 + ((wid + (p >> 2)) & 7)) * 2 + (p & 1)] = u32x2{o[0], o[1]}; else qrow[64 * j] = u32x2{o[0], o[1]};
     }
     if (lane == 0) xs[row] = s;
+    if constexpr (BLK) {
+        __syncthreads();
+        const int row0 = row - wid;
+        int8_t* const blk = xq + (size_t(row0 >> 5) * size_t(K >> 5)) * 1024;
+        const u32x4* t16 = reinterpret_cast<const u32x4*>(tile);
+#pragma unroll
+        for (int j = 0; j < CH / 2 + CH % 2; ++j) {   // K / 16 pieces x 8 rows of 16 bytes, 512 per pass
+            const int idx = int(threadIdx.x) + 512 * j, c = idx >> 3, r = idx & 7;
+            if (CH % 2 == 0 || c < K / 16)
+                *reinterpret_cast<u32x4*>(blk + size_t(c >> 1) * 1024 + (c & 1) * 512 + ((row0 + r) & 31) * 16) = t16[c * 8 + ((r + (c >> 1)) & 7)];
+        }
+    }
 }
 
 // fn(K / 512 as a compile-time constant), 1 ... 8: the kernels that keep a row in a wave's registers.
@@ -1434,6 +1449,27 @@ int scmx_moe_combine(const uint16_t* y, const int32_t* pos, const uint16_t* scor
         moe_combine_kernel<4><<<dim3(Mp), dim3(NT), size_t(K) * 4 + 72 * 4, (hipStream_t)stream>>>(y, pos, scores, sscore, res,
                                                                                                     w, eps, h, xq, xs, M, K, topk);
     return check_launch("moe_combine");
+}
+
+int scmx_moe_combine_blocked(const uint16_t* y, const int32_t* pos, const uint16_t* scores, const uint16_t* sscore, const uint16_t* res,
+                             const uint16_t* w, float eps, uint16_t* h, int8_t* xq, float* xs, int M, int Mp, int K, int topk,
+                             void* stream) {
+    if (!y || !pos || !scores || !res || !h || !xq || !w || !xs || Mp < M || Mp % 32 || topk < 1 || topk > 65536 || K % 512 || K > 2048 ||
+        !row_shape_ok("moe_combine_blocked", M, K, 2048) ||
+        (uintptr_t(y) | uintptr_t(res) | uintptr_t(h) | uintptr_t(w) | uintptr_t(xq)) % 16) {
+        set_error("moe_combine_blocked: need all of y, pos, scores, res, w, h, xq and xs (16-byte aligned), M <= Mp with Mp %% 32 == 0 (%d), "
+                  "topk in 1..65536 and K %% 512 == 0, K <= 2048 (%d)", Mp, K);
+        return SCMX_ERR_ARG;
+    }
+    if (Mp == 0) return SCMX_OK;
+    auto go = [&](auto kernel) {
+        kernel<<<dim3(unsigned(Mp) / 8u), dim3(512), 0, (hipStream_t)stream>>>(y, pos, scores, sscore, res, w, eps, h, xq, xs, M, Mp, topk);
+    };
+    if (K == 512) go(moe_combine_wave_kernel<1, true>);
+    else if (K == 1024) go(moe_combine_wave_kernel<2, true>);
+    else if (K == 1536) go(moe_combine_wave_kernel<3, true>);
+    else go(moe_combine_wave_kernel<4, true>);
+    return check_launch("moe_combine_blocked");
 }
 
 }  // extern "C"

@@ -253,7 +253,7 @@ PyMODINIT_FUNC PyInit__binding() {
         ENTRY(scmx_swiglu_quant), ENTRY(scmx_qkv_headnorm), ENTRY(scmx_qkv_headnorm_rope), ENTRY(scmx_qkv_fullnorm),
         ENTRY(scmx_qkv_fullnorm_rope), ENTRY(scmx_attn_decode), ENTRY(scmx_attn_decode_qkv), ENTRY(scmx_attn_prefill), ENTRY(scmx_attn_prefill_split),
         ENTRY(scmx_gemv), ENTRY(scmx_gemv_rows), ENTRY(scmx_route_topk), ENTRY(scmx_norm_linear), ENTRY(scmx_route_sort), ENTRY(scmx_moe_mm),
-        ENTRY(scmx_moe_mm_i8), ENTRY(scmx_moe_mm_blocked), ENTRY(scmx_moe_gather_blocked), ENTRY(scmx_act_quant_sorted), ENTRY(scmx_moe_combine), ENTRY(scmx_rot_quant), ENTRY(scmx_mxfp4_to_sc),
+        ENTRY(scmx_moe_mm_i8), ENTRY(scmx_moe_mm_blocked), ENTRY(scmx_moe_gather_blocked), ENTRY(scmx_act_quant_sorted), ENTRY(scmx_moe_combine), ENTRY(scmx_moe_combine_blocked), ENTRY(scmx_rot_quant), ENTRY(scmx_mxfp4_to_sc),
         ENTRY(scmx_quantize_sc), ENTRY(scmx_quantize_family),
         QUERY(scmx_linear_w4a8_workspace), QUERY(scmx_gemv_rows_workspace), QUERY(scmx_mm_w4a8_prefers_blocked), QUERY(scmx_moe_mm_takes_slots),
         {"gemv", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&gemv)), METH_FASTCALL, nullptr},

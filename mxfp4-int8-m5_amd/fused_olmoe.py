@@ -140,7 +140,7 @@ class FusedOlmoe:
         logits = S.linear_bf16(xn[:M], nw["mlp.gate"])
         return sc_moe.route(logits, self.args.num_experts_per_tok, renorm=self.args.norm_topk_prob)
 
-    def _experts(self, xq, xs, inds, scores, h, nn, ex, L, quant=True):
+    def _experts(self, xq, xs, inds, scores, h, nn, ex, L, quant=True, blocked=False):
         a = self.args
         E, F2, D = a.num_experts, 2 * a.intermediate_size, a.hidden_size
         R = L * a.num_experts_per_tok
@@ -164,7 +164,7 @@ class FusedOlmoe:
             yd = sc_moe.moe_mm_i8(xq2, R, sc_moe.unpack_experts(cd, bd, D, F2 // 2), sd, off, tstart, maxt, D, 1, xs2, tile=t)
         else:
             yd = sc_moe.expert_mlp(xq, xs, R, ex["gu"], ex["down"], tok, off, tstart, maxt, tm, self.fmt)
-        return sc_moe.moe_combine(yd, pos, scores, h, nn, self.eps, L, quant=quant)
+        return sc_moe.moe_combine(yd, pos, scores, h, nn, self.eps, L, quant=quant, blocked=blocked)
 
     def hidden(self, ids, cache=None):
         """Final normed hidden states [L, D] for prompt ids [L]."""
@@ -173,20 +173,20 @@ class FusedOlmoe:
         cache = cache if cache is not None else self.make_cache(max(4096, ids.numel()))
         h, L, Mp = embed_rows(self.embed, ids)
         nl = len(self.layers)
-        xq, xs = S.rmsnorm_quant(h, self.layers[0][0]["input_layernorm"], self.eps, Mp)
+        # prefill-sized GEMMs on packed weights read their activations in 32x32 blocks (the quantizers write either layout)
+        blk = {g: isinstance(w.unpack(), S.PackedWq) and S.prefers_blocked(Mp, w.N, w.K) for g, w in self.layers[0][1].items()}
+        xq, xs = S.rmsnorm_quant(h, self.layers[0][0]["input_layernorm"], self.eps, Mp, blocked=blk["qkv"])
         for i, (nw, ws, ex) in enumerate(self.layers):
             y = S.mm_epi(xq, ws["qkv"].unpack(), xs, ws["qkv"].wscale, 1)
             o = self._attention(cache[i], nw, y, L)
-            wo = ws["o"].unpack()   # a prefill-sized GEMM on packed weights reads its activations in 32x32 blocks
-            blocked = isinstance(wo, S.PackedWq) and S.prefers_blocked(Mp, ws["o"].N, ws["o"].K)
-            xq, xs = S.act_quant_blocked(o, Mp) if blocked else S.act_quant(o, Mp)
-            h = S.mm_epi(xq, wo, xs, ws["o"].wscale, 2, res=h)
+            xq, xs = S.act_quant_blocked(o, Mp) if blk["o"] else S.act_quant(o, Mp)
+            h = S.mm_epi(xq, ws["o"].unpack(), xs, ws["o"].wscale, 2, res=h)
             xq, xs, xn = S.rmsnorm_quant_n(h, nw["post_attention_layernorm"], self.eps)
             inds, scores = self.route(nw, xn, L)
             if self.record is not None:
                 self.record.append((inds, scores))
             nn = self.layers[i + 1][0]["input_layernorm"] if i + 1 < nl else self.norm
-            h, xq, xs = self._experts(xq, xs, inds, scores, h, nn, ex, L)
+            h, xq, xs = self._experts(xq, xs, inds, scores, h, nn, ex, L, quant=i + 1 < nl, blocked=blk["qkv"])
         return S.rmsnorm(h[:L], self.norm, self.eps)
 
     def logits(self, h):

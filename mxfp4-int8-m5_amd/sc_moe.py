@@ -169,11 +169,13 @@ def unpack_experts(codes, bcodes, N, K):
     return S.unpack_i8(codes.reshape(-1), bcodes.reshape(E * N, -1), E * N, K, lazy=False)
 
 
-def moe_combine(y, pos, scores, res, w, eps, M, quant=True):
+def moe_combine(y, pos, scores, res, w, eps, M, quant=True, blocked=False):
     """y bf16 [R, K] (sorted assignments), pos int32 [M*topk], scores bf16 [M, topk], res [Mp, K] ->
     (h [Mp, K], xq int8 [Mp, K], xscale [Mp]) with xq = INT8(rms_norm(h, w)); quant=False returns xq = xs = None.
+    blocked: xq as a BlockedXq (the layout of act_quant_blocked) where the shape allows it (Mp % 32 == 0, K % 512 == 0, K <= 2048) and
+    the rows are as many as the kernel that writes it is made for (1024), by rows otherwise.
     (The reference keeps this in e2e/fused_olmoe.py:87-97.)"""
-    return _combine(y, pos, scores, None, res, w, eps, M, quant)
+    return _combine(y, pos, scores, None, res, w, eps, M, quant, blocked)
 
 
 def moe_combine_split(y, pos, scores, sscore, res, w, eps, M):
@@ -181,12 +183,14 @@ def moe_combine_split(y, pos, scores, sscore, res, w, eps, M):
     return _combine(y, pos, scores, sscore, res, w, eps, M, False)
 
 
-def _combine(y, pos, scores, sscore, res, w, eps, M, quant):
+def _combine(y, pos, scores, sscore, res, w, eps, M, quant, blocked=False):
     Mp, K = res.shape
     topk = scores.shape[1] + (1 if sscore is not None else 0)
     h = torch.empty_like(res)
     xq = _lib.native().empty_i8(res, Mp, K) if quant else None
     xs = _lib.native().empty_f32(res, Mp) if quant else None
-    _lib.native().scmx_moe_combine(y, pos, scores, sscore, res, w if quant else None, S._eps(eps) if quant else 0.0, h, xq,
-                                   xs, M, Mp, K, topk)
-    return h, xq, xs
+    blocked = (blocked and quant and Mp % 32 == 0 and Mp >= 1024 and K % 512 == 0 and K <= 2048
+               and not (y.data_ptr() | res.data_ptr() | w.data_ptr()) % 16)
+    combine = _lib.native().scmx_moe_combine_blocked if blocked else _lib.native().scmx_moe_combine
+    combine(y, pos, scores, sscore, res, w if quant else None, S._eps(eps) if quant else 0.0, h, xq, xs, M, Mp, K, topk)
+    return h, S.BlockedXq(xq.reshape(-1), Mp, K) if blocked else xq, xs

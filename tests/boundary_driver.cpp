@@ -305,6 +305,12 @@ int main() {
     expect(scmx_moe_mm_i8(xq, f0, nullptr, 100, nullptr, f1, ci, ci, 4, 64, 8, 128, 1, out, nullptr), SCMX_ERR_ARG, "moe_mm_i8 null wq");
     expect(scmx_moe_combine(h[0], ci, h[1], nullptr, h[2], nullptr, 0.0f, oh[0], oq, of, 4, 4, 128, 8, nullptr), SCMX_ERR_ARG,
            "moe_combine quantization without norm weight");
+    expect(scmx_moe_combine_blocked(h[0], ci, h[1], nullptr, h[2], h[3], 1e-5f, oh[0], oq, of, 4, 40, 2048, 8, nullptr), SCMX_ERR_ARG,
+           "moe_combine_blocked Mp % 32");
+    expect(scmx_moe_combine_blocked(h[0], ci, h[1], nullptr, h[2], h[3], 1e-5f, oh[0], oq, of, 4, 32, 2560, 8, nullptr), SCMX_ERR_ARG,
+           "moe_combine_blocked K > 2048");
+    expect(scmx_moe_combine_blocked(h[0], ci, h[1], nullptr, h[2], nullptr, 1e-5f, oh[0], oq, of, 4, 32, 2048, 8, nullptr), SCMX_ERR_ARG,
+           "moe_combine_blocked null w");
     expect(scmx_moe_combine(h[0], ci, h[1], nullptr, h[2], nullptr, 0.0f, oh[0], nullptr, nullptr, 5, 4, 128, 8, nullptr), SCMX_ERR_ARG,
            "moe_combine Mp < M");
     expect(scmx_rot_quant(h[0], f0, oq, of, 4, 4, 100, nullptr), SCMX_ERR_ARG, "rot_quant K % 32");
@@ -399,6 +405,8 @@ int main() {
         expect_valid(scmx_moe_mm_blocked(&fmt, xq, f0, 4096, codes, bc, f1, ci, ci, 64, 2048, k, 3, out, nullptr), "moe_mm_blocked");
     }
     expect_valid(scmx_moe_mm_i8(xq, f0, nullptr, 600, xq, f1, ci, ci, 8, 64, 256, 512, 0, out, nullptr), "moe_mm_i8");
+    for (int k : {512, 1024, 1536, 2048})
+        expect_valid(scmx_moe_combine_blocked(h[0], ci, h[1], nullptr, h[2], h[3], 1e-5f, oh[0], oq, of, 200, 256, k, 8, nullptr), "moe_combine_blocked");
     expect_valid(scmx_moe_combine(h[0], ci, h[1], nullptr, h[2], h[3], 1e-5f, oh[0], oq, of, 200, 256, 2048, 8, nullptr), "moe_combine");
     expect_valid(scmx_rot_quant(h[0], f0, oq, of, 17, 128, 1536, nullptr), "rot_quant");
     expect_valid(scmx_mxfp4_to_sc(bc, obc, of, oi[0], 4096, 2048, nullptr), "mxfp4_to_sc");
@@ -491,6 +499,9 @@ int main() {
                       "fuzz moe_mm_blocked");
         expect_status(scmx_moe_mm_i8(xq, f0, nullptr, r(), xq, f1, ci, ci, r(), r(), r(), r(), int(rng() % 6) - 1, out, nullptr),
                       "fuzz moe_mm_i8");
+        expect_status(scmx_moe_combine_blocked(h[0], ci, h[1], (const uint16_t*)maybe(h[4]), h[2], (const uint16_t*)maybe(h[3]), 1e-5f, oh[0],
+                                               (int8_t*)maybe(oq), of, r(), r(), r(), r(), nullptr),
+                      "fuzz moe_combine_blocked");
         expect_status(scmx_moe_combine(h[0], ci, h[1], (const uint16_t*)maybe(h[4]), h[2], (const uint16_t*)maybe(h[3]), 1e-5f, oh[0],
                                        (int8_t*)maybe(oq), of, r(), r(), r(), r(), nullptr),
                       "fuzz moe_combine");
