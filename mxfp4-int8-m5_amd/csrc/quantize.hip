@@ -132,6 +132,33 @@ __device__ __forceinline__ float fp4_sq_err(const float (&x)[BLOCK], float scale
     return r0 + r1;
 }
 
+// The same for weights born in bf16, as half-precision pairs: two conversions, a packed difference and a dot product per
+// two weights, two instructions a weight for three.  Scaled to magnitudes below 8 their eight bits fit half precision
+// down to 2^-17.  A difference is a multiple of its weight's last bit and no larger than the weight (or below 5 at a last
+// bit of 2^-5, where it saturates), so it is exact too, and the dot product adds exact squares in float32.  What is
+// smaller rounds to zero at every exponent tried, as all below 1/8 does: it adds the same to all three sums, whatever is
+// left of it.  The others' squares are multiples of 2^-20: two sums differ by that or not at all.
+template <int BLOCK>
+__device__ __forceinline__ float fp4_sq_err_half(const half2_t (&x)[BLOCK / 2], float scale) {
+    float r0 = 0.0f, r1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < BLOCK / 2; i += 4) {   // the conversion writes one byte and keeps the others: four share a register
+        uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(0u, x[i], scale, 0);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(c, x[i + 1], scale, 1);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(c, x[i + 2], scale, 2);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(c, x[i + 3], scale, 3);
+        const half2_t d0 = half2_t(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(c, scale, 0)) - x[i];
+        const half2_t d1 = half2_t(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(c, scale, 1)) - x[i + 1];
+        const half2_t d2 = half2_t(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(c, scale, 2)) - x[i + 2];
+        const half2_t d3 = half2_t(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(c, scale, 3)) - x[i + 3];
+        r0 = __builtin_amdgcn_fdot2(d0, d0, r0, false);
+        r1 = __builtin_amdgcn_fdot2(d1, d1, r1, false);
+        r0 = __builtin_amdgcn_fdot2(d2, d2, r0, false);
+        r1 = __builtin_amdgcn_fdot2(d3, d3, r1, false);
+    }
+    return r0 + r1;
+}
+
 // Eight weights' codes at a power-of-two scale, signs included: a word of the packed layout.
 __device__ __forceinline__ uint32_t fp4_word(const float* x, float scale) {
     uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[0], x[1], scale, 0);
@@ -149,13 +176,20 @@ __device__ __forceinline__ uint32_t unsigned_zeros(uint32_t c) {
 // sums. The codes come from the conversion, which takes a midpoint to the even code where the host takes the lower one.
 // bf16 weights have eight bits: 2^-12 smaller, one on a midpoint lies below it and no other changes sides.  float32
 // weights are converted as they are and 2^-23 smaller: where both agree so does the host (a midpoint whose even code is
-// the lower one, or none near); the others' blocks take the arithmetic.  12288 x 2048 bf16: 22.2 us; 28.8 with that
-// arithmetic for every weight, 44 with the near ties summed by one lane of the wave, 234 us with a lane per weight and
-// every candidate in float64 across lanes.
+// the lower one, or none near); the others' blocks take the arithmetic.  That arithmetic for every weight took 28.8 us
+// where the conversion's 22.2 stood beside it, near ties summed by one lane of the wave 44, a lane per weight and every
+// candidate in float64 across lanes 234 (12288 x 2048, bf16, 32-blocks).
+// Registers decide how many waves hide the conversions' latency: four a SIMD need 128 a thread.  16-blocks are held to
+// that; bf16 32-blocks fit only if the weights are read again for their codes (L2 has them) instead of kept over the
+// barrier; float32 32-blocks fit neither way.  us, before / with half-precision trials / so bounded, 12288 x 2048: bf16
+// 32-blocks 24.3 / 23.9 / 21.8 (bounded without reading again 24.7; five or six waves 29), 16-blocks 47.7 / 47.8 / 31.6;
+// float32 32-blocks 28.9 (bounded 32.3, read again 31.5), 16-blocks 50.4 / - / 35.9.  4096 x 12288: bf16 47.1 -> 39.7
+// and 70.8 -> 50.2, float32 16-blocks 76.3 -> 67.3.
 template <int BLOCK, bool BF16>
-__global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict__ w, uint32_t* __restrict__ codes,
-                                                         uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
-                                                         int64_t N, int K, int rows, bool vec) {
+__global__ __launch_bounds__(QNT, BLOCK == 16 || BF16 ? 4 : 1) void quantize_sc_kernel(
+    const void* __restrict__ w, uint32_t* __restrict__ codes, uint8_t* __restrict__ bcodes, float* __restrict__ wscale,
+    int64_t N, int K, int rows, bool vec) {
+    constexpr bool AGAIN = BLOCK == 32 && BF16;   // the weights are read again for their codes
     extern __shared__ int s_e[];   // rows x nb block exponents, then the rows' smallest allowed and lowest exponents
     const int nb = K / BLOCK;
     const size_t row0 = size_t(blockIdx.x) * rows;
@@ -185,10 +219,20 @@ __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict
             if (amax > 0.0f) {
                 // floor(log2 amax) of a float32-born value is its binary exponent
                 e0 = int((__double_as_longlong(double(amax)) >> 52) & 0x7FF) - 1023 - 2;
-                float x[BLOCK];
+                float s0, sm, sp;
+                if constexpr (BF16) {
+                    half2_t x[BLOCK / 2];
 #pragma unroll
-                for (int i = 0; i < BLOCK; ++i) x[i] = __builtin_amdgcn_ldexpf(v[i], -e0);
-                const float s0 = fp4_sq_err<BLOCK>(x, 1.0f), sm = fp4_sq_err<BLOCK>(x, 0.5f), sp = fp4_sq_err<BLOCK>(x, 2.0f);
+                    for (int i = 0; i < BLOCK; i += 2)
+                        x[i / 2] = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_ldexpf(v[i], -e0),
+                                                                                         __builtin_amdgcn_ldexpf(v[i + 1], -e0)));
+                    s0 = fp4_sq_err_half<BLOCK>(x, 1.0f), sm = fp4_sq_err_half<BLOCK>(x, 0.5f), sp = fp4_sq_err_half<BLOCK>(x, 2.0f);
+                } else {
+                    float x[BLOCK];
+#pragma unroll
+                    for (int i = 0; i < BLOCK; ++i) x[i] = __builtin_amdgcn_ldexpf(v[i], -e0);
+                    s0 = fp4_sq_err<BLOCK>(x, 1.0f), sm = fp4_sq_err<BLOCK>(x, 0.5f), sp = fp4_sq_err<BLOCK>(x, 2.0f);
+                }
                 // A float32 sum of 32 squares of exact differences is within 32 half-ulps (2e-6) of the exact one, the
                 // host's float64 sum within 1e-14: apart by more than 1e-5, the sums order alike.  (Below 1e-30 squares
                 // underflow.)
@@ -260,7 +304,7 @@ __global__ __launch_bounds__(QNT) void quantize_sc_kernel(const void* __restrict
     // ---- codes (sim/make_testcase.py:36-39, e2e/sc_format.py:72-73) ------------------------------------------------
     for (int b = tid; b < total; b += QNT) {
         const size_t at = base + size_t(b) * BLOCK;
-        if (total > QNT) load_block<BLOCK, BF16>(w, at, vec, v);   // more than one block per thread: read them again
+        if (AGAIN || total > QNT) load_block<BLOCK, BF16>(w, at, vec, v);   // (or more than one block per thread)
         const int e = max(s_e[b], s_floor[b / nb]);
         uint32_t c[BLOCK / 8], open = 1u;
         if (e > -100 && e < 120) {   // (its scale is an ordinary float32)
