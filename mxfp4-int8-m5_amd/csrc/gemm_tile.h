@@ -92,13 +92,19 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // round trip to memory
     __shared__ __attribute__((aligned(16))) float s_xs[BM], s_ws[BN];
     // SwiGLU: the sigmoid's table (8 KB), copied to LDS while the first operands are on their way, where it costs the CU
-    // no workgroup (all but the packed expert tiles); the lookups go to memory otherwise.  A wave's 64 gates lie in some
-    // 30 cache lines, which the vector L1 serves one after the other.  With the 65536-entry table of silu(g) in memory,
-    // two conversions and one lookup at a time instead of two, 12288 x 2048 at 2048 rows took 57.3 us for 53.0, at 1500
-    // 51.1 for 49.4, at 256 12.0 for 11.1; 6144 x 4096 at 6000 rows 152.5 for 148.4.
+    // no workgroup.  The packed expert tiles, three of whose workgroups fill the CU's LDS, copy it over their stages once
+    // the K loop is done, behind the waves' output tiles: one trip to the L2 and a barrier, hidden by the other workgroups
+    // (SIG_LATE).  A wave's 64 gates lie in some 30 cache lines, which the vector L1 would serve one after the other.
+    // With the 65536-entry table of silu(g) in memory, two conversions and one lookup at a time instead of two, 12288 x
+    // 2048 at 2048 rows took 57.3 us for 53.0, at 1500 51.1 for 49.4, at 256 12.0 for 11.1; 6144 x 4096 at 6000 rows 152.5
+    // for 148.4.  A sparse block of 257 experts, 2000 tokens, whose gate|up runs packed tiles: 257.5 with the lookups in
+    // memory, 253.3 with the late copy.
     constexpr int CU_WGS = OCC * 4 * 64 / (NT * KG) > 1 ? OCC * 4 * 64 / (NT * KG) : 1;
     constexpr bool SIG = !PK && SMEM_BYTES + (BM + BN) * 4 + int(sizeof(uint16_t)) * 2 * int(SIGMOID_ENTRIES) <= 160 * 1024 / CU_WGS;
     __shared__ __attribute__((aligned(16))) uint16_t s_sig[SIG ? 2 * SIGMOID_ENTRIES : 8];
+    constexpr int SIG_AT = WGM * WGN * WTM * (WTN + 16);   // behind the waves' output tiles
+    constexpr bool SIG_LATE = PK && SIG_AT + int(sizeof(uint16_t)) * 2 * int(SIGMOID_ENTRIES) <= SMEM_BYTES;
+    uint16_t* const sig = SIG ? s_sig : reinterpret_cast<uint16_t*>(smem + (SIG_LATE ? SIG_AT : 0));
     auto swz = [](int row, int chunk) { return row * BK + ((chunk ^ ((row / RPB) & (CPR - 1))) << 4); };
     // packed weight rows (64 bytes, 4 chunks): 4 rows per sweep of the banks, chunk c of row r at c ^ ((r / 4) % 4)
     auto swzp = [](int row, int chunk) { return row * (BK / 2) + ((chunk ^ ((row >> 2) & 3)) << 4); };
@@ -236,12 +242,18 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 
     constexpr int SIG_PER = (2 * int(SIGMOID_ENTRIES) / 8 + NT * KG - 1) / (NT * KG);   // 16-byte pieces of the table a thread copies
     [[maybe_unused]] u32x4 sig_reg[SIG_PER];
-    const bool sig_copy = SIG && a.epi == SCMX_EPI_SWIGLU;
-    if (sig_copy) {
+    auto load_sig = [&] {
 #pragma unroll
         for (int j = 0; j < SIG_PER; ++j)
             sig_reg[j] = reinterpret_cast<const u32x4*>(a.silu)[min(int(threadIdx.x) + j * NT * KG, 2 * int(SIGMOID_ENTRIES) / 8 - 1)];
-    }
+    };
+    auto store_sig = [&](uint16_t* to) {
+#pragma unroll
+        for (int j = 0; j < SIG_PER; ++j)
+            if (int(threadIdx.x) + j * NT * KG < 2 * int(SIGMOID_ENTRIES) / 8) reinterpret_cast<u32x4*>(to)[int(threadIdx.x) + j * NT * KG] = sig_reg[j];
+    };
+    const bool sig_copy = SIG && a.epi == SCMX_EPI_SWIGLU, late_sig = SIG_LATE && a.epi == SCMX_EPI_SWIGLU;
+    if (sig_copy) load_sig();
 
     // Two register sets hold the global loads of two K steps in flight.
     struct Staged {
@@ -453,11 +465,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int j = 0; j < WS_PER; ++j)
             if (tid + j * NT < BN) s_ws[tid + j * NT] = ws_reg[j];
     }
-    if (sig_copy) {
-#pragma unroll
-        for (int j = 0; j < SIG_PER; ++j)
-            if (int(threadIdx.x) + j * NT * KG < 2 * int(SIGMOID_ENTRIES) / 8) reinterpret_cast<u32x4*>(s_sig)[int(threadIdx.x) + j * NT * KG] = sig_reg[j];
-    }
+    if (sig_copy) store_sig(s_sig);
     if constexpr (AD) load_ad(0, 0);
     store_lds(r0, 0, 0);
     store_lds(r1, 1, BK);
@@ -772,7 +780,12 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // columns of one row, the unit every epilogue works on.  Results go through a per-wave LDS tile so that global
     // stores are 16 bytes per lane over whole contiguous row segments.
     const int N = a.N;
+    if (late_sig) load_sig();
     __syncthreads();   // every wave is done reading the staging buffers
+    if (late_sig) {
+        store_sig(sig);
+        __syncthreads();
+    }
     if constexpr (KG > 1) {   // the groups' partial sums meet in group 0 (register r of thread t at word r * NT + t)
         if (kg > 0) {
             int32_t* sums = reinterpret_cast<int32_t*>(smem + PART_BASE + (kg - 1) * PART_BYTES);
@@ -847,7 +860,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
                 y[r] = __fmul_rn(__fmul_rn(float(acc[i][j][4 * g + r]), xs), w4[r]);
             uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
             if (epi == SCMX_EPI_SWIGLU) {   // (g, g, u, u) -> two outputs
-                const uint32_t o = swiglu_lut2(SIG ? s_sig : a.silu, y[0], y[1], y[2], y[3]);
+                const uint32_t o = swiglu_lut2(SIG || SIG_LATE ? sig : a.silu, y[0], y[1], y[2], y[3]);
                 if (W)
                     *reinterpret_cast<uint32_t*>(wtile + row * rsb + col) = o;
                 else if (m < row_end && n < N)

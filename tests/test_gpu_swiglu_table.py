@@ -10,12 +10,14 @@ from tests.util import F32, blocked_layout, dev, host, product_format
 pytestmark = pytest.mark.gpu
 
 
-# few rows; tiles from blocked activations and by rows; expert slots of 64 (the packed tile, whose lookups go to memory), 128 and 256 rows
-@pytest.mark.parametrize("path,m", [("blocked", 5), ("blocked", 300), ("rows", 300), (64, 70), (128, 70), (256, 70)])
-def test_every_gate(path, m):
+# few rows; tiles from blocked activations and by rows; expert slots of 64 (the packed tiles, which copy the table behind their K loop:
+# eight waves up to K = 512, four beyond), 128 and 256 rows
+@pytest.mark.parametrize("path,m,k", [("blocked", 5, 256), ("blocked", 300, 256), ("rows", 300, 256), (64, 70, 256), (64, 70, 768), (64, 20, 768),
+                                      (128, 70, 256), (256, 70, 256)])
+def test_every_gate(path, m, k):
     from mxfp4_int8_m5_amd import sc_kernels as S
     from mxfp4_int8_m5_amd import sc_moe as M
-    n, k = 4 * 32768, 256
+    n = 4 * 32768
     gate = bf16.from_bits(np.arange(65536, dtype=np.uint32).astype(np.uint16))
     ws = np.empty((n // 4, 4), F32)
     ws[:, 0], ws[:, 1], ws[:, 2], ws[:, 3] = gate[0::2], gate[1::2], F32(1.0), F32(-0.3984375)
