@@ -92,7 +92,7 @@ void launch_grouped(const GemmArgs& a, int bmode, int tm, hipStream_t s) {
         else
             launch_tile<64, 128, 128, 1, 4, 2, 2, true, true, 1, 0, 32, FP4_MODES>(a, bmode, max_tiles, s);
     } else
-        launch_tile<64, 128, 128, 2, 4>(a, bmode, max_tiles, s);
+        launch_tile<64, 128, 128, 2, 4, 4>(a, bmode, max_tiles, s);
 }
 
 }  // namespace scmx

@@ -15,10 +15,10 @@ void launch_rows(const GemmArgs& a, int bmode, int tile, hipStream_t s) {
         case 0: return launch_tile<256, 256, 64, 2, 4, 1, 2>(a, bmode, rows256, s);
         case 1: return launch_tile<256, 128, 128, 4, 2, 1, 3>(a, bmode, rows256, s);
         case 2: return launch_tile<128, 128, 128, 4, 2, 1, 3>(a, bmode, rows128, s);
-        case 3: return launch_tile<128, 64, 128, 4, 2>(a, bmode, rows128, s);
+        case 3: return launch_tile<128, 64, 128, 4, 2, 4>(a, bmode, rows128, s);
         case 5: return launch_tile<64, 64, 128, 2, 2, 1, 2, false, false, 2>(a, bmode, rows64, s);
         case 6: return launch_tile<64, 32, 128, 2, 1, 1, 2, false, false, 4>(a, bmode, rows64, s);
-        default: return launch_tile<64, 64, 128, 2, 2>(a, bmode, rows64, s);
+        default: return launch_tile<64, 64, 128, 2, 2, 3>(a, bmode, rows64, s);
     }
 }
 

@@ -9,7 +9,7 @@ void launch_rows_idle(const GemmArgs& a, int bmode, int tile, hipStream_t s) {
         case 0: return launch_tile<256, 256, 64, 2, 4, 1, 2, false, false, 1, 0, 32>(a, bmode, rows256, s);
         case 1: return launch_tile<256, 128, 128, 4, 2, 1, 3, false, false, 1, 0, 32>(a, bmode, rows256, s);
         case 2: return launch_tile<128, 128, 128, 4, 2, 1, 3, false, false, 1, 0, 32>(a, bmode, rows128, s);
-        default: return launch_tile<128, 64, 128, 4, 2, 1, 2, false, false, 1, 0, 32>(a, bmode, rows128, s);
+        default: return launch_tile<128, 64, 128, 4, 2, 4, 2, false, false, 1, 0, 32>(a, bmode, rows128, s);
     }
 }
 

@@ -40,6 +40,8 @@ namespace scmx {
 // pass through LDS; every wave loads the fragments of its own rows from memory, two K steps ahead: four runs of 256
 // bytes from the blocked layout, sixteen of 64 from rows.  Waves must then not share rows (WGN = 1, or few column
 // groups), and only the weight rows of a stage exist in LDS.
+//
+// OCC: waves a SIMD that the tile's registers and LDS leave room for at least, and with them the workgroups that share a CU.
 template <int BM, int BN, int BK, int WGM, int WGN, int BMODE, int OCC = 1, int FD = 2, bool SKIP = false, bool PK = false,
           int KG = 1, int ADM = 0, int MF = 16>
 __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const GemmArgs a) {
@@ -91,19 +93,26 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
     // scales of the tile's rows and columns, fetched before the K loop so that the epilogue does not start with a
     // round trip to memory
     __shared__ __attribute__((aligned(16))) float s_xs[BM], s_ws[BN];
-    // SwiGLU: the sigmoid's table (8 KB), copied to LDS while the first operands are on their way, where it costs the CU
-    // no workgroup.  The packed expert tiles, three of whose workgroups fill the CU's LDS, copy it over their stages once
-    // the K loop is done, behind the waves' output tiles: one trip to the L2 and a barrier, hidden by the other workgroups
-    // (SIG_LATE).  A wave's 64 gates lie in some 30 cache lines, which the vector L1 would serve one after the other.
+    // SwiGLU: the sigmoid's table (8 KB), copied to LDS while the first operands are on their way, where the CU then still
+    // holds the workgroups that OCC counts on.  The others (three packed expert tiles fill the CU's LDS, as do two staged
+    // ones of 64x128, two of 128x64 and three of 64x64) copy it over their stages once the K loop is done, behind the
+    // waves' output tiles: one trip to the L2 and a barrier, hidden by the other workgroups (SIG_LATE).  A wave's 64 gates
+    // lie in some 30 cache lines, which the vector L1 would serve one after the other.
     // With the 65536-entry table of silu(g) in memory, two conversions and one lookup at a time instead of two, 12288 x
     // 2048 at 2048 rows took 57.3 us for 53.0, at 1500 51.1 for 49.4, at 256 12.0 for 11.1; 6144 x 4096 at 6000 rows 152.5
     // for 148.4.  A sparse block of 257 experts, 2000 tokens, whose gate|up runs packed tiles: 257.5 with the lookups in
-    // memory, 253.3 with the late copy.
+    // memory, 253.3 with the late copy.  An early copy that takes a workgroup from the CU costs every epilogue, us early /
+    // late, scaled output and SwiGLU: 64x128 with table decode, 257 experts of 1024 x 2048, 60 rows each, 329 / 234 and
+    // 334 / 238, with INT8 weights 145 / 128 and 149 / 128; 128x64, 12288 x 1152 at 160 rows, 11.5 / 9.3 and 12.5 / 10.2;
+    // 64x64, 49152 x 1024 at 50 rows, 10.4 / 8.8 and 10.7 / 9.2.
+    constexpr int SIG_BYTES = int(sizeof(uint16_t)) * 2 * int(SIGMOID_ENTRIES);
     constexpr int CU_WGS = OCC * 4 * 64 / (NT * KG) > 1 ? OCC * 4 * 64 / (NT * KG) : 1;
-    constexpr bool SIG = !PK && SMEM_BYTES + (BM + BN) * 4 + int(sizeof(uint16_t)) * 2 * int(SIGMOID_ENTRIES) <= 160 * 1024 / CU_WGS;
+    constexpr int CU_SHARE = 160 * 1024 / CU_WGS, LDS_BYTES = SMEM_BYTES + (BM + BN) * 4;
+    static_assert(LDS_BYTES <= CU_SHARE, "the workgroups that OCC counts on fit the CU's LDS");
+    constexpr bool SIG = !PK && LDS_BYTES + SIG_BYTES <= CU_SHARE;
     __shared__ __attribute__((aligned(16))) uint16_t s_sig[SIG ? 2 * SIGMOID_ENTRIES : 8];
     constexpr int SIG_AT = WGM * WGN * WTM * (WTN + 16);   // behind the waves' output tiles
-    constexpr bool SIG_LATE = PK && SIG_AT + int(sizeof(uint16_t)) * 2 * int(SIGMOID_ENTRIES) <= SMEM_BYTES;
+    constexpr bool SIG_LATE = !SIG && KG == 1 && SIG_AT + SIG_BYTES <= SMEM_BYTES;
     uint16_t* const sig = SIG ? s_sig : reinterpret_cast<uint16_t*>(smem + (SIG_LATE ? SIG_AT : 0));
     auto swz = [](int row, int chunk) { return row * BK + ((chunk ^ ((row / RPB) & (CPR - 1))) << 4); };
     // packed weight rows (64 bytes, 4 chunks): 4 rows per sweep of the banks, chunk c of row r at c ^ ((r / 4) % 4)

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import bf16, layout, linear
-from tests.util import F32, blocked_layout, dev, host, product_format
+from tests.util import F32, FORMATS, blocked_layout, dev, host, product_format, random_packed
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +43,33 @@ def test_every_gate(path, m, k):
         assert torch.equal(rows.isnan(), nan[r].expand_as(rows))
         assert torch.equal(rows.view(torch.int16)[:, ~nan[r]], want[r].view(torch.int16)[~nan[r]].expand(len(rows), -1))
     assert host(nan).sum() < 2000
+
+
+# staged tiles several of which share a CU copy the table behind their K loop as well: expert slots of 64 rows where K is no multiple of
+# 256 (one K step, odd and even counts of them), 64x64 by rows
+@pytest.mark.parametrize("path,m,k", [(64, 70, 128), (64, 70, 384), (64, 20, 896), ("rows", 50, 128), ("rows", 64, 384)])
+def test_every_gate_where_workgroups_share_a_cu(path, m, k):
+    test_every_gate(path, m, k)
+
+
+# 128x64 by rows, with more tiles than CUs and fewer, rows and columns that end inside a tile; 64x64; the tiles of test_gemm_tile_choice.py
+SHARED = [(3, 160, 12288, 1152), (3, 131, 11656, 1152), (3, 67, 8288, 128), (4, 300, 6144, 512), (4, 300, 6152, 896)]
+
+
+@pytest.mark.parametrize("epi", [1, 2, 3])
+@pytest.mark.parametrize("tile,m,n,k", SHARED)
+def test_epilogues_where_workgroups_share_a_cu(tile, m, n, k, epi):
+    """INT8 weights, the published format and table decode, bit for bit against the oracle's epilogue of the exact sums."""
+    from mxfp4_int8_m5_amd import sc_kernels as S
+    from tests.test_gpu_gemm_tiles import product
+    rng = np.random.default_rng(m + n + epi)
+    xq = rng.integers(-127, 128, (m, k)).astype(np.int8)
+    xs = (2.0 ** -7 * (0.5 + rng.random(m))).astype(F32)
+    res = bf16.to_bits(rng.standard_normal((m, n)).astype(F32)) if epi == 2 else None
+    for fmt in (FORMATS[0], FORMATS[4]):
+        c, b, w, q = random_packed(rng, n, k, fmt)
+        want = linear.epilogue(host(product(dev(xq), dev(q))), xs, w, epi, res)
+        forms = [S.PackedWq(dev(c), dev(b), n, k, product_format(fmt), dev(w))] + ([dev(q)] if fmt is FORMATS[0] else [])
+        for wq in forms:
+            got = S.mm_epi(dev(xq), wq, dev(xs), dev(w), epi, res=dev(res) if epi == 2 else None)
+            assert np.array_equal(host(got), want)
