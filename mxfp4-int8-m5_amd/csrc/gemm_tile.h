@@ -251,6 +251,7 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
 
     constexpr int SIG_PER = (2 * int(SIGMOID_ENTRIES) / 8 + NT * KG - 1) / (NT * KG);   // 16-byte pieces of the table a thread copies
     [[maybe_unused]] u32x4 sig_reg[SIG_PER];
+    static_assert(alignof(silu_ce::Table) % sizeof(u32x4) == 0, "the table is read in whole pieces");
     auto load_sig = [&] {
 #pragma unroll
         for (int j = 0; j < SIG_PER; ++j)

@@ -55,7 +55,7 @@ constexpr uint16_t sigmoid_bits(uint16_t gb) {   // gb: not a NaN
     return to_bf16((g < 0.0f) ? y : round_bf16(1.0f - y));
 }
 
-struct Table {
+struct alignas(16) Table {             // (kernels copy it in pieces of 16 bytes)
     uint16_t v[2 * SIGMOID_ENTRIES];   // of g >= 0, then of g < 0
 };
 constexpr Table make() {

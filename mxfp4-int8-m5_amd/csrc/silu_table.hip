@@ -17,7 +17,7 @@ const uint16_t* silu_table_device() {
     const uint16_t* p = cached[dev].load(std::memory_order_acquire);
     if (!p) {
         void* addr = nullptr;
-        if (hipGetSymbolAddress(&addr, HIP_SYMBOL(g_silu_table)) != hipSuccess) return nullptr;
+        if (hipGetSymbolAddress(&addr, HIP_SYMBOL(g_silu_table)) != hipSuccess || uintptr_t(addr) % alignof(silu_ce::Table)) return nullptr;
         p = reinterpret_cast<const uint16_t*>(addr);
         cached[dev].store(p, std::memory_order_release);
     }

@@ -1,5 +1,6 @@
-"""What the compiler gave each GEMM tile (registers and LDS, from the built library's kernel descriptors) against what the choice of a
-tile counts on: as many workgroups on a CU as the cost tables of gemm.hip and the comments of gemm_grouped.hip say."""
+"""What the compiler made of the GEMM tiles, read from the built library: the registers and LDS of each against what the choice of a
+tile counts on -- as many workgroups on a CU as the cost tables of gemm.hip and the comments of gemm_grouped.hip say --, and the
+place of the sigmoid's table."""
 import re
 import struct
 
@@ -12,8 +13,8 @@ CU_LDS, SIMDS, REGISTERS, MOST_WAVES = 160 * 1024, 4, 512, 8   # gfx950: a CU's 
 FIELDS = ("bm", "bn", "bk", "wgm", "wgn", "bmode", "occ", "fd", "skip", "pk", "kg", "adm", "mf")
 
 
-def descriptors():
-    """The metadata of every kernel in the library: the code objects of its offload bundles, their AMDGPU notes."""
+def code_objects():
+    """The GPU's ELF files in the library's offload bundles."""
     import mxfp4_int8_m5_amd as pkg
     with open(pkg._lib.LIB_PATH, "rb") as f:
         lib = f.read()
@@ -24,7 +25,7 @@ def descriptors():
         for _ in range(entries):
             start, size, n = struct.unpack_from("<QQQ", lib, p)
             if b"gfx950" in lib[p + 24:p + 24 + n]:
-                yield from notes(lib[at + start:at + start + size])
+                yield lib[at + start:at + start + size]
             p += 24 + n
         at = lib.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
 
@@ -35,12 +36,14 @@ def sections(elf):
     return [struct.unpack_from("<IIQQQQIIQQ", elf, first + i * size) for i in range(count)]
 
 
-def notes(elf):
-    for _, kind, _, _, at, _, _, _, _, _ in sections(elf):
-        if kind == 7:   # SHT_NOTE
-            name, desc, note = struct.unpack_from("<III", elf, at)
-            if note == 32:   # NT_AMDGPU_METADATA
-                yield from msgpack.unpackb(elf[at + 12 + (name + 3 & ~3):][:desc])["amdhsa.kernels"]
+def descriptors():
+    """The metadata of every kernel: the code objects' AMDGPU notes."""
+    for elf in code_objects():
+        for _, kind, _, _, at, _, _, _, _, _ in sections(elf):
+            if kind == 7:   # SHT_NOTE
+                name, desc, note = struct.unpack_from("<III", elf, at)
+                if note == 32:   # NT_AMDGPU_METADATA
+                    yield from msgpack.unpackb(elf[at + 12 + (name + 3 & ~3):][:desc])["amdhsa.kernels"]
 
 
 @pytest.fixture(scope="module")
@@ -84,3 +87,20 @@ def test_the_epilogue_tests_reach_their_tiles():
     from tests.test_gemm_tile_choice import chosen
     from tests.test_gpu_swiglu_table import SHARED
     assert [chosen("ROW_TILES", *s) for _, *s in SHARED] == [t for t, *_ in SHARED]
+
+
+def test_the_sigmoid_table_is_aligned():
+    """The tiles copy it in pieces of 16 bytes: the section that holds it has to be placed on one, and its place in there."""
+    found = 0
+    for elf in code_objects():
+        parts = sections(elf)
+        for _, kind, _, _, at, size, link, _, _, entry in parts:
+            if kind != 11:   # SHT_DYNSYM
+                continue
+            names = parts[link][4]
+            for i in range(at, at + size, entry):
+                name, _, _, section, value, _ = struct.unpack_from("<IBBHQQ", elf, i)
+                if section and b"g_silu_table" in elf[names + name:elf.index(b"\0", names + name)]:
+                    found += 1
+                    assert parts[section][8] % 16 == 0 and value % 16 == 0
+    assert found == 1
