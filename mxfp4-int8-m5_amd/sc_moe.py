@@ -127,23 +127,49 @@ def takes_slots(R, n_experts, K, tm, fmt):
     return tm == 256 and bool(_lib.native().scmx_moe_mm_takes_slots(fmt.c, R, n_experts, K))
 
 
+def slots_pay(R, n_experts, N, K, gathered):
+    """Whether a grouped GEMM on N columns and 256-row tiles is faster from slots than by rows, what fills them included: the copy of
+    `gathered` rows (6 - 10 us and R * K bytes), or the quantization, which writes either layout.  Slots always take one tile of 256 rows
+    and 128 columns; by rows the launch chooses, and cuts a few tiles into pairs of 128 rows that reach more CUs.  Lines for 256 CUs, in
+    256 x 256 tiles of the experts if none had more rows than that; 589 problems (4 ... 257 experts, 512 ... 4352 columns and reductions,
+    96 ... 1500 rows an expert, four formats, skewed routing): 1.4 per cent over the faster form on average for gate|up, 0.4 for
+    down, where slots from 2048 columns on cost 4.3 and slots for all 3.3, and up to 2.05 and 1.6 times the rows' time.  us by rows /
+    from slots:
+    - quantized rows: 8 experts of 2048 x 1024, 100 rows 15.3 / 19.4, 150 rows 21.5 / 20.2; 16 of 768 x 768, 110 rows 0.8 times as
+      fast, 300 rows 1.23; 64 of 2048 x 1024, 400 rows 106 / 99.  Columns that the 256x256 tile does not take (not a multiple of 256,
+      under 1024) are 256x128 by rows as well: 6 of 640 x 1280, 1053 rows 0.86 times as fast.
+    - gathered rows: 8 of 2048 x 2048, 100 rows 16.4 / 29.4, 400 rows 38.3 / 35.8; 32 of 2048 x 1024, 110 / 180 / 300 rows 0.8 ... 0.97 /
+      0.95 / 1.01 times as fast; 64 of 2048 x 2048, 100 ... 400 rows 82 / 77, 98 / 88, 119 / 102, 172 / 169; under 128 rows 64 of 2048 x
+      1024 0.93 ... 1.03 and 16 of 8192 x 4096, whose code lines are read twice, 0.90 ... 1.0.  Less than 2048 columns do not earn the
+      copy: 128 of 1536 x 2048, 100 ... 400 rows 0.98, 1.0, 0.98, 0.91."""
+    rows, tiles, cus = R / n_experts, n_experts * -(-N // 256), 256
+    if not gathered:
+        wide = N % 256 == 0 or N >= 1024
+        return tiles > cus // 4 or (wide and (rows >= 256 or tiles * rows > 43 * cus))
+    if N < 2048:
+        return False
+    if rows < 128:
+        return tiles > cus and 1536 <= K < 4096
+    return tiles > cus or (rows >= 200 and tiles > cus // 2 and K >= 1024)
+
+
 def expert_mlp(xq, xs, R, gate_up, down, tok, off, tstart, max_tiles, tm, fmt):
     """Gate|up with SwiGLU, INT8, down of the routed experts on packed weights: xq int8 [M, D] with the token of each sorted row in tok,
     gate_up / down = (codes, bcodes, wscale) stacked over the experts -> bf16 [R, D] by sorted row.  With 256-row tiles the activations
-    go through slots in the blocked layout where that pays: always for down, whose quantization writes them, for gate|up from
-    2048 columns on (the copy costs R * D bytes, what it gains grows with R * D * columns).  Both GEMMs, quantization and copy, us
-    without / with slots, 64 experts of 2048 x 2048 and 2048 x 1024, skewed routing: 8000 rows 126 / 117, 12000 169 / 149, 24000
-    260 / 236, 48000 425 / 416, 24000 in e2m1/B16/M1..10 261 / 247; 16 of 4096 x 4096 264 / 225; 257 of 1024 x 2048, 54000
-    rows: gate|up 197 / 229 with the copy, down 145 / 136."""
+    go through slots in the blocked layout where that pays.  Both GEMMs, quantization and copy, us without / with slots, 64 experts of
+    2048 x 2048 and 2048 x 1024, skewed routing: 8000 rows 126 / 117, 12000 169 / 149, 24000 260 / 236, 48000 425 / 416, 24000 in
+    e2m1/B16/M1..10 261 / 247; 16 of 4096 x 4096 264 / 225; 257 of 1024 x 2048, 54000 rows: down 145 / 136.  Working memory beyond the
+    outputs: (ceil(R / 256) + E) * 256 * K bytes of slots for each of the two, one after the other (24000 rows over 64 experts:
+    83 MB at K = 2048), where rows take R * K for down and gate|up nothing."""
     (cg, bg, sg), (cd, bd, sd) = gate_up, down
     E, F2 = sg.shape
     D, K2, tile = sd.shape[1], F2 // 2, (tm, 64, 4)
-    if F2 >= 2048 and takes_slots(R, E, D, tm, fmt):
+    if slots_pay(R, E, F2, D, True) and takes_slots(R, E, D, tm, fmt):
         slots, xs = gather_blocked(xq, xs, tok, R, off, tstart)
         act = moe_mm_blocked(slots, xs, R, D, cg, bg, sg, off, tstart, F2, 3, fmt)
     else:
         act = moe_mm(xq, R, cg, bg, sg, off, tstart, max_tiles, F2, 3, xs, tile=tile, gather=tok, fmt=fmt)
-    if takes_slots(R, E, K2, tm, fmt):
+    if slots_pay(R, E, D, K2, False) and takes_slots(R, E, K2, tm, fmt):
         slots, xs = act_quant_sorted(act, R, off, tstart)
         return moe_mm_blocked(slots, xs, R, K2, cd, bd, sd, off, tstart, D, 1, fmt)
     xq, xs = S.act_quant(act, R)

@@ -78,12 +78,12 @@ def test_table_formats_are_refused():
         M.moe_mm_blocked(z.view(torch.int8), z.float(), 10, 256, z, z.view(torch.uint8), z.float().reshape(4, -1), z, z, 8, 1, fmt)
 
 
-@pytest.mark.parametrize("d,f2,rows", [(512, 2048, 300), (512, 1024, 300), (256, 2048, 90)])   # both GEMMs from slots; down alone; neither
-def test_expert_mlp_is_its_parts(d, f2, rows):
+@pytest.mark.parametrize("d,f2,rows", [(512, 2048, 300), (512, 1024, 300), (256, 2048, 90)])   # down from slots, wide and narrow; neither
+def test_expert_mlp_is_its_parts(d, f2, rows, e=5):
     from mxfp4_int8_m5_amd import sc_kernels as S
     from mxfp4_int8_m5_amd import sc_moe as M
     rng = np.random.default_rng(d + f2)
-    e, m = 5, rows * 5 // 2
+    m = rows * e // 2
     gu, dn = ([torch.stack(t) for t in zip(*[weights(rng, n, k, "published")[:3] for _ in range(e)])] for n, k in ((f2, d), (d, f2 // 2)))
     inds = dev(rng.permuted(np.tile(np.arange(e), (m, 1)), axis=1)[:, :2].astype(np.int32))
     tm = M.row_tile(2 * m, e)
@@ -94,3 +94,10 @@ def test_expert_mlp_is_its_parts(d, f2, rows):
     hq, hs = S.act_quant(act, 2 * m)
     want = M.moe_mm(hq, 2 * m, *dn, off, ts, mt, d, 1, hs, tile=(tm, 64, 4), fmt=fmt)
     assert torch.equal(M.expert_mlp(xq, xs, 2 * m, gu, dn, tok, off, ts, mt, tm, fmt).view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("d,f2,rows,e", [(512, 2048, 150, 40), (1024, 2048, 220, 18)])   # more tiles than CUs; fewer, and many rows
+def test_expert_mlp_from_slots_throughout(d, f2, rows, e):
+    from mxfp4_int8_m5_amd import sc_moe as M
+    assert M.slots_pay(rows * e, e, f2, d, True) and M.slots_pay(rows * e, e, d, f2 // 2, False)
+    test_expert_mlp_is_its_parts(d, f2, rows, e)
