@@ -174,7 +174,7 @@ class FusedOlmoe:
         h, L, Mp = embed_rows(self.embed, ids)
         nl = len(self.layers)
         # prefill-sized GEMMs on packed weights read their activations in 32x32 blocks (the quantizers write either layout)
-        blk = {g: isinstance(w.unpack(), S.PackedWq) and S.prefers_blocked(Mp, w.N, w.K) for g, w in self.layers[0][1].items()}
+        blk = {g: w.stays_packed() and S.prefers_blocked(Mp, w.N, w.K) for g, w in self.layers[0][1].items()}
         xq, xs = S.rmsnorm_quant(h, self.layers[0][0]["input_layernorm"], self.eps, Mp, blocked=blk["qkv"])
         for i, (nw, ws, ex) in enumerate(self.layers):
             y = S.mm_epi(xq, ws["qkv"].unpack(), xs, ws["qkv"].wscale, 1)

@@ -51,6 +51,10 @@ class PackedWeight:
             return self.wq
         return S.unpack_i8(self.codes, self.bcodes, self.N, self.K, fmt=self.fmt)
 
+    def stays_packed(self):
+        """Whether unpack() hands out packed weights (and costs nothing), not an INT8 tensor."""
+        return self.wq is None and S.FUSE_UNPACK
+
     def nbytes(self):
         return sum(t.numel() * t.element_size() for t in (self.codes, self.bcodes, self.wscale))
 
