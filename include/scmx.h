@@ -112,8 +112,9 @@ int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* 
                          const uint8_t* bcodes, const float* wscale, const uint16_t* res, void* out, int epi, int M,
                          int N, int K, void* stream);
 
-/* 1 when a dense problem of this shape runs faster from blocked activations (by the tiles
- * that read them or by the few-row kernel), 0 when the row layout is the one to quantize into; what scmx_linear_w4a8 decides by.  No device work. */
+/* 1 when a dense problem of this shape runs faster from blocked activations (by the tiles that read them or by the few-row
+ * kernel), 0 when the row layout is the one to quantize into.  scmx_linear_w4a8 decides by the same rule, but that it takes
+ * blocks for 97 ... 128 rows on 1376 ... 2048 columns with long reductions, where this answer stays 0.  No device work. */
 int scmx_mm_w4a8_prefers_blocked(int M, int N, int K);
 
 /* Whole dense W4A8 linear on a bf16 input: activation quantization prologue + scmx_mm_w4a8, one call (the activations

@@ -97,10 +97,10 @@ static TileChoice fastest_tile(const Cand* cand, int first, int last, long M, lo
 // which some formats do not take (launch_dense), never decides: the same layout with and without it on 250 000 drawn
 // problems.
 enum { BY_ROWS = 0, BLOCKED = 1 };   // and FEW_ROWS
-static int dense_layout(const scmx_format* fmt, int M, int N, int K) {
+static int dense_layout(const scmx_format* fmt, int M, int N, int K, int most = SKINNY_MAX_ROWS / 16) {
     const int cus = device_cus();
     const bool small = M <= SKINNY_MAX_ROWS, candidate = small && long(M + 15) / 16 * 16 * N <= 480000;   // (beyond: not measured)
-    const float few = candidate ? 1.0f + 0.9f * skinny_time(M, N, K, cus) : 1e30f;
+    const float few = candidate ? 1.0f + 0.9f * skinny_time(M, N, K, cus, most) : 1e30f;
     const float least = fmaxf(3.8f, 2.41f + 0.157f / 128.0f * float(K));
     if (few < least) return FEW_ROWS;
     const float rows = fastest_tile(ROW_TILES, small ? 0 : 5, 6, M, N, K, cus).us;
@@ -236,7 +236,10 @@ int scmx_mm_w4a8_blocked(const scmx_format* fmt, const int8_t* xq, const float* 
 
 int scmx_mm_w4a8_prefers_blocked(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    return dense_layout(nullptr, M, N, K) != BY_ROWS;
+    // Callers keep the answer they have had for 97 ... 128 rows on 1376 ... 2048 columns and K beyond 3000, by rows (2048 x 4096
+    // at 128 rows 8.3 us and 2.8 for the quantization), from before the few-row kernel cut such rows into groups of four tiles
+    // (6.5 and 3.3); the whole linear, which lays its rows out itself, and who hands over blocks get the groups.
+    return dense_layout(nullptr, M, N, K, 3) != BY_ROWS;
 }
 
 // The fused layer quantizes into whichever layout suits the shape (dense_layout).  Both layouts take (M rounded up to

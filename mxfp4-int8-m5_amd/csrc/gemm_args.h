@@ -37,7 +37,7 @@ enum { B_INT8 = 0, B_PACKED_DEFAULT = 1, B_PACKED_GENERIC = 2, B_PACKED_B16 = 3,
 
 constexpr int SKINNY_MAX_ROWS = 128;
 // The few-row kernel's time (us) on a dense problem of up to SKINNY_MAX_ROWS rows, activations in the blocked layout.
-float skinny_time(int M, int N, int K, int cus);
+float skinny_time(int M, int N, int K, int cus, int most = SKINNY_MAX_ROWS / 16);
 void launch_skinny(const GemmArgs& a, int bmode, hipStream_t s);
 void launch_rows(const GemmArgs& a, int bmode, int tile, hipStream_t s);
 void launch_rows_idle(const GemmArgs& a, int bmode, int tile, hipStream_t s);

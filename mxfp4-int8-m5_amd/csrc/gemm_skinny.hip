@@ -158,15 +158,15 @@ static int row_groups(int tiles, int columns, int cus) {
 }
 
 // Its time in us beside what any launch costs.  A CU runs `turns` = ceil(N / 16 / CUs) workgroups, each of which walks its
-// weights and the rows of activations of its group (five row tiles run as six, seven as eight).  Fitted to 1002 problems (13
-// widths 896 ... 28672, 27 reductions 512 ... 14336, 16 ... 128 rows): within 5 per cent.
-float skinny_time(int M, int N, int K, int cus) {
+// weights and the rows of activations of its group (five row tiles run as six, seven as eight); groups of more than `most`
+// tiles are taken for one.  The coefficients were fitted to one group (1002 problems, weights from HBM); with weights in the
+// L2, as a loop over one layer has them, a launch takes 2.3 us and 0.8 of this, 5 per cent off on average and 13 at the
+// 95th percentile, in one group and in several alike (963 problems: 13 widths 512 ... 24576, 12 reductions 512 ... 12288,
+// 16 ... 128 rows).
+float skinny_time(int M, int N, int K, int cus, int most) {
     const int columns = (N + 15) / 16, turns = columns <= cus ? 1 : (columns + cus - 1) / cus;
     const int rows16 = (M + 15) / 16, groups = row_groups(rows16, columns, cus), share = (rows16 + groups - 1) / groups;
-    // Groups of more than three row tiles (97 ... 128 rows on 1376 ... 2048 columns) are launched but not counted on: which
-    // layout callers have been told to give such a problem's activations stays as it was (2048 x 4096 at 128 rows by rows,
-    // 8.6 us where the groups take 7.2).
-    const int tiles = share > 3 ? rows16 : share;
+    const int tiles = share > most ? rows16 : share;
     const float more = 16.0f * float((tiles == 5 ? 6 : tiles == 7 ? 8 : tiles) - 1), k = float(K);
     return K <= 2048 ? 0.33f + 1.6e-5f * k + float(turns) * k * (5.6e-4f + 1.19e-5f * more)
                      : 1.31e-4f * k - 0.3f + float(turns) * k * (6.8e-4f + 1.03e-5f * more);

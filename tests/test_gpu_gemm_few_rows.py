@@ -36,3 +36,9 @@ def test_equals_the_tiled_kernel(m, n, k, name):
         assert np.array_equal(host(S.mm_epi(xb, wq, xsb, ws, epi, **kw)), host(S.mm_epi(xr, wq, xs, ws, epi, **kw))), epi
     y = S.linear_w4a8(x, codes, bc, ws, n, 1, fmt=fmt)
     assert np.array_equal(host(y), host(S.mm_epi(xr, wq, xs, ws, 1)))
+
+
+@pytest.mark.parametrize("name", [*FORMATS, "generic"])
+@pytest.mark.parametrize("m,n,k", [(97, 1376, 2176), (112, 1544, 4224), (128, 2048, 4096)])
+def test_two_groups_of_four_row_tiles(m, n, k, name):
+    test_equals_the_tiled_kernel(m, n, k, name)
