@@ -344,24 +344,17 @@ def attn_splits(rows):
     return 1 if rows <= 1024 else 8 if rows <= 8192 else 16
 
 
-def _decode_ranges(rows, hq, hk, d):
-    """The same for any number of heads.  16 heads of 128 over 8 KV heads, attention and merge in a graph, us with 1 / 8 / 16 / 32
-    ranges: 300 rows 6.2 / 6.8 / 6.2 / 6.9, 500 7.6 / 6.6 / 6.3 / 7.0, 1000 11.6 / 7.0 / 6.5 / 6.9, 3000 26.9 / 9.4 / 7.9 / 8.0, 6000 57 /
-    15.1 / 13.9 / 9.2, 12000 110 / 22.6 / 20.8 / 14.1; up to 512 rows the second launch costs a host-bound loop more than it gives.
-    32 ranges let the kernel serve two query heads of a KV head from one reading of the cache, which it does beyond 3072 rows.  They
-    pay where the rows of all query heads, K and V, are more than 29 MB, by 16 / 32 ranges: 16 heads of 128 3200 rows 7.8 / 8.3, 4096
-    9.2 / 8.3; 8 of 128 4096 7.8 / 8.3, 6000 8.9 / 9.0, 12000 15.3 / 10.6; 4 of 128 6000 8.7 / 8.9, 12000 11.6 / 10.6; 32 of 128 3200
-    13.4 / 10.3; 16 of 64 6000 7.4 / 8.2, 12000 13.7 / 9.1; 32 of 64 3200 8.1 / 9.8, 6000 13.1 / 10.1; 8 of 64 12000 8.4 / 8.9; 8 of 256
-    3200 10.0 / 9.8, 4096 12.1 / 10.3.  (Groups of two, four and eight alike; 32 heads over 2 KV heads, whose rows the L2 holds, 6000
-    14.0 / 15.0, 12000 21.4 / 20.2.)
+def _decode_ranges(rows, hq, hk):
+    """The same for any number of heads.  16 heads, us with 8 / 16 ranges: 160 rows 6.2 / 6.3, 500 6.4 / 6.3, 1000 7.3 / 6.8, 3000 10.5 /
+    9.5, 6000 15.0 / 13.7, 12000 26.6 / 23.4 (32 ranges 22.2); up to 512 rows the second launch costs a host-bound loop more than it gives
+    (300 rows 6.2 with one).  32 ranges let the kernel serve two query heads of a KV head from one reading of the cache, which it does
+    beyond 3072 rows (8 KV heads: 6000 rows 12.0, 12000 15.2; up to there it cuts them into 16).
     With the position on the device `rows` is the cache's, and a short context in a longer cache pays for a merge that finds little
-    or nothing to do, with 1 / 16 / 32 ranges: 30 rows 4.1 / 5.5 / 5.8, 128 4.7 / 6.2 / 6.1, 300 6.2 / 6.3 / 6.7 (32 heads 6.2 / 7.2 / 7.8,
-    32 of 256 - / 7.8 / 8.7); from about 300 rows on the ranges win."""
+    or nothing to do: in a graph, with 1 range / in a longer cache, 30 rows 4.2 / 5.7, 128 4.7 / 6.2, 300 6.2 / 6.4; from about 300 rows on
+    the ranges win."""
     if hq > 32:
         return attn_splits(rows)
-    if rows <= 512:
-        return 1
-    return 32 if rows > 3072 and hq // hk % 2 == 0 and rows * max(hq, 8) * d > 7 << 20 else 16
+    return 1 if rows <= 512 else 16 if rows <= 3072 or hq // hk % 2 else 32
 
 
 def _split_workspace(splits, hq, d, like):
@@ -377,7 +370,7 @@ def attn_decode(q, kcache, vcache, n, scale=None, splits=None):
     out = _lib.native().empty_bf16(q, 1, hq * d)
     dev_pos = n if torch.is_tensor(n) else None
     if splits is None:
-        splits = _decode_ranges(rows if dev_pos is not None else int(n), hq, hk, d)
+        splits = _decode_ranges(rows if dev_pos is not None else int(n), hq, hk)
     work = _split_workspace(splits, hq, d, q)
     _lib.native().scmx_attn_decode(q, kcache, vcache, dev_pos, 0 if dev_pos is not None else int(n), out, hq, hk, d, rows,
                                    float(scale if scale is not None else d ** -0.5), work, splits)
@@ -429,7 +422,7 @@ def attn_decode_qkv(y, qn, kn, eps, hq, hk, d, kcache, vcache, pos, inv_freq, sc
     dev_pos = pos if torch.is_tensor(pos) else None
     assert dev_pos is None or dev_pos.dtype == torch.int64
     if splits is None:
-        splits = _decode_ranges(kcache.shape[1] if dev_pos is not None else int(pos) + 1, hq, hk, d)
+        splits = _decode_ranges(kcache.shape[1] if dev_pos is not None else int(pos) + 1, hq, hk)
     work = _split_workspace(splits, hq, d, y)
     _lib.native().scmx_attn_decode_qkv(y, qn, kn, _eps(eps), inv_freq, dev_pos, 0 if dev_pos is not None else int(pos),
                                        kcache, vcache, out, hq, hk, d, kcache.shape[1],
