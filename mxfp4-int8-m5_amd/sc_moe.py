@@ -131,17 +131,18 @@ def slots_pay(R, n_experts, N, K, gathered):
     """Whether a grouped GEMM on N columns and 256-row tiles is faster from slots than by rows, what fills them included: the copy of
     `gathered` rows (6 - 10 us and R * K bytes), or the quantization, which writes either layout.  Slots always take one tile of 256 rows
     and 128 columns; by rows the launch chooses, and cuts a few tiles into pairs of 128 rows that reach more CUs.  Lines for 256 CUs, in
-    256 x 256 tiles of the experts if none had more rows than that; 589 problems (4 ... 257 experts, 512 ... 4352 columns and reductions,
-    96 ... 1500 rows an expert, four formats, skewed routing): 1.4 per cent over the faster form on average for gate|up, 0.4 for
-    down, where slots from 2048 columns on cost 4.3 and slots for all 3.3, and up to 2.05 and 1.6 times the rows' time.  us by rows /
-    from slots:
+    256 x 256 tiles of the experts if none had more rows than that; 795 problems (4 ... 257 experts, 512 ... 4352 columns and reductions,
+    96 ... 1500 rows an expert, four formats, skewed routing, 206 of them with weights from HBM): 1.7 per cent over the faster form on
+    average for gate|up, 0.4 for down, where slots from 2048 columns on cost 4.5 and slots for all 3.7, and up to 2.05 and 1.8 times
+    the rows' time.  us by rows / from slots:
     - quantized rows: 8 experts of 2048 x 1024, 100 rows 15.3 / 19.4, 150 rows 21.5 / 20.2; 16 of 768 x 768, 110 rows 0.8 times as
       fast, 300 rows 1.23; 64 of 2048 x 1024, 400 rows 106 / 99.  Columns that the 256x256 tile does not take (not a multiple of 256,
       under 1024) are 256x128 by rows as well: 6 of 640 x 1280, 1053 rows 0.86 times as fast.
-    - gathered rows: 8 of 2048 x 2048, 100 rows 16.4 / 29.4, 400 rows 38.3 / 35.8; 32 of 2048 x 1024, 110 / 180 / 300 rows 0.8 ... 0.97 /
-      0.95 / 1.01 times as fast; 64 of 2048 x 2048, 100 ... 400 rows 82 / 77, 98 / 88, 119 / 102, 172 / 169; under 128 rows 64 of 2048 x
-      1024 0.93 ... 1.03 and 16 of 8192 x 4096, whose code lines are read twice, 0.90 ... 1.0.  Less than 2048 columns do not earn the
-      copy: 128 of 1536 x 2048, 100 ... 400 rows 0.98, 1.0, 0.98, 0.91."""
+    - gathered rows: 8 of 2048 x 2048, 100 rows 16.4 / 29.4, 400 rows 38.3 / 35.8; 16 of 4096 x 2048, 110 / 180 / 300 rows 0.91 ... 1.16 /
+      0.96 ... 1.01 / 1.05 ... 1.11 times as fast; 32 of 2048 x 2048, 220 / 300 / 400 rows 0.96 / 1.04 / 1.01; 64 of 2048 x 2048, 100 ...
+      400 rows 82 / 77, 98 / 88, 119 / 102, 172 / 169; under 128 rows 64 of 2048 x 1024 0.93 ... 1.03 and 16 of 8192 x 4096, whose code
+      lines are read twice, 0.90 ... 1.0.  Less than 2048 columns do not earn the copy: 128 of 1536 x 2048, 100 ... 400 rows 0.98, 1.0,
+      0.98, 0.91."""
     rows, tiles, cus = R / n_experts, n_experts * -(-N // 256), 256
     if not gathered:
         wide = N % 256 == 0 or N >= 1024
@@ -150,7 +151,7 @@ def slots_pay(R, n_experts, N, K, gathered):
         return False
     if rows < 128:
         return tiles > cus and 1536 <= K < 4096
-    return tiles > cus or (rows >= 200 and tiles > cus // 2 and K >= 1024)
+    return tiles > cus or (rows >= 256 and tiles > cus // 2 and K >= 1024)
 
 
 def expert_mlp(xq, xs, R, gate_up, down, tok, off, tstart, max_tiles, tm, fmt):

@@ -96,7 +96,7 @@ def test_expert_mlp_is_its_parts(d, f2, rows, e=5):
     assert torch.equal(M.expert_mlp(xq, xs, 2 * m, gu, dn, tok, off, ts, mt, tm, fmt).view(torch.int16), want.view(torch.int16))
 
 
-@pytest.mark.parametrize("d,f2,rows,e", [(512, 2048, 150, 40), (1024, 2048, 220, 18)])   # more tiles than CUs; fewer, and many rows
+@pytest.mark.parametrize("d,f2,rows,e", [(512, 2048, 150, 40), (1024, 2048, 280, 18)])   # more tiles than CUs; fewer, and many rows
 def test_expert_mlp_from_slots_throughout(d, f2, rows, e):
     from mxfp4_int8_m5_amd import sc_moe as M
     assert M.slots_pay(rows * e, e, f2, d, True) and M.slots_pay(rows * e, e, d, f2 // 2, False)
