@@ -101,3 +101,13 @@ def test_expert_mlp_from_slots_throughout(d, f2, rows, e):
     from mxfp4_int8_m5_amd import sc_moe as M
     assert M.slots_pay(rows * e, e, f2, d, True) and M.slots_pay(rows * e, e, d, f2 // 2, False)
     test_expert_mlp_is_its_parts(d, f2, rows, e)
+
+
+@pytest.mark.parametrize("k", [4096, 8192, 8320, 8704, 12288])   # beyond 8192: the quantizer's codes pass through LDS in two turns
+def test_slots_of_long_rows(k):
+    test_slots_hold_the_sorted_rows(25, k)
+
+
+@pytest.mark.parametrize("k", [4096, 8704, 12288])
+def test_grouped_product_of_long_rows(k):
+    test_grouped_product_from_slots(25, 132, k, "published")
