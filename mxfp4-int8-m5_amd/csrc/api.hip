@@ -234,8 +234,8 @@ struct SortedRows {
     }
 };
 template <int CH, bool BLK, bool WHOLE, bool SORT = false>
-__global__ __launch_bounds__(BLK ? 512 : 256, !BLK && WHOLE && CH <= 12 ? 1 : CH <= 12 ? 4 : CH <= 16 ? 3 : 1) void act_quant_wave_kernel(const uint16_t* __restrict__ x, int8_t* __restrict__ xq,
-                                                                         float* __restrict__ xs, int M, int Mp, int K_any, SortedRows sort) {
+__global__ __launch_bounds__(BLK ? 512 : 256, !BLK && WHOLE && CH <= 12 ? 1 : CH <= 12 ? 4 : CH <= 16 ? 3 : 1) void act_quant_wave_kernel(
+    const uint16_t* __restrict__ x, int8_t* __restrict__ xq, float* __restrict__ xs, int M, int Mp, int K_any, SortedRows sort) {
     const int K = WHOLE ? 512 * CH : K_any;   // WHOLE: every lane has all of its CH pieces
     constexpr int RPW = BLK ? 8 : 4;
     constexpr int TURN = CH > 16 ? CH / 2 : CH;   // pieces whose codes are in LDS at once (at most 64 KB)
@@ -534,7 +534,8 @@ static void launch_act_quant_rows(const uint16_t* x, int8_t* xq, float* xs, int 
 template <bool BLK, bool SORT = false>
 static bool launch_act_quant_waves(const uint16_t* x, int8_t* xq, float* xs, int M, int Mp, int K, hipStream_t st, SortedRows sort = {}) {
     if (K % 32 || K > (BLK ? 12288 : 8192)) return false;
-    const dim3 grid(SORT ? unsigned(M) / 8u + unsigned(sort.n_experts) : BLK ? unsigned(Mp) / 8u : (unsigned(Mp) + 3u) / 4u), block(BLK ? 512 : 256);
+    const dim3 grid(SORT ? unsigned(M) / 8u + unsigned(sort.n_experts) : BLK ? unsigned(Mp) / 8u : (unsigned(Mp) + 3u) / 4u);
+    const dim3 block(BLK ? 512 : 256);
     auto go = [&](auto ch) {
         constexpr int CH = decltype(ch)::value;
         if (K == 512 * CH) act_quant_wave_kernel<CH, BLK, true, SORT><<<grid, block, 0, st>>>(x, xq, xs, M, Mp, K, sort);
@@ -664,8 +665,8 @@ int scmx_moe_gather_blocked(const int8_t* xq, const float* xscale, const int32_t
         return SCMX_ERR_ARG;
     }
     if (R == 0) return SCMX_OK;
-    moe_gather_blocked_kernel<<<dim3(unsigned(R) / 32u + unsigned(n_experts)), dim3(256), 0, (hipStream_t)stream>>>(xq, xscale, gather, s, K,
-                                                                                                                out, out_scale);
+    const dim3 grid(unsigned(R) / 32u + unsigned(n_experts));
+    moe_gather_blocked_kernel<<<grid, dim3(256), 0, (hipStream_t)stream>>>(xq, xscale, gather, s, K, out, out_scale);
     return check_launch("moe_gather_blocked");
 }
 

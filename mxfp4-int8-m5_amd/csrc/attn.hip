@@ -20,8 +20,9 @@ constexpr int ANT = 512;
 constexpr int ATTN_SINGLE_MAX = 128;   // rows up to which a split launch falls back to one workgroup per head: one turn of its loads
 
 // A launch of this many ranges may serve the query heads of a KV head two at a time (kernel below), and does so with more
-// rows than these: 16 heads, 8 KV heads, us with 32 ranges two heads at a time / 16 ranges one at a time: 300 rows 7.5 /
-// 6.3, 1000 7.5 / 6.8, 3000 9.8 / 9.7, 6000 12.0 / 13.8, 12000 15.2 / 20.4.
+// rows than these.  16 heads of 128 over 8 KV heads, sixteen caches in turn, attention and merge in a graph, us with 32 ranges
+// two heads at a time / 16 ranges one at a time (in the grid of 32): 300 rows 7.7 / 6.8, 1000 8.2 / 7.4, 2000 8.4 / 7.8, 3000
+// 9.0 / 8.9; against a launch of 16 ranges 4096 10.2 / 12.1, 6000 11.9 / 14.9, 12000 15.8 / 21.4.
 constexpr int ATTN_PAIR_RANGES = 32, ATTN_PAIR_MIN = 3072;
 
 // What the fused variant needs besides the attention operands: the token's q|k|v row as the qkv projection wrote it,
@@ -102,9 +103,9 @@ struct AttnDecode {
     // of them, the output is written; else the unnormalised results, maxima and sums go to `part` (and part_other).
     template <int HEADS>
     static __device__ __forceinline__ void run(Shared& s, const uint16_t* __restrict__ q, uint16_t* __restrict__ kc,
-                                               uint16_t* __restrict__ vc, int head, int other, int hq, int hk, int rows, int n, int row0, int row1,
-                                               bool append, float scale, const QkvArgs& x, const Token& token, bool whole, uint16_t* __restrict__ out,
-                                               float* part, float* part_other) {
+                                               uint16_t* __restrict__ vc, int head, int other, int hq, int hk, int rows, int n,
+                                               int row0, int row1, bool append, float scale, const QkvArgs& x, const Token& token,
+                                               bool whole, uint16_t* __restrict__ out, float* part, float* part_other) {
         const int tid = threadIdx.x, grp = tid / LPR, c = tid % LPR, lane = tid & 63, wave = tid >> 6;
         const int kvh = head / (hq / hk);
         const uint16_t* kbase = kc + size_t(kvh) * rows * D + 8 * c;
@@ -341,7 +342,8 @@ __global__ __launch_bounds__(ANT) void attn_decode_kernel(const uint16_t* __rest
     const bool append = range == 0 && (both ? min(head, other) : head) % (hq / hk) == 0;
     if constexpr (PAIR) {
         if (both) {
-            A::template run<2>(s, q, kc, vc, head, other, hq, hk, rows, n, row0, row1, append, scale, x, token, false, out, part(head), part(other));
+            A::template run<2>(s, q, kc, vc, head, other, hq, hk, rows, n, row0, row1, append, scale, x, token, false, out, part(head),
+                               part(other));
             return;
         }
     }
@@ -391,9 +393,11 @@ static void launch_attn(int d, hipStream_t st, const uint16_t* q, uint16_t* kc, 
         constexpr int D = decltype(dim)::value;
         const bool pair = splits >= ATTN_PAIR_RANGES && splits % 2 == 0 && hq / hk % 2 == 0;
         if (pair)
-            attn_decode_kernel<D, FUSED, true><<<dim3(hq / 2, splits), dim3(ANT), 0, st>>>(q, kc, vc, pos_dev, n, out, hq, hk, rows, scale, x, partial);
+            attn_decode_kernel<D, FUSED, true><<<dim3(hq / 2, splits), dim3(ANT), 0, st>>>(q, kc, vc, pos_dev, n, out, hq, hk, rows, scale,
+                                                                                           x, partial);
         else
-            attn_decode_kernel<D, FUSED, false><<<dim3(hq, splits), dim3(ANT), 0, st>>>(q, kc, vc, pos_dev, n, out, hq, hk, rows, scale, x, partial);
+            attn_decode_kernel<D, FUSED, false><<<dim3(hq, splits), dim3(ANT), 0, st>>>(q, kc, vc, pos_dev, n, out, hq, hk, rows, scale, x,
+                                                                                        partial);
         if (splits > 32) attn_merge_kernel<D, 64><<<dim3(hq), dim3(MERGE_NT), 0, st>>>(partial, out, splits, pair, pos_dev, n, rows);
         else if (splits > 16) attn_merge_kernel<D, 32><<<dim3(hq), dim3(MERGE_NT), 0, st>>>(partial, out, splits, pair, pos_dev, n, rows);
         else if (splits > 1) attn_merge_kernel<D, 16><<<dim3(hq), dim3(MERGE_NT), 0, st>>>(partial, out, splits, pair, pos_dev, n, rows);

@@ -34,8 +34,8 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
     // activations in the blocked layout (rows padded to whole 32-row blocks): block (m / 32, k / 32), 16-byte halves of k
     const int8_t* ap[TILES];
 #pragma unroll
-    for (int t = 0; t < TILES; ++t)
-        ap[t] = a.xq + (size_t(min(tile0 + t, (M - 1) / 16) >> 1) * (K / 32) + g) * 1024 + (16 * ((tile0 + t) & 1) + r) * 16;   // (a tile past M: any block)
+    for (int t = 0; t < TILES; ++t)   // (a tile past M: any block)
+        ap[t] = a.xq + (size_t(min(tile0 + t, (M - 1) / 16) >> 1) * (K / 32) + g) * 1024 + (16 * ((tile0 + t) & 1) + r) * 16;
 
     struct Weights {
         u32x4 w;
@@ -148,10 +148,11 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(const GemmArgs a) {
 
 // Groups that the 16-row tiles are cut into, a workgroup each: as many as the CUs that a workgroup per 16 columns leaves idle
 // allow.  What a workgroup takes beyond the latency of its loads is its activations through the vector L1 (48 rows of 6144:
-// 295 KB at 64 bytes a clock); the weights that several then decode come from the L2.  us with one group / several: 2048 x
-// 6144 at 40 rows 7.5 / 6.8 (two), 64 8.3 / 6.9, 128 11.3 / 8.5; 896 x 4864 at 40 rows 6.4 / 5.3 (three), 128 9.6 / 5.9
-// (four); 2048 x 2048 at 128 5.6 / 4.5.  Groups beyond that share CUs: 4096 x 4096 at 40 rows 6.6 / 9.1, 2048 x 6144 in
-// three 9.5.
+// 295 KB at 64 bytes a clock); the weights that several then decode come from one L2 where the groups of a column land on
+// one XCD, which they do with a multiple of eight columns of workgroups (2048, 1152 and 896 wide layers, not 1376).  us
+// with one group / several: 2048 x 6144 at 40 rows 7.5 / 6.8 (two), 64 8.3 / 6.9, 128 11.3 / 8.5; 896 x 4864 at 40 rows 6.4
+// / 5.3 (three), 128 9.6 / 5.9 (four); 2048 x 2048 at 128 5.6 / 4.5.  Groups beyond that share CUs: 4096 x 4096 at 40 rows
+// 6.6 / 9.1, 2048 x 6144 in three 9.5.
 static int row_groups(int tiles, int columns, int cus) {
     const int room = max(1, cus / columns), per = (tiles + room - 1) / room;
     return (tiles + per - 1) / per;

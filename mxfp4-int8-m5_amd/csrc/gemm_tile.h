@@ -249,18 +249,18 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         ws_reg[j] = (a.xscale && c < BN && n0 + c < a.N) ? a.wscale[size_t(expert) * a.N + n0 + c] : 0.0f;
     }
 
-    constexpr int SIG_PER = (2 * int(SIGMOID_ENTRIES) / 8 + NT * KG - 1) / (NT * KG);   // 16-byte pieces of the table a thread copies
+    constexpr int SIG_PIECES = SIG_BYTES / 16, SIG_PER = (SIG_PIECES + NT * KG - 1) / (NT * KG);   // pieces a thread copies
     [[maybe_unused]] u32x4 sig_reg[SIG_PER];
     static_assert(alignof(silu_ce::Table) % sizeof(u32x4) == 0, "the table is read in whole pieces");
     auto load_sig = [&] {
 #pragma unroll
         for (int j = 0; j < SIG_PER; ++j)
-            sig_reg[j] = reinterpret_cast<const u32x4*>(a.silu)[min(int(threadIdx.x) + j * NT * KG, 2 * int(SIGMOID_ENTRIES) / 8 - 1)];
+            sig_reg[j] = reinterpret_cast<const u32x4*>(a.silu)[min(int(threadIdx.x) + j * NT * KG, SIG_PIECES - 1)];
     };
     auto store_sig = [&](uint16_t* to) {
 #pragma unroll
         for (int j = 0; j < SIG_PER; ++j)
-            if (int(threadIdx.x) + j * NT * KG < 2 * int(SIGMOID_ENTRIES) / 8) reinterpret_cast<u32x4*>(to)[int(threadIdx.x) + j * NT * KG] = sig_reg[j];
+            if (int(threadIdx.x) + j * NT * KG < SIG_PIECES) reinterpret_cast<u32x4*>(to)[int(threadIdx.x) + j * NT * KG] = sig_reg[j];
     };
     const bool sig_copy = SIG && a.epi == SCMX_EPI_SWIGLU, late_sig = SIG_LATE && a.epi == SCMX_EPI_SWIGLU;
     if (sig_copy) load_sig();
@@ -457,10 +457,11 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int s = 0; s < KS; ++s)
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
-                const u32x4 v = ADR ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR ? i : 0] + s * 64, k0, 0)
-                                : DEAL ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[DEAL ? i : 0] + s * (MF == 32 ? 1024 : 2048), k0 * 32, 0)
-                                : MF == 32 ? __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[MF == 32 && !DEAL ? i : 0] + s * 1024, k0 * 32, 0)
-                                    : __builtin_amdgcn_raw_buffer_load_b128(ra, ad_src[ADR || MF == 32 ? 0 : i / 2] + s * 2048 + (i & 1) * 256, k0 * 32, 0);
+                // a block of 32 rows holds an MF = 32 fragment, or those of an even i and the next
+                const int at = ADR               ? ad_src[i] + s * 64
+                               : DEAL || MF == 32 ? ad_src[i] + s * (MF == 32 ? 1024 : 2048)
+                                                  : ad_src[i / 2] + s * 2048 + (i & 1) * 256;
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(ra, at, ADR ? k0 : k0 * 32, 0);
                 fad[buf][s][i] = v4i{int(v[0]), int(v[1]), int(v[2]), int(v[3])};
             }
     };
@@ -507,7 +508,8 @@ __global__ __launch_bounds__(WGM* WGN* KG * 64, OCC) void gemm_kernel(const Gemm
         for (int i = 0; i < PMI; ++i)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                if (!SKIP || i < mi_active) f[h][i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + (((4 * kp + 2 * part + h) ^ sw) << 4));
+                if (!SKIP || i < mi_active)
+                    f[h][i] = *reinterpret_cast<const v4i*>(src + a_frag + i * 32 * BK + (((4 * kp + 2 * part + h) ^ sw) << 4));
     };
     auto load_pw = [&](const int8_t* src, int kp, v4i (&f)[PNI]) __attribute__((always_inline)) {
 #pragma unroll

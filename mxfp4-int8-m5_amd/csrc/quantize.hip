@@ -180,8 +180,9 @@ __device__ __forceinline__ uint32_t unsigned_zeros(uint32_t c) {
 // where the conversion's 22.2 stood beside it, near ties summed by one lane of the wave 44, a lane per weight and every
 // candidate in float64 across lanes 234 (12288 x 2048, bf16, 32-blocks).
 // Registers decide how many waves hide the conversions' latency: four a SIMD need 128 a thread.  16-blocks are held to
-// that; bf16 32-blocks fit only if the weights are read again for their codes (L2 has them) instead of kept over the
-// barrier; float32 32-blocks fit neither way.  us, before / with half-precision trials / so bounded, 12288 x 2048: bf16
+// that, at the price of 40 spilled registers (most around the float64 sums of near ties, which few blocks take); bf16
+// 32-blocks fit only if the weights are read again for their codes (L2 has them) instead of kept over the barrier; float32
+// 32-blocks fit neither way.  us, before / with half-precision trials / so bounded, 12288 x 2048: bf16
 // 32-blocks 24.3 / 23.9 / 21.8 (bounded without reading again 24.7; five or six waves 29), 16-blocks 47.7 / 47.8 / 31.6;
 // float32 32-blocks 28.9 (bounded 32.3, read again 31.5), 16-blocks 50.4 / - / 35.9.  4096 x 12288: bf16 47.1 -> 39.7
 // and 70.8 -> 50.2, float32 16-blocks 76.3 -> 67.3.

@@ -320,7 +320,8 @@ __global__ __launch_bounds__(NT) void swiglu_quant_kernel(const int32_t* __restr
             g[i] = __fmul_rn(__fmul_rn(float(g4[i]), xsr), wg[i]);
             u[i] = __fmul_rn(__fmul_rn(float(u4[i]), xsr), wu[i]);
         }
-        *reinterpret_cast<u32x2*>(srow + 4 * c) = u32x2{swiglu_lut2(silu, g[0], g[1], u[0], u[1]), swiglu_lut2(silu, g[2], g[3], u[2], u[3])};
+        *reinterpret_cast<u32x2*>(srow + 4 * c) =
+            u32x2{swiglu_lut2(silu, g[0], g[1], u[0], u[1]), swiglu_lut2(silu, g[2], g[3], u[2], u[3])};
     }
     __syncthreads();
     block_quant_row(srow, F, xq + size_t(row) * F, xs + row, red);
@@ -873,7 +874,8 @@ __global__ __launch_bounds__(BLK ? 512 : 256) void moe_combine_wave_kernel(const
                                                                float eps, uint16_t* __restrict__ h, int8_t* __restrict__ xq,
                                                                float* __restrict__ xs, int M, int Mp, int topk) {
     constexpr int K = 512 * CH;
-    const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), row = int(blockIdx.x) * (BLK ? 8 : 4) + wid, lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
+    const int row = int(blockIdx.x) * (BLK ? 8 : 4) + wid;
     if (row >= Mp) return;   // wave-uniform (BLK: never)
     const int nsc = sscore ? topk - 1 : topk;
     auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
@@ -960,7 +962,8 @@ __global__ __launch_bounds__(BLK ? 512 : 256) void moe_combine_wave_kernel(const
         for (int j = 0; j < CH / 2 + CH % 2; ++j) {   // K / 16 pieces x 8 rows of 16 bytes, 512 per pass
             const int idx = int(threadIdx.x) + 512 * j, c = idx >> 3, r = idx & 7;
             if (CH % 2 == 0 || c < K / 16)
-                *reinterpret_cast<u32x4*>(blk + size_t(c >> 1) * 1024 + (c & 1) * 512 + ((row0 + r) & 31) * 16) = t16[c * 8 + ((r + (c >> 1)) & 7)];
+                *reinterpret_cast<u32x4*>(blk + size_t(c >> 1) * 1024 + (c & 1) * 512 + ((row0 + r) & 31) * 16) =
+                    t16[c * 8 + ((r + (c >> 1)) & 7)];
         }
     }
 }
@@ -1457,8 +1460,8 @@ int scmx_moe_combine_blocked(const uint16_t* y, const int32_t* pos, const uint16
     if (!y || !pos || !scores || !res || !h || !xq || !w || !xs || Mp < M || Mp % 32 || topk < 1 || topk > 65536 || K % 512 || K > 2048 ||
         !row_shape_ok("moe_combine_blocked", M, K, 2048) ||
         (uintptr_t(y) | uintptr_t(res) | uintptr_t(h) | uintptr_t(w) | uintptr_t(xq)) % 16) {
-        set_error("moe_combine_blocked: need all of y, pos, scores, res, w, h, xq and xs (16-byte aligned), M <= Mp with Mp %% 32 == 0 (%d), "
-                  "topk in 1..65536 and K %% 512 == 0, K <= 2048 (%d)", Mp, K);
+        set_error("moe_combine_blocked: need all of y, pos, scores, res, w, h, xq and xs (16-byte aligned), M <= Mp with "
+                  "Mp %% 32 == 0 (%d), topk in 1..65536 and K %% 512 == 0, K <= 2048 (%d)", Mp, K);
         return SCMX_ERR_ARG;
     }
     if (Mp == 0) return SCMX_OK;

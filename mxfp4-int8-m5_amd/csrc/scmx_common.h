@@ -121,7 +121,9 @@ __device__ __forceinline__ uint32_t swiglu_lut2(const uint16_t* __restrict__ tab
     const u16x2 from = __builtin_elementwise_sub_sat(twice, u16x2{2 * SIGMOID_FIRST, 2 * SIGMOID_FIRST});
     const u16x2 at = __builtin_elementwise_min(from, u16x2{2 * SIGMOID_ENTRIES - 2, 2 * SIGMOID_ENTRIES - 2});
     const uint32_t e = __builtin_bit_cast(uint32_t, at) | ((g >> 3) & 0x10001000u);
-    const auto entry = [&](uint32_t byte) { return bf16_to_f32(*reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(table) + byte)); };
+    const auto entry = [&](uint32_t byte) {
+        return bf16_to_f32(*reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(table) + byte));
+    };
     const uint32_t silu = f32_to_bf16x2(__fmul_rn(bf16_lo(g), entry(e & 0xFFFFu)), __fmul_rn(bf16_hi(g), entry(e >> 16)));
     return f32_to_bf16x2(__fmul_rn(bf16_lo(silu), bf16_lo(u)), __fmul_rn(bf16_hi(silu), bf16_hi(u)));
 }

@@ -1,7 +1,7 @@
 // Python binding of the C ABI for torch tensors: `_binding`, a module whose functions are the entry points of
-// include/scmx.h that enqueue work (and four of its queries), under the same names and with the same arguments except the last.  A pointer argument
-// takes a tensor (contiguous, on the GPU), None or an integer address; a format argument an object whose buffer is the
-// scmx_format; the stream is the caller's current one and is not passed.  A negative status raises.
+// include/scmx.h that enqueue work (and four of its queries), under the same names and with the same arguments except the
+// last.  A pointer argument takes a tensor (contiguous, on the GPU), None or an integer address; a format argument an object
+// whose buffer is the scmx_format; the stream is the caller's current one and is not passed.  A negative status raises.
 //
 // A decode step is a few hundred calls of a few microseconds of GPU work each, so the host's share per call decides: through
 // ctypes a call cost 8-10 us (argument conversion; pointers, stream and format descriptor made in Python each time).  One
@@ -194,8 +194,8 @@ PyObject* gemv(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const at::Tensor* xscale = pro == 0 ? plain(args[2]) : x;
         const at::Tensor* res = epi == SCMX_EPI_RES ? plain(args[8]) : x;
         const at::Tensor* nw = pro == 2 ? plain(args[13]) : x;
-        if (!x || !codes || !bcodes || !wscale || !xscale || !res || !nw || x->dim() < 1 || x->dim() > 2 || (pro == 2 && !PyFloat_Check(args[14])))
-            Py_RETURN_NONE;
+        if (!x || !codes || !bcodes || !wscale || !xscale || !res || !nw || x->dim() < 1 || x->dim() > 2) Py_RETURN_NONE;
+        if (pro == 2 && !PyFloat_Check(args[14])) Py_RETURN_NONE;
         const at::Tensor* eidx = args[9] == Py_None ? nullptr : plain(args[9], at::ScalarType::Int);
         const int64_t rows = x->dim() == 2 ? x->size(0) : 1, K64 = x->size(-1), slots64 = eidx ? eidx->numel() : 0;
         if ((args[9] != Py_None && !eidx) || N < 0 || K64 > INT32_MAX || slots64 > INT32_MAX - 1 || (!eidx && rows > 8)) Py_RETURN_NONE;
@@ -219,8 +219,8 @@ PyObject* gemv(PyObject*, PyObject* const* args, Py_ssize_t n) {
             const auto *s = static_cast<const float*>(ptr(wscale));
             auto* o = static_cast<uint16_t*>(out.data_ptr());
             if (eidx) {
-                rc = scmx_gemv(fmt, ptr(x), xs, c, b, s, rs, o, epi, pro, w, eps, batch, N, K, static_cast<const int32_t*>(ptr(eidx)), int(slots64),
-                               xstride, shared, c10::hip::getCurrentHIPStream().stream());
+                rc = scmx_gemv(fmt, ptr(x), xs, c, b, s, rs, o, epi, pro, w, eps, batch, N, K, static_cast<const int32_t*>(ptr(eidx)),
+                               int(slots64), xstride, shared, c10::hip::getCurrentHIPStream().stream());
             } else {
                 const size_t need = batch > 1 ? scmx_gemv_rows_workspace(fmt, pro, batch, N, K) : 0;
                 const at::Tensor work = need ? at::empty({int64_t(need)}, options.dtype(at::ScalarType::Byte)) : at::Tensor();
@@ -253,9 +253,11 @@ PyMODINIT_FUNC PyInit__binding() {
         ENTRY(scmx_swiglu_quant), ENTRY(scmx_qkv_headnorm), ENTRY(scmx_qkv_headnorm_rope), ENTRY(scmx_qkv_fullnorm),
         ENTRY(scmx_qkv_fullnorm_rope), ENTRY(scmx_attn_decode), ENTRY(scmx_attn_decode_qkv), ENTRY(scmx_attn_prefill), ENTRY(scmx_attn_prefill_split),
         ENTRY(scmx_gemv), ENTRY(scmx_gemv_rows), ENTRY(scmx_route_topk), ENTRY(scmx_norm_linear), ENTRY(scmx_route_sort), ENTRY(scmx_moe_mm),
-        ENTRY(scmx_moe_mm_i8), ENTRY(scmx_moe_mm_blocked), ENTRY(scmx_moe_gather_blocked), ENTRY(scmx_act_quant_sorted), ENTRY(scmx_moe_combine), ENTRY(scmx_moe_combine_blocked), ENTRY(scmx_rot_quant), ENTRY(scmx_mxfp4_to_sc),
+        ENTRY(scmx_moe_mm_i8), ENTRY(scmx_moe_mm_blocked), ENTRY(scmx_moe_gather_blocked), ENTRY(scmx_act_quant_sorted),
+        ENTRY(scmx_moe_combine), ENTRY(scmx_moe_combine_blocked), ENTRY(scmx_rot_quant), ENTRY(scmx_mxfp4_to_sc),
         ENTRY(scmx_quantize_sc), ENTRY(scmx_quantize_family),
-        QUERY(scmx_linear_w4a8_workspace), QUERY(scmx_gemv_rows_workspace), QUERY(scmx_mm_w4a8_prefers_blocked), QUERY(scmx_moe_mm_takes_slots),
+        QUERY(scmx_linear_w4a8_workspace), QUERY(scmx_gemv_rows_workspace), QUERY(scmx_mm_w4a8_prefers_blocked),
+        QUERY(scmx_moe_mm_takes_slots),
         {"gemv", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&gemv)), METH_FASTCALL, nullptr},
         EMPTY(bf16, BFloat16), EMPTY(i8, Char), EMPTY(u8, Byte), EMPTY(i32, Int), EMPTY(f32, Float),
         {nullptr, nullptr, 0, nullptr}};

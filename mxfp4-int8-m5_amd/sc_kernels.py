@@ -345,13 +345,18 @@ def attn_splits(rows):
 
 
 def _decode_ranges(rows, hq, hk):
-    """The same for any number of heads.  16 heads, us with 8 / 16 ranges: 160 rows 6.2 / 6.3, 500 6.4 / 6.3, 1000 7.3 / 6.8, 3000 10.5 /
-    9.5, 6000 15.0 / 13.7, 12000 26.6 / 23.4 (32 ranges 22.2); up to 512 rows the second launch costs a host-bound loop more than it gives
-    (300 rows 6.2 with one).  32 ranges let the kernel serve two query heads of a KV head from one reading of the cache, which it does
-    beyond 3072 rows (8 KV heads: 6000 rows 12.0, 12000 15.2; up to there it cuts them into 16).
+    """The same for any number of heads.  16 heads of 128 over 8 KV heads, attention and merge in a graph, one cache again and again, us
+    with 1 / 8 / 16 ranges: 300 rows 6.2 / 6.8 / 6.2, 500 7.6 / 6.6 / 6.3, 1000 11.6 / 7.0 / 6.5, 3000 27 / 9.4 / 7.9; up to 512 rows the
+    second launch costs a host-bound loop more than it gives.  32 ranges let the kernel serve two query heads of a KV head from one
+    reading of the cache, which it does beyond 3072 rows (up to there it cuts them into 16).  24 caches in turn, as the layers of a
+    model read theirs, 16 / 32 ranges: 3200 rows 10.6 / 9.8, 6000 14.5 / 11.6, 12000 21.7 / 15.8; 32 heads 14.0 / 12.6, 19.5 / 15.4, 33.7 /
+    20.7; 8 heads 8.8 / 8.7, 11.3 / 10.6, 16.4 / 13.3; 16 heads of 64 8.3 / 8.3, 9.8 / 9.4, 14.1 / 11.6, of 256 15.8 / 12.7, 22.6 /
+    16.6, 36.4 / 25.1; groups of four and eight like those of two.  16 ranges stay better up to 5000 rows for 8 heads of 64 (3200 7.5 /
+    8.3) and to 8000 where 16 heads share a KV head (32 over 2: 10.9 / 12.4, 13.9 / 15.0, 21.9 / 20.4); with the one cache of a loop in
+    the L2 also 16 heads of 128 to 3500 rows, 8 of 128 and 16 of 64 to 6000.
     With the position on the device `rows` is the cache's, and a short context in a longer cache pays for a merge that finds little
-    or nothing to do: in a graph, with 1 range / in a longer cache, 30 rows 4.2 / 5.7, 128 4.7 / 6.2, 300 6.2 / 6.4; from about 300 rows on
-    the ranges win."""
+    or nothing to do, with 1 / 16 / 32 ranges: 30 rows 4.1 / 5.5 / 5.8, 128 4.7 / 6.2 / 6.1, 300 6.2 / 6.3 / 6.7 (32 heads of 256 - / 7.8 /
+    8.7); from about 300 rows on the ranges win."""
     if hq > 32:
         return attn_splits(rows)
     return 1 if rows <= 512 else 16 if rows <= 3072 or hq // hk % 2 else 32

@@ -37,11 +37,13 @@ DOWN = {True: ["sort", "slots"], False: ["quant", "rows"]}
 
 # both sides of each line: few tiles, where the rows' launch spreads over more CUs; rows an expert; narrow layers; reductions
 @pytest.mark.parametrize("E,D,F2,rows,gate,down", [
-    (8, 2048, 2048, 110, False, False), (8, 2048, 2048, 180, False, True), (4, 2048, 4096, 180, False, False), (4, 2048, 4096, 300, False, True),
-    (8, 768, 2048, 180, False, False), (6, 640, 2560, 1053, False, False), (16, 1024, 2048, 110, False, False), (16, 1024, 2048, 300, False, True),
-    (32, 2048, 2048, 110, False, True), (32, 2048, 2048, 220, False, True), (32, 2048, 2048, 300, True, True), (32, 512, 2048, 300, False, True), (48, 1536, 2048, 110, True, True),
-    (64, 1024, 2048, 110, False, True), (64, 1024, 2048, 150, True, True), (64, 2048, 2048, 110, True, True), (16, 4096, 8192, 110, False, True),
-    (16, 4096, 8192, 150, True, True), (128, 2048, 1536, 400, False, True)])
+    (8, 2048, 2048, 110, False, False), (8, 2048, 2048, 180, False, True), (4, 2048, 4096, 180, False, False),
+    (4, 2048, 4096, 300, False, True), (8, 768, 2048, 180, False, False), (6, 640, 2560, 1053, False, False),
+    (16, 1024, 2048, 110, False, False), (16, 1024, 2048, 300, False, True), (32, 2048, 2048, 110, False, True),
+    (32, 2048, 2048, 220, False, True), (32, 2048, 2048, 300, True, True), (32, 512, 2048, 300, False, True),
+    (48, 1536, 2048, 110, True, True), (64, 1024, 2048, 110, False, True), (64, 1024, 2048, 150, True, True),
+    (64, 2048, 2048, 110, True, True), (16, 4096, 8192, 110, False, True), (16, 4096, 8192, 150, True, True),
+    (128, 2048, 1536, 400, False, True)])
 def test_layout_by_size(passes, E, D, F2, rows, gate, down):
     assert passes(E, D, F2, E * rows) == GATE[gate] + DOWN[down]
 
