@@ -90,8 +90,9 @@ static TileChoice fastest_tile(const Cand* cand, int first, int last, long M, lo
 // kernel (blocked as well) or the row tiles, by their models.  The quantizer takes 0.3 us longer for blocks.  Beyond
 // the few-row kernel's range only the row tiles with K groups were ever the fastest of all (up to 1.4 times, narrow
 // layers); within it the blocked tiles have to be a tenth faster (wide layers at 100 rows and more are: 128 x 12288 x
-// 2048 9.3 us for 10.7). The few-row kernel's model takes no launch in.  On the 61 problems of up to 128 rows the
-// choice costs 0.1 per cent over the fastest kernel on average.  Formats whose codes are looked up: a tile's weights
+// 2048 9.3 us for 10.7). The few-row kernel's model takes no launch in.  On 334 drawn problems of 9 ... 128 rows (512 ...
+// 12400 columns and reductions, three formats, weights from HBM) whole linears cost 0.2 per cent over the fastest form on
+// average, 6.5 at most.  Formats whose codes are looked up: a tile's weights
 // are decoded again by each of its row groups, once by the few-row kernel, which is worth half as much again. No table
 // gives less than `least`, so the smallest calls, which the host bounds, look no further.  The four-wave 256x128 tile,
 // which some formats do not take (launch_dense), never decides: the same layout with and without it on 250 000 drawn
